@@ -37,8 +37,9 @@ CLI = os.path.join(HERE, "bin", "hpdbscan")
 HDF5_PREFIX = os.environ.get("HDF5_PREFIX", "/opt/conda")
 ROCM_LIB = "/opt/rocm/lib"
 
-SOURCES = ["capi.hip", "scan.hip", "radix_sort.hip", "grid.hip", "index.hip", "dbscan.hip",
-           "boxes.hip", "server.cpp"]
+# "file.hip:MACRO=value": one part of a file compiled in parts (side by side)
+SOURCES = ["capi.hip", "scan.hip", "radix_sort.hip", "grid.hip", "index.hip",
+           *(f"dbscan.hip:HPD_DBSCAN_PART={p}" for p in range(4)), "boxes.hip", "server.cpp"]
 
 ARCH = os.environ.get("HPD_OFFLOAD_ARCH", "gfx950")
 
@@ -65,11 +66,19 @@ def compile_flags() -> list[str]:
     ]
 
 
+def object_path(src: str, macro: str = "") -> str:
+    part = "_" + macro.rpartition("=")[2] if macro else ""
+    return os.path.join(BUILD, os.path.splitext(src)[0] + part + ".o")
+
+
 def _compile(src: str, verbose: bool) -> str:
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+    src, _, macro = src.partition(":")
+    obj = object_path(src, macro)
     lang = ["-x", "hip"] if src.endswith(".hip") else []
     flags = compile_flags() if src.endswith(".hip") else [
         "-O3", "-std=c++17", "-fPIC", "-Wall", f"-I{INCLUDE}", "-pthread"]
+    if macro:
+        flags = [*flags, f"-D{macro}"]
     cmd = [hipcc(), *flags, *lang, "-c", os.path.join(CSRC, src), "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)

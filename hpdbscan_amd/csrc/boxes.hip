@@ -30,6 +30,7 @@
 
 #include "boxes.hpp"
 #include "hpdbscan_capi.h"
+#include "collect.hpp"
 #include "common.hpp"
 #include "grid.hpp"
 #include "index.hpp"
@@ -331,13 +332,13 @@ __global__ __launch_bounds__(kThreads) void k_box_table(const K* __restrict__ ke
 
 // The occupied cells from the boxes (a cell's first slot starts a box):
 // cell u = the u-th box with cbflag set; ucell / ustart as the cell runs
-// give them (ustart[m] = n), bcell per box.  The boxes walk a bounded grid.
+// give them (ustart[m] = n), bcell per box, cbox per cell.  The boxes walk a bounded grid.
 template <typename K>
 __global__ __launch_bounds__(kThreads) void k_cells_of_boxes(
     const K* __restrict__ keys, int64_t n, int shift, const int32_t* __restrict__ bstart,
     Count nbox_c, const uint32_t* __restrict__ cbflag, const uint32_t* __restrict__ cbscan,
     int32_t* __restrict__ bcell, K* __restrict__ ucell, int32_t* __restrict__ ustart,
-    const uint32_t* __restrict__ ncells_dev) {
+    int32_t* __restrict__ cbox, const uint32_t* __restrict__ ncells_dev) {
     const int64_t nbox = nbox_c.get();
     for (int64_t b = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; b < nbox;
          b += static_cast<int64_t>(gridDim.x) * kThreads) {
@@ -347,42 +348,17 @@ __global__ __launch_bounds__(kThreads) void k_cells_of_boxes(
             const int32_t s0 = bstart[b];
             ucell[u] = keys[s0] >> shift;
             ustart[u] = s0;
+            cbox[u] = static_cast<int32_t>(b);
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) ustart[*ncells_dev] = static_cast<int32_t>(n);
-}
-
-// first box of every cell; cbox[m] = number of boxes
-__global__ __launch_bounds__(kThreads) void k_cell_boxes(const int32_t* __restrict__ bcell,
-                                                         Count nbox_c, Count m_c,
-                                                         int32_t* __restrict__ cbox) {
-    const int32_t m = static_cast<int32_t>(m_c.get());
-    const int32_t nbox = static_cast<int32_t>(nbox_c.get());
-    const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (b < nbox && (b == 0 || bcell[b] != bcell[b - 1])) cbox[bcell[b]] = b;
-    if (b == 0) cbox[m] = nbox;
-}
-
-template <typename U>
-__device__ __forceinline__ U wave_min_u(U v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const U w = __shfl_xor(v, o, 64);
-        v = w < v ? w : v;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ustart[*ncells_dev] = static_cast<int32_t>(n);
+        cbox[*ncells_dev] = static_cast<int32_t>(nbox);
     }
-    return v;
-}
-template <typename U>
-__device__ __forceinline__ U wave_max_u(U v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const U w = __shfl_xor(v, o, 64);
-        v = w > v ? w : v;
-    }
-    return v;
 }
 
-// tight flag per box: dist2(extent) <= EPS2 in the reference's order
+// flags per box: tight (dist2(extent) <= EPS2 in the reference's order),
+// full, in a cell that can hold cores
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_box_tight(const OrdKey<T>* __restrict__ bbox,
                                                         Count nbox_c,
@@ -390,12 +366,14 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const OrdKey<T>* __restr
                                                         const int32_t* __restrict__ bcell,
                                                         const int32_t* __restrict__ job_of_cell,
                                                         const JobParams<T>* __restrict__ jobs,
+                                                        const uint8_t* __restrict__ cell_core,
                                                         uint8_t* __restrict__ btight,
                                                         unsigned int* __restrict__ nloose) {
     const int32_t nbox = static_cast<int32_t>(nbox_c.get());
     const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (b >= nbox) return;
-    const JobParams<T>& jp = jobs[job_of_cell[bcell[b]]];
+    const int32_t u = bcell[b];
+    const JobParams<T>& jp = jobs[job_of_cell[u]];
     T lo[D], hi[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
@@ -406,8 +384,26 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const OrdKey<T>* __restr
     const int32_t size = bstart[b + 1] - bstart[b];
     // bit 0: tight; bit 1: tight and at least minPts rows (all rows core)
     btight[b] = static_cast<uint8_t>((tight ? 1 : 0) |
-                                     ((tight && static_cast<uint32_t>(size) >= jp.min_pts) ? 2 : 0));
+                                     ((tight && static_cast<uint32_t>(size) >= jp.min_pts) ? 2 : 0) |
+                                     (cell_core[u] ? 4 : 0));
     if (!tight && size > 1) atomicAdd(nloose, 1u);
+}
+
+// Whether a core row of a box, [q0, q1), is within eps of the row of a lane
+// in `act` (wave-uniform answer, first hit stops).
+template <typename T, int D>
+__device__ __forceinline__ bool any_pair(const T* __restrict__ soa, int64_t ld,
+                                         const uint8_t* __restrict__ core, int32_t q0, int32_t q1,
+                                         const T* pc, bool act, T eps2) {
+    const uint64_t rows = ballot(act);
+    if (walk_wide(rows, q1 - q0))
+        return __any(wide_any<T, D>(soa, ld, core, q0, q1, pc, eps2, rows, true));
+    bool hit = false;
+    auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
+        if (cq && act && within<D>(pc, qc, eps2)) hit = true;
+    };
+    auto stop = [&] { return static_cast<bool>(__any(hit)); };
+    return visit_range<T, D>(soa, ld, core, nullptr, q0, q1, body, stop);
 }
 
 // Box-level hook: every box with cores points at some box of a smaller
@@ -421,7 +417,7 @@ __global__ __launch_bounds__(kThreads) void k_box_hook(
     const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nitems_c,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rcells, const OrdKey<T>* __restrict__ bbox,
+    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
     const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
     const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
     const int32_t* __restrict__ rcenter, int32_t* __restrict__ bparent) {
@@ -454,7 +450,7 @@ __global__ __launch_bounds__(kThreads) void k_box_hook(
         // nearest neighbours are there, so the first hit comes soonest; boxes
         // before b only
         for_each_row_box<T, D>(
-            r0, r1, uniform(rcenter[u]), rcells, cbox, bstart, bbox, bmincore,
+            r0, r1, uniform(rcenter[u]), rboxes, bstart, bbox, bmincore,
             [&](int32_t b2, const double* lo, const double* hi, int32_t q0, int32_t q1,
                 int32_t mincore) {
                 if (mincore == INT_MAX) return false;  // no cores
@@ -463,14 +459,8 @@ __global__ __launch_bounds__(kThreads) void k_box_hook(
                 const bool act = pcore && gmin2 <= gap2_max;
                 if (!__any(act)) return false;
                 // a core row within eps of the whole box is within eps of its cores
-                bool hit = act && gmax2 <= full2;
-                if (!__any(hit)) {
-                    auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
-                        if (cq && act && within<D>(pc, qc, eps2)) hit = true;
-                    };
-                    auto stop = [&] { return static_cast<bool>(__any(hit)); };
-                    if (!visit_range<T, D>(soa, ld, core, nullptr, q0, q1, body, stop)) return false;
-                }
+                const bool hit = act && gmax2 <= full2;
+                if (!__any(hit) && !any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return false;
                 if (lane_id() == 0) bparent[b] = b2;
                 return true;
             },
@@ -488,7 +478,7 @@ __global__ __launch_bounds__(kThreads) void k_box_root_join(
     const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nitems_c,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rcells, const OrdKey<T>* __restrict__ bbox,
+    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
     const int32_t* __restrict__ rsnap, const uint8_t* __restrict__ core,
     const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
     const int32_t* __restrict__ rcenter, int32_t* bparent) {
@@ -515,7 +505,7 @@ __global__ __launch_bounds__(kThreads) void k_box_root_join(
         const int32_t r0 = uniform(static_cast<int32_t>(roff[u]));
         const int32_t r1 = uniform(static_cast<int32_t>(roff[u + 1]));
         for_each_row_box<T, D>(
-            r0, r1, uniform(rcenter[u]), rcells, cbox, bstart, bbox, rsnap,
+            r0, r1, uniform(rcenter[u]), rboxes, bstart, bbox, rsnap,
             [&](int32_t b2, const double* lo, const double* hi, int32_t q0, int32_t q1,
                 int32_t s2) {
                 if (s2 < 0 || s2 == b) return false;  // no cores, or b's own tree
@@ -523,12 +513,7 @@ __global__ __launch_bounds__(kThreads) void k_box_root_join(
                 point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
                 const bool act = pcore && gmin2 <= gap2_max;
                 if (!__any(act)) return false;
-                bool hit = false;
-                auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
-                    if (cq && act && within<D>(pc, qc, eps2)) hit = true;
-                };
-                auto stop = [&] { return static_cast<bool>(__any(hit)); };
-                if (!visit_range<T, D>(soa, ld, core, nullptr, q0, q1, body, stop)) return false;
+                if (!any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return false;
                 if (lane_id() == 0) uf_unite(bparent, b, b2);
                 return true;
             });
@@ -542,7 +527,7 @@ __global__ __launch_bounds__(kThreads) void k_box_root_join(
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_box_scan(
     Count nbox_c, const int32_t* __restrict__ bcell, const int32_t* __restrict__ cbox,
-    const uint32_t* __restrict__ roff, const int2* __restrict__ rcells,
+    const uint32_t* __restrict__ roff, const int2* __restrict__ rboxes,
     const OrdKey<T>* __restrict__ bbox, const int32_t* __restrict__ job_of_cell,
     const JobParams<T>* __restrict__ jobs, const int32_t* __restrict__ rsnap,
     uint32_t* __restrict__ cnt, int32_t* __restrict__ list, unsigned long long* __restrict__ total,
@@ -565,9 +550,8 @@ __global__ __launch_bounds__(kThreads) void k_box_scan(
             hi[j] = box_hi<T, D>(bbox, b, j);
         }
         for (uint32_t r = roff[u]; r < roff[u + 1]; ++r) {
-            const int2 cs = rcells[r];
-            const int32_t e1 = cbox[cs.y];
-            for (int32_t b2 = max(cbox[cs.x], b + 1); b2 < e1; ++b2) {
+            const int2 bs = rboxes[r];
+            for (int32_t b2 = max(bs.x, b + 1); b2 < bs.y; ++b2) {
                 const int32_t s2 = rsnap[b2];
                 if (s2 < 0 || s2 == sb) continue;
                 double gap2 = 0.0;
@@ -657,13 +641,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union_list(
                 rb = uniform(uf_find(bparent, rb));
                 rb2 = uniform(uf_find(bparent, rb2));
                 if (rb2 == rb) continue;
-                bool hit = false;
-                auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
-                    if (cq && act && within<D>(pc, qc, eps2)) hit = true;
-                };
-                auto stop = [&] { return static_cast<bool>(__any(hit)); };
-                if (visit_range<T, D>(soa, ld, core, nullptr, bcast(q0l, j), bcast(q1l, j), body,
-                                      stop)) {
+                if (any_pair<T, D>(soa, ld, core, bcast(q0l, j), bcast(q1l, j), pc, act, eps2)) {
                     if (lane_id() == 0) uf_unite(bparent, rb, rb2);
                     rb = uniform(uf_find(bparent, b));
                 }
@@ -741,7 +719,7 @@ __global__ __launch_bounds__(kThreads) void k_box_hook_small(
     const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nlist_c,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rcells, const int32_t* __restrict__ rcenter,
+    const int2* __restrict__ rboxes, const int32_t* __restrict__ rcenter,
     const OrdKey<T>* __restrict__ bbox, const int32_t* __restrict__ bmincore,
     const uint8_t* __restrict__ core, const int32_t* __restrict__ job_of_cell,
     const JobParams<T>* __restrict__ jobs, int32_t* __restrict__ bparent) {
@@ -767,10 +745,10 @@ __global__ __launch_bounds__(kThreads) void k_box_hook_small(
     for (int32_t k = -1; k < r1 - r0; ++k) {
         const int32_t r = k < 0 ? center : r0 + k;
         if (k >= 0 && r == center) continue;
-        const int2 cs = rcells[r];
-        const int32_t e0 = cbox[cs.x];
+        const int2 bs = rboxes[r];
+        const int32_t e0 = bs.x;
         if (e0 >= b) continue;  // only boxes before b
-        const int32_t e1 = min(cbox[cs.y], b);
+        const int32_t e1 = min(bs.y, b);
         // the own row from the own cell's first box on, wrapping round
         const int32_t len = e1 - e0;
         const int32_t own = cbox[u];
@@ -904,38 +882,21 @@ __global__ __launch_bounds__(kThreads) void k_select_items(Count nitems_c,
         [&](int64_t i, unsigned int pos) { out[pos] = items[i]; });
 }
 
-__global__ __launch_bounds__(kThreads) void k_core_full(int64_t n,
-                                                        const int32_t* __restrict__ box_of_slot,
-                                                        const uint8_t* __restrict__ btight,
-                                                        const int32_t* __restrict__ bstart,
-                                                        const uint32_t* __restrict__ inrow,
-                                                        uint8_t* __restrict__ core,
-                                                        int32_t* __restrict__ bmincore) {
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (s >= n) return;
-    const int32_t b = box_of_slot[s];
-    const bool full = (btight[b] & 2) != 0;
-    core[s] = full ? 1 : 0;
-    if (full && bstart[b] == s) bmincore[b] = static_cast<int32_t>(inrow[s]);
-}
-
-// the chunks holding a row of a box that is not tight with >= minPts rows
-__global__ __launch_bounds__(kThreads) void k_select_core_chunks(
-    Count nitems_c, const int2* __restrict__ items, const int32_t* __restrict__ ustart,
-    const int32_t* __restrict__ box_of_slot, const uint8_t* __restrict__ btight,
-    int2* __restrict__ out, unsigned int* __restrict__ count) {
-    const int32_t nitems = static_cast<int32_t>(nitems_c.get());
-    block_select(
-        nitems, count,
-        [&](int64_t i) {
-            const int2 it = items[i];
-            const int32_t last = min(it.y + kWave, ustart[it.x + 1]) - 1;
-            const int32_t b1 = box_of_slot[last];
-            for (int32_t b = box_of_slot[it.y]; b <= b1; ++b)
-                if (!(btight[b] & 2)) return true;
-            return false;
-        },
-        [&](int64_t i, unsigned int pos) { out[pos] = items[i]; });
+__global__ __launch_bounds__(kThreads) void k_core_init(
+    int64_t n, const int32_t* __restrict__ box_of_slot, const uint8_t* __restrict__ btight,
+    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
+    const uint32_t* __restrict__ inrow, uint8_t* __restrict__ core, int32_t* __restrict__ bmincore,
+    int2* __restrict__ rows, unsigned int* __restrict__ nrows) {
+    block_collect(n, rows, nrows, [&](int64_t s, int2& v) {
+        const int32_t b = box_of_slot[s];
+        const uint8_t t = btight[b];
+        const bool full = (t & 2) != 0;
+        core[s] = full ? 1 : 0;
+        if (bstart[b] == s) bmincore[b] = full ? static_cast<int32_t>(inrow[s]) : INT_MAX;
+        if (full || !(t & 4)) return false;
+        v = make_int2(static_cast<int32_t>(s), bcell[b]);
+        return true;
+    });
 }
 
 // root of every box's hook tree -> rsnap (-1 for boxes without cores)
@@ -963,7 +924,7 @@ __device__ __forceinline__ void box_union_item(
     const T* __restrict__ soa, int64_t ld, const int2* __restrict__ bitems,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rcells, const OrdKey<T>* __restrict__ bbox,
+    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
     const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
     const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
     const int32_t* __restrict__ rsnap, int32_t* bparent, int32_t wid) {
@@ -991,9 +952,9 @@ __device__ __forceinline__ void box_union_item(
     const int32_t r0 = uniform(static_cast<int32_t>(roff[u]));
     const int32_t r1 = uniform(static_cast<int32_t>(roff[u + 1]));
     for (int32_t r = r0; r < r1; ++r) {
-        const int2 cs = rcells[r];
-        const int32_t e0 = uniform(cbox[uniform(cs.x)]);
-        const int32_t e1 = uniform(cbox[uniform(cs.y)]);
+        const int2 bs = rboxes[r];
+        const int32_t e0 = uniform(bs.x);
+        const int32_t e1 = uniform(bs.y);
         for (int32_t b2 = max(e0, b + 1); b2 < e1; ++b2) {
             // joined by the hook forest already, or no cores (rsnap -1)
             const int32_t s2 = uniform(rsnap[b2]);
@@ -1015,13 +976,8 @@ __device__ __forceinline__ void box_union_item(
             const int32_t rb2 = uniform(uf_find(bparent, b2));
             rb = uniform(uf_find(bparent, rb));
             if (rb2 == rb) continue;
-            bool hit = false;
-            auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
-                if (cq && act && within<D>(pc, qc, eps2)) hit = true;
-            };
-            auto stop = [&] { return static_cast<bool>(__any(hit)); };
-            if (visit_range<T, D>(soa, ld, core, nullptr, uniform(bstart[b2]),
-                                  uniform(bstart[b2 + 1]), body, stop)) {
+            if (any_pair<T, D>(soa, ld, core, uniform(bstart[b2]), uniform(bstart[b2 + 1]), pc, act,
+                               eps2)) {
                 if (lane_id() == 0) uf_unite(bparent, rb, rb2);
                 rb = uniform(uf_find(bparent, b));
             }
@@ -1038,7 +994,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
     const T* __restrict__ soa, int64_t ld, const int2* __restrict__ bitems, int32_t nitems,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rcells, const OrdKey<T>* __restrict__ bbox,
+    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
     const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
     const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
     const int32_t* __restrict__ rsnap, int32_t* bparent,
@@ -1048,7 +1004,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
     for (int32_t wid = uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
                                static_cast<int32_t>(threadIdx.x >> 6));
          wid < nitems; wid += stride)
-        box_union_item<T, D>(soa, ld, bitems, bstart, bcell, cbox, roff, rcells, bbox, bmincore,
+        box_union_item<T, D>(soa, ld, bitems, bstart, bcell, cbox, roff, rboxes, bbox, bmincore,
                              core, job_of_cell, jobs, rsnap, bparent, wid);
 }
 
@@ -1217,7 +1173,7 @@ template <typename K>
 void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* bstart,
                            uint32_t* nbox_dev, uint32_t* cbflag, uint32_t* cbscan,
                            uint32_t* scan_tmp, int32_t* bcell, K* ucell, int32_t* ustart,
-                           uint32_t* ncells_dev, hipStream_t s) {
+                           int32_t* cbox, uint32_t* ncells_dev, hipStream_t s) {
     const Count nb{n, nbox_dev};
     exclusive_scan_u32_dev(cbflag, cbscan, nb, scan_tmp, s);
     copy_at_count(cbscan, nbox_dev, ncells_dev, s);
@@ -1225,13 +1181,8 @@ void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* b
     hipLaunchKernelGGL(k_cells_of_boxes<K>, dim3(static_cast<unsigned>(want < 4096 ? want : 4096)),
                        dim3(kThreads), 0, s, keys, n, shift, bstart, nb,
                        static_cast<const uint32_t*>(cbflag), static_cast<const uint32_t*>(cbscan),
-                       bcell, ucell, ustart, static_cast<const uint32_t*>(ncells_dev));
+                       bcell, ucell, ustart, cbox, static_cast<const uint32_t*>(ncells_dev));
     HPD_HIP(hipGetLastError());
-}
-
-void launch_cell_boxes(const int32_t* bcell, Count nbox, Count m, int32_t* cbox, hipStream_t s) {
-    hipLaunchKernelGGL(k_cell_boxes, dim3(blocks_for(nbox.host > 0 ? nbox.host : 1, kThreads)),
-                       dim3(kThreads), 0, s, bcell, nbox, m, cbox);
 }
 
 void launch_box_items(const int32_t* bstart, Count nbox, uint32_t* cnt, uint32_t* scan_tmp,
@@ -1253,12 +1204,13 @@ void launch_box_items_fill(const int32_t* bstart, Count nbox, const uint32_t* of
 }
 
 template <typename T, int D>
-void launch_box_tight(const BoxArgs<T>& a, uint8_t* btight, unsigned int* nloose, hipStream_t s) {
+void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
+                      unsigned int* nloose, hipStream_t s) {
     using U = OrdKey<T>;
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_tight<T, D>), dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0,
                        s, reinterpret_cast<const U*>(a.bbox), Count{a.nbox, a.nbox_dev}, a.bstart,
-                       a.bcell, a.job_of_cell, a.jobs, btight, nloose);
+                       a.bcell, a.job_of_cell, a.jobs, cell_core, btight, nloose);
 }
 
 // A grid of waves for a count of work items: one wave per item of a
@@ -1275,7 +1227,7 @@ inline unsigned wave_blocks(Count items) {
 }
 
 template <typename T, int D>
-void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
                      Count nlist, int32_t* bparent, int32_t* big, unsigned int* nbig,
                      hipStream_t s) {
@@ -1288,12 +1240,12 @@ void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcel
         // soonest), the small ones one thread each
         const Count nb{nlist.host, nbig};
         hipLaunchKernelGGL((k_box_hook<T, D>), dim3(wave_blocks(nb)), dim3(kThreads), 0, s, a.soa,
-                           a.ld, big, nb, a.bstart, a.bcell, a.cbox, roff, rcells,
+                           a.ld, big, nb, a.bstart, a.bcell, a.cbox, roff, rboxes,
                            reinterpret_cast<const U*>(a.bbox), bmincore, core, a.job_of_cell, a.jobs,
                            a.rcenter, bparent);
         hipLaunchKernelGGL((k_box_hook_small<T, D>), dim3(blocks_for(nlist.host, kThreads)),
                            dim3(kThreads), 0, s, a.soa, a.ld, blist, nlist, a.bstart, a.bcell,
-                           a.cbox, roff, rcells, a.rcenter, reinterpret_cast<const U*>(a.bbox),
+                           a.cbox, roff, rboxes, a.rcenter, reinterpret_cast<const U*>(a.bbox),
                            bmincore, core, a.job_of_cell, a.jobs, bparent);
     }
 }
@@ -1306,13 +1258,13 @@ void launch_box_roots(Count nbox, const int32_t* bmincore, int32_t* bparent, int
 }
 
 template <typename T, int D>
-void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                           const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
                           Count nlist, int32_t* bparent, hipStream_t s) {
     using U = OrdKey<T>;
     if (nlist.host <= 0) return;
     hipLaunchKernelGGL((k_box_root_join<T, D>), dim3(wave_blocks(nlist)), dim3(kThreads), 0, s,
-                       a.soa, a.ld, blist, nlist, a.bstart, a.bcell, a.cbox, roff, rcells,
+                       a.soa, a.ld, blist, nlist, a.bstart, a.bcell, a.cbox, roff, rboxes,
                        reinterpret_cast<const U*>(a.bbox), rsnap, core, a.job_of_cell, a.jobs,
                        a.rcenter, bparent);
 }
@@ -1325,20 +1277,14 @@ void launch_select_boxes(Count nbox, int mode, const int32_t* v, int32_t* list,
                        s, nbox, mode, v, list, count, bstart);
 }
 
-void launch_core_full(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
-                      const int32_t* bstart, const uint32_t* inrow, uint8_t* core,
-                      int32_t* bmincore, hipStream_t s) {
+void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
+                      const int32_t* bstart, const int32_t* bcell, const uint32_t* inrow,
+                      uint8_t* core, int32_t* bmincore, int2* rows, unsigned int* nrows,
+                      hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_core_full, dim3(blocks_for(n, kThreads)), dim3(kThreads), 0, s, n,
-                       box_of_slot, btight, bstart, inrow, core, bmincore);
-}
-
-void launch_select_core_chunks(Count nitems, const int2* items, const int32_t* ustart,
-                               const int32_t* box_of_slot, const uint8_t* btight, int2* out,
-                               unsigned int* count, hipStream_t s) {
-    if (nitems.host <= 0) return;
-    hipLaunchKernelGGL(k_select_core_chunks, dim3(blocks_for(nitems.host, kSelectSpan)),
-                       dim3(kThreads), 0, s, nitems, items, ustart, box_of_slot, btight, out, count);
+    hipLaunchKernelGGL(k_core_init, dim3(collect_blocks(n)), dim3(kCollectThreads), 0, s, n,
+                       box_of_slot, btight, bstart, bcell, inrow, core, bmincore, rows, nrows);
+    HPD_HIP(hipGetLastError());
 }
 
 void launch_select_items(Count nitems, const int2* items, const uint32_t* off, int2* out,
@@ -1355,7 +1301,7 @@ int32_t small_union_rows(int64_t n, int64_t nbox) {
 }
 
 template <typename T, int D>
-void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* rsnap,
                      int32_t* bparent, hipStream_t s, const unsigned long long* only_over,
                      unsigned long long cap) {
@@ -1364,19 +1310,19 @@ void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcel
     const int64_t waves = std::min<int64_t>(a.nbitems, 32768);
     hipLaunchKernelGGL((k_box_union<T, D>), dim3(blocks_for(waves, kWavesPerBlock)),
                        dim3(kThreads), 0, s, a.soa, a.ld, a.bitems, a.nbitems, a.bstart, a.bcell,
-                       a.cbox, roff, rcells, reinterpret_cast<const U*>(a.bbox), bmincore, core,
+                       a.cbox, roff, rboxes, reinterpret_cast<const U*>(a.bbox), bmincore, core,
                        a.job_of_cell, a.jobs, rsnap, bparent, only_over, cap);
 }
 
 template <typename T, int D>
-void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* rsnap, uint32_t* cnt, int32_t* list,
                      unsigned long long* total, hipStream_t s,
                      const unsigned long long* total_chk, unsigned long long cap) {
     using U = OrdKey<T>;
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_scan<T, D>), dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0,
-                       s, Count{a.nbox, a.nbox_dev}, a.bcell, a.cbox, roff, rcells,
+                       s, Count{a.nbox, a.nbox_dev}, a.bcell, a.cbox, roff, rboxes,
                        reinterpret_cast<const U*>(a.bbox), a.job_of_cell, a.jobs, rsnap, cnt, list,
                        total, total_chk, cap);
 }
@@ -1460,8 +1406,8 @@ void launch_positions(int64_t n, int32_t m, const int32_t* box_of_slot, const in
     template void launch_gather_boxes<T, D>(const T*, int64_t, const uint32_t*, T*, int64_t,      \
                                             const int32_t*, const int32_t*, void*, void*,         \
                                             hipStream_t);                                         \
-    template void launch_box_tight<T, D>(const BoxArgs<T>&, uint8_t*, unsigned int*,             \
-                                         hipStream_t);                                            \
+    template void launch_box_tight<T, D>(const BoxArgs<T>&, const uint8_t*, uint8_t*,            \
+                                         unsigned int*, hipStream_t);                                            \
     template void launch_box_hook<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,          \
                                         const int32_t*, const uint8_t*, const int32_t*, Count,    \
                                         int32_t*, int32_t*, unsigned int*, hipStream_t);          \
@@ -1502,9 +1448,11 @@ template void launch_box_table<uint64_t>(const uint64_t*, int64_t, const uint32_
                                          hipStream_t, int, uint32_t*);
 template void launch_cells_of_boxes<uint32_t>(const uint32_t*, int64_t, int, const int32_t*,
                                               uint32_t*, uint32_t*, uint32_t*, uint32_t*, int32_t*,
-                                              uint32_t*, int32_t*, uint32_t*, hipStream_t);
+                                              uint32_t*, int32_t*, int32_t*, uint32_t*,
+                                              hipStream_t);
 template void launch_cells_of_boxes<uint64_t>(const uint64_t*, int64_t, int, const int32_t*,
                                               uint32_t*, uint32_t*, uint32_t*, uint32_t*, int32_t*,
-                                              uint64_t*, int32_t*, uint32_t*, hipStream_t);
+                                              uint64_t*, int32_t*, int32_t*, uint32_t*,
+                                              hipStream_t);
 
 }  // namespace hpd

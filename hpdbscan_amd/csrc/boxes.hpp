@@ -56,14 +56,14 @@ void launch_box_table(const K* keys, int64_t n, const uint32_t* cflags, const ui
                       uint32_t* cbflag = nullptr);
 // The occupied cells from the boxes of launch_box_table (every cell starts
 // a box): ucell, ustart (ustart[m] = n) and *ncells_dev as launch_cells
-// gives them, and bcell per box, from one scan over the boxes instead of
-// a flag pass and a scan over all n slots.  cbscan: n + 1 words.
+// gives them, bcell per box and cbox (first box per cell, cbox[m] = number
+// of boxes), from one scan over the boxes instead of a flag pass and a scan
+// over all n slots.  cbscan: n + 1 words.
 template <typename K>
 void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* bstart,
                            uint32_t* nbox_dev, uint32_t* cbflag, uint32_t* cbscan,
                            uint32_t* scan_tmp, int32_t* bcell, K* ucell, int32_t* ustart,
-                           uint32_t* ncells_dev, hipStream_t s);
-void launch_cell_boxes(const int32_t* bcell, Count nbox, Count m, int32_t* cbox, hipStream_t s);
+                           int32_t* cbox, uint32_t* ncells_dev, hipStream_t s);
 
 // cnt[b] = 64-slot chunks of box b, scanned in place; *total_dev = chunks
 void launch_box_items(const int32_t* bstart, Count nbox, uint32_t* cnt, uint32_t* scan_tmp,
@@ -71,10 +71,12 @@ void launch_box_items(const int32_t* bstart, Count nbox, uint32_t* cnt, uint32_t
 void launch_box_items_fill(const int32_t* bstart, Count nbox, const uint32_t* off, Count nitems,
                            int2* items, hipStream_t s);
 
-// btight[b]: bit 0 tight, bit 1 tight with >= minPts rows; *nloose counts
-// boxes of two or more rows that are not tight
+// btight[b]: bit 0 tight, bit 1 tight with >= minPts rows, bit 2 in a cell
+// that can hold cores (cell_core); *nloose counts boxes of two or more rows
+// that are not tight
 template <typename T, int D>
-void launch_box_tight(const BoxArgs<T>& a, uint8_t* btight, unsigned int* nloose, hipStream_t s);
+void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
+                      unsigned int* nloose, hipStream_t s);
 
 // Components of the boxes with cores:
 //   launch_select_boxes  list of the boxes with cores (mode 0, v = bmincore),
@@ -97,28 +99,27 @@ constexpr int kRootJoinRounds = D <= 3 ? 1 : 2;
 void launch_select_boxes(Count nbox, int mode, const int32_t* v, int32_t* list,
                          unsigned int* count, hipStream_t s, const int32_t* bstart = nullptr);
 template <typename T, int D>
-void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
                      Count nlist, int32_t* bparent, int32_t* big, unsigned int* nbig,
                      hipStream_t s);
 void launch_box_roots(Count nbox, const int32_t* bmincore, int32_t* bparent, int32_t* rsnap,
                       hipStream_t s);
 template <typename T, int D>
-void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                           const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
                           Count nlist, int32_t* bparent, hipStream_t s);
-// the box chunks (items) of the boxes with open pairs (off[b+1] > off[b])
 // core[s] = 1 for the rows of tight boxes with >= minPts rows (btight bit 1),
-// 0 for every other row; for those boxes bmincore[b] = inrow[bstart[b]]
-// (every row is core and a box holds its rows in input order)
-void launch_core_full(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
-                      const int32_t* bstart, const uint32_t* inrow, uint8_t* core,
-                      int32_t* bmincore, hipStream_t s);
-// out[..] = the chunks (cell, first row) of items holding a row outside
-// those boxes; *count += their number
-void launch_select_core_chunks(Count nitems, const int2* items, const int32_t* ustart,
-                               const int32_t* box_of_slot, const uint8_t* btight, int2* out,
-                               unsigned int* count, hipStream_t s);
+// 0 for every other row; bmincore[b] = inrow[bstart[b]] for those boxes
+// (every row is core and a box holds its rows in input order), INT_MAX for
+// the others; rows[..] = the other rows whose cell can hold cores (btight
+// bit 2), as (slot, cell), *nrows += their number
+void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
+                      const int32_t* bstart, const int32_t* bcell, const uint32_t* inrow,
+                      uint8_t* core, int32_t* bmincore, int2* rows, unsigned int* nrows,
+                      hipStream_t s);
+// out[..] = the box chunks (items) of the boxes with open pairs (off[b+1] >
+// off[b]); *count += their number
 // (with min_rows > 0: only chunks of boxes of more than min_rows rows; the
 // thread-per-box union of launch_box_union_list takes the others)
 void launch_select_items(Count nitems, const int2* items, const uint32_t* off, int2* out,
@@ -135,7 +136,7 @@ int32_t small_union_rows(int64_t n, int64_t nbox);
 // only_over (optional): the join runs only when *only_over > cap, i.e. when
 // the open-pair lists did not fit (decided on the device, no host check).
 template <typename T, int D>
-void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* rsnap,
                      int32_t* bparent, hipStream_t s, const unsigned long long* only_over = nullptr,
                      unsigned long long cap = 0);
@@ -151,7 +152,7 @@ void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcel
 // both do nothing when *total_chk > cap, and launch_box_join with the same
 // check runs exactly then.
 template <typename T, int D>
-void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rcells,
+void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* rsnap, uint32_t* cnt, int32_t* list,
                      unsigned long long* total, hipStream_t s,
                      const unsigned long long* total_chk = nullptr, unsigned long long cap = 0);

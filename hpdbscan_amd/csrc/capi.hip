@@ -320,6 +320,7 @@ private:
 // Neighbour rows of one run are indexed with 32-bit offsets (signed in the
 // kernels' loops).
 constexpr uint64_t kMaxNeighborRows = 0x7fffffffull;
+constexpr int kWaveRows = 64;  // rows of a work item
 
 static void check_neighbor_rows(uint64_t total) {
     if (total > kMaxNeighborRows)
@@ -359,7 +360,7 @@ static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
     b += sizeof(T) * 2 * D * (mm_blocks + nj) + 4 * (mm_blocks + nj + 2) + 64;  // min/max
     b += sizeof(JobParams<T>) * nj + 4 * nn;   // job table, job of every cell
     if (one_thread) b += 8 * nn + 4 * nn + nn + 4;  // ambiguous rows, f, involved, flag
-    b += 8 * (16 + kNoiseStripes);            // statistics, counters, noise counters
+    b += 8 * 16;                               // statistics, counters
     b += 54 * 256 + 64 * 1024;                 // alignment
     return b;
 }
@@ -397,10 +398,10 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     int32_t* cmax = A.take_n<int32_t>(nn);
     int32_t* rcenter = A.take_n<int32_t>(nn);
     int32_t* job_of_cell = A.take_n<int32_t>(nn);
-    unsigned long long* dstats = A.take_n<unsigned long long>(16 + kNoiseStripes);
-    uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);  // m, ranges, items, boxes, box items, loose
-    unsigned long long* noise_stripes = dstats + 16;
-    HPD_HIP(hipMemsetAsync(dstats, 0, (16 + kNoiseStripes) * sizeof(unsigned long long), s));
+    unsigned long long* dstats = A.take_n<unsigned long long>(16);
+    // m, ranges, items, boxes, box items, loose, rows to count, non-core rows
+    uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
+    HPD_HIP(hipMemsetAsync(dstats, 0, 16 * sizeof(unsigned long long), s));
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx.host_scratch);
 
     // cell ids (spatial_index.h:144-165), offset by the job's key base; in
@@ -469,7 +470,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
                             &counters[3], nullptr, 2 * D, static_cast<int>(sizeof(T)), s, sub_bits,
                             flags);
         launch_cells_of_boxes<K>(keys, n, sub_bits, bstart, &counters[3], flags, flags + nn + 1,
-                                 tmp, bcell, ucell, ustart, &counters[0], s);
+                                 tmp, bcell, ucell, ustart, cbox, &counters[0], s);
         launch_gather_boxes<T, D>(rows_sorted ? nullptr : pts, n, inrow_of_slot, soa, ld,
                                   box_of_slot, bstart, bbox, bpart, s);
     } else if (!rows_sorted) {
@@ -491,10 +492,10 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     }
     tm.mark(M_SORT);
 
-    // neighbour ranges (spatial_index.h:682-737) and work items
-    uint32_t* ccnt = boxes ? A.take_n<uint32_t>(nn + 1) : nullptr;
+    // neighbour ranges (spatial_index.h:682-737)
+    uint8_t* cell_core = boxes ? A.take_n<uint8_t>(nn) : nullptr;
     // the count pass keeps the rows it finds in scratch64 (idle until the
-    // union) when every cell's 3^(D-1) rows fit, and the fill copies them
+    // core count) when every cell's 3^(D-1) rows fit, and the fill copies them
     int32_t stash_rows = 1;
     for (int j = 1; j < D; ++j) stash_rows *= 3;
     int2* stash = scratch64 && static_cast<uint64_t>(m) * static_cast<uint64_t>(stash_rows) <= nn
@@ -502,28 +503,20 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
                       : nullptr;
     // up to 27 rows per cell (D <= 4): the copy puts the nearest rows first
     const bool by_class = stash && D <= 4;
-    launch_neighbor_count<K, T>(ucell, ustart, host_count(m), jobs, njobs, job_of_cell, nranges, ccnt,
-                                &dstats[0], &dstats[4], stash, stash_rows, rcenter, by_class, s,
-                                ctab);
-    launch_chunk_counts(ustart, host_count(m), nchunks, s);
-    // box mode: dense-cell chunks and sparse-cell rows as separate work
-    // lists; their per-cell counts live in the (now unused) run flags
-    uint32_t* dcnt = flags;
-    uint32_t* scnt = flags + nn + 1;
-    if (boxes) launch_split_counts(ustart, host_count(m), ctx.sparse_max, dcnt, scnt, s);
-    // the per-cell counts, scanned together (totals at entry m)
+    launch_neighbor_count<K, T>(ucell, ustart, host_count(m), jobs, njobs, job_of_cell, nranges,
+                                cell_core, &dstats[0], &dstats[4], stash, stash_rows, rcenter,
+                                by_class, s, ctab);
+    // the per-cell counts, scanned together (totals at entry m); box mode
+    // has no use for the 64-row chunks of every cell unless the union runs on
+    // rows or the one-thread border rule meets an ambiguous row
+    if (!boxes) launch_chunk_counts(ustart, host_count(m), nchunks, s);
     ScanSet counts{};
     int ncounts = 0;
     counts.a[ncounts++] = nranges;
-    counts.a[ncounts++] = nchunks;
-    if (boxes) {
-        counts.a[ncounts++] = ccnt;
-        counts.a[ncounts++] = dcnt;
-        counts.a[ncounts++] = scnt;
-    }
+    if (!boxes) counts.a[ncounts++] = nchunks;
     exclusive_scan_set_u32(counts, ncounts, m, tmp, tmp_words, s);
     if (boxes) {
-        // the box chunks (counted and scanned) and the tight flags (their
+        // the box chunks (counted and scanned) and the box flags (their
         // loose count decides the union) before the read-back below
         launch_box_items(bstart, host_count(nbox), bcnt, tmp, &counters[4], s);
         BoxArgs<T> bt;
@@ -533,18 +526,13 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         bt.bbox = bbox;
         bt.jobs = jobs;
         bt.job_of_cell = job_of_cell;
-        launch_box_tight<T, D>(bt, btight, &counters[5], s);
+        launch_box_tight<T, D>(bt, cell_core, btight, &counters[5], s);
     }
     // the scans' totals into the counters (one launch), then one read-back
     // of the 64-bit row total (dstats[4]) and the counters (dstats + 8)
     WordCopies totals;
     totals.add(&nranges[m], &counters[1]);
-    totals.add(&nchunks[m], &counters[2]);
-    if (boxes) {
-        totals.add(&ccnt[m], &counters[11]);
-        totals.add(&dcnt[m], &counters[6]);
-        totals.add(&scnt[m], &counters[7]);
-    }
+    if (!boxes) totals.add(&nchunks[m], &counters[2]);
     copy_words(totals, s);
     unsigned long long* hs_rows = reinterpret_cast<unsigned long long*>(ctx.host_scratch) + 12;
     HPD_HIP(hipMemcpyAsync(hs_rows, &dstats[4], 10 * sizeof(unsigned long long),
@@ -555,49 +543,44 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     // 64-bit total first
     check_neighbor_rows(*hs_rows);
     const uint32_t total_ranges = hc[1];
-    const int32_t ncitems = boxes ? static_cast<int32_t>(hc[11]) : 0;
-    const int32_t nitems = static_cast<int32_t>(hc[2]);
-    const int32_t nditems = boxes ? static_cast<int32_t>(hc[6]) : 0;
-    const int32_t nsitems = boxes ? static_cast<int32_t>(hc[7]) : 0;
     const int32_t nbitems = boxes ? static_cast<int32_t>(hc[4]) : 0;
     // every box of two or more rows is tight: the union runs on boxes
     const bool all_tight = boxes && hc[5] == 0;
+    const bool one_thread = ctx.border_rule == HPD_BORDER_ONE_THREAD;
+    // the row-level tables: slot and cell ranges of the neighbour rows and the
+    // chunks of every cell (at most one per cell and one per 64 rows)
+    const bool row_tables = !all_tight || one_thread;
+    const size_t max_items =
+        boxes ? static_cast<size_t>(m) + nn / kWaveRows + 1 : static_cast<size_t>(hc[2]);
 
-    X.reserve(2 * align_up(static_cast<size_t>(total_ranges) * sizeof(int2), 256) +
-                    align_up(static_cast<size_t>(nitems) * sizeof(int2), 256) +
-                    align_up(static_cast<size_t>(nbitems) * sizeof(int2), 256) +
-                    align_up(static_cast<size_t>(nditems) * sizeof(int2), 256) +
-                    align_up(static_cast<size_t>(nsitems) * sizeof(int2), 256) +
-                    align_up(static_cast<size_t>(nbitems) * sizeof(int2), 256) +
-                    2 * align_up(static_cast<size_t>(ncitems) * sizeof(int2), 256) + 2048);
-    int2* ranges = X.take_n<int2>(total_ranges);
-    int2* rcells = X.take_n<int2>(total_ranges);
-    int2* items = X.take_n<int2>(static_cast<size_t>(nitems));
+    const size_t range_bytes = align_up(static_cast<size_t>(total_ranges) * sizeof(int2), 256);
+    X.reserve((boxes ? range_bytes : 0) + (row_tables ? 2 * range_bytes : 0) +
+              (row_tables ? align_up(max_items * sizeof(int2), 256) : 0) +
+              2 * align_up(static_cast<size_t>(nbitems) * sizeof(int2), 256) + 2048);
+    int2* rboxes = boxes ? X.take_n<int2>(total_ranges) : nullptr;
+    int2* ranges = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
+    int2* rcells = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
+    int2* items = row_tables ? X.take_n<int2>(max_items) : nullptr;
     int2* bitems = boxes ? X.take_n<int2>(static_cast<size_t>(nbitems)) : nullptr;
-    int2* ditems = boxes ? X.take_n<int2>(static_cast<size_t>(nditems)) : nullptr;
-    int2* sitems = boxes ? X.take_n<int2>(static_cast<size_t>(nsitems)) : nullptr;
     int2* uitems = boxes ? X.take_n<int2>(static_cast<size_t>(nbitems)) : nullptr;
-    int2* citems = boxes ? X.take_n<int2>(static_cast<size_t>(ncitems)) : nullptr;
-    int2* citems_need = boxes ? X.take_n<int2>(static_cast<size_t>(ncitems)) : nullptr;
-    if (stash)
-        launch_neighbor_copy(stash, stash_rows, ustart, m, nranges, ranges, rcells, rcenter,
-                             by_class, s);
+    if (boxes && stash)
+        launch_neighbor_copy(stash, stash_rows, m, nranges, cbox, rboxes, rcenter, by_class, s);
+    else if (boxes)
+        launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
+                                   nullptr, rboxes, rcenter, s, ctab, cbox);
     else
-        launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges, ranges,
-                                   rcells, rcenter, s, ctab);
-    launch_work_items(ustart, host_count(m), nchunks, host_count(nitems), items, s);
-    if (boxes) {
-        launch_split_items(ustart, host_count(m), ctx.sparse_max, dcnt, scnt, ditems,
-                           host_count(nditems), sitems, s);
-        launch_expand_chunks(ccnt, host_count(m), ustart, host_count(ncitems), citems, s);
-    }
+        launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
+                                   ranges, rcells, rcenter, s);
+    if (!boxes)
+        launch_work_items(ustart, host_count(m), nchunks, host_count(static_cast<int64_t>(hc[2])),
+                          items, s);
 
     DbscanArgs<T> a;
     a.soa = soa;
     a.n = n;
     a.ld = ld;
     a.items = items;
-    a.nitems = nitems;
+    a.nitems = boxes ? 0 : static_cast<int32_t>(hc[2]);
     a.ustart = ustart;
     a.roff = nranges;
     a.ranges = ranges;
@@ -613,7 +596,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     BoxArgs<T> ba;
     bool box_union = false;
     if (boxes) {
-        launch_cell_boxes(bcell, host_count(nbox), host_count(m), cbox, s);
         launch_box_items_fill(bstart, host_count(nbox), bcnt, host_count(nbitems), bitems, s);
         ba.soa = soa;
         ba.ld = ld;
@@ -633,18 +615,27 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         a.bstart = bstart;
         a.bcell = bcell;
         a.bbox = bbox;
-        a.sparse_core = ctx.sparse_core;
+        a.rboxes = rboxes;
         a.bmincore = bmincore;
-        fill_i32(bmincore, INT_MAX, nbox, s);
-        a.ditems = ditems;
-        a.nditems = nditems;
-        a.citems = citems;
-        a.ncitems = ncitems;
-        a.citems_need = citems_need;
-        a.ncitems_need_dev = &counters[12];
-        a.sitems = sitems;
-        a.nsitems = nsitems;
+        // both row lists in scratch64, before and after the union
+        a.crows = reinterpret_cast<int2*>(scratch64);
+        a.ncrows_dev = &counters[6];
+        a.brows = reinterpret_cast<int2*>(scratch64);
+        a.nbrows_dev = &counters[7];
     }
+    // box mode: the row-level tables when they turn out to be needed (the
+    // neighbour rows ascending again, their own-row index with them)
+    auto fill_row_tables = [&] {
+        launch_chunk_counts(ustart, host_count(m), nchunks, s);
+        exclusive_scan_u32(nchunks, nchunks, m, tmp, &nchunks[m], s);
+        uint32_t* h = reinterpret_cast<uint32_t*>(ctx.host_scratch) + 64;
+        HPD_HIP(hipMemcpyAsync(h, &nchunks[m], sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        HPD_HIP(hipStreamSynchronize(s));
+        a.nitems = static_cast<int32_t>(*h);
+        launch_work_items(ustart, host_count(m), nchunks, host_count(a.nitems), items, s);
+        launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
+                                   ranges, rcells, rcenter, s);
+    };
     tm.mark(M_INDEX);
 
     launch_core<T, D>(a, core, ctx.count_tests ? &dstats[7] : nullptr, s, tm.event(M_CORE0));
@@ -662,13 +653,13 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         // (the slot-level union's rsnap is free in box mode: the list of
         // the larger boxes)
         launch_select_boxes(host_count(nbox), 2, bmincore, rsnap, &counters[14], s, bstart);
-        launch_box_hook<T, D>(ba, nranges, rcells, bmincore, core, blist,
+        launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist,
                               Count{nbox, &counters[8], true}, bparent, rsnap, &counters[14], s);
         launch_box_roots(host_count(nbox), bmincore, bparent, compmin, s);
         for (int round = 0; round < kRootJoinRounds<D>; ++round) {
             HPD_HIP(hipMemsetAsync(&counters[9], 0, sizeof(uint32_t), s));
             launch_select_boxes(host_count(nbox), 1, compmin, blist, &counters[9], s);
-            launch_box_root_join<T, D>(ba, nranges, rcells, compmin, core, blist,
+            launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, blist,
                                        Count{nbox, &counters[9]}, bparent, s);
             launch_box_roots(host_count(nbox), bmincore, bparent, compmin, s);
         }
@@ -678,7 +669,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         int32_t* list = reinterpret_cast<int32_t*>(scratch64);
         unsigned long long cap = 2 * static_cast<unsigned long long>(nn);
         if (ctx.open_pair_limit > 0 && ctx.open_pair_limit < cap) cap = ctx.open_pair_limit;
-        launch_box_scan<T, D>(ba, nranges, rcells, compmin, bcnt, nullptr, &dstats[5], s);
+        launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, nullptr, &dstats[5], s);
         // offsets (meaningful when the total fits; the kernels that use them
         // check the 64-bit total on the device, and the full join runs
         // instead when it does not fit) and the chunks of the boxes that
@@ -688,10 +679,10 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         const int32_t small_rows = small_union_rows(n, nbox);
         launch_select_items(host_count(nbitems), bitems, bcnt, uitems, &counters[10], s, bstart,
                             small_rows);
-        launch_box_scan<T, D>(ba, nranges, rcells, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
+        launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
         launch_box_union_list<T, D>(ba, uitems, Count{nbitems, &counters[10]}, core, bcnt, list,
                                     bparent, s, &dstats[5], cap, small_rows);
-        launch_box_join<T, D>(ba, nranges, rcells, bmincore, core, compmin, bparent, s, &dstats[5],
+        launch_box_join<T, D>(ba, nranges, rboxes, bmincore, core, compmin, bparent, s, &dstats[5],
                               cap);
         tm.mark(M_JOIN1);
         launch_box_clusters(host_count(nbox), bmincore, bcell, cbox, bstart, inrow_of_slot, ustart,
@@ -700,6 +691,8 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     } else {
         if (boxes) {
             // a loose box: the slot-level union needs the sorted positions
+            // and the row-level tables
+            fill_row_tables();
             launch_positions(n, m, box_of_slot, bcell, inrow_of_slot,
                              reinterpret_cast<uint32_t*>(keys), vals_free,
                              reinterpret_cast<uint32_t*>(keys_free),
@@ -710,7 +703,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         launch_union_points<T, D>(a, core, parent, rsnap, cmin, cmax, compmin, s);
     }
     tm.mark(M_UNION);
-    const bool one_thread = ctx.border_rule == HPD_BORDER_ONE_THREAD;
     int2* amb = one_thread ? A.take_n<int2>(nn) : nullptr;
     // box mode reads rootslot only under the one-thread border rule; without
     // it the rows of full boxes are labelled in input order, through a table
@@ -729,7 +721,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
                           &dstats[1], s, full_ok);
     tm.mark(M_BORDER0);
     launch_border<T, D>(a, core, box_union ? bcluster : nullptr, rootslot, cmin, cmax, labels,
-                        &dstats[2], amb, noise_stripes, s);
+                        &dstats[2], amb, s);
 
     unsigned long long* hs = reinterpret_cast<unsigned long long*>(ctx.host_scratch);
     HPD_HIP(hipMemcpyAsync(hs, dstats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
@@ -740,6 +732,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         // the reference's choice at one thread for the border rows next to
         // two or more clusters (hpdbscan.h:74-92)
         const int32_t namb = static_cast<int32_t>(hs[3]);
+        if (box_union) fill_row_tables();
         if (boxes && !a.pos_of_slot) {  // the relaxation compares sorted positions
             launch_positions(n, m, box_of_slot, bcell, inrow_of_slot,
                              reinterpret_cast<uint32_t*>(keys), vals_free,
@@ -804,17 +797,14 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
 enum StaticSlot : int {
     SS_M = 0,          // occupied cells
     SS_RANGES = 1,     // neighbour rows
-    SS_ITEMS = 2,      // 64-row chunks of every cell
     SS_NBOX = 3,       // boxes
     SS_BITEMS = 4,     // 64-slot chunks of every box
     SS_LOOSE = 5,      // boxes of two or more rows that are not tight
-    SS_DITEMS = 6,     // chunks of dense cells
-    SS_SITEMS = 7,     // rows of sparse cells
+    SS_CROWS = 6,      // rows to count
+    SS_BROWS = 7,      // non-core rows
     SS_NLIST = 8,      // boxes with cores
     SS_JOIN0 = 9,      // roots of the first root-join round
     SS_UITEMS = 10,    // box chunks with open pairs
-    SS_CITEMS = 11,    // chunks of cells with >= minPts candidates
-    SS_NEED = 12,      // those holding a row outside the full tight boxes
     SS_JOIN1 = 13,     // roots of the second round
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
@@ -835,8 +825,8 @@ static inline int64_t range_bound(int64_t n) {
 
 template <typename T, int D>
 static size_t static_aux_bytes(int64_t n) {
-    return 2 * align_up(static_cast<size_t>(range_bound<D>(n)) * sizeof(int2), 256) +
-           7 * align_up(static_cast<size_t>(item_bound(n)) * sizeof(int2), 256) + 4096;
+    return align_up(static_cast<size_t>(range_bound<D>(n)) * sizeof(int2), 256) +
+           2 * align_up(static_cast<size_t>(item_bound(n)) * sizeof(int2), 256) + 4096;
 }
 
 template <typename T, int D>
@@ -849,7 +839,7 @@ static size_t static_main_bytes(int64_t n, int32_t njobs) {
 // else (no read-back, no synchronisation, no memset), in the workspace the
 // caller reserved and started taking from; jobs / bfirst_dev hold the
 // host-made job table (row ranges, eps2, minPts, reciprocals) and min/max
-// blocks.  sc (SS_WORDS words) and dstats (16 + kNoiseStripes words) end up
+// blocks.  sc (SS_WORDS words) and dstats (16 words) end up
 // holding the counts read afterwards.
 template <typename T, int D>
 static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
@@ -865,8 +855,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     const int64_t IB = item_bound(n);
     // zeroed by a kernel (no memset in a graph)
     fill_i32(reinterpret_cast<int32_t*>(sc), 0, SS_WORDS, s);
-    fill_i32(reinterpret_cast<int32_t*>(dstats), 0, 2 * (16 + kNoiseStripes), s);
-    unsigned long long* noise_stripes = dstats + 16;
+    fill_i32(reinterpret_cast<int32_t*>(dstats), 0, 2 * 16, s);
 
     // min / max, then every job's grid on the device
     T* part = A.take_n<T>(static_cast<size_t>(nblocks) * 2 * D + 1);
@@ -916,7 +905,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     uint8_t* btight = A.take_n<uint8_t>(nn);
     void* bbox = A.take(2 * D * sizeof(T) * nn);
     void* bpart = A.take(gather_part_bytes(n, D, static_cast<int>(sizeof(T))));
-    uint32_t* ccnt = A.take_n<uint32_t>(nn + 1);
+    uint8_t* cell_core = A.take_n<uint8_t>(nn);
 
     // cell ids and the sort (passes past the key's bits do nothing)
     launch_cell_ids<T, D, K>(pts, n, jobs, njobs, sub_k, sub_bits, keys_a, vals_a, s);
@@ -929,49 +918,24 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
                         bstart, bcell, box_of_slot, &sc[SS_NBOX], nullptr, 2 * D,
                         static_cast<int>(sizeof(T)), s, sub_bits, flags);
     launch_cells_of_boxes<K>(keys, n, sub_bits, bstart, &sc[SS_NBOX], flags, flags + nn + 1, tmp,
-                             bcell, ucell, ustart, &sc[SS_M], s);
+                             bcell, ucell, ustart, cbox, &sc[SS_M], s);
     launch_gather_boxes<T, D>(pts, n, inrow_of_slot, soa, ld, box_of_slot, bstart, bbox, bpart, s);
 
     // neighbour rows and work lists, counted and laid out on the device
     const Count M{n, &sc[SS_M]};
     const Count NB{n, &sc[SS_NBOX]};
-    uint32_t* dcnt = flags;
-    uint32_t* scnt = flags + nn + 1;
-    launch_neighbor_count<K, T>(ucell, ustart, M, jobs, njobs, job_of_cell, nranges, ccnt,
+    launch_neighbor_count<K, T>(ucell, ustart, M, jobs, njobs, job_of_cell, nranges, cell_core,
                                 &dstats[0], &dstats[4], nullptr, 1, rcenter, false, s);
-    launch_chunk_counts(ustart, M, nchunks, s);
-    launch_split_counts(ustart, M, ctx.sparse_max, dcnt, scnt, s);
-    ScanSet counts{};
-    counts.a[0] = nranges;
-    counts.a[1] = nchunks;
-    counts.a[2] = ccnt;
-    counts.a[3] = dcnt;
-    counts.a[4] = scnt;
-    exclusive_scan_set_u32(counts, 5, n, tmp, tmp_words, s, &sc[SS_M]);
+    exclusive_scan_u32_dev(nranges, nranges, M, tmp, s);
     copy_at_count(nranges, &sc[SS_M], &sc[SS_RANGES], s);
-    copy_at_count(nchunks, &sc[SS_M], &sc[SS_ITEMS], s);
-    copy_at_count(ccnt, &sc[SS_M], &sc[SS_CITEMS], s);
-    copy_at_count(dcnt, &sc[SS_M], &sc[SS_DITEMS], s);
-    copy_at_count(scnt, &sc[SS_M], &sc[SS_SITEMS], s);
     launch_box_items(bstart, NB, bcnt, tmp, &sc[SS_BITEMS], s);
 
     const int64_t R = range_bound<D>(n);
-    int2* ranges = X.take_n<int2>(static_cast<size_t>(R));
-    int2* rcells = X.take_n<int2>(static_cast<size_t>(R));
-    int2* items = X.take_n<int2>(static_cast<size_t>(IB));
+    int2* rboxes = X.take_n<int2>(static_cast<size_t>(R));
     int2* bitems = X.take_n<int2>(static_cast<size_t>(IB));
-    int2* ditems = X.take_n<int2>(static_cast<size_t>(IB));
-    int2* sitems = X.take_n<int2>(static_cast<size_t>(IB));
     int2* uitems = X.take_n<int2>(static_cast<size_t>(IB));
-    int2* citems = X.take_n<int2>(static_cast<size_t>(IB));
-    int2* citems_need = X.take_n<int2>(static_cast<size_t>(IB));
-    launch_neighbor_fill<K, T>(ucell, ustart, M, jobs, job_of_cell, nranges, ranges, rcells, rcenter,
-                               s);
-    launch_work_items(ustart, M, nchunks, Count{IB, &sc[SS_ITEMS]}, items, s);
-    launch_split_items(ustart, M, ctx.sparse_max, dcnt, scnt, ditems, Count{IB, &sc[SS_DITEMS]},
-                       sitems, s);
-    launch_expand_chunks(ccnt, M, ustart, Count{IB, &sc[SS_CITEMS]}, citems, s);
-    launch_cell_boxes(bcell, NB, M, cbox, s);
+    launch_neighbor_fill<K, T>(ucell, ustart, M, jobs, job_of_cell, nranges, nullptr, rboxes,
+                               rcenter, s, nullptr, cbox);
     launch_box_items_fill(bstart, NB, bcnt, Count{IB, &sc[SS_BITEMS]}, bitems, s);
 
     BoxArgs<T> ba;
@@ -988,19 +952,15 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     ba.jobs = jobs;
     ba.job_of_cell = job_of_cell;
     ba.rcenter = rcenter;
-    launch_box_tight<T, D>(ba, btight, &sc[SS_LOOSE], s);
-    fill_i32(bmincore, INT_MAX, n, s);
+    launch_box_tight<T, D>(ba, cell_core, btight, &sc[SS_LOOSE], s);
 
     DbscanArgs<T> a;
     a.soa = soa;
     a.n = n;
     a.ld = ld;
-    a.items = items;
-    a.nitems = static_cast<int32_t>(IB);
     a.ustart = ustart;
     a.roff = nranges;
-    a.ranges = ranges;
-    a.rcells = rcells;
+    a.rboxes = rboxes;
     a.rcenter = rcenter;
     a.m = static_cast<int32_t>(n);
     a.jobs = jobs;
@@ -1014,45 +974,37 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     a.bstart = bstart;
     a.bcell = bcell;
     a.bbox = bbox;
-    a.sparse_core = ctx.sparse_core;
     a.bmincore = bmincore;
-    a.ditems = ditems;
-    a.nditems = static_cast<int32_t>(IB);
-    a.nditems_dev = &sc[SS_DITEMS];
-    a.citems = citems;
-    a.ncitems = static_cast<int32_t>(IB);
-    a.ncitems_dev = &sc[SS_CITEMS];
-    a.citems_need = citems_need;
-    a.ncitems_need_dev = &sc[SS_NEED];
-    a.sitems = sitems;
-    a.nsitems = static_cast<int32_t>(n);
-    a.nsitems_dev = &sc[SS_SITEMS];
+    a.crows = reinterpret_cast<int2*>(scratch64);
+    a.ncrows_dev = &sc[SS_CROWS];
+    a.brows = reinterpret_cast<int2*>(scratch64);
+    a.nbrows_dev = &sc[SS_BROWS];
     launch_core<T, D>(a, core, ctx.count_tests ? &dstats[7] : nullptr, s);
 
     // the box union (its result is discarded when a box is loose)
     int32_t* blist = parent;
     launch_select_boxes(NB, 0, bmincore, blist, &sc[SS_NLIST], s);
     launch_select_boxes(NB, 2, bmincore, hook_big, &sc[SS_HOOKBIG], s, bstart);
-    launch_box_hook<T, D>(ba, nranges, rcells, bmincore, core, blist, Count{n, &sc[SS_NLIST]},
+    launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, Count{n, &sc[SS_NLIST]},
                           bparent, hook_big, &sc[SS_HOOKBIG], s);
     launch_box_roots(NB, bmincore, bparent, compmin, s);
     for (int round = 0; round < kRootJoinRounds<D>; ++round) {
         uint32_t* cnt = &sc[round == 0 ? SS_JOIN0 : SS_JOIN1];
         launch_select_boxes(NB, 1, compmin, blist, cnt, s);
-        launch_box_root_join<T, D>(ba, nranges, rcells, compmin, core, blist, Count{n, cnt}, bparent,
+        launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, blist, Count{n, cnt}, bparent,
                                    s);
         launch_box_roots(NB, bmincore, bparent, compmin, s);
     }
     int32_t* list = reinterpret_cast<int32_t*>(scratch64);
     const unsigned long long cap = 2 * static_cast<unsigned long long>(nn);
-    launch_box_scan<T, D>(ba, nranges, rcells, compmin, bcnt, nullptr, &dstats[5], s);
+    launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, nullptr, &dstats[5], s);
     exclusive_scan_u32_dev(bcnt, bcnt, NB, tmp, s);
     // (the box count is on the device: the small boxes' pairs always one
     // thread per box, the static pipeline's batches of small clouds being
     // sparse)
     launch_select_items(Count{IB, &sc[SS_BITEMS]}, bitems, bcnt, uitems, &sc[SS_UITEMS], s, bstart,
                         kSmallUnionRows);
-    launch_box_scan<T, D>(ba, nranges, rcells, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
+    launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
     launch_box_union_list<T, D>(ba, uitems, Count{IB, &sc[SS_UITEMS]}, core, bcnt, list, bparent, s,
                                 &dstats[5], cap, kSmallUnionRows);
     launch_box_clusters(NB, bmincore, bcell, cbox, bstart, inrow_of_slot, ustart, bparent,
@@ -1066,8 +1018,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
                                     &sc[SS_ROWTAB], s);
     launch_label_cores<T>(a, core, bcluster, parent, compmin, nullptr, cmin, cmax, labels,
                           &dstats[1], s, &sc[SS_ROWTAB]);
-    launch_border<T, D>(a, core, bcluster, rootslot, cmin, cmax, labels, &dstats[2], nullptr,
-                        noise_stripes, s);
+    launch_border<T, D>(a, core, bcluster, rootslot, cmin, cmax, labels, &dstats[2], nullptr, s);
 }
 
 // Ends a stream capture if the body throws halfway.
@@ -1098,7 +1049,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     JobParams<T>* jobs_dev = A.take_n<JobParams<T>>(static_cast<size_t>(njobs));
     int32_t* bfirst_dev = A.take_n<int32_t>(static_cast<size_t>(njobs) + 1);
     uint32_t* sc = A.take_n<uint32_t>(SS_WORDS);
-    unsigned long long* dstats = A.take_n<unsigned long long>(16 + kNoiseStripes);
+    unsigned long long* dstats = A.take_n<unsigned long long>(16);
 
     // host-made part of the job table: row ranges, eps2, minPts, reciprocals
     HostArray<JobParams<T>, 1> hj(static_cast<size_t>(njobs));

@@ -38,6 +38,7 @@
 
 #include "boxes.hpp"
 #include "cellkey.hpp"
+#include "collect.hpp"
 #include "common.hpp"
 #include "dbscan.hpp"
 #include "grid.hpp"
@@ -78,42 +79,19 @@ __device__ __forceinline__ bool fetch_chunk(const int2* __restrict__ items, int3
     return true;
 }
 
-// Chunk of work item wid (no bounds check).
-__device__ __forceinline__ void chunk_at(const int2* __restrict__ items, int32_t wid,
-                                         const int32_t* __restrict__ ustart,
-                                         const uint32_t* __restrict__ roff, Chunk& c) {
-    const int2 it = items[wid];
-    c.u = uniform(it.x);
-    c.first = uniform(it.y);
-    c.end = uniform(ustart[c.u + 1]);
-    c.r0 = uniform(static_cast<int32_t>(roff[c.u]));
-    c.r1 = uniform(static_cast<int32_t>(roff[c.u + 1]));
-}
+// Lanes per row of the row-group kernels, and the rows of a box up to which
+// the box's lane walks it by itself.
+template <int D>
+constexpr int kGroup = D <= 3 ? 8 : 16;
+constexpr int kLaneRows = 16;
 
-// Number of work items: host-known, or written by an earlier kernel.
-__device__ __forceinline__ int32_t item_count(int32_t host, const unsigned int* dev) {
-    return dev ? uniform(static_cast<int32_t>(*dev)) : host;
-}
-
-// The work item of the calling wave: one wave per item where the grid covers
-// the host-known count or its bound (waves past a device-written count
-// exit); the waves of a smaller grid walk items wid, wid + wave_stride(), ...
+// Persistent grids: wave w of them takes items w, w + wave_stride(), ...
 __device__ __forceinline__ int32_t first_wave() {
     return uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
                    static_cast<int32_t>(threadIdx.x >> 6));
 }
 __device__ __forceinline__ int32_t wave_stride() {
     return static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-}
-
-// The boxes of chunk c's neighbour rows (for_each_row_box).
-template <typename T, int D, typename Fn>
-__device__ __forceinline__ void for_each_nbr_box(const DbscanArgs<T>& a, const Chunk& c,
-                                                 const int32_t* __restrict__ tag, Fn&& fn,
-                                                 bool own_cell_first = false) {
-    for_each_row_box<T, D>(c.r0, c.r1, uniform(a.rcenter[c.u]), a.rcells, a.cbox, a.bstart,
-                           static_cast<const OrdKey<T>*>(a.bbox), tag, fn, INT_MAX,
-                           own_cell_first ? uniform(a.cbox[c.u]) : -1);
 }
 
 __device__ __forceinline__ int32_t wave_min(int32_t v) {
@@ -171,251 +149,105 @@ __global__ __launch_bounds__(kThreads) void k_core(const DbscanArgs<T> a, uint8_
     (void)ncore;
 }
 
-// Box-mode core counts.  For every neighbour box: lanes whose row is farther
-// than eps from the box's bounding box skip it, lanes whose row is within
-// eps of the box's farthest corner count all its rows, the other lanes
-// test the box's rows one by one.  Exactness: with d the exact distance
-// and gmin2 <= d^2 <= gmax2, the reference's float expression is within a
-// few ulps of d^2, so gmin2 > EPS2 (1 + 1e-5) (+ 1e-30) rules every member
-// out and gmax2 <= EPS2 (1 - 1e-5) rules every member in.
-// kCount: also add the row-row distance tests executed to *ntests (an
-// instrumented variant: the count is one more live value in a kernel that
-// has no VGPR to spare at 8 waves per SIMD)
+// Box-mode core counts: the rows listed in a.crows (rows outside the full
+// boxes, in cells that can hold cores), G lanes per row, a neighbour box per
+// lane.  A box farther than eps from the row (bounding box) is skipped, one
+// within eps of its farthest corner counts whole, the others are tested row
+// by row: small ones by their lane, larger ones by the whole wave with the
+// candidates on the lanes.  Exactness: with d the exact distance and gmin2
+// <= d^2 <= gmax2, the reference's float expression is within a few ulps of
+// d^2, so gmin2 > EPS2 (1 + 1e-5) (+ 1e-30) rules every member out and
+// gmax2 <= EPS2 (1 - 1e-5) rules every member in.
+//
+// Bound by latency (list -> cell -> box ranges -> boxes) and VALU issue of
+// the box tests.  kCount: also add the row-row distance tests executed to
+// *ntests (the instrumented variant).
 template <typename T, int D, bool kCount = false>
-__device__ __forceinline__ void core_boxes_item(const DbscanArgs<T>& a, uint8_t* __restrict__ core,
-                                                unsigned long long* __restrict__ ntests,
-                                                int32_t wid) {
-    Chunk c;
-    chunk_at(a.ditems, wid, a.ustart, a.roff, c);
-    uint32_t tests = 0;  // row-row distance tests executed (lanes x rows visited)
-    // the first group's neighbour boxes are loaded ahead, beside the rows
-    // and their boxes (the chunk was selected because a row needs counting)
-    const int32_t center = uniform(a.rcenter[c.u]);
-    const int32_t own_box = uniform(a.cbox[c.u]);
-    RowBoxes pre;
-    row_boxes(c.r0, c.r1, center, 0, a.rcells, a.cbox, INT_MAX, pre.rb0, pre.rcnt);
-    const JobParams<T>& jp = a.jobs[uniform(a.job_of_cell[c.u])];
-    const T eps2 = jp.eps2;
-    const uint32_t min_pts = jp.min_pts;
-    const double gap2_max = jp.gap2_max;
-    const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-    const int32_t p = c.first + lane_id();
-    const bool valid = p < c.end;
-    T pc[D];
-    load_row<T, D>(a.soa, a.ld, valid ? p : c.first, pc);
-    uint32_t cnt = 0;
-    // rows of a tight box with >= minPts rows are core without counting
-    const int32_t bp = valid ? a.box_of_slot[p] : -1 - lane_id();
-    const bool full = valid && (a.btight[bp] & 2);
-    if (full) cnt = min_pts;
-    bool need = valid && cnt < min_pts;
-    if (__any(need)) {
-        // the group's boxes are first classified against the bounding box of
-        // the rows still counting, one box per lane: a box farther than eps
-        // from all of them is skipped, one within eps of all of them counts
-        // whole for every row (both exactly as the per-row tests below would
-        // decide, box_box bounding them monotonically); only the others are
-        // walked box by box
-        double clo[D], chi[D];
-        rows_bbox<T, D>(pc, need, clo, chi);
-        for_each_row_box_group<T, D>(
-            c.r0, c.r1, center, a.rcells, a.cbox, a.bstart,
-            static_cast<const OrdKey<T>*>(a.bbox), nullptr,
-            [&](int32_t nk, int32_t bl, const double* lol, const double* hil, int32_t q0l,
-                int32_t q1l, int32_t) {
-                double cmin2, cmax2;
-                box_box<D>(clo, chi, lol, hil, cmin2, cmax2);
-                const bool mine = lane_id() < nk;
-                const bool all_in = mine && cmax2 <= full2;
-                const bool some = mine && !all_in && cmin2 <= gap2_max;
-                uint32_t add = all_in ? static_cast<uint32_t>(q1l - q0l) : 0u;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) add += __shfl_xor(add, o, 64);
-                if (need) cnt += add;
-                need = valid && cnt < min_pts;
-                const uint64_t somem = ballot(some);
-                const uint64_t needm = ballot(need);
-                if (D <= 4 && __popcll(needm) < __popcll(somem)) {
-                    // fewer rows than boxes to decide: row by row, every
-                    // box on its lane at once (the same point-box test as
-                    // box by box below); the boxes within eps of a row's
-                    // farthest corner count whole, the others that are
-                    // near it are marked for the row and tested row by row
-                    uint64_t part_rows = 0;  // on a box's lane: rows it is partial for
-                    for (uint64_t rows = needm; rows != 0; rows &= rows - 1) {
-                        const int r = static_cast<int>(__builtin_ctzll(rows));
-                        double v[D];
-#pragma unroll
-                        for (int e = 0; e < D; ++e) v[e] = bcast(static_cast<double>(pc[e]), r);
-                        double gmin2, gmax2;
-                        point_box_dd<D>(lol, hil, v, gmin2, gmax2);
-                        const bool near = some && gmin2 <= gap2_max;
-                        const bool whole = near && gmax2 <= full2;
-                        uint32_t w = whole ? static_cast<uint32_t>(q1l - q0l) : 0u;
-#pragma unroll
-                        for (int o = 32; o > 0; o >>= 1) w += __shfl_xor(w, o, 64);
-                        if (lane_id() == r) cnt += w;
-                        if (near && !whole) part_rows |= uint64_t{1} << r;
-                    }
-                    need = valid && cnt < min_pts;
-                    for (uint64_t todo = ballot(part_rows != 0); todo != 0 && __any(need);
-                         todo &= todo - 1) {
-                        const int j = static_cast<int>(__builtin_ctzll(todo));
-                        const bool part = need && ((bcast64(part_rows, j) >> lane_id()) & 1);
-                        if (__any(part)) {
-                            const uint32_t lanes = static_cast<uint32_t>(__popcll(ballot(part)));
-                            auto body = [&](int32_t, const T* qc, uint8_t, int32_t) {
-                                cnt += (part && within<D>(pc, qc, eps2)) ? 1u : 0u;
-                                if constexpr (kCount) tests += lanes;
-                            };
-                            auto stop = [&] {
-                                return static_cast<bool>(__all(!part || cnt >= min_pts));
-                            };
-                            visit_range<T, D>(a.soa, a.ld, nullptr, nullptr, bcast(q0l, j),
-                                              bcast(q1l, j), body, stop);
-                        }
-                        need = valid && cnt < min_pts;
-                    }
-                    return !__any(need);
-                }
-                for (uint64_t todo = somem; todo != 0 && __any(need); todo &= todo - 1) {
-                    const int j = static_cast<int>(__builtin_ctzll(todo));
-                    double lo[D], hi[D];
-#pragma unroll
-                    for (int e = 0; e < D; ++e) {
-                        lo[e] = bcast(lol[e], j);
-                        hi[e] = bcast(hil[e], j);
-                    }
-                    const int32_t q0 = bcast(q0l, j), q1 = bcast(q1l, j);
-                    double gmin2, gmax2;
-                    point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
-                    const bool near = need && gmin2 <= gap2_max;
-                    if (!__any(near)) continue;
-                    const bool whole = near && gmax2 <= full2;
-                    if (whole) cnt += static_cast<uint32_t>(q1 - q0);
-                    const bool part = near && !whole;
-                    if (__any(part)) {
-                        const uint32_t lanes = static_cast<uint32_t>(__popcll(ballot(part)));
-                        auto body = [&](int32_t, const T* qc, uint8_t, int32_t) {
-                            cnt += (part && within<D>(pc, qc, eps2)) ? 1u : 0u;
-                            if constexpr (kCount) tests += lanes;
-                        };
-                        auto stop = [&] { return static_cast<bool>(__all(!part || cnt >= min_pts)); };
-                        visit_range<T, D>(a.soa, a.ld, nullptr, nullptr, q0, q1, body, stop);
-                    }
-                    need = valid && cnt < min_pts;
-                }
-                return !__any(need);
-            },
-            INT_MAX, own_box, &pre);
-    }
-    const bool is_core = valid && cnt >= min_pts;
-    if (valid) core[p] = is_core ? 1 : 0;
-    if constexpr (kCount)
-        if (tests != 0 && lane_id() == 0) atomicAdd(ntests, static_cast<unsigned long long>(tests));
-    if (a.bmincore) {
-        // smallest core input row per box.  A box holds its rows in input
-        // order, and every row of a tight box with >= minPts rows is core:
-        // its value is its first slot's input row, stored by that lane (no
-        // atomics on one address from every chunk of a large box).  Other
-        // boxes: one inside this chunk is stored by its first lane, one that
-        // extends past it is merged atomically.
-        const uint32_t row = valid ? a.inrow[p] : 0u;
-        if (full && a.bstart[bp] == p) a.bmincore[bp] = static_cast<int32_t>(row);
-        const int32_t m =
-            run_suffix_min<int32_t>(is_core && !full ? static_cast<int32_t>(row) : INT_MAX, bp);
-        const bool first = run_head(bp);  // every lane takes part in the shuffles
-        if (valid && first && m != INT_MAX) {
-            if (a.bstart[bp] >= c.first && a.bstart[bp + 1] <= c.first + kWave)
-                a.bmincore[bp] = m;
-            else
-                atomicMin(&a.bmincore[bp], m);
-        }
-    }
-}
-
-// One wave per work item.
-template <typename T, int D, bool kCount = false>
-__global__ __launch_bounds__(kThreads, 8) void k_core_boxes(const DbscanArgs<T> a,
-                                                         uint8_t* __restrict__ core,
-                                                         unsigned long long* __restrict__ ntests) {
-    const int32_t wid = first_wave();
-    if (wid < item_count(a.nditems, a.nditems_dev))
-        core_boxes_item<T, D, kCount>(a, core, ntests, wid);
-}
-
-// The waves walk items wid0, wid0 + 1, ...: the items of a device-written
-// count beyond what a one-wave-per-item grid covered.  The walk keeps the
-// arguments live across items, more than the 64 VGPRs of 8 waves per SIMD
-// hold without spilling, so it runs at 4.
-template <typename T, int D, bool kCount = false>
-__global__ __launch_bounds__(kThreads, 4) void k_core_boxes_walk(
-    const DbscanArgs<T> a, uint8_t* __restrict__ core, unsigned long long* __restrict__ ntests,
-    int32_t wid0) {
-    const int32_t nwork = item_count(a.nditems, a.nditems_dev);
-    for (int32_t wid = wid0 + first_wave(); wid < nwork; wid += wave_stride())
-        core_boxes_item<T, D, kCount>(a, core, ntests, wid);
-}
-
-// Thread-per-row core counts for the rows of sparse cells (a.sitems): the
-// same box-by-box count as k_core_boxes, with every thread walking its own
-// row's neighbourhood.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_core_sparse(const DbscanArgs<T> a,
-                                                          uint8_t* __restrict__ core,
-                                                          unsigned long long* __restrict__ ncore) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    bool is_core = false;
-    if (i < item_count(a.nsitems, a.nsitems_dev)) {
-        const int2 it = a.sitems[i];
+__global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
+                                                        uint8_t* __restrict__ core,
+                                                        unsigned long long* __restrict__ ntests) {
+    constexpr int G = kGroup<D>;
+    constexpr int kPer = 64 / G;  // rows of a wave
+    const int32_t nrows = uniform(static_cast<int32_t>(*a.ncrows_dev));
+    const int gl = lane_id() & (G - 1);
+    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    unsigned long long tests = 0;
+    for (int32_t base = first_wave() * kPer; base < nrows; base += wave_stride() * kPer) {
+        const int32_t i = base + lane_id() / G;
+        const bool on = i < nrows;
+        const int2 it = a.crows[on ? i : nrows - 1];
         const int32_t p = it.x, u = it.y;
-        const int32_t b = a.box_of_slot[p];
-        {
-            const JobParams<T>& jp = a.jobs[a.job_of_cell[u]];
-            const uint32_t min_pts = jp.min_pts;
-            uint32_t cnt = (a.btight[b] & 2) ? min_pts : 0u;
-            if (cnt < min_pts) {
-                const T eps2 = jp.eps2;
-                const double gap2_max = jp.gap2_max;
-                const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-                const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
-                T pc[D];
-                load_row<T, D>(a.soa, a.ld, p, pc);
-                // the own row first, from the own cell's first box on
-                const int32_t r0 = static_cast<int32_t>(a.roff[u]);
-                const int32_t nr = static_cast<int32_t>(a.roff[u + 1]) - r0;
-                const int32_t center = a.rcenter[u];
-                const int32_t own = a.cbox[u];
-                for (int32_t k = -1; k < nr && cnt < min_pts; ++k) {
-                    const int32_t r = k < 0 ? center : r0 + k;
-                    if (k >= 0 && r == center) continue;
-                    const int2 cs = a.rcells[r];
-                    const int32_t e0 = a.cbox[cs.x], len = a.cbox[cs.y] - e0;
-                    const int32_t rot = (k < 0 && own > e0 && own < e0 + len) ? own - e0 : 0;
-                    for (int32_t t = 0; t < len && cnt < min_pts; ++t) {
-                        const int32_t b2 = e0 + (t + rot < len ? t + rot : t + rot - len);
-                        double gmin2, gmax2;
-                        point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
-                        if (gmin2 > gap2_max) continue;
-                        const int32_t q0 = a.bstart[b2], q1 = a.bstart[b2 + 1];
-                        if (gmax2 <= full2) {
-                            cnt += static_cast<uint32_t>(q1 - q0);
-                            continue;
-                        }
-                        for (int32_t q = q0; q < q1 && cnt < min_pts; ++q) {
-                            T qc[D];
-                            load_row<T, D>(a.soa, a.ld, q, qc);
-                            cnt += within<D>(pc, qc, eps2) ? 1u : 0u;
-                        }
+        T pc[D];
+        load_row<T, D>(a.soa, a.ld, p, pc);
+        const int32_t r0 = static_cast<int32_t>(a.roff[u]);
+        const int32_t r1 = static_cast<int32_t>(a.roff[u + 1]);
+        const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
+        const T eps2 = jp.eps2;
+        const uint32_t min_pts = jp.min_pts;
+        const double gap2_max = jp.gap2_max;
+        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
+        uint32_t cnt = 0;
+        bool need = on && min_pts > 0;
+        group_boxes<G>(need, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, INT_MAX,
+                       [&](bool valid, int32_t b) {
+            int32_t q0 = 0, q1 = 0;
+            bool part = false;
+            uint32_t w = 0;
+            if (valid) {
+                double gmin2, gmax2;
+                point_box<T, D>(bbox, b, pc, gmin2, gmax2);
+                q0 = a.bstart[b];
+                q1 = a.bstart[b + 1];
+                const bool near = gmin2 <= gap2_max;
+                const bool whole = near && gmax2 <= full2;
+                if (whole) w = static_cast<uint32_t>(q1 - q0);
+                part = near && !whole;
+            }
+            cnt += group_sum<G>(w);
+            need = need && cnt < min_pts;
+            if (__any(need && part)) {
+                const bool lane_walk = q1 - q0 <= kLaneRows;
+                uint32_t c = 0;
+                if (need && part && lane_walk) {
+                    for (int32_t q = q0; q < q1; ++q) {
+                        T qc[D];
+                        load_row<T, D>(a.soa, a.ld, q, qc);
+                        c += within<D>(pc, qc, eps2) ? 1u : 0u;
                     }
+                    if constexpr (kCount) tests += static_cast<unsigned long long>(q1 - q0);
+                }
+                cnt += group_sum<G>(c);
+                need = need && cnt < min_pts;
+                for (uint64_t todo = ballot(need && part && !lane_walk); todo != 0;
+                     todo &= todo - 1) {
+                    const int j = static_cast<int>(__builtin_ctzll(todo));
+                    if (!((ballot(need) >> j) & 1)) continue;  // an earlier box was enough
+                    T pr[D];
+#pragma unroll
+                    for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], j);
+                    const uint32_t left =
+                        static_cast<uint32_t>(bcast(static_cast<int32_t>(min_pts - cnt), j));
+                    uint32_t visited = 0;
+                    const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, bcast(q0, j),
+                                                          bcast(q1, j), pr, bcast(eps2, j), left,
+                                                          visited);
+                    if (lane_id() / G == j / G) {
+                        cnt += got;
+                        need = need && cnt < min_pts;
+                    }
+                    if constexpr (kCount)
+                        if (lane_id() == 0) tests += visited;
                 }
             }
-            is_core = cnt >= min_pts;
-            core[p] = is_core ? 1 : 0;
-            if (is_core && a.bmincore) atomicMin(&a.bmincore[b], static_cast<int32_t>(a.inrow[p]));
+            return !need;
+        });
+        // (launch_core_rows_init wrote 0 for every listed row)
+        if (on && gl == 0 && cnt >= min_pts) {
+            core[p] = 1;
+            atomicMin(&a.bmincore[a.box_of_slot[p]], static_cast<int32_t>(a.inrow[p]));
         }
     }
-    (void)ncore;
+    if constexpr (kCount) block_add<kThreads>(tests, ntests);
 }
 
 template <typename T, int D>
@@ -530,10 +362,7 @@ __global__ __launch_bounds__(kThreads) void k_label_cores(
 }
 
 // Box mode: core labels one thread per slot (the cluster of a core is its
-// box's); cmin / cmax are not needed there.
-// 8 waves on each of the 1024 SIMDs
-constexpr unsigned kLabelBlocks = 2048;
-
+// box's); the other rows go to `rows` as (slot, cell) for k_border_rows.
 // skip_full (with *full_ok set): the rows of full boxes (btight bit 2) were
 // labelled in input order (k_label_full_rows) and are skipped here.
 template <typename T>
@@ -543,24 +372,26 @@ __global__ __launch_bounds__(kThreads) void k_label_cores_boxes(
     const int32_t* __restrict__ bcell, const int32_t* __restrict__ bcluster,
     const uint32_t* __restrict__ inrow, int64_t* __restrict__ labels,
     int32_t* __restrict__ rootslot, unsigned long long* __restrict__ ncore, bool one_job,
-    const uint8_t* __restrict__ skip_full, const unsigned int* __restrict__ full_ok) {
+    const uint8_t* __restrict__ skip_full, const unsigned int* __restrict__ full_ok,
+    int2* __restrict__ rows, unsigned int* __restrict__ nrows) {
     if (skip_full && *full_ok == 0) skip_full = nullptr;
-    // grid-stride over at most kLabelBlocks blocks, so that the core count
-    // of the run statistics (folded in here) takes few atomics
-    unsigned long long cores = 0;
-    for (int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; p < n;
-         p += static_cast<int64_t>(gridDim.x) * kThreads) {
-        if (!core[p]) continue;
-        ++cores;  // every core, the row-order ones included
+    unsigned long long cores = 0;  // of the run statistics
+    block_collect(n, rows, nrows, [&](int64_t p, int2& v) {
         const int32_t b = box_of_slot[p];
-        if (skip_full && (skip_full[b] & 2)) continue;
+        if (!core[p]) {
+            v = make_int2(static_cast<int32_t>(p), bcell[b]);
+            return true;
+        }
+        ++cores;  // every core, the row-order ones included
+        if (skip_full && (skip_full[b] & 2)) return false;
         const int32_t r = bcluster[b];
         if (rootslot) rootslot[p] = r;
         // one job starts at row 0
         const int64_t first_pos = one_job ? 0 : jobs[job_of_cell[bcell[b]]].row_begin;
         labels[inrow[p]] = -(static_cast<int64_t>(r) - first_pos + 1);
-    }
-    if (ncore) block_add<kThreads>(cores, ncore);
+        return false;
+    });
+    block_add<kThreads>(cores, ncore);
 }
 
 // Row-order labels of full boxes.  A table indexed by cell key (the sort's
@@ -728,191 +559,111 @@ __global__ __launch_bounds__(kThreads) void k_border(const DbscanArgs<T> a,
 // Box-mode border labels: every core of a box lies in the box's cluster
 // (bcluster), so a non-core row only needs, per neighbour box whose cluster
 // could change its answer, one within-eps core of that box (or a box within
-// eps as a whole).  A box is skipped for a lane when its cluster is the
-// lane's current one, or larger while the lane has not yet met two
-// clusters; the smallest adjacent cluster and the two-cluster flag come out
-// exact.
-// Noise rows of the wave, added to one of kNoiseStripes counters (picked by
-// the wave's index): one counter per wave would serialise the atomics of
-// all waves with noise on one address.  k_sum_stripes adds them up.
-__device__ __forceinline__ void count_noise_rows(bool is_noise, unsigned long long* noise) {
-    if (!noise) return;
-    const uint64_t nz = ballot(is_noise);
-    if (lane_id() == 0 && nz) {
-        const uint32_t w = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-        atomicAdd(&noise[w & (kNoiseStripes - 1)], static_cast<unsigned long long>(__popcll(nz)));
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void k_sum_stripes(const unsigned long long* __restrict__ v,
-                                                          unsigned long long* __restrict__ out) {
-    unsigned long long t = 0;
-    for (int i = threadIdx.x; i < kNoiseStripes; i += kThreads) t += v[i];
-    block_add<kThreads>(t, out);
-}
-
+// eps as a whole).  G lanes per listed row, a box per lane, as in
+// k_core_rows; a box is skipped when its cluster is the row's current one, or
+// larger once two clusters were met; the smallest adjacent cluster and the
+// two-cluster flag come out exact.  stats[0] += noise rows, stats[1] += rows
+// next to two or more clusters.
 template <typename T, int D>
-__device__ __forceinline__ void border_boxes_item(
-    const DbscanArgs<T>& a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
-    const uint32_t* __restrict__ order, int64_t* __restrict__ labels,
-    unsigned long long* __restrict__ stats, int2* __restrict__ amb_list,
-    unsigned long long* __restrict__ noise, int32_t wid) {
-    Chunk c;
-    chunk_at(a.ditems, wid, a.ustart, a.roff, c);
-    const JobParams<T>& jp = a.jobs[uniform(a.job_of_cell[c.u])];
-    const T eps2 = jp.eps2;
-    const double gap2_max = jp.gap2_max;
-    const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-    const int64_t first_pos = jp.row_begin;
-    const int32_t p = c.first + lane_id();
-    const bool valid = p < c.end;
-    const bool active = valid && !core[p];
-    if (!__any(active)) return;
-    T pc[D];
-    load_row<T, D>(a.soa, a.ld, valid ? p : c.first, pc);
-    int32_t best = INT_MAX;
-    bool amb = false;
-    for_each_nbr_box<T, D>(a, c, bcluster, [&](int32_t, const double* lo, const double* hi,
-                                               int32_t q0, int32_t q1, int32_t cl) {
-        if (cl < 0) return false;  // no cores
-        const bool want = active && cl != best && (cl < best || !amb);
-        if (!__any(want)) return false;
-        double gmin2, gmax2;
-        point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
-        const bool near = want && gmin2 <= gap2_max;
-        if (!__any(near)) return false;
-        bool hit = near && gmax2 <= full2;
-        const bool part = near && !hit;
-        if (__any(part)) {
-            auto body = [&](int32_t, const T* qc, uint8_t cq, int32_t) {
-                if (part && !hit && cq && within<D>(pc, qc, eps2)) hit = true;
-            };
-            auto stop = [&] { return static_cast<bool>(__all(!part || hit)); };
-            visit_range<T, D>(a.soa, a.ld, core, nullptr, q0, q1, body, stop);
-        }
-        if (hit) {
-            if (best != INT_MAX) amb = true;
-            best = min(best, cl);
-        }
-        return false;
-    }, true);
-    if (active) labels[order[p]] = best == INT_MAX ? 0 : static_cast<int64_t>(best) - first_pos + 1;
-    count_noise_rows(active && best == INT_MAX, noise);
-    const bool is_amb = active && amb;
-    const uint64_t amb_mask = ballot(is_amb);
-    const unsigned long long namb = __popcll(amb_mask);
-    unsigned long long base = 0;
-    if (lane_id() == 0) {
-        if (namb) base = atomicAdd(&stats[1], namb);
-    }
-    if (amb_list && namb) {
-        base = __shfl(base, 0, 64);
-        if (is_amb)
-            amb_list[base + static_cast<unsigned long long>(__popcll(amb_mask & lanemask_lt()))] =
-                make_int2(p, c.u);
-    }
-}
-
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads, 8) void k_border_boxes(
+__global__ __launch_bounds__(kThreads) void k_border_rows(
     const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
-    const uint32_t* __restrict__ order, int64_t* __restrict__ labels,
-    unsigned long long* __restrict__ stats, int2* __restrict__ amb_list,
-    unsigned long long* __restrict__ noise) {
-    const int32_t wid = first_wave();
-    if (wid < item_count(a.nditems, a.nditems_dev))
-        border_boxes_item<T, D>(a, core, bcluster, order, labels, stats, amb_list, noise, wid);
-}
-
-// k_border_boxes with the waves walking items wid0, ... (as k_core_boxes_walk).
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads, 4) void k_border_boxes_walk(
-    const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
-    const uint32_t* __restrict__ order, int64_t* __restrict__ labels,
-    unsigned long long* __restrict__ stats, int2* __restrict__ amb_list,
-    unsigned long long* __restrict__ noise, int32_t wid0) {
-    const int32_t nwork = item_count(a.nditems, a.nditems_dev);
-    for (int32_t wid = wid0 + first_wave(); wid < nwork; wid += wave_stride())
-        border_boxes_item<T, D>(a, core, bcluster, order, labels, stats, amb_list, noise, wid);
-}
-
-// Thread-per-row border labels for the non-core rows of sparse cells
-// (a.sitems); same box-by-box search as k_border_boxes.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_border_sparse(const DbscanArgs<T> a,
-                                                            const uint8_t* __restrict__ core,
-                                                            const int32_t* __restrict__ bcluster,
-                                                            int64_t* __restrict__ labels,
-                                                            unsigned long long* __restrict__ stats,
-                                                            int2* __restrict__ amb_list,
-                                                            unsigned long long* __restrict__ noise) {
-    const int64_t s = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    bool active = false, amb = false;
-    int32_t best = INT_MAX, p = 0, u = 0;
-    if (s < item_count(a.nsitems, a.nsitems_dev)) {
-        const int2 it = a.sitems[s];
-        p = it.x;
-        u = it.y;
-        active = !core[p];
-    }
-    if (active) {
-        const JobParams<T>& jp = a.jobs[a.job_of_cell[u]];
+    const int2* __restrict__ rows, const unsigned int* __restrict__ nrows_dev,
+    int64_t* __restrict__ labels, unsigned long long* __restrict__ stats,
+    int2* __restrict__ amb_list) {
+    constexpr int G = kGroup<D>;
+    constexpr int kPer = 64 / G;
+    const int32_t nrows = uniform(static_cast<int32_t>(*nrows_dev));
+    const int gl = lane_id() & (G - 1);
+    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    unsigned long long noise = 0;
+    for (int32_t base = first_wave() * kPer; base < nrows; base += wave_stride() * kPer) {
+        const int32_t i = base + lane_id() / G;
+        const bool on = i < nrows;
+        const int2 it = rows[on ? i : nrows - 1];
+        const int32_t p = it.x, u = it.y;
+        T pc[D];
+        load_row<T, D>(a.soa, a.ld, p, pc);
+        const int32_t r0 = static_cast<int32_t>(a.roff[u]);
+        const int32_t r1 = static_cast<int32_t>(a.roff[u + 1]);
+        const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
         const double gap2_max = jp.gap2_max;
         const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-        const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
-        T pc[D];
-        load_row<T, D>(a.soa, a.ld, p, pc);
-        // the own row first, from the own cell's first box on: the own
-        // cluster is found first and its other boxes are skipped
-        const int32_t r0 = static_cast<int32_t>(a.roff[u]);
-        const int32_t nr = static_cast<int32_t>(a.roff[u + 1]) - r0;
-        const int32_t center = a.rcenter[u];
-        const int32_t own = a.cbox[u];
-        for (int32_t k = -1; k < nr; ++k) {
-            const int32_t r = k < 0 ? center : r0 + k;
-            if (k >= 0 && r == center) continue;
-            const int2 cs = a.rcells[r];
-            const int32_t e0 = a.cbox[cs.x], len = a.cbox[cs.y] - e0;
-            const int32_t rot = (k < 0 && own > e0 && own < e0 + len) ? own - e0 : 0;
-            for (int32_t t = 0; t < len; ++t) {
-                const int32_t b2 = e0 + (t + rot < len ? t + rot : t + rot - len);
-                const int32_t cl = bcluster[b2];
-                if (cl < 0 || cl == best || (cl > best && amb)) continue;
+        int32_t best = INT_MAX, worst = -1;  // smallest, largest adjacent cluster so far
+        group_boxes<G>(on, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, INT_MAX,
+                       [&](bool valid, int32_t b) {
+            const int32_t cl = valid ? bcluster[b] : -1;
+            auto wanted = [&] { return cl >= 0 && cl != best && (cl < best || best == worst); };
+            int32_t q0 = 0, q1 = 0;
+            bool part = false, hit = false;
+            if (wanted()) {
                 double gmin2, gmax2;
-                point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
-                if (gmin2 > gap2_max) continue;
-                bool hit = gmax2 <= full2;
-                const int32_t q1 = a.bstart[b2 + 1];
-                for (int32_t q = a.bstart[b2]; q < q1 && !hit; ++q) {
-                    if (!core[q]) continue;
-                    T qc[D];
-                    load_row<T, D>(a.soa, a.ld, q, qc);
-                    hit = within<D>(pc, qc, eps2);
+                point_box<T, D>(bbox, b, pc, gmin2, gmax2);
+                q0 = a.bstart[b];
+                q1 = a.bstart[b + 1];
+                const bool near = gmin2 <= gap2_max;
+                hit = near && gmax2 <= full2;
+                part = near && !hit;
+            }
+            if (__any(hit)) {
+                best = min(best, group_min<G>(hit ? cl : INT_MAX));
+                worst = max(worst, group_max<G>(hit ? cl : -1));
+            }
+            const bool lane_walk = q1 - q0 <= kLaneRows;
+            if (__any(part)) {
+                bool h = false;
+                if (part && lane_walk && wanted()) {
+                    for (int32_t q = q0; q < q1 && !h; ++q) {
+                        if (!core[q]) continue;
+                        T qc[D];
+                        load_row<T, D>(a.soa, a.ld, q, qc);
+                        h = within<D>(pc, qc, eps2);
+                    }
                 }
-                if (hit) {
-                    if (best != INT_MAX) amb = true;
-                    best = min(best, cl);
+                if (__any(h)) {
+                    best = min(best, group_min<G>(h ? cl : INT_MAX));
+                    worst = max(worst, group_max<G>(h ? cl : -1));
+                }
+                for (uint64_t todo = ballot(part && !lane_walk && wanted()); todo != 0;
+                     todo &= todo - 1) {
+                    const int j = static_cast<int>(__builtin_ctzll(todo));
+                    if (!((ballot(wanted()) >> j) & 1)) continue;
+                    T pr[D];
+#pragma unroll
+                    for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], j);
+                    uint32_t visited = 0;
+                    if (wide_count<T, D>(a.soa, a.ld, core, bcast(q0, j), bcast(q1, j), pr,
+                                         bcast(eps2, j), 1u, visited) != 0) {
+                        const int32_t c = bcast(cl, j);
+                        if (lane_id() / G == j / G) {
+                            best = min(best, c);
+                            worst = max(worst, c);
+                        }
+                    }
                 }
             }
+            return false;
+        });
+        const bool lead = on && gl == 0;
+        if (lead) {
+            labels[a.inrow[p]] =
+                best == INT_MAX ? 0 : static_cast<int64_t>(best) - jp.row_begin + 1;
+            noise += best == INT_MAX ? 1 : 0;
         }
-        labels[a.inrow[p]] =
-            best == INT_MAX ? 0 : static_cast<int64_t>(best) - jp.row_begin + 1;
+        const bool is_amb = lead && best != INT_MAX && best != worst;
+        const uint64_t amb_mask = ballot(is_amb);
+        if (amb_mask == 0) continue;
+        unsigned long long at = 0;
+        if (lane_id() == 0)
+            at = atomicAdd(&stats[1], static_cast<unsigned long long>(__popcll(amb_mask)));
+        if (amb_list) {
+            at = __shfl(at, 0, 64);
+            if (is_amb)
+                amb_list[at + static_cast<unsigned long long>(__popcll(amb_mask & lanemask_lt()))] =
+                    make_int2(p, u);
+        }
     }
-    count_noise_rows(active && best == INT_MAX, noise);
-    const bool is_amb = active && amb;
-    const uint64_t amb_mask = ballot(is_amb);
-    const unsigned long long namb = __popcll(amb_mask);
-    unsigned long long base = 0;
-    if (lane_id() == 0) {
-        if (namb) base = atomicAdd(&stats[1], namb);
-    }
-    if (amb_list && namb) {
-        base = __shfl(base, 0, 64);
-        if (is_amb)
-            amb_list[base + static_cast<unsigned long long>(__popcll(amb_mask & lanemask_lt()))] =
-                make_int2(p, u);
-    }
+    block_add<kThreads>(noise, &stats[0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1088,31 +839,18 @@ __global__ __launch_bounds__(kThreads) void k_fill2(int32_t* __restrict__ a, int
 
 inline unsigned blocks_for(int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
 
-// Waves for the chunk items of the core and border kernels.  A host-known
-// count gets one wave per item.  A count that an earlier kernel wrote (the
-// host holds a bound, n + n / 64 for chunks) gets one wave per item up to a
-// likely count, n / 8 + n / 64 (cells of 8 rows on average; every wave past
-// the count exits at once, and each costs a dispatch), and a small walking
-// grid for the items beyond it, which exits at once when there are none.
-constexpr int64_t kMaxItemWaves = int64_t{1} << 24;
-constexpr int64_t kTailWaves = 16384;
-struct ItemGrid {
-    int64_t waves = 0;  // one-wave-per-item grid: items [0, waves)
-    bool tail = false;  // a walking grid for items [waves, count)
-};
-inline ItemGrid item_grid(int64_t bound, bool device_count, int64_t n) {
-    ItemGrid g;
-    const int64_t likely = device_count ? n / 8 + n / 64 + 64 : bound;
-    g.waves = std::min(bound, std::min(likely, kMaxItemWaves));
-    g.tail = bound > g.waves;
-    return g;
+// Blocks of a persistent grid of the row-group kernels over at most n rows:
+// 8 blocks on each of the 256 CUs.
+template <int D>
+inline unsigned row_blocks(int64_t n) {
+    return static_cast<unsigned>(
+        std::min<int64_t>((n * kGroup<D> + kThreads - 1) / kThreads, 2048));
 }
-
 
 }  // namespace
 
 // *out += number of nonzero flags among f[0, n)
-void count_flags(const uint8_t* f, int64_t n, unsigned long long* out, hipStream_t s) {
+static void count_flags(const uint8_t* f, int64_t n, unsigned long long* out, hipStream_t s) {
     if (n <= 0) return;
     const int64_t want = (n + kThreads - 1) / kThreads;
     const unsigned grid = static_cast<unsigned>(want < 2048 ? want : 2048);
@@ -1121,7 +859,7 @@ void count_flags(const uint8_t* f, int64_t n, unsigned long long* out, hipStream
 }
 
 // *out += number of zero labels (noise rows) among labels[0, n)
-void count_noise(const int64_t* labels, int64_t n, unsigned long long* out, hipStream_t s) {
+static void count_noise(const int64_t* labels, int64_t n, unsigned long long* out, hipStream_t s) {
     if (n <= 0) return;
     const int64_t want = (n + kThreads - 1) / kThreads;
     const unsigned grid = static_cast<unsigned>(want < 2048 ? want : 2048);
@@ -1134,58 +872,24 @@ void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntes
                  hipEvent_t count_start) {
     unsigned long long* ncore = nullptr;  // (the other core kernels count nothing)
     if (count_start) HPD_HIP(hipEventRecord(count_start, s));  // (no box pass: all of it)
-    if (a.nitems <= 0) return;
     if constexpr (std::is_floating_point<T>::value) {
         if (a.bbox) {
-            DbscanArgs<T> ac = a;
-            if (!a.sparse_core) {  // the chunks of every cell that can hold cores
-                ac.ditems = a.citems ? a.citems : a.items;
-                ac.nditems = a.citems ? a.ncitems : a.nitems;
-                ac.nditems_dev = a.citems ? a.ncitems_dev : nullptr;
-                ac.nsitems = 0;
-            }
-            if (a.citems && !a.sparse_core && a.citems_need && a.bmincore) {
-                // rows of tight boxes with >= minPts rows are core, every other
-                // row starts non-core (no row of a cell outside citems is
-                // core); only the chunks holding another row are counted
-                launch_core_full(a.n, a.box_of_slot, a.btight, a.bstart, a.inrow, core, a.bmincore,
-                                 s);
-                launch_select_core_chunks(Count{a.ncitems, a.ncitems_dev}, a.citems, a.ustart,
-                                          a.box_of_slot, a.btight, a.citems_need,
-                                          a.ncitems_need_dev, s);
-                ac.ditems = a.citems_need;
-                ac.nditems_dev = a.ncitems_need_dev;
-            } else if (a.citems && !a.sparse_core) {  // rows of the other cells are not core
-                HPD_HIP(hipMemsetAsync(core, 0, static_cast<size_t>(a.n), s));
-            }
-            const ItemGrid g = item_grid(ac.nditems, ac.nditems_dev != nullptr, a.n);
+            // rows of tight boxes with >= minPts rows are core, every other
+            // row starts non-core; the rows that can be core are listed
+            launch_core_init(a.n, a.box_of_slot, a.btight, a.bstart, a.bcell, a.inrow, core,
+                             a.bmincore, a.crows, a.ncrows_dev, s);
             if (count_start) HPD_HIP(hipEventRecord(count_start, s));
-            if (g.waves > 0) {
-                if (ntests)
-                    hipLaunchKernelGGL((k_core_boxes<T, D, true>),
-                                       dim3(blocks_for(g.waves, kWavesPerBlock)), dim3(kThreads), 0,
-                                       s, ac, core, ntests);
-                else
-                    hipLaunchKernelGGL((k_core_boxes<T, D>),
-                                       dim3(blocks_for(g.waves, kWavesPerBlock)), dim3(kThreads), 0,
-                                       s, ac, core, nullptr);
-            }
-            if (g.tail) {
-                if (ntests)
-                    hipLaunchKernelGGL((k_core_boxes_walk<T, D, true>),
-                                       dim3(blocks_for(kTailWaves, kWavesPerBlock)), dim3(kThreads),
-                                       0, s, ac, core, ntests, static_cast<int32_t>(g.waves));
-                else
-                    hipLaunchKernelGGL((k_core_boxes_walk<T, D>),
-                                       dim3(blocks_for(kTailWaves, kWavesPerBlock)), dim3(kThreads),
-                                       0, s, ac, core, nullptr, static_cast<int32_t>(g.waves));
-            }
-            if (ac.nsitems > 0)
-                hipLaunchKernelGGL((k_core_sparse<T, D>), dim3(blocks_for(ac.nsitems, kThreads)),
-                                   dim3(kThreads), 0, s, ac, core, ncore);
+            if (ntests)
+                hipLaunchKernelGGL((k_core_rows<T, D, true>), dim3(row_blocks<D>(a.n)),
+                                   dim3(kThreads), 0, s, a, core, ntests);
+            else
+                hipLaunchKernelGGL((k_core_rows<T, D>), dim3(row_blocks<D>(a.n)), dim3(kThreads), 0,
+                                   s, a, core, nullptr);
+            HPD_HIP(hipGetLastError());
             return;
         }
     }
+    if (a.nitems <= 0) return;
     hipLaunchKernelGGL((k_core<T, D>), dim3(blocks_for(a.nitems, kWavesPerBlock)), dim3(kThreads),
                        0, s, a, core, ncore);
     HPD_HIP(hipGetLastError());
@@ -1235,10 +939,10 @@ void launch_label_cores(const DbscanArgs<T>& a, const uint8_t* core, const int32
                         const unsigned int* full_ok) {
     if (a.n <= 0) return;
     if (bcluster && a.bcell) {
-        const unsigned grid = std::min<unsigned>(blocks_for(a.n, kThreads), kLabelBlocks);
-        hipLaunchKernelGGL(k_label_cores_boxes<T>, dim3(grid), dim3(kThreads), 0, s, a.n, a.jobs,
-                           a.job_of_cell, core, a.box_of_slot, a.bcell, bcluster, a.inrow, labels,
-                           rootslot, ncore, a.njobs == 1, full_ok ? a.btight : nullptr, full_ok);
+        hipLaunchKernelGGL(k_label_cores_boxes<T>, dim3(collect_blocks(a.n)), dim3(kThreads), 0, s,
+                           a.n, a.jobs, a.job_of_cell, core, a.box_of_slot, a.bcell, bcluster,
+                           a.inrow, labels, rootslot, ncore, a.njobs == 1,
+                           full_ok ? a.btight : nullptr, full_ok, a.brows, a.nbrows_dev);
         HPD_HIP(hipGetLastError());
         return;
     }
@@ -1255,31 +959,15 @@ void launch_label_cores(const DbscanArgs<T>& a, const uint8_t* core, const int32
 template <typename T, int D>
 void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* bcluster,
                    const int32_t* rootslot, const int32_t* cmin, const int32_t* cmax,
-                   int64_t* labels, unsigned long long* stats, int2* amb_list,
-                   unsigned long long* noise_stripes, hipStream_t s) {
+                   int64_t* labels, unsigned long long* stats, int2* amb_list, hipStream_t s) {
     if (a.n <= 0) return;
     const unsigned gw = blocks_for(a.nitems, kWavesPerBlock);
     if constexpr (std::is_floating_point<T>::value) {
         if (bcluster && a.bbox) {
-            const ItemGrid g = item_grid(a.nditems, a.nditems_dev != nullptr, a.n);
-            if (g.waves > 0)
-                hipLaunchKernelGGL((k_border_boxes<T, D>), dim3(blocks_for(g.waves, kWavesPerBlock)),
-                                   dim3(kThreads), 0, s, a, core, bcluster, a.inrow, labels, stats,
-                                   amb_list, noise_stripes);
-            if (g.tail)
-                hipLaunchKernelGGL((k_border_boxes_walk<T, D>),
-                                   dim3(blocks_for(kTailWaves, kWavesPerBlock)), dim3(kThreads), 0,
-                                   s, a, core, bcluster, a.inrow, labels, stats, amb_list,
-                                   noise_stripes, static_cast<int32_t>(g.waves));
-            if (a.nsitems > 0)
-                hipLaunchKernelGGL((k_border_sparse<T, D>), dim3(blocks_for(a.nsitems, kThreads)),
-                                   dim3(kThreads), 0, s, a, core, bcluster, labels, stats,
-                                   amb_list, noise_stripes);
-            if (noise_stripes)
-                hipLaunchKernelGGL(k_sum_stripes, dim3(1), dim3(kThreads), 0, s,
-                                   static_cast<const unsigned long long*>(noise_stripes), &stats[0]);
-            else
-                count_noise(labels, a.n, &stats[0], s);
+            hipLaunchKernelGGL((k_border_rows<T, D>), dim3(row_blocks<D>(a.n)), dim3(kThreads), 0,
+                               s, a, core, bcluster, static_cast<const int2*>(a.brows),
+                               static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
+                               amb_list);
             HPD_HIP(hipGetLastError());
             return;
         }
@@ -1326,8 +1014,7 @@ void launch_one_thread_assign(const DbscanArgs<T>& a, const uint8_t* core, const
                                             int32_t*, int32_t*, int32_t*, int32_t*, hipStream_t); \
     template void launch_border<T, D>(const DbscanArgs<T>&, const uint8_t*, const int32_t*,       \
                                       const int32_t*, const int32_t*, const int32_t*, int64_t*,   \
-                                      unsigned long long*, int2*, unsigned long long*,            \
-                                      hipStream_t);                                               \
+                                      unsigned long long*, int2*, hipStream_t);                   \
     template void launch_one_thread_mark<T, D>(const DbscanArgs<T>&, const uint8_t*,              \
                                                const int32_t*, const int2*, int32_t, uint8_t*,    \
                                                int32_t*, hipStream_t);                            \
@@ -1347,14 +1034,29 @@ void launch_one_thread_assign(const DbscanArgs<T>& a, const uint8_t* core, const
     HPD_INST_DBSCAN(T, 7)        \
     HPD_INST_DBSCAN(T, 8)
 
-HPD_FOR_EACH_DTYPE(HPD_INST_DBSCAN_ALL_D)
+// The build compiles this file in parts (HPD_DBSCAN_PART), each a share of
+// the element types, so that they compile in parallel.
+#ifndef HPD_DBSCAN_PART
+#define HPD_DBSCAN_PART 0
+#endif
+#if HPD_DBSCAN_PART == 0
+#define HPD_FOR_EACH_PART_DTYPE(X) X(float)
+#elif HPD_DBSCAN_PART == 1
+#define HPD_FOR_EACH_PART_DTYPE(X) X(double)
+#elif HPD_DBSCAN_PART == 2
+#define HPD_FOR_EACH_PART_DTYPE(X) X(int8_t) X(int16_t) X(int32_t) X(int64_t)
+#else
+#define HPD_FOR_EACH_PART_DTYPE(X) X(uint8_t) X(uint16_t) X(uint32_t) X(uint64_t)
+#endif
+
+HPD_FOR_EACH_PART_DTYPE(HPD_INST_DBSCAN_ALL_D)
 
 #define HPD_INST_LABEL_CORES(T)                                                                \
     template void launch_label_cores<T>(const DbscanArgs<T>&, const uint8_t*, const int32_t*,  \
                                         int32_t*, const int32_t*, int32_t*, int32_t*, int32_t*, \
                                         int64_t*, unsigned long long*, hipStream_t,      \
                                         const unsigned int*);
-HPD_FOR_EACH_DTYPE(HPD_INST_LABEL_CORES)
+HPD_FOR_EACH_PART_DTYPE(HPD_INST_LABEL_CORES)
 
 #define HPD_INST_FULL_ROWS(T, D, K)                                                             \
     template void launch_label_full_rows<T, D, K>(const T*, const DbscanArgs<T>&, int, int,     \
@@ -1377,8 +1079,11 @@ HPD_FOR_EACH_DTYPE(HPD_INST_LABEL_CORES)
     HPD_INST_FULL_ROWS(T, 6, uint64_t)     \
     HPD_INST_FULL_ROWS(T, 7, uint64_t)     \
     HPD_INST_FULL_ROWS(T, 8, uint64_t)
+#if HPD_DBSCAN_PART == 0
 HPD_INST_FULL_ROWS_ALL(float)
+#elif HPD_DBSCAN_PART == 1
 HPD_INST_FULL_ROWS_ALL(double)
+#endif
 
 
 }  // namespace hpd

@@ -37,30 +37,17 @@ struct DbscanArgs {
     const int32_t* bstart = nullptr;
     const int32_t* bcell = nullptr;         // occupied cell of every box
     const void* bbox = nullptr;
-    // box mode: the core count and the border pass take the chunks of dense
-    // cells from ditems (one wave each) and the rows of sparse cells from
-    // sitems, (row, cell) per row (one thread each)
-    const int2* ditems = nullptr;
-    int32_t nditems = 0;
-    const int2* sitems = nullptr;
-    int32_t nsitems = 0;
-    const uint32_t* nsitems_dev = nullptr;  // static pipeline: nsitems in device memory
-    const uint32_t* ncitems_dev = nullptr;  // static pipeline: ncitems in device memory
-    bool sparse_core = false;  // core count split too (else one wave per chunk of every cell)
-    // chunks of the cells with >= minPts candidates: the only cells that can
-    // hold cores (core flags of the others stay 0; null: every chunk)
-    const int2* citems = nullptr;
-    int32_t ncitems = 0;
-    // box mode without the core split: scratch for the chunks of citems
-    // holding a row outside the tight boxes of >= minPts rows (those rows
-    // are core without counting), and a device counter (zeroed) for them
-    int2* citems_need = nullptr;
-    unsigned int* ncitems_need_dev = nullptr;
-    // when not null, the number of work items of ditems is read from here
-    // (nditems is then only the grid's bound)
-    const unsigned int* nditems_dev = nullptr;
+    // box mode: box ranges of the neighbour rows (in place of rcells)
+    const int2* rboxes = nullptr;
+    // box mode: the rows to count (outside the full boxes, in cells that can
+    // hold cores) and the non-core rows of the border pass, as (slot, cell),
+    // with their numbers (device words, zeroed by the caller)
+    int2* crows = nullptr;
+    unsigned int* ncrows_dev = nullptr;
+    int2* brows = nullptr;
+    unsigned int* nbrows_dev = nullptr;
     // box mode: the core count also writes the smallest input row of a core
-    // row per box (pre-filled with INT_MAX; stays INT_MAX without cores)
+    // row per box (INT_MAX without cores)
     int32_t* bmincore = nullptr;
 };
 
@@ -114,15 +101,12 @@ void launch_label_full_rows(const T* pts, const DbscanArgs<T>& a, int sub_k, int
 // Border and noise labels of the non-core rows (in box mode box by box:
 // all cores of a box share its cluster).  stats[0] += noise rows,
 // stats[1] += ambiguous border rows; when amb_list is given it receives
-// (slot, cell) of each ambiguous border row (capacity n).  noise_stripes
-// (kNoiseStripes zeroed counters, or null) lets the box kernels count the
-// noise rows as they label them instead of a pass over the labels.
-constexpr int kNoiseStripes = 1024;
+// (slot, cell) of each ambiguous border row (capacity n).  Box mode takes
+// the rows that launch_label_cores listed in a.brows.
 template <typename T, int D>
 void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* bcluster,
                    const int32_t* rootslot, const int32_t* cmin, const int32_t* cmax,
-                   int64_t* labels, unsigned long long* stats, int2* amb_list,
-                   unsigned long long* noise_stripes, hipStream_t s);
+                   int64_t* labels, unsigned long long* stats, int2* amb_list, hipStream_t s);
 
 // The reference's one-thread border choice for the namb ambiguous rows:
 // mark the touched clusters (involved, indexed by cluster position, zeroed

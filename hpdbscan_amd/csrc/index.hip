@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_count(const K* __restrict
                                                              int32_t njobs,
                                                              int32_t* __restrict__ job_of_cell,
                                                              uint32_t* __restrict__ nranges,
-                                                             uint32_t* __restrict__ core_chunks,
+                                                             uint8_t* __restrict__ cell_core,
                                                              unsigned long long* __restrict__ sumcand,
                                                              unsigned long long* __restrict__ rows_total,
                                                              int2* __restrict__ stash,
@@ -224,9 +224,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_count(const K* __restrict
         count_u = static_cast<uint64_t>(ustart[u + 1] - ustart[u]);
         // the reference queries a row only with >= minPts candidates
         // (hpdbscan.h:74); with fewer, no row of the cell can be core
-        if (core_chunks)
-            core_chunks[u] = cand >= jobs[j].min_pts ? static_cast<uint32_t>((count_u + kWave - 1) / kWave)
-                                                     : 0u;
+        if (cell_core) cell_core[u] = cand >= jobs[j].min_pts ? 1 : 0;
     }
     // *sumcand += Σ over rows of the cell of |candidates| = count_u * cand;
     // *rows_total += the cell's neighbour rows (their 64-bit total is checked
@@ -245,7 +243,8 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_fill(const K* __restrict_
                                                             int2* __restrict__ ranges,
                                                             int2* __restrict__ rcells,
                                                             int32_t* __restrict__ rcenter,
-                                                            const int32_t* __restrict__ ctab) {
+                                                            const int32_t* __restrict__ ctab,
+                                                            const int32_t* __restrict__ cbox) {
     const int32_t m = static_cast<int32_t>(mc.get());
     const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
     if (u >= m) return;
@@ -261,22 +260,20 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_fill(const K* __restrict_
                      if (!ctab) from = ab.y;
                      if (ab.y > ab.x) {
                          if (is_center) center = static_cast<int32_t>(w);
-                         rcells[w] = ab;
-                         ranges[w++] = make_int2(ustart[ab.x], ustart[ab.y]);
+                         if (ranges) ranges[w] = make_int2(ustart[ab.x], ustart[ab.y]);
+                         rcells[w++] = cbox ? make_int2(cbox[ab.x], cbox[ab.y]) : ab;
                      }
                  });
     rcenter[u] = center;
 }
 
-// The fill from the count pass's stash: the same ranges, rcells and rcenter
-// as k_neighbor_rows_fill, without searching again.
+// The fill from the count pass's stash: the same box ranges and rcenter as
+// k_neighbor_rows_fill, without searching again.
 __global__ __launch_bounds__(256) void k_neighbor_rows_copy(const int2* __restrict__ stash,
-                                                            int32_t stash_rows,
-                                                            const int32_t* __restrict__ ustart,
-                                                            int32_t m,
+                                                            int32_t stash_rows, int32_t m,
                                                             const uint32_t* __restrict__ roff,
-                                                            int2* __restrict__ ranges,
-                                                            int2* __restrict__ rcells,
+                                                            const int32_t* __restrict__ cbox,
+                                                            int2* __restrict__ rboxes,
                                                             int32_t* rcenter, bool by_class) {
     const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
     if (u >= m) return;
@@ -285,8 +282,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_copy(const int2* __restri
     if (!by_class) {
         for (uint32_t k = 0; k < cnt; ++k) {
             const int2 ab = mine[k];
-            rcells[w0 + k] = ab;
-            ranges[w0 + k] = make_int2(ustart[ab.x], ustart[ab.y]);
+            rboxes[w0 + k] = make_int2(cbox[ab.x], cbox[ab.y]);
         }
         rcenter[u] = static_cast<int32_t>(w0) + rcenter[u];  // local index from the count pass
         return;
@@ -300,10 +296,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_copy(const int2* __restri
             const int2 e = mine[k];
             const uint32_t x = static_cast<uint32_t>(e.x), y = static_cast<uint32_t>(e.y);
             if (((x >> 31) | ((y >> 31) << 1)) != c) continue;
-            const int2 ab = make_int2(static_cast<int32_t>(x & 0x7fffffffu),
-                                      static_cast<int32_t>(y & 0x7fffffffu));
-            rcells[w] = ab;
-            ranges[w] = make_int2(ustart[ab.x], ustart[ab.y]);
+            rboxes[w] = make_int2(cbox[x & 0x7fffffffu], cbox[y & 0x7fffffffu]);
             ++w;
         }
     }
@@ -315,11 +308,10 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_copy(const int2* __restri
 // their class's place.
 template <int R>
 __global__ __launch_bounds__(256) void k_neighbor_rows_copy_class(const int2* __restrict__ stash,
-                                                                  const int32_t* __restrict__ ustart,
                                                                   int32_t m,
                                                                   const uint32_t* __restrict__ roff,
-                                                                  int2* __restrict__ ranges,
-                                                                  int2* __restrict__ rcells,
+                                                                  const int32_t* __restrict__ cbox,
+                                                                  int2* __restrict__ rboxes,
                                                                   int32_t* __restrict__ rcenter) {
     const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
     if (u >= m) return;
@@ -335,8 +327,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_copy_class(const int2* __
             const int2 v = mine[k];
             const uint32_t x = static_cast<uint32_t>(v.x), y = static_cast<uint32_t>(v.y);
             cls[k] = (x >> 31) | ((y >> 31) << 1);
-            e[k] = make_int2(static_cast<int32_t>(x & 0x7fffffffu),
-                             static_cast<int32_t>(y & 0x7fffffffu));
+            e[k] = make_int2(cbox[x & 0x7fffffffu], cbox[y & 0x7fffffffu]);
             n1 += cls[k] == 1 ? 1u : 0u;
             n2 += cls[k] == 2 ? 1u : 0u;
         }
@@ -347,8 +338,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_copy_class(const int2* __
         if (cls[k] > 3) continue;
         const uint32_t c = cls[k];
         const uint32_t w = c == 0 ? p0++ : c == 1 ? p1++ : c == 2 ? p2++ : p3++;
-        rcells[w] = e[k];
-        ranges[w] = make_int2(ustart[e[k].x], ustart[e[k].y]);
+        rboxes[w] = e[k];
     }
     rcenter[u] = static_cast<int32_t>(w0);  // the own row is the only one of class 0
 }
@@ -382,58 +372,7 @@ __global__ __launch_bounds__(256) void k_expand_chunks(const uint32_t* __restric
     items[w] = make_int2(lo, start[lo] + kWave * (w - static_cast<int32_t>(off[lo])));
 }
 
-// Per cell: 64-row chunks if the cell has more than `sparse_max` rows
-// (dense), else its rows one by one (sparse).
-__global__ __launch_bounds__(256) void k_split_counts(const int32_t* __restrict__ ustart, Count mc,
-                                                      int32_t sparse_max,
-                                                      uint32_t* __restrict__ dcnt,
-                                                      uint32_t* __restrict__ scnt) {
-    const int32_t m = static_cast<int32_t>(mc.get());
-    const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (u >= m) return;
-    const int32_t c = ustart[u + 1] - ustart[u];
-    const bool sparse = c <= sparse_max;
-    dcnt[u] = sparse ? 0u : static_cast<uint32_t>((c + kWave - 1) / kWave);
-    scnt[u] = sparse ? static_cast<uint32_t>(c) : 0u;
-}
-
-__global__ __launch_bounds__(256) void k_split_items(const int32_t* __restrict__ ustart, Count mc,
-                                                     int32_t sparse_max,
-                                                     const uint32_t* __restrict__ doff,
-                                                     const uint32_t* __restrict__ soff,
-                                                     int2* __restrict__ ditems,
-                                                     int2* __restrict__ sitems) {
-    const int32_t m = static_cast<int32_t>(mc.get());
-    const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (u >= m) return;
-    const int32_t s = ustart[u], e = ustart[u + 1];
-    if (e - s <= sparse_max) {
-        uint32_t w = soff[u];
-        for (int32_t p = s; p < e; ++p) sitems[w++] = make_int2(p, u);
-    }
-    (void)doff;
-    (void)ditems;
-}
-
 }  // namespace
-
-void launch_split_counts(const int32_t* ustart, Count m, int32_t sparse_max, uint32_t* dcnt,
-                         uint32_t* scnt, hipStream_t s) {
-    if (m.host <= 0) return;
-    hipLaunchKernelGGL(k_split_counts, dim3(blocks_for(m.host, 256)), dim3(256), 0, s, ustart, m,
-                       sparse_max, dcnt, scnt);
-    HPD_HIP(hipGetLastError());
-}
-
-void launch_split_items(const int32_t* ustart, Count m, int32_t sparse_max, const uint32_t* doff,
-                        const uint32_t* soff, int2* ditems, Count nditems, int2* sitems,
-                        hipStream_t s) {
-    if (m.host <= 0) return;
-    hipLaunchKernelGGL(k_split_items, dim3(blocks_for(m.host, 256)), dim3(256), 0, s, ustart, m,
-                       sparse_max, doff, soff, ditems, sitems);
-    launch_expand_chunks(doff, m, ustart, nditems, ditems, s);
-    HPD_HIP(hipGetLastError());
-}
 
 void launch_expand_chunks(const uint32_t* off, Count ngroups, const int32_t* start, Count total,
                           int2* items, hipStream_t s) {
@@ -459,12 +398,12 @@ void launch_cells(const K* keys, int64_t n, int shift, uint32_t* flags, uint32_t
 template <typename K, typename T>
 void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
                            const JobParams<T>* jobs, int32_t njobs, int32_t* job_of_cell,
-                           uint32_t* nranges, uint32_t* core_chunks, unsigned long long* sumcand,
+                           uint32_t* nranges, uint8_t* cell_core, unsigned long long* sumcand,
                            unsigned long long* rows_total, int2* stash, int32_t stash_rows,
                            int32_t* rcenter, bool by_class, hipStream_t s, const int32_t* ctab) {
     if (m.host <= 0) return;
     hipLaunchKernelGGL((k_neighbor_rows_count<K, T>), dim3(blocks_for(m.host, 256)), dim3(256), 0, s,
-                       ucell, ustart, m, jobs, njobs, job_of_cell, nranges, core_chunks, sumcand,
+                       ucell, ustart, m, jobs, njobs, job_of_cell, nranges, cell_core, sumcand,
                        rows_total, stash, stash_rows, rcenter, by_class, ctab);
     HPD_HIP(hipGetLastError());
 }
@@ -478,19 +417,19 @@ void launch_cell_table(const K* ucell, Count m, int32_t* ctab, uint64_t ids, hip
     HPD_HIP(hipGetLastError());
 }
 
-void launch_neighbor_copy(const int2* stash, int32_t stash_rows, const int32_t* ustart, int32_t m,
-                          const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
-                          bool by_class, hipStream_t s) {
+void launch_neighbor_copy(const int2* stash, int32_t stash_rows, int32_t m, const uint32_t* roff,
+                          const int32_t* cbox, int2* rboxes, int32_t* rcenter, bool by_class,
+                          hipStream_t s) {
     const dim3 grid(blocks_for(m, 256));
     if (by_class && stash_rows == 9)
-        hipLaunchKernelGGL(k_neighbor_rows_copy_class<9>, grid, dim3(256), 0, s, stash, ustart, m,
-                           roff, ranges, rcells, rcenter);
+        hipLaunchKernelGGL(k_neighbor_rows_copy_class<9>, grid, dim3(256), 0, s, stash, m, roff,
+                           cbox, rboxes, rcenter);
     else if (by_class && stash_rows == 27)
-        hipLaunchKernelGGL(k_neighbor_rows_copy_class<27>, grid, dim3(256), 0, s, stash, ustart, m,
-                           roff, ranges, rcells, rcenter);
+        hipLaunchKernelGGL(k_neighbor_rows_copy_class<27>, grid, dim3(256), 0, s, stash, m, roff,
+                           cbox, rboxes, rcenter);
     else
-        hipLaunchKernelGGL(k_neighbor_rows_copy, grid, dim3(256), 0, s, stash, stash_rows, ustart, m,
-                           roff, ranges, rcells, rcenter, by_class);
+        hipLaunchKernelGGL(k_neighbor_rows_copy, grid, dim3(256), 0, s, stash, stash_rows, m, roff,
+                           cbox, rboxes, rcenter, by_class);
     HPD_HIP(hipGetLastError());
 }
 
@@ -498,10 +437,10 @@ template <typename K, typename T>
 void launch_neighbor_fill(const K* ucell, const int32_t* ustart, Count m,
                           const JobParams<T>* jobs, const int32_t* job_of_cell,
                           const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
-                          hipStream_t s, const int32_t* ctab) {
+                          hipStream_t s, const int32_t* ctab, const int32_t* cbox) {
     if (m.host <= 0) return;
     hipLaunchKernelGGL((k_neighbor_rows_fill<K, T>), dim3(blocks_for(m.host, 256)), dim3(256), 0, s,
-                       ucell, ustart, m, jobs, job_of_cell, roff, ranges, rcells, rcenter, ctab);
+                       ucell, ustart, m, jobs, job_of_cell, roff, ranges, rcells, rcenter, ctab, cbox);
     HPD_HIP(hipGetLastError());
 }
 
@@ -527,24 +466,26 @@ HPD_INST_INDEX(uint64_t)
 #define HPD_INST_ROWS(T)                                                                        \
     template void launch_neighbor_count<uint32_t, T>(const uint32_t*, const int32_t*, Count,    \
                                                      const JobParams<T>*, int32_t, int32_t*,    \
-                                                     uint32_t*, uint32_t*, unsigned long long*, \
+                                                     uint32_t*, uint8_t*, unsigned long long*,  \
                                                      unsigned long long*, int2*, int32_t,       \
                                                      int32_t*, bool, hipStream_t,               \
                                                      const int32_t*);                           \
     template void launch_neighbor_count<uint64_t, T>(const uint64_t*, const int32_t*, Count,    \
                                                      const JobParams<T>*, int32_t, int32_t*,    \
-                                                     uint32_t*, uint32_t*, unsigned long long*, \
+                                                     uint32_t*, uint8_t*, unsigned long long*,  \
                                                      unsigned long long*, int2*, int32_t,       \
                                                      int32_t*, bool, hipStream_t,               \
                                                      const int32_t*);                           \
     template void launch_neighbor_fill<uint32_t, T>(const uint32_t*, const int32_t*, Count,     \
                                                     const JobParams<T>*, const int32_t*,        \
                                                     const uint32_t*, int2*, int2*, int32_t*,    \
-                                                    hipStream_t, const int32_t*);               \
+                                                    hipStream_t, const int32_t*,                \
+                                                    const int32_t*);                            \
     template void launch_neighbor_fill<uint64_t, T>(const uint64_t*, const int32_t*, Count,     \
                                                     const JobParams<T>*, const int32_t*,        \
                                                     const uint32_t*, int2*, int2*, int32_t*,    \
-                                                    hipStream_t, const int32_t*);
+                                                    hipStream_t, const int32_t*,                \
+                                                    const int32_t*);
 HPD_FOR_EACH_DTYPE(HPD_INST_ROWS)
 
 }  // namespace hpd

@@ -17,8 +17,8 @@ void launch_cells(const K* keys, int64_t n, int shift, uint32_t* flags, uint32_t
                   K* ucell, int32_t* ustart, uint32_t* ncells_dev, hipStream_t s);
 
 // job_of_cell[u] = job of cell u; nranges[u] = number of non-empty
-// neighbour rows of cell u; core_chunks[u] (when not null) = 64-row chunks
-// of cell u if it has >= minPts candidates, else 0; adds
+// neighbour rows of cell u; cell_core[u] (when not null) = 1 if cell u has
+// >= minPts candidates (only then can it hold cores), else 0; adds
 // Σ_u count(u) * |candidates(u)| to *sumcand and Σ_u nranges[u] to
 // *rows_total (64-bit, unlike the scan of nranges).  With a stash (m * stash_rows
 // entries, stash_rows >= the most neighbour rows a cell can have) the
@@ -29,7 +29,7 @@ void launch_cells(const K* keys, int64_t n, int shift, uint32_t* flags, uint32_t
 template <typename K, typename T>
 void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
                            const JobParams<T>* jobs, int32_t njobs, int32_t* job_of_cell,
-                           uint32_t* nranges, uint32_t* core_chunks, unsigned long long* sumcand,
+                           uint32_t* nranges, uint8_t* cell_core, unsigned long long* sumcand,
                            unsigned long long* rows_total, int2* stash, int32_t stash_rows,
                            int32_t* rcenter, bool by_class, hipStream_t s,
                            const int32_t* ctab = nullptr);
@@ -40,33 +40,28 @@ void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
 template <typename K>
 void launch_cell_table(const K* ucell, Count m, int32_t* ctab, uint64_t ids, hipStream_t s);
 
-// launch_neighbor_fill's output from the count pass's stash (roff scanned);
-// with by_class the rows of each cell go nearest first (own row, then by
-// the number of offset dimensions) instead of ascending
-void launch_neighbor_copy(const int2* stash, int32_t stash_rows, const int32_t* ustart, int32_t m,
-                          const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
-                          bool by_class, hipStream_t s);
+// Box mode: launch_neighbor_fill's box ranges and rcenter from the count
+// pass's stash (roff scanned); with by_class the rows of each cell go
+// nearest first (own row, then by the number of offset dimensions) instead of
+// ascending
+void launch_neighbor_copy(const int2* stash, int32_t stash_rows, int32_t m, const uint32_t* roff,
+                          const int32_t* cbox, int2* rboxes, int32_t* rcenter, bool by_class,
+                          hipStream_t s);
 
 // ranges[roff[u] ..) = [first row, end row) of each non-empty neighbour row,
 // ascending; rcells[..] = [first, end) occupied-cell index of the same row;
-// rcenter[u] = index (into ranges) of the row holding cell u itself
+// rcenter[u] = index (into ranges) of the row holding cell u itself.  With
+// cbox (first box of every cell) rcells gets the rows' box ranges
+// [cbox[first], cbox[end]) instead: the box kernels then read them in one
+// load, not three dependent ones.  ranges may be null.
 template <typename K, typename T>
 void launch_neighbor_fill(const K* ucell, const int32_t* ustart, Count m,
                           const JobParams<T>* jobs, const int32_t* job_of_cell,
                           const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
-                          hipStream_t s, const int32_t* ctab = nullptr);
+                          hipStream_t s, const int32_t* ctab = nullptr,
+                          const int32_t* cbox = nullptr);
 
 void launch_chunk_counts(const int32_t* ustart, Count m, uint32_t* nchunks, hipStream_t s);
-
-// Work split of the neighbour kernels: cells with more than sparse_max rows
-// give one item (cell, first row) per 64-row chunk (dcnt: chunks per cell),
-// the others one item (row, cell) per row (scnt: rows per cell).  doff /
-// soff are the exclusive scans of dcnt / scnt.
-void launch_split_counts(const int32_t* ustart, Count m, int32_t sparse_max, uint32_t* dcnt,
-                         uint32_t* scnt, hipStream_t s);
-void launch_split_items(const int32_t* ustart, Count m, int32_t sparse_max, const uint32_t* doff,
-                        const uint32_t* soff, int2* ditems, Count nditems, int2* sitems,
-                        hipStream_t s);
 
 // items[w] = (g, start[g] + 64 * (w - off[g])) for the `total` 64-row chunks
 // of ngroups groups (off: exclusive scan of chunk counts, ngroups + 1 entries)

@@ -9,6 +9,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "common.hpp"
+
 namespace hpd {
 
 template <typename T, int D>
@@ -135,6 +137,79 @@ __device__ __forceinline__ double bcast(double v, int j) {
     return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
 }
 
+__device__ __forceinline__ float bcast(float v, int j) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+}
+
+// Candidates on the lanes: how many of the rows [qb, qe) (with flags: of
+// those whose flag is set) are within eps of the wave-uniform row pr, counted
+// until the count reaches `limit` (a look after every kWideStep rows; the
+// result is exact below the limit and at least the limit otherwise).
+// visit_range reads 16 candidates an iteration for up to 64 rows at once;
+// with a few rows that leaves the lanes idle and a box of a million rows is
+// one wave's chain of 65k dependent iterations.  Here an iteration reads
+// kWideStep rows, coalesced.  visited += rows read.
+constexpr int kWideLoads = 4;
+constexpr int kWideStep = 64 * kWideLoads;
+// Rows of a wave up to which a box of more than kWideMinRows rows is walked
+// row by row with the candidates on the lanes: an iteration of either walk
+// costs about one load latency and 16 x 4 tests, so 256 candidates of one
+// row cost what 16 candidates of all 64 do.  One-wave chains were the whole
+// core count of 100M skewed 2-D rows (7.85 ms for 2.3M tests).
+constexpr int kWideRows = 8;
+constexpr int kWideMinRows = 64;
+
+template <typename T, int D>
+__device__ __forceinline__ uint32_t wide_count(const T* __restrict__ soa, int64_t ld,
+                                               const uint8_t* __restrict__ flags, int32_t qb,
+                                               int32_t qe, const T* pr, T eps2, uint32_t limit,
+                                               uint32_t& visited) {
+    uint32_t cnt = 0;
+    const int lane = __lane_id();
+    for (int32_t a = qb; a < qe && cnt < limit; a += kWideStep) {
+        T c[kWideLoads][D];
+        uint8_t f[kWideLoads];
+#pragma unroll
+        for (int k = 0; k < kWideLoads; ++k) {
+            const int32_t q = min(a + k * 64 + lane, qe - 1);
+            load_row<T, D>(soa, ld, q, c[k]);
+            f[k] = flags ? flags[q] : uint8_t(1);
+        }
+#pragma unroll
+        for (int k = 0; k < kWideLoads; ++k) {
+            const bool in = a + k * 64 + lane < qe && f[k] && within<D>(pr, c[k], eps2);
+            cnt += static_cast<uint32_t>(__popcll(__ballot(in)));
+        }
+        visited += static_cast<uint32_t>(min(kWideStep, qe - a));
+    }
+    return cnt;
+}
+
+// The rows of the lanes in `rows` walked as above; true on the lanes whose
+// row has a candidate (with flags: a flagged one) within eps.
+template <typename T, int D>
+__device__ __forceinline__ bool wide_any(const T* __restrict__ soa, int64_t ld,
+                                         const uint8_t* __restrict__ flags, int32_t qb, int32_t qe,
+                                         const T* pc, T eps2, uint64_t rows, bool first_only) {
+    bool hit = false;
+    uint32_t visited = 0;
+    for (; rows != 0; rows &= rows - 1) {
+        const int r = static_cast<int>(__builtin_ctzll(rows));
+        T pr[D];
+#pragma unroll
+        for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], r);
+        const bool h = wide_count<T, D>(soa, ld, flags, qb, qe, pr, eps2, 1u, visited) != 0;
+        if (__lane_id() == r) hit = h;
+        if (h && first_only) break;
+    }
+    return hit;
+}
+
+// Whether a walk of n candidate rows for the lanes of `rows` goes row by row.
+__device__ __forceinline__ bool walk_wide(uint64_t rows, int32_t n) {
+    return n > kWideMinRows && __popcll(rows) <= kWideRows;
+}
+
 // Squared distances from a row to the box [lo, hi] (double): gmin2 to its
 // nearest point, gmax2 to its farthest corner.
 template <int D>
@@ -171,8 +246,7 @@ __device__ __forceinline__ void point_box_lh(const double* lo, const double* hi,
 // earlier boxes: a visit that stops early sees the own cell's boxes first.
 template <typename T, int D, typename Fn>
 __device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t center,
-                                                 const int2* __restrict__ rcells,
-                                                 const int32_t* __restrict__ cbox,
+                                                 const int2* __restrict__ rboxes,
                                                  const int32_t* __restrict__ bstart,
                                                  const OrdKey<T>* __restrict__ bbox,
                                                  const int32_t* __restrict__ tag, Fn&& fn,
@@ -184,9 +258,9 @@ __device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t
         int32_t rb0 = 0, rcnt = 0;
         if (i < nrows) {
             const int32_t r = i == 0 ? center : (r0 + i - 1 < center ? r0 + i - 1 : r0 + i);
-            const int2 cs = rcells[r];
-            rb0 = cbox[cs.x];
-            rcnt = max(0, min(cbox[cs.y], bmax) - rb0);  // boxes below bmax only
+            const int2 bs = rboxes[r];
+            rb0 = bs.x;
+            rcnt = max(0, min(bs.y, bmax) - rb0);  // boxes below bmax only
         }
         int32_t incl = rcnt;  // inclusive prefix over the lanes
 #pragma unroll
@@ -233,90 +307,81 @@ __device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t
     }
 }
 
-// The same visit as for_each_row_box, handed to fn a group of up to 64 boxes
-// at a time with one box per lane: fn(nk, bl, lol, hil, q0l, q1l, tagl) gets
-// the group's size nk (wave-uniform) and, on lanes below nk, the lane's box,
-// its bounding box, rows and tag (lanes at or above nk repeat the group's
-// last box); it returns true to stop the visit.  Boxes keep the visiting
-// order of for_each_row_box (lane order inside a group).  Lets a kernel
-// classify a whole group against the bounding box of its rows in parallel
-// and walk only the boxes that need row tests.
-// The boxes of the neighbour rows g0 + lane of the visiting order (own row
-// first): the first box rb0 and the number rcnt below bmax (0 past the rows).
-__device__ __forceinline__ void row_boxes(int32_t r0, int32_t r1, int32_t center, int32_t g0,
-                                          const int2* __restrict__ rcells,
-                                          const int32_t* __restrict__ cbox, int32_t bmax,
-                                          int32_t& rb0, int32_t& rcnt) {
-    const int32_t i = g0 + __lane_id();
-    rb0 = 0;
-    rcnt = 0;
-    if (i < r1 - r0) {
-        const int32_t r = i == 0 ? center : (r0 + i - 1 < center ? r0 + i - 1 : r0 + i);
-        const int2 cs = rcells[r];
-        rb0 = cbox[cs.x];
-        rcnt = max(0, min(cbox[cs.y], bmax) - rb0);
+// A wave split into groups of G lanes, each with a neighbourhood of its own:
+// the boxes of the neighbour rows [r0, r1) of an occupied cell (box ranges
+// rboxes, the own row `center` first, from the cell's first box `own` on and
+// wrapping round, then the other rows in stored order) are handed out G at a
+// time, one per lane.  fn(valid, b) runs for the whole wave at once (it may
+// use wave-wide operations), with the lane's box b where valid; what it
+// returns must be equal over a group: true ends that group's visit.  Only
+// boxes below bmax are visited.  All arguments but G are per lane, equal over
+// a group; inactive groups take part in the wave-wide steps only.
+//
+// Why groups: a neighbourhood holds some 10-30 boxes, so a whole wave per
+// row, box or cell leaves most lanes without one, and a thread per row or box
+// walks them as a chain of dependent loads.
+template <int G, typename Fn>
+__device__ __forceinline__ void group_boxes(bool active, int32_t r0, int32_t r1, int32_t center,
+                                            int32_t own, const int2* __restrict__ rboxes,
+                                            int32_t bmax, Fn&& fn) {
+    const int gl = __lane_id() & (G - 1);
+    const int32_t nrows = r1 - r0;
+    for (int32_t g0 = 0; __any(active && g0 < nrows); g0 += G) {
+        // G rows at a time, one per lane
+        const int32_t i = g0 + gl;
+        int32_t b0 = 0, cnt = 0;
+        if (active && i < nrows) {
+            const int32_t r = i == 0 ? center : (r0 + i - 1 < center ? r0 + i - 1 : r0 + i);
+            const int2 bs = rboxes[r];
+            b0 = bs.x;
+            cnt = max(0, min(bs.y, bmax) - b0);
+        }
+        // the own row starts at box `own`
+        const int32_t rot = g0 == 0 && gl == 0 && own > b0 && own < b0 + cnt ? own - b0 : 0;
+        int32_t incl = cnt;
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) {
+            const int32_t t = __shfl_up(incl, o, G);
+            if (gl >= o) incl += t;
+        }
+        const int32_t excl = incl - cnt;
+        const int32_t total = __shfl(incl, G - 1, G);
+        const int32_t rot0 = __shfl(rot, 0, G);
+        const int32_t n0 = __shfl(cnt, 0, G);
+        for (int32_t k0 = 0; __any(active && k0 < total); k0 += G) {
+            const int32_t kk = k0 + gl;
+            int32_t row = 0;  // the last row whose first box is at or before kk
+#pragma unroll
+            for (int st = G / 2; st > 0; st >>= 1) {
+                const int32_t e = __shfl(excl, row + st, G);
+                if (e <= kk) row += st;
+            }
+            int32_t local = kk - __shfl(excl, row, G);
+            if (g0 == 0 && row == 0) local += local + rot0 < n0 ? rot0 : rot0 - n0;
+            const int32_t b = __shfl(b0, row, G) + local;
+            if (fn(active && kk < total, b)) active = false;
+        }
     }
 }
 
-// pre (optional): row_boxes of the first group, loaded by the caller ahead
-// of its own loads so that the two overlap.
-struct RowBoxes {
-    int32_t rb0, rcnt;
-};
-
-template <typename T, int D, typename Fn>
-__device__ __forceinline__ void for_each_row_box_group(int32_t r0, int32_t r1, int32_t center,
-                                                       const int2* __restrict__ rcells,
-                                                       const int32_t* __restrict__ cbox,
-                                                       const int32_t* __restrict__ bstart,
-                                                       const OrdKey<T>* __restrict__ bbox,
-                                                       const int32_t* __restrict__ tag, Fn&& fn,
-                                                       int32_t bmax = INT_MAX,
-                                                       int32_t first = -1,
-                                                       const RowBoxes* pre = nullptr) {
-    const int32_t nrows = r1 - r0;
-    const int lane = __lane_id();
-    for (int32_t g0 = 0; g0 < nrows; g0 += 64) {
-        int32_t rb0, rcnt;
-        if (g0 == 0 && pre) {
-            rb0 = pre->rb0;
-            rcnt = pre->rcnt;
-        } else {
-            row_boxes(r0, r1, center, g0, rcells, cbox, bmax, rb0, rcnt);
-        }
-        int32_t incl = rcnt;  // inclusive prefix over the lanes
+// Sum, minimum and maximum over a group of G lanes.
+template <int G>
+__device__ __forceinline__ uint32_t group_sum(uint32_t v) {
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int32_t t = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += t;
-        }
-        const int32_t excl = incl - rcnt;
-        const int32_t total = bcast(incl, 63);
-        const int32_t grows = min(64, nrows - g0);
-        int32_t rot = 0, rot_n = 0;
-        if (g0 == 0 && first >= 0) {
-            const int32_t b0 = bcast(rb0, 0);
-            rot_n = bcast(rcnt, 0);
-            rot = (first >= b0 && first < b0 + rot_n) ? first - b0 : 0;
-        }
-        for (int32_t k0 = 0; k0 < total; k0 += 64) {
-            const int32_t kk = min(k0 + lane, total - 1);
-            int32_t row = 0;  // last row whose first box index is <= kk
-            for (int32_t t = 1; t < grows; ++t) row = bcast(excl, t) <= kk ? t : row;
-            int32_t local = kk - __shfl(excl, row, 64);
-            if (row == 0 && rot > 0) local = local + rot < rot_n ? local + rot : local + rot - rot_n;
-            const int32_t bl = __shfl(rb0, row, 64) + local;
-            double lol[D], hil[D];
+    for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+template <int G>
+__device__ __forceinline__ int32_t group_min(int32_t v) {
 #pragma unroll
-            for (int j = 0; j < D; ++j) {
-                lol[j] = box_lo<T, D>(bbox, bl, j);
-                hil[j] = box_hi<T, D>(bbox, bl, j);
-            }
-            const int32_t q0l = bstart[bl], q1l = bstart[bl + 1];
-            const int32_t tagl = tag ? tag[bl] : 0;
-            if (fn(min(64, total - k0), bl, lol, hil, q0l, q1l, tagl)) return;
-        }
-    }
+    for (int o = G / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+    return v;
+}
+template <int G>
+__device__ __forceinline__ int32_t group_max(int32_t v) {
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    return v;
 }
 
 // Box-to-box squared distances (double): gmin2 between the nearest points
