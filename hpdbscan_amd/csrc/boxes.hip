@@ -43,12 +43,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
-// boxes of at most kSmallBox rows are hooked one thread per box, with at
-// most kSmallTests distance tests per box pair
-constexpr int kSmallBox = 32;
-constexpr int kSmallTests = 512;
-
-
 inline unsigned blocks_for(int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
 
 // Rows in slot order: coordinates (SoA); with it the bounding box of every
@@ -406,480 +400,316 @@ __device__ __forceinline__ bool any_pair(const T* __restrict__ soa, int64_t ld,
     return visit_range<T, D>(soa, ld, core, nullptr, q0, q1, body, stop);
 }
 
-// Box-level hook: every box with cores points at some box of a smaller
-// index holding a core within eps of one of its cores (searched from the
-// box's first 64-row chunk, stopping at the first hit; any such box will
-// do, and a box without one stays a root).  parent
-// stays <= the box index, so the hooks form a forest whose trees are
-// connected sets of boxes.
+// Whether a core row of slots [s0, s1) is within eps of a core row of box b2
+// (slots [q0, q1)), by the whole wave (every argument wave-uniform): 64 rows
+// of [s0, s1) at a time on the lanes; a row within eps of the whole box
+// answers at once, one farther than eps from its bounding box is left out,
+// the others meet the box's rows.
 template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_hook(
-    const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nitems_c,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
-    const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
-    const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
-    const int32_t* __restrict__ rcenter, int32_t* __restrict__ bparent) {
-    const int32_t nitems = static_cast<int32_t>(nitems_c.get());
-    const int32_t stride = static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-    // waves walk the items wid, wid + stride, ... (one each when the grid
-    // covers them)
-    for (int32_t wid = uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
-                               static_cast<int32_t>(threadIdx.x >> 6));
-         wid < nitems; wid += stride) [&] {
-        // boxes with cores of more than kSmallBox rows; one hook per box is
-        // enough: its first chunk looks for it (a missed link is found by
-        // the exact union later)
-        const int32_t b = uniform(blist[wid]);
-        const int2 it = make_int2(b, uniform(bstart[b]));
-        const int32_t end = uniform(bstart[b + 1]);
-        const int32_t p = it.y + lane_id();
-        const bool pcore = p < end && core[p];
-        if (!__any(pcore)) return;
-        const int32_t u = uniform(bcell[b]);
-        const JobParams<T>& jp = jobs[uniform(job_of_cell[u])];
+__device__ __forceinline__ bool wave_pair(const T* __restrict__ soa, int64_t ld,
+                                          const uint8_t* __restrict__ core,
+                                          const OrdKey<T>* __restrict__ bbox, int32_t s0,
+                                          int32_t s1, int32_t b2, int32_t q0, int32_t q1, T eps2,
+                                          double gap2_max, double full2) {
+    for (int32_t c = s0; c < s1; c += kWave) {
+        const int32_t p = c + lane_id();
+        const bool pcore = p < s1 && core[p];
+        if (!__any(pcore)) continue;
+        T pc[D];
+        load_row<T, D>(soa, ld, pcore ? p : c, pc);
+        double gmin2, gmax2;
+        point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
+        const bool act = pcore && gmin2 <= gap2_max;
+        if (__any(act && gmax2 <= full2)) return true;
+        if (__any(act) && any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return true;
+    }
+    return false;
+}
+
+// The same by one lane, for boxes of few rows.
+template <typename T, int D>
+__device__ __forceinline__ bool lane_pair(const T* __restrict__ soa, int64_t ld,
+                                          const uint8_t* __restrict__ core, int32_t s0, int32_t s1,
+                                          int32_t q0, int32_t q1, T eps2) {
+    for (int32_t p = s0; p < s1; ++p) {
+        if (!core[p]) continue;
+        T pc[D];
+        load_row<T, D>(soa, ld, p, pc);
+        for (int32_t q = q0; q < q1; ++q) {
+            if (!core[q]) continue;
+            T qc[D];
+            load_row<T, D>(soa, ld, q, qc);
+            if (within<D>(pc, qc, eps2)) return true;
+        }
+    }
+    return false;
+}
+
+// The pair kernels below take the boxes with cores from blist, a group of G
+// lanes per box, a neighbour box per lane (group_boxes); box pairs of up to
+// kLanePair rows by rows are tested by their lane, larger ones by the wave.
+constexpr int kLanePair = 64;
+
+// squared distances between two bounding boxes: nearest and farthest points
+template <typename T, int D>
+__device__ __forceinline__ void box_gap(const OrdKey<T>* __restrict__ bbox, int32_t b2,
+                                        const double* lo, const double* hi, double& gap2,
+                                        double& far2) {
+    gap2 = 0.0;
+    far2 = 0.0;
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+        const double l2 = box_lo<T, D>(bbox, b2, j), h2 = box_hi<T, D>(bbox, b2, j);
+        const double g = fmax(0.0, fmax(l2 - hi[j], lo[j] - h2));
+        const double f = fmax(h2 - lo[j], hi[j] - l2);
+        gap2 += g * g;
+        far2 += f * f;
+    }
+}
+
+// Hook forest (kJoin false): every listed box points at some earlier box
+// holding a core within eps of one of its cores, the own neighbour row
+// searched first from the own cell on (any such box will do, and a box
+// without one stays a root; larger boxes search from their first 64 rows
+// only, here and in the root join: a missed link is found by the exact union
+// later).  bparent stays <=
+// the box index, so the hooks form a forest whose trees are connected sets
+// of boxes.
+// Root join (kJoin): every root of that forest (blist) looks through its
+// whole neighbourhood for the first box of another tree (rsnap) holding a
+// within-eps core pair and joins the two trees (union-find, smaller root on
+// top).  One round merges most trees of a cluster, so far fewer pairs stay
+// open for the union.
+// tag: bmincore (INT_MAX: no cores) for the hook, rsnap (-1) for the join.
+template <typename T, int D, bool kJoin>
+__global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
+                                                       const uint32_t* __restrict__ roff,
+                                                       const int2* __restrict__ rboxes,
+                                                       const int32_t* __restrict__ tag,
+                                                       const uint8_t* __restrict__ core,
+                                                       const int32_t* __restrict__ blist,
+                                                       const unsigned int* __restrict__ nlist_dev,
+                                                       int32_t* bparent) {
+    constexpr int G = kGroup<D>;
+    constexpr int kPer = 64 / G;
+    const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
+    const int gl = lane_id() & (G - 1);
+    const int grp = lane_id() / G;
+    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    for (int32_t base = first_wave() * kPer; base < nlist; base += wave_stride() * kPer) {
+        const bool on = base + grp < nlist;
+        const int32_t b = blist[on ? base + grp : nlist - 1];
+        const int32_t s0 = a.bstart[b], s1 = a.bstart[b + 1];
+        const int32_t u = a.bcell[b];
+        const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
         const double gap2_max = jp.gap2_max;
         const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-        T pc[D];
-        load_row<T, D>(soa, ld, pcore ? p : it.y, pc);
-        const int32_t r0 = uniform(static_cast<int32_t>(roff[u]));
-        const int32_t r1 = uniform(static_cast<int32_t>(roff[u + 1]));
-        // the cell's own row first, from the own cell's first box: the box's
-        // nearest neighbours are there, so the first hit comes soonest; boxes
-        // before b only
-        for_each_row_box<T, D>(
-            r0, r1, uniform(rcenter[u]), rboxes, bstart, bbox, bmincore,
-            [&](int32_t b2, const double* lo, const double* hi, int32_t q0, int32_t q1,
-                int32_t mincore) {
-                if (mincore == INT_MAX) return false;  // no cores
-                double gmin2, gmax2;
-                point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
-                const bool act = pcore && gmin2 <= gap2_max;
-                if (!__any(act)) return false;
-                // a core row within eps of the whole box is within eps of its cores
-                const bool hit = act && gmax2 <= full2;
-                if (!__any(hit) && !any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return false;
-                if (lane_id() == 0) bparent[b] = b2;
-                return true;
-            },
-            b, uniform(cbox[u]));
-    }();
-}
-
-// Root join: every root of the hook forest (a box without an earlier
-// within-eps core pair) looks through its whole neighbourhood for the first
-// box of another tree holding a within-eps core pair and joins the two
-// trees (union-find, smaller root on top).  One round merges most trees of
-// a cluster, so far fewer pairs stay open for the union.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_root_join(
-    const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nitems_c,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
-    const int32_t* __restrict__ rsnap, const uint8_t* __restrict__ core,
-    const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
-    const int32_t* __restrict__ rcenter, int32_t* bparent) {
-    const int32_t nitems = static_cast<int32_t>(nitems_c.get());
-    const int32_t stride = static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-    // waves walk the items wid, wid + stride, ... (one each when the grid
-    // covers them)
-    for (int32_t wid = uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
-                               static_cast<int32_t>(threadIdx.x >> 6));
-         wid < nitems; wid += stride) [&] {
-        // roots of the forest, each searched from its first chunk
-        const int32_t b = uniform(blist[wid]);
-        const int2 it = make_int2(b, uniform(bstart[b]));
-        const int32_t end = uniform(bstart[b + 1]);
-        const int32_t p = it.y + lane_id();
-        const bool pcore = p < end && core[p];
-        if (!__any(pcore)) return;
-        const int32_t u = uniform(bcell[b]);
-        const JobParams<T>& jp = jobs[uniform(job_of_cell[u])];
-        const T eps2 = jp.eps2;
-        const double gap2_max = jp.gap2_max;
-        T pc[D];
-        load_row<T, D>(soa, ld, pcore ? p : it.y, pc);
-        const int32_t r0 = uniform(static_cast<int32_t>(roff[u]));
-        const int32_t r1 = uniform(static_cast<int32_t>(roff[u + 1]));
-        for_each_row_box<T, D>(
-            r0, r1, uniform(rcenter[u]), rboxes, bstart, bbox, rsnap,
-            [&](int32_t b2, const double* lo, const double* hi, int32_t q0, int32_t q1,
-                int32_t s2) {
-                if (s2 < 0 || s2 == b) return false;  // no cores, or b's own tree
-                double gmin2, gmax2;
-                point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
-                const bool act = pcore && gmin2 <= gap2_max;
-                if (!__any(act)) return false;
-                if (!any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return false;
-                if (lane_id() == 0) uf_unite(bparent, b, b2);
-                return true;
-            });
-    }();
-}
-
-// Box pairs the hook forest leaves open: one thread per box b finds every
-// later box b2 with cores in a different hook tree whose bounding box is
-// within eps of b's.  Count pass (list == nullptr): cnt[b] = their number;
-// fill pass: the b2 go to list[off[b] ..].
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_scan(
-    Count nbox_c, const int32_t* __restrict__ bcell, const int32_t* __restrict__ cbox,
-    const uint32_t* __restrict__ roff, const int2* __restrict__ rboxes,
-    const OrdKey<T>* __restrict__ bbox, const int32_t* __restrict__ job_of_cell,
-    const JobParams<T>* __restrict__ jobs, const int32_t* __restrict__ rsnap,
-    uint32_t* __restrict__ cnt, int32_t* __restrict__ list, unsigned long long* __restrict__ total,
-    const unsigned long long* __restrict__ total_chk, unsigned long long cap) {
-    const int32_t nbox = static_cast<int32_t>(nbox_c.get());
-    // fill pass of the static pipeline: nothing to write when the pairs
-    // exceed the list (the host path then takes over)
-    if (list && total_chk && *total_chk > cap) return;
-    const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    uint32_t k = (list && b < nbox) ? cnt[b] : 0u;
-    // the fill pass walks only the boxes the count pass found pairs for
-    const int32_t sb = b < nbox && (!list || cnt[b + 1] > k) ? rsnap[b] : -1;
-    if (sb >= 0) {
-        const int32_t u = bcell[b];
-        const double gap2_max = jobs[job_of_cell[u]].gap2_max;
         double lo[D], hi[D];
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             lo[j] = box_lo<T, D>(bbox, b, j);
             hi[j] = box_hi<T, D>(bbox, b, j);
         }
-        for (uint32_t r = roff[u]; r < roff[u + 1]; ++r) {
-            const int2 bs = rboxes[r];
-            for (int32_t b2 = max(bs.x, b + 1); b2 < bs.y; ++b2) {
-                const int32_t s2 = rsnap[b2];
-                if (s2 < 0 || s2 == sb) continue;
-                double gap2 = 0.0;
-#pragma unroll
-                for (int j = 0; j < D; ++j) {
-                    const double g = fmax(0.0, fmax(box_lo<T, D>(bbox, b2, j) - hi[j],
-                                                    lo[j] - box_hi<T, D>(bbox, b2, j)));
-                    gap2 += g * g;
-                }
-                if (gap2 > gap2_max) continue;
-                if (list) list[k] = b2;
-                ++k;
-            }
-        }
-    }
-    if (!list) {
-        if (b < nbox) cnt[b] = k;
-        // 64-bit total, so that the caller can check it before a 32-bit scan
-        block_add<kThreads>(k, total);
-    }
-}
-
-// Union over the open pairs: one wave per 64-slot chunk of a box b; the
-// chunk's core rows (lanes) meet the boxes of b's open list one by one.  A
-// pair is skipped when the two boxes are joined by now (live roots) or no
-// core of the chunk is within eps of the other box's bounding box;
-// otherwise the other box's cores stream through the wave until the first
-// within-eps pair, which joins the boxes.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_union_list(
-    const T* __restrict__ soa, int64_t ld, const int2* __restrict__ bitems, Count nitems_c,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const OrdKey<T>* __restrict__ bbox, const uint8_t* __restrict__ core,
-    const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
-    const uint32_t* __restrict__ off, const int32_t* __restrict__ list, int32_t* bparent,
-    const unsigned long long* __restrict__ total_chk, unsigned long long cap) {
-    if (total_chk && *total_chk > cap) return;  // no list was written
-    const int32_t nitems = static_cast<int32_t>(nitems_c.get());
-    const int32_t stride = static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-    // waves walk the items wid, wid + stride, ... (one each when the grid
-    // covers them)
-    for (int32_t wid = uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
-                               static_cast<int32_t>(threadIdx.x >> 6));
-         wid < nitems; wid += stride) [&] {
-        const int2 it = bitems[wid];
-        const int32_t b = uniform(it.x);
-        const uint32_t l0 = uniform(static_cast<int32_t>(off[b]));
-        const uint32_t l1 = uniform(static_cast<int32_t>(off[b + 1]));
-        if (l0 == l1) return;
-        const int32_t end = uniform(bstart[b + 1]);
-        const int32_t p = it.y + lane_id();
-        const bool pcore = p < end && core[p];
-        if (!__any(pcore)) return;
-        const JobParams<T>& jp = jobs[uniform(job_of_cell[uniform(bcell[b])])];
-        const T eps2 = jp.eps2;
-        const double gap2_max = jp.gap2_max;
-        T pc[D];
-        load_row<T, D>(soa, ld, pcore ? p : it.y, pc);
-        int32_t rb = uniform(uf_find(bparent, b));
-        for (uint32_t L0 = l0; L0 < l1; L0 += kWave) {
-            // lanes fetch 64 partners at once: box, bounding box, rows, and a
-            // root (roots only merge, so an equal root is final)
-            const uint32_t li = min(L0 + static_cast<uint32_t>(lane_id()), l1 - 1);
-            const int32_t b2l = list[li];
-            double lol[D], hil[D];
-    #pragma unroll
-            for (int j = 0; j < D; ++j) {
-                lol[j] = box_lo<T, D>(bbox, b2l, j);
-                hil[j] = box_hi<T, D>(bbox, b2l, j);
-            }
-            const int32_t q0l = bstart[b2l], q1l = bstart[b2l + 1];
-            const int32_t r2l = uf_find(bparent, b2l);
-            const int32_t nk = static_cast<int32_t>(min(static_cast<uint32_t>(kWave), l1 - L0));
-            for (int32_t j = 0; j < nk; ++j) {
-                double lo[D], hi[D];
-    #pragma unroll
-                for (int e = 0; e < D; ++e) {
-                    lo[e] = bcast(lol[e], j);
-                    hi[e] = bcast(hil[e], j);
-                }
-                double gmin2, gmax2;
-                point_box_lh<T, D>(lo, hi, pc, gmin2, gmax2);
-                const bool act = pcore && gmin2 <= gap2_max;
-                if (!__any(act)) continue;
-                int32_t rb2 = bcast(r2l, j);
-                if (rb2 == rb) continue;
-                rb = uniform(uf_find(bparent, rb));
-                rb2 = uniform(uf_find(bparent, rb2));
-                if (rb2 == rb) continue;
-                if (any_pair<T, D>(soa, ld, core, bcast(q0l, j), bcast(q1l, j), pc, act, eps2)) {
-                    if (lane_id() == 0) uf_unite(bparent, rb, rb2);
-                    rb = uniform(uf_find(bparent, b));
+        int32_t link = -1;  // equal over the group
+        group_boxes<G>(on, static_cast<int32_t>(roff[u]), static_cast<int32_t>(roff[u + 1]),
+                       a.rcenter[u], a.cbox[u], rboxes, 0, kJoin ? INT_MAX : b,
+                       [&](bool valid, int32_t b2) {
+            bool open = false, hit = false;
+            int32_t q0 = 0, q1 = 0;
+            if (valid) {
+                const int32_t t = tag[b2];
+                if (kJoin ? (t >= 0 && t != b) : t != INT_MAX) {
+                    double gap2, far2;
+                    box_gap<T, D>(bbox, b2, lo, hi, gap2, far2);
+                    open = gap2 <= gap2_max;
+                    hit = far2 <= full2;
+                    q0 = a.bstart[b2];
+                    q1 = a.bstart[b2 + 1];
                 }
             }
-        }
-    }();
-}
-
-// Union over the open pairs of the boxes of at most small_rows rows, one
-// thread per box (a wave per box would leave most of its lanes idle): the
-// box's core rows meet each listed box whose root differs -- a row within
-// eps of the other box's whole bounding box joins at once, a row farther
-// than eps from it skips it, and otherwise the rows are tested against the
-// other box's cores until the first within-eps pair.  Every pair is decided
-// exactly (no test budget), as in k_box_union_list.
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_union_small(
-    const T* __restrict__ soa, int64_t ld, Count nbox_c, const int32_t* __restrict__ bstart,
-    const int32_t* __restrict__ bcell, const OrdKey<T>* __restrict__ bbox,
-    const uint8_t* __restrict__ core, const int32_t* __restrict__ job_of_cell,
-    const JobParams<T>* __restrict__ jobs, const uint32_t* __restrict__ off,
-    const int32_t* __restrict__ list, int32_t* bparent,
-    const unsigned long long* __restrict__ total_chk, unsigned long long cap, int32_t small_rows) {
-    if (total_chk && *total_chk > cap) return;  // no list was written
-    const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (b >= static_cast<int32_t>(nbox_c.get())) return;
-    const uint32_t l0 = off[b], l1 = off[b + 1];
-    if (l0 == l1) return;
-    const int32_t s0 = bstart[b], s1 = bstart[b + 1];
-    if (s1 - s0 > small_rows) return;  // one wave per chunk instead
-    const JobParams<T>& jp = jobs[job_of_cell[bcell[b]]];
-    const T eps2 = jp.eps2;
-    const double gap2_max = jp.gap2_max;
-    const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-    for (uint32_t L = l0; L < l1; ++L) {
-        const int32_t b2 = list[L];
-        int32_t r = uf_find(bparent, b);
-        const int32_t r2 = uf_find(bparent, b2);
-        if (r == r2) continue;
-        const int32_t t0 = bstart[b2], t1 = bstart[b2 + 1];
-        bool hit = false;
-        for (int32_t p = s0; p < s1 && !hit; ++p) {
-            if (!core[p]) continue;
-            T pc[D];
-            load_row<T, D>(soa, ld, p, pc);
-            double gmin2, gmax2;
-            point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
-            if (gmin2 > gap2_max) continue;
-            if (gmax2 <= full2) {  // within eps of all of b2, its cores included
-                hit = true;
-                break;
-            }
-            for (int32_t q = t0; q < t1; ++q) {
-                if (!core[q]) continue;
-                T qc[D];
-                load_row<T, D>(soa, ld, q, qc);
-                if (within<D>(pc, qc, eps2)) {
-                    hit = true;
-                    break;
+            const uint64_t gmask = ((G < 64 ? (uint64_t{1} << G) : 0) - 1) << (grp * G);
+            uint64_t hits = ballot(hit) & gmask;
+            if (hits == 0 && open) {
+                const int64_t tests = static_cast<int64_t>(s1 - s0) * (q1 - q0);
+                if (tests <= kLanePair) {
+                    hit = lane_pair<T, D>(a.soa, a.ld, core, s0, s1, q0, q1, eps2);
+                    open = false;
                 }
             }
-        }
-        if (hit) uf_unite(bparent, r, r2);
-    }
-}
-
-// Hook of a small box (at most kSmallBox rows), one thread per box: the
-// box's core rows meet the earlier boxes of its neighbourhood, own neighbour
-// row first; a box pair gets at most kSmallTests distance tests (rows
-// farther than eps from the other box's bounding box take none) before the
-// search moves on: a missed hook only leaves work for the exact union.
-
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_hook_small(
-    const T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ blist, Count nlist_c,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rboxes, const int32_t* __restrict__ rcenter,
-    const OrdKey<T>* __restrict__ bbox, const int32_t* __restrict__ bmincore,
-    const uint8_t* __restrict__ core, const int32_t* __restrict__ job_of_cell,
-    const JobParams<T>* __restrict__ jobs, int32_t* __restrict__ bparent) {
-    const int32_t nlist = static_cast<int32_t>(nlist_c.get());
-    const int32_t i = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= nlist) return;
-    const int32_t b = blist[i];
-    const int32_t s0 = bstart[b], s1 = bstart[b + 1];
-    if (s1 - s0 > kSmallBox) return;  // k_box_hook's
-    const int32_t u = bcell[b];
-    const JobParams<T>& jp = jobs[job_of_cell[u]];
-    const T eps2 = jp.eps2;
-    const double gap2_max = jp.gap2_max;
-    const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-    double blo[D], bhi[D];
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        blo[j] = box_lo<T, D>(bbox, b, j);
-        bhi[j] = box_hi<T, D>(bbox, b, j);
-    }
-    const int32_t r0 = static_cast<int32_t>(roff[u]), r1 = static_cast<int32_t>(roff[u + 1]);
-    const int32_t center = rcenter[u];
-    for (int32_t k = -1; k < r1 - r0; ++k) {
-        const int32_t r = k < 0 ? center : r0 + k;
-        if (k >= 0 && r == center) continue;
-        const int2 bs = rboxes[r];
-        const int32_t e0 = bs.x;
-        if (e0 >= b) continue;  // only boxes before b
-        const int32_t e1 = min(bs.y, b);
-        // the own row from the own cell's first box on, wrapping round
-        const int32_t len = e1 - e0;
-        const int32_t own = cbox[u];
-        const int32_t rot = (k < 0 && own > e0 && own < e1) ? own - e0 : 0;
-        for (int32_t t = 0; t < len; ++t) {
-            const int32_t b2 = e0 + (t + rot < len ? t + rot : t + rot - len);
-            if (bmincore[b2] == INT_MAX) continue;
-            // the two bounding boxes: beyond eps of each other, nothing to
-            // test; every pair within eps, the boxes' cores meet
-            double gap2 = 0.0, far2 = 0.0;
-#pragma unroll
-            for (int j = 0; j < D; ++j) {
-                const double lo = box_lo<T, D>(bbox, b2, j), hi = box_hi<T, D>(bbox, b2, j);
-                const double g = fmax(0.0, fmax(lo - bhi[j], blo[j] - hi));
-                const double f = fmax(hi - blo[j], bhi[j] - lo);
-                gap2 += g * g;
-                far2 += f * f;
-            }
-            if (gap2 > gap2_max) continue;
-            if (far2 <= full2) {
-                bparent[b] = b2;
-                return;
-            }
-            const int32_t t0 = bstart[b2], t1 = bstart[b2 + 1];
-            int tests = 0;
-            for (int32_t p = s0; p < s1 && tests < kSmallTests; ++p) {
-                if (!core[p]) continue;
-                T pc[D];
-                load_row<T, D>(soa, ld, p, pc);
-                double gmin2, gmax2;
-                point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
-                if (gmin2 > gap2_max) continue;
-                if (gmax2 <= full2) {  // within eps of all of b2, its cores included
-                    bparent[b] = b2;
-                    return;
-                }
-                for (int32_t q = t0; q < t1 && tests < kSmallTests; ++q) {
-                    if (!core[q]) continue;
-                    ++tests;
-                    T qc[D];
-                    load_row<T, D>(soa, ld, q, qc);
-                    if (within<D>(pc, qc, eps2)) {
-                        bparent[b] = b2;
-                        return;
+            const bool none = hits == 0;
+            hits = none ? ballot(hit) & gmask : hits;
+            // (the ballot above is taken by every lane: `none` differs
+            // between groups only in which value they keep)
+            bool done = hits != 0;
+            for (uint64_t todo = ballot(open && !done); todo != 0; todo &= todo - 1) {
+                const int j = static_cast<int>(__builtin_ctzll(todo));
+                if ((ballot(done) >> j) & 1) continue;
+                const int32_t t0 = bcast(s0, j);
+                if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, min(bcast(s1, j), t0 + kWave),
+                                    bcast(b2, j), bcast(q0, j), bcast(q1, j), bcast(eps2, j),
+                                    bcast(gap2_max, j), bcast(full2, j))) {
+                    if (grp == j / G) {
+                        done = true;
+                        hits = uint64_t{1} << j;
                     }
                 }
             }
+            if (hits != 0) link = __shfl(b2, static_cast<int>(__builtin_ctzll(hits)), 64);
+            return done;
+        });
+        if (on && gl == 0 && link >= 0) {
+            if (kJoin) uf_unite(bparent, b, link);
+            else bparent[b] = link;
         }
     }
 }
 
-// Stream compaction with one atomic per block: block `blockIdx.x` takes
-// the kSelectPer * kThreads consecutive indices from blockIdx.x *
-// kSelectSpan, wave w the 64 * kSelectPer of them from w * 64 * kSelectPer,
-// in rounds of 64.  The waves' counts meet in LDS, thread 0 reserves the
-// block's range with one atomicAdd, and every taken index i is emitted at
-// its place in the range (input order inside a block; blocks in the order
-// of their reservations).  One reservation per wave instead serialises
-// thousands of atomics on one address.
-constexpr int kSelectPer = 8;
-constexpr int kSelectSpan = kThreads * kSelectPer;
+// The exact union: every listed box meets the later boxes of its
+// neighbourhood that are in another snapshot tree (rsnap) and within eps
+// (bounding boxes) -- the open pairs, counted in *nopen.  A pair is skipped
+// when the two boxes are joined by now (live roots); two boxes wholly within
+// eps of each other join at once; small pairs are tested by their lane; a
+// pair with a box of more than kHeavyRows rows leaves an entry per kHeavyRows
+// of that box in heavy (up to heavy_cap entries; beyond, the wave tests it
+// here) and the others are tested by the wave.
+constexpr int kHeavyRows = 2048;
 
-template <typename Take, typename Emit>
-__device__ __forceinline__ void block_select(int64_t n, unsigned int* count, Take take,
-                                             Emit emit) {
-    __shared__ unsigned int wcount[kWavesPerBlock];
-    __shared__ unsigned int bbase;
-    const int w = static_cast<int>(threadIdx.x >> 6);
-    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kSelectSpan +
-                       static_cast<int64_t>(w) * kWave * kSelectPer + lane_id();
-    uint64_t masks[kSelectPer];
-    unsigned int total = 0;
+template <typename T, int D>
+__global__ __launch_bounds__(kThreads) void k_box_union(
+    const BoxArgs<T> a, const uint32_t* __restrict__ roff, const int2* __restrict__ rboxes,
+    const int32_t* __restrict__ rsnap, const uint8_t* __restrict__ core,
+    const int32_t* __restrict__ blist, const unsigned int* __restrict__ nlist_dev,
+    int32_t* bparent, int2* __restrict__ heavy, unsigned long long* __restrict__ nheavy,
+    unsigned long long heavy_cap, unsigned long long* __restrict__ nopen) {
+    constexpr int G = kGroup<D>;
+    constexpr int kPer = 64 / G;
+    const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
+    const int grp = lane_id() / G;
+    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    unsigned long long opened = 0;
+    for (int32_t base = first_wave() * kPer; base < nlist; base += wave_stride() * kPer) {
+        const bool on = base + grp < nlist;
+        const int32_t b = blist[on ? base + grp : nlist - 1];
+        const int32_t s0 = a.bstart[b], s1 = a.bstart[b + 1];
+        const int32_t sb = rsnap[b];
+        const int32_t u = a.bcell[b];
+        const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
+        const T eps2 = jp.eps2;
+        const double gap2_max = jp.gap2_max;
+        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
+        double lo[D], hi[D];
 #pragma unroll
-    for (int r = 0; r < kSelectPer; ++r) {
-        const int64_t i = i0 + r * kWave;
-        masks[r] = ballot(i < n && take(i));
-        total += static_cast<unsigned int>(__popcll(masks[r]));
+        for (int j = 0; j < D; ++j) {
+            lo[j] = box_lo<T, D>(bbox, b, j);
+            hi[j] = box_hi<T, D>(bbox, b, j);
+        }
+        const int32_t r0 = static_cast<int32_t>(roff[u]);
+        group_boxes<G>(on, r0, static_cast<int32_t>(roff[u + 1]), r0, -1, rboxes, b + 1, INT_MAX,
+                       [&](bool valid, int32_t b2) {
+            const int32_t s2 = valid ? rsnap[b2] : -1;
+            bool open = false, whole = false;
+            if (s2 >= 0 && s2 != sb) {
+                double gap2, far2;
+                box_gap<T, D>(bbox, b2, lo, hi, gap2, far2);
+                open = gap2 <= gap2_max;
+                whole = far2 <= full2;
+                opened += open ? 1 : 0;
+            }
+            if (!__any(open)) return false;
+            int32_t q0 = 0, q1 = 0;
+            if (open) {
+                const int32_t r = uf_find(bparent, sb), r2 = uf_find(bparent, s2);
+                open = r != r2;
+                if (open) {
+                    q0 = a.bstart[b2];
+                    q1 = a.bstart[b2 + 1];
+                    const int64_t tests = static_cast<int64_t>(s1 - s0) * (q1 - q0);
+                    if (whole || tests <= kLanePair) {
+                        if (whole || lane_pair<T, D>(a.soa, a.ld, core, s0, s1, q0, q1, eps2))
+                            uf_unite(bparent, r, r2);
+                        open = false;
+                    }
+                }
+            }
+            for (uint64_t todo = ballot(open); todo != 0; todo &= todo - 1) {
+                const int j = static_cast<int>(__builtin_ctzll(todo));
+                const int32_t bj = bcast(b, j), b2j = bcast(b2, j);
+                const int32_t r = uniform(uf_find(bparent, bj));
+                const int32_t r2 = uniform(uf_find(bparent, b2j));
+                if (r == r2) continue;
+                const int32_t t0 = bcast(s0, j), t1 = bcast(s1, j);
+                const int32_t v0 = bcast(q0, j), v1 = bcast(q1, j);
+                if (max(t1 - t0, v1 - v0) > kHeavyRows) {
+                    // the larger box by parts, each against the other box
+                    const bool mine = t1 - t0 >= v1 - v0;
+                    const int32_t x0 = mine ? t0 : v0, x1 = mine ? t1 : v1;
+                    const int32_t k = (x1 - x0 + kHeavyRows - 1) / kHeavyRows;
+                    unsigned long long at = 0;
+                    if (lane_id() == 0) at = atomicAdd(nheavy, static_cast<unsigned long long>(k));
+                    at = bcast64(at, 0);
+                    const bool fits = at + static_cast<unsigned long long>(k) <= heavy_cap;
+                    // (the entries of a range that does not fit do nothing)
+                    for (int32_t e = lane_id(); e < k && at + e < heavy_cap; e += kWave)
+                        heavy[at + e] = fits ? make_int2(x0 + e * kHeavyRows, mine ? b2j : bj)
+                                             : make_int2(-1, -1);
+                    if (fits) continue;
+                }
+                if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, t1, b2j, v0, v1, bcast(eps2, j),
+                                    bcast(gap2_max, j), bcast(full2, j)) &&
+                    lane_id() == 0)
+                    uf_unite(bparent, r, r2);
+            }
+            return false;
+        });
     }
-    if (lane_id() == 0) wcount[w] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned int t = 0;
-#pragma unroll
-        for (int k = 0; k < kWavesPerBlock; ++k) t += wcount[k];
-        bbase = t ? atomicAdd(count, t) : 0u;
-    }
-    __syncthreads();
-    unsigned int base = bbase;
-    for (int k = 0; k < w; ++k) base += wcount[k];
-    const uint64_t lt = lanemask_lt();
-#pragma unroll
-    for (int r = 0; r < kSelectPer; ++r) {
-        if ((masks[r] >> lane_id()) & 1ull)
-            emit(i0 + r * kWave, base + static_cast<unsigned int>(__popcll(masks[r] & lt)));
-        base += static_cast<unsigned int>(__popcll(masks[r]));
+    block_add<kThreads>(opened, nopen);
+}
+
+// The heavy entries (first slot of a part of a box, other box), one wave
+// each: the part's core rows against the other box, unless the two are
+// joined by now (looked at again every 64 rows).
+template <typename T, int D>
+__global__ __launch_bounds__(kThreads) void k_box_union_heavy(
+    const BoxArgs<T> a, const int32_t* __restrict__ box_of_slot, const uint8_t* __restrict__ core,
+    int32_t* bparent, const int2* __restrict__ heavy,
+    const unsigned long long* __restrict__ nheavy, unsigned long long heavy_cap) {
+    const unsigned long long found = *nheavy;
+    const int32_t n = uniform(static_cast<int32_t>(found < heavy_cap ? found : heavy_cap));
+    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    for (int32_t w = first_wave(); w < n; w += wave_stride()) {
+        const int32_t x0 = uniform(heavy[w].x), b2 = uniform(heavy[w].y);
+        if (x0 < 0) continue;
+        const int32_t b = uniform(box_of_slot[x0]);
+        const int32_t x1 = min(uniform(a.bstart[b + 1]), x0 + kHeavyRows);
+        const int32_t q0 = uniform(a.bstart[b2]), q1 = uniform(a.bstart[b2 + 1]);
+        const JobParams<T>& jp = a.jobs[uniform(a.job_of_cell[uniform(a.bcell[b])])];
+        const double full2 = static_cast<double>(jp.eps2) * (1.0 - 1e-5);
+        for (int32_t c = x0; c < x1; c += kWave) {
+            const int32_t r = uniform(uf_find(bparent, b));
+            const int32_t r2 = uniform(uf_find(bparent, b2));
+            if (r == r2) break;
+            if (wave_pair<T, D>(a.soa, a.ld, core, bbox, c, min(c + kWave, x1), b2, q0, q1, jp.eps2,
+                                jp.gap2_max, full2)) {
+                if (lane_id() == 0) uf_unite(bparent, r, r2);
+                break;
+            }
+        }
     }
 }
 
-// list[...] = every box b with (mode 0) cores (v = bmincore != INT_MAX) /
-// (mode 1) v[b] == b (a root); *count += their number
-__global__ __launch_bounds__(kThreads) void k_select_boxes(Count nbox_c, int mode,
-                                                           const int32_t* __restrict__ v,
-                                                           int32_t* __restrict__ list,
-                                                           unsigned int* __restrict__ count,
-                                                           const int32_t* __restrict__ bstart) {
-    const int32_t nbox = static_cast<int32_t>(nbox_c.get());
-    block_select(
-        nbox, count,
-        [&](int64_t b) {
-            if (mode == 1) return v[b] == static_cast<int32_t>(b);
-            return v[b] != INT_MAX && (mode == 0 || bstart[b + 1] - bstart[b] > kSmallBox);
-        },
-        [&](int64_t b, unsigned int pos) { list[pos] = static_cast<int32_t>(b); });
-}
-
-// the 64-slot chunks of the boxes that have open pairs (off[b+1] > off[b])
-__global__ __launch_bounds__(kThreads) void k_select_items(Count nitems_c,
-                                                           const int2* __restrict__ items,
-                                                           const uint32_t* __restrict__ off,
-                                                           const int32_t* __restrict__ bstart,
-                                                           int32_t min_rows,
-                                                           int2* __restrict__ out,
-                                                           unsigned int* __restrict__ count) {
-    const int32_t nitems = static_cast<int32_t>(nitems_c.get());
-    block_select(
-        nitems, count,
-        [&](int64_t i) {
-            const int32_t b = items[i].x;
-            return off[b + 1] > off[b] && (!bstart || bstart[b + 1] - bstart[b] > min_rows);
-        },
-        [&](int64_t i, unsigned int pos) { out[pos] = items[i]; });
+// list[...] = every box with cores (v = bmincore != INT_MAX); *count +=
+// their number; every box a root of its own (bparent)
+__global__ __launch_bounds__(kThreads) void k_list_boxes(Count nbox_c,
+                                                         const int32_t* __restrict__ bmincore,
+                                                         int32_t* __restrict__ list,
+                                                         unsigned int* __restrict__ count,
+                                                         int32_t* __restrict__ bparent) {
+    block_collect(nbox_c.get(), list, count, [&](int64_t b, int32_t& v) {
+        v = static_cast<int32_t>(b);
+        bparent[b] = v;
+        return bmincore[b] != INT_MAX;
+    });
 }
 
 __global__ __launch_bounds__(kThreads) void k_core_init(
@@ -899,113 +729,21 @@ __global__ __launch_bounds__(kThreads) void k_core_init(
     });
 }
 
-// root of every box's hook tree -> rsnap (-1 for boxes without cores)
+// root of every box's tree -> rsnap (-1 for boxes without cores); with a
+// list, the roots go there (*count += their number)
 __global__ __launch_bounds__(kThreads) void k_box_roots(Count nbox_c,
                                                         const int32_t* __restrict__ bmincore,
                                                         int32_t* bparent,
-                                                        int32_t* __restrict__ rsnap) {
-    const int32_t nbox = static_cast<int32_t>(nbox_c.get());
-    const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (b >= nbox) return;
-    rsnap[b] = bmincore[b] == INT_MAX ? -1 : uf_find(bparent, b);
-}
-
-// Box-level union: one wave per 64-slot chunk of a box with cores; lanes
-// own the chunk's rows.  Neighbour boxes come from the cell's neighbour rows
-// (cells [a, b) -> boxes [cbox[a], cbox[b])); each unordered box pair is
-// tested by the chunks of its lower box.  A pair is skipped when the boxes
-// are already joined (live roots) or their bounding boxes are farther apart
-// than eps; otherwise the lanes whose row is a core within eps of the other
-// box's bounding box test the other box's cores as they stream through the
-// wave, until the first within-eps pair, which joins the two boxes.
-// One chunk of k_box_union.
-template <typename T, int D>
-__device__ __forceinline__ void box_union_item(
-    const T* __restrict__ soa, int64_t ld, const int2* __restrict__ bitems,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
-    const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
-    const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
-    const int32_t* __restrict__ rsnap, int32_t* bparent, int32_t wid) {
-    const int2 it = bitems[wid];
-    const int32_t b = uniform(it.x);
-    if (bmincore[b] == INT_MAX) return;
-    const int32_t sb = uniform(rsnap[b]);
-    const int32_t end = uniform(bstart[b + 1]);
-    const int32_t p = it.y + lane_id();
-    const bool pcore = p < end && core[p];
-    if (!__any(pcore)) return;
-    const int32_t u = uniform(bcell[b]);
-    const JobParams<T>& jp = jobs[uniform(job_of_cell[u])];
-    const T eps2 = jp.eps2;
-    const double gap2_max = jp.gap2_max;
-    T pc[D];
-    load_row<T, D>(soa, ld, pcore ? p : it.y, pc);
-    double lo[D], hi[D];
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        lo[j] = box_lo<T, D>(bbox, b, j);
-        hi[j] = box_hi<T, D>(bbox, b, j);
-    }
-    int32_t rb = uniform(uf_find(bparent, b));
-    const int32_t r0 = uniform(static_cast<int32_t>(roff[u]));
-    const int32_t r1 = uniform(static_cast<int32_t>(roff[u + 1]));
-    for (int32_t r = r0; r < r1; ++r) {
-        const int2 bs = rboxes[r];
-        const int32_t e0 = uniform(bs.x);
-        const int32_t e1 = uniform(bs.y);
-        for (int32_t b2 = max(e0, b + 1); b2 < e1; ++b2) {
-            // joined by the hook forest already, or no cores (rsnap -1)
-            const int32_t s2 = uniform(rsnap[b2]);
-            if (s2 == sb || s2 < 0) continue;
-            double gap2 = 0.0, pgap2 = 0.0;
-#pragma unroll
-            for (int j = 0; j < D; ++j) {
-                const double lo2 = box_lo<T, D>(bbox, b2, j);
-                const double hi2 = box_hi<T, D>(bbox, b2, j);
-                const double g = fmax(0.0, fmax(lo2 - hi[j], lo[j] - hi2));
-                gap2 += g * g;
-                const double v = static_cast<double>(pc[j]);
-                const double h = fmax(0.0, fmax(lo2 - v, v - hi2));
-                pgap2 += h * h;
-            }
-            if (gap2 > gap2_max) continue;
-            const bool act = pcore && pgap2 <= gap2_max;
-            if (!__any(act)) continue;
-            const int32_t rb2 = uniform(uf_find(bparent, b2));
-            rb = uniform(uf_find(bparent, rb));
-            if (rb2 == rb) continue;
-            if (any_pair<T, D>(soa, ld, core, uniform(bstart[b2]), uniform(bstart[b2 + 1]), pc, act,
-                               eps2)) {
-                if (lane_id() == 0) uf_unite(bparent, rb, rb2);
-                rb = uniform(uf_find(bparent, b));
-            }
-        }
-    }
-}
-
-// The full union walk: every box chunk against the later boxes of its
-// neighbourhood.  The fallback when the open-pair lists do not fit, so it is
-// launched on a small grid whose waves walk the chunks (only_over: run only
-// when *only_over > cap, decided on the device).
-template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_union(
-    const T* __restrict__ soa, int64_t ld, const int2* __restrict__ bitems, int32_t nitems,
-    const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
-    const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
-    const int2* __restrict__ rboxes, const OrdKey<T>* __restrict__ bbox,
-    const int32_t* __restrict__ bmincore, const uint8_t* __restrict__ core,
-    const int32_t* __restrict__ job_of_cell, const JobParams<T>* __restrict__ jobs,
-    const int32_t* __restrict__ rsnap, int32_t* bparent,
-    const unsigned long long* __restrict__ only_over, unsigned long long cap) {
-    if (only_over && *only_over <= cap) return;
-    const int32_t stride = static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-    for (int32_t wid = uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
-                               static_cast<int32_t>(threadIdx.x >> 6));
-         wid < nitems; wid += stride)
-        box_union_item<T, D>(soa, ld, bitems, bstart, bcell, cbox, roff, rboxes, bbox, bmincore,
-                             core, job_of_cell, jobs, rsnap, bparent, wid);
+                                                        int32_t* __restrict__ rsnap,
+                                                        int32_t* __restrict__ list,
+                                                        unsigned int* __restrict__ count) {
+    block_collect(nbox_c.get(), list, count, [&](int64_t i, int32_t& v) {
+        const int32_t b = static_cast<int32_t>(i);
+        const int32_t r = bmincore[b] == INT_MAX ? -1 : uf_find(bparent, b);
+        rsnap[b] = r;
+        v = b;
+        return list && r == b;
+    });
 }
 
 // Cluster ids.  A sorted position orders rows by (occupied cell, input
@@ -1077,17 +815,6 @@ __global__ __launch_bounds__(kThreads) void k_box_cluster(Count nbox_c,
     bcluster[b] = bmincore[b] == INT_MAX ? -1 : compmin[uf_find(bparent, b)];
 }
 
-__global__ __launch_bounds__(kThreads) void k_box_items_count(const int32_t* __restrict__ bstart,
-                                                              Count nbox_c,
-                                                              uint32_t* __restrict__ cnt) {
-    const int32_t nbox = static_cast<int32_t>(nbox_c.get());
-    const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (b >= nbox) return;
-    cnt[b] = static_cast<uint32_t>((bstart[b + 1] - bstart[b] + kWave - 1) / kWave);
-}
-
-
-
 __global__ __launch_bounds__(kThreads) void k_fill_u64(unsigned long long* __restrict__ a,
                                                        unsigned long long v, int64_t n) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
@@ -1098,11 +825,6 @@ __global__ __launch_bounds__(kThreads) void k_fill_i32(int32_t* __restrict__ a, 
                                                        int64_t n) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i < n) a[i] = v;
-}
-
-__global__ __launch_bounds__(kThreads) void k_iota_i32(int32_t* __restrict__ a, int64_t n) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i < n) a[i] = static_cast<int32_t>(i);
 }
 
 }  // namespace
@@ -1185,24 +907,6 @@ void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* b
     HPD_HIP(hipGetLastError());
 }
 
-void launch_box_items(const int32_t* bstart, Count nbox, uint32_t* cnt, uint32_t* scan_tmp,
-                      uint32_t* total_dev, hipStream_t s) {
-    if (nbox.host > 0)
-        hipLaunchKernelGGL(k_box_items_count, dim3(blocks_for(nbox.host, kThreads)), dim3(kThreads),
-                           0, s, bstart, nbox, cnt);
-    if (nbox.dev) {
-        exclusive_scan_u32_dev(cnt, cnt, nbox, scan_tmp, s);
-        copy_at_count(cnt, nbox.dev, total_dev, s);
-    } else {
-        exclusive_scan_u32(cnt, cnt, nbox.host, scan_tmp, total_dev, s);
-    }
-}
-
-void launch_box_items_fill(const int32_t* bstart, Count nbox, const uint32_t* off, Count nitems,
-                           int2* items, hipStream_t s) {
-    launch_expand_chunks(off, nbox, bstart, nitems, items, s);
-}
-
 template <typename T, int D>
 void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
                       unsigned int* nloose, hipStream_t s) {
@@ -1213,68 +917,40 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
                        a.bcell, a.job_of_cell, a.jobs, cell_core, btight, nloose);
 }
 
-// A grid of waves for a count of work items: one wave per item of a
-// host-known count (the kernels' wave loops then run once), at most
-// kMaxItemWaves, which walk a larger count.  For a count an earlier kernel
-// wrote (the host holds a bound, n or n + n / 64) one wave per item up to an
-// eighth of the bound, which walk the items beyond it: every wave past the
-// count costs a dispatch.
-constexpr int64_t kMaxItemWaves = int64_t{1} << 24;
-inline unsigned wave_blocks(Count items) {
-    int64_t w = items.dev && !items.tight ? std::min(items.host, items.host / 8 + 64) : items.host;
-    w = std::min(w, kMaxItemWaves);
-    return blocks_for(w > 0 ? w : 1, kWavesPerBlock);
+void launch_list_boxes(Count nbox, const int32_t* bmincore, int32_t* list, unsigned int* count,
+                       int32_t* bparent, hipStream_t s) {
+    if (nbox.host <= 0) return;
+    hipLaunchKernelGGL(k_list_boxes, dim3(collect_blocks(nbox.host)), dim3(kThreads), 0, s, nbox,
+                       bmincore, list, count, bparent);
+    HPD_HIP(hipGetLastError());
 }
 
 template <typename T, int D>
 void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
-                     Count nlist, int32_t* bparent, int32_t* big, unsigned int* nbig,
-                     hipStream_t s) {
-    using U = OrdKey<T>;
-    if (a.nbox > 0)
-        hipLaunchKernelGGL(k_iota_i32, dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0, s,
-                           bparent, static_cast<int64_t>(a.nbox));
-    if (nlist.host > 0) {
-        // the larger boxes one wave each (first: their hooks are found
-        // soonest), the small ones one thread each
-        const Count nb{nlist.host, nbig};
-        hipLaunchKernelGGL((k_box_hook<T, D>), dim3(wave_blocks(nb)), dim3(kThreads), 0, s, a.soa,
-                           a.ld, big, nb, a.bstart, a.bcell, a.cbox, roff, rboxes,
-                           reinterpret_cast<const U*>(a.bbox), bmincore, core, a.job_of_cell, a.jobs,
-                           a.rcenter, bparent);
-        hipLaunchKernelGGL((k_box_hook_small<T, D>), dim3(blocks_for(nlist.host, kThreads)),
-                           dim3(kThreads), 0, s, a.soa, a.ld, blist, nlist, a.bstart, a.bcell,
-                           a.cbox, roff, rboxes, a.rcenter, reinterpret_cast<const U*>(a.bbox),
-                           bmincore, core, a.job_of_cell, a.jobs, bparent);
-    }
+                     const unsigned int* nlist, int32_t* bparent, hipStream_t s) {
+    if (a.nbox <= 0) return;
+    hipLaunchKernelGGL((k_box_link<T, D, false>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0,
+                       s, a, roff, rboxes, bmincore, core, blist, nlist, bparent);
+    HPD_HIP(hipGetLastError());
 }
 
 void launch_box_roots(Count nbox, const int32_t* bmincore, int32_t* bparent, int32_t* rsnap,
-                      hipStream_t s) {
+                      int32_t* list, unsigned int* count, hipStream_t s) {
     if (nbox.host <= 0) return;
-    hipLaunchKernelGGL(k_box_roots, dim3(blocks_for(nbox.host, kThreads)), dim3(kThreads), 0, s,
-                       nbox, bmincore, bparent, rsnap);
+    hipLaunchKernelGGL(k_box_roots, dim3(collect_blocks(nbox.host)), dim3(kThreads), 0, s, nbox,
+                       bmincore, bparent, rsnap, list, count);
+    HPD_HIP(hipGetLastError());
 }
 
 template <typename T, int D>
 void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                          const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
-                          Count nlist, int32_t* bparent, hipStream_t s) {
-    using U = OrdKey<T>;
-    if (nlist.host <= 0) return;
-    hipLaunchKernelGGL((k_box_root_join<T, D>), dim3(wave_blocks(nlist)), dim3(kThreads), 0, s,
-                       a.soa, a.ld, blist, nlist, a.bstart, a.bcell, a.cbox, roff, rboxes,
-                       reinterpret_cast<const U*>(a.bbox), rsnap, core, a.job_of_cell, a.jobs,
-                       a.rcenter, bparent);
-}
-
-void launch_select_boxes(Count nbox, int mode, const int32_t* v, int32_t* list,
-                         unsigned int* count, hipStream_t s, const int32_t* bstart) {
-    if (nbox.host <= 0) return;
-    if (mode == 2 && !bstart) throw Error(HPD_EINVAL, "launch_select_boxes: mode 2 needs bstart");
-    hipLaunchKernelGGL(k_select_boxes, dim3(blocks_for(nbox.host, kSelectSpan)), dim3(kThreads), 0,
-                       s, nbox, mode, v, list, count, bstart);
+                          const int32_t* rsnap, const uint8_t* core, const int32_t* roots,
+                          const unsigned int* nroots, int32_t* bparent, hipStream_t s) {
+    if (a.nbox <= 0) return;
+    hipLaunchKernelGGL((k_box_link<T, D, true>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0,
+                       s, a, roff, rboxes, rsnap, core, roots, nroots, bparent);
+    HPD_HIP(hipGetLastError());
 }
 
 void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
@@ -1287,62 +963,21 @@ void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btig
     HPD_HIP(hipGetLastError());
 }
 
-void launch_select_items(Count nitems, const int2* items, const uint32_t* off, int2* out,
-                         unsigned int* count, hipStream_t s, const int32_t* bstart,
-                         int32_t min_rows) {
-    if (nitems.host <= 0) return;
-    hipLaunchKernelGGL(k_select_items, dim3(blocks_for(nitems.host, kSelectSpan)), dim3(kThreads),
-                       0, s, nitems, items, off, min_rows > 0 ? bstart : nullptr, min_rows, out,
-                       count);
-}
-
-int32_t small_union_rows(int64_t n, int64_t nbox) {
-    return nbox > 0 && n < kSmallUnionMean * nbox ? kSmallUnionRows : 0;
-}
-
 template <typename T, int D>
-void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                     const int32_t* bmincore, const uint8_t* core, const int32_t* rsnap,
-                     int32_t* bparent, hipStream_t s, const unsigned long long* only_over,
-                     unsigned long long cap) {
-    using U = OrdKey<T>;
-    if (a.nbitems <= 0) return;
-    const int64_t waves = std::min<int64_t>(a.nbitems, 32768);
-    hipLaunchKernelGGL((k_box_union<T, D>), dim3(blocks_for(waves, kWavesPerBlock)),
-                       dim3(kThreads), 0, s, a.soa, a.ld, a.bitems, a.nbitems, a.bstart, a.bcell,
-                       a.cbox, roff, rboxes, reinterpret_cast<const U*>(a.bbox), bmincore, core,
-                       a.job_of_cell, a.jobs, rsnap, bparent, only_over, cap);
-}
-
-template <typename T, int D>
-void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                     const int32_t* rsnap, uint32_t* cnt, int32_t* list,
-                     unsigned long long* total, hipStream_t s,
-                     const unsigned long long* total_chk, unsigned long long cap) {
-    using U = OrdKey<T>;
+void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
+                      const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
+                      const unsigned int* nlist, const int32_t* box_of_slot, int2* heavy,
+                      unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
+                      unsigned long long* nopen, hipStream_t s) {
     if (a.nbox <= 0) return;
-    hipLaunchKernelGGL((k_box_scan<T, D>), dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0,
-                       s, Count{a.nbox, a.nbox_dev}, a.bcell, a.cbox, roff, rboxes,
-                       reinterpret_cast<const U*>(a.bbox), a.job_of_cell, a.jobs, rsnap, cnt, list,
-                       total, total_chk, cap);
-}
-
-template <typename T, int D>
-void launch_box_union_list(const BoxArgs<T>& a, const int2* items, Count nitems,
-                           const uint8_t* core, const uint32_t* off, const int32_t* list,
-                           int32_t* bparent, hipStream_t s, const unsigned long long* total_chk,
-                           unsigned long long cap, int32_t small_rows) {
-    using U = OrdKey<T>;
-    if (a.nbox > 0 && small_rows > 0)
-        hipLaunchKernelGGL((k_box_union_small<T, D>), dim3(blocks_for(a.nbox, kThreads)),
-                           dim3(kThreads), 0, s, a.soa, a.ld, Count{a.nbox, a.nbox_dev}, a.bstart,
-                           a.bcell, reinterpret_cast<const U*>(a.bbox), core, a.job_of_cell,
-                           a.jobs, off, list, bparent, total_chk, cap, small_rows);
-    if (nitems.host <= 0) return;
-    hipLaunchKernelGGL((k_box_union_list<T, D>), dim3(wave_blocks(nitems)), dim3(kThreads), 0, s,
-                       a.soa, a.ld, items, nitems, a.bstart, a.bcell,
-                       reinterpret_cast<const U*>(a.bbox), core, a.job_of_cell, a.jobs, off, list,
-                       bparent, total_chk, cap);
+    hipLaunchKernelGGL((k_box_union<T, D>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0, s, a,
+                       roff, rboxes, rsnap, core, blist, nlist, bparent, heavy, nheavy, heavy_cap,
+                       nopen);
+    // (its waves leave at once when there are no entries)
+    hipLaunchKernelGGL((k_box_union_heavy<T, D>), dim3(group_blocks<1>(a.nrows)), dim3(kThreads), 0,
+                       s, a, box_of_slot, core, bparent, static_cast<const int2*>(heavy),
+                       static_cast<const unsigned long long*>(nheavy), heavy_cap);
+    HPD_HIP(hipGetLastError());
 }
 
 void fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s) {
@@ -1409,23 +1044,16 @@ void launch_positions(int64_t n, int32_t m, const int32_t* box_of_slot, const in
     template void launch_box_tight<T, D>(const BoxArgs<T>&, const uint8_t*, uint8_t*,            \
                                          unsigned int*, hipStream_t);                                            \
     template void launch_box_hook<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,          \
-                                        const int32_t*, const uint8_t*, const int32_t*, Count,    \
-                                        int32_t*, int32_t*, unsigned int*, hipStream_t);          \
+                                        const int32_t*, const uint8_t*, const int32_t*,           \
+                                        const unsigned int*, int32_t*, hipStream_t);              \
     template void launch_box_root_join<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,     \
                                              const int32_t*, const uint8_t*, const int32_t*,      \
-                                             Count, int32_t*, hipStream_t);                       \
-    template void launch_box_join<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,          \
-                                        const int32_t*, const uint8_t*, const int32_t*, int32_t*, \
-                                        hipStream_t, const unsigned long long*,                   \
-                                        unsigned long long);                                      \
-    template void launch_box_scan<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,          \
-                                        const int32_t*, uint32_t*, int32_t*,                      \
-                                        unsigned long long*, hipStream_t,                         \
-                                        const unsigned long long*, unsigned long long);           \
-    template void launch_box_union_list<T, D>(const BoxArgs<T>&, const int2*, Count,               \
-                                              const uint8_t*, const uint32_t*, const int32_t*,    \
-                                              int32_t*, hipStream_t, const unsigned long long*,   \
-                                              unsigned long long, int32_t);
+                                             const unsigned int*, int32_t*, hipStream_t);         \
+    template void launch_box_union<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,         \
+                                         const int32_t*, const uint8_t*, const int32_t*,          \
+                                         const unsigned int*, const int32_t*, int2*,              \
+                                         unsigned long long*, unsigned long long, int32_t*,       \
+                                         unsigned long long*, hipStream_t);
 #define HPD_INST_BOX_ALL_D(T) \
     HPD_INST_BOX_KEYS(T, 1)   \
     HPD_INST_BOX_KEYS(T, 2)   \

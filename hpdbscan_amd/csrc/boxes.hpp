@@ -23,10 +23,10 @@ struct BoxArgs {
     const int32_t* bstart = nullptr;   // first slot of every box, [nbox + 1]
     const int32_t* bcell = nullptr;    // occupied cell of every box
     const int32_t* cbox = nullptr;     // first box of every cell, [m + 1]
-    const int2* bitems = nullptr;      // (box, first slot) per 64-slot chunk
-    int32_t nbitems = 0;
     void* bbox = nullptr;              // ordered-key min/max per box and dim
     const JobParams<T>* jobs = nullptr;
+    int32_t njobs = 1;
+    int64_t nrows = 0;
     const int32_t* job_of_cell = nullptr;
     const int32_t* rcenter = nullptr;  // index of every cell's own neighbour row
 };
@@ -65,12 +65,6 @@ void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* b
                            uint32_t* scan_tmp, int32_t* bcell, K* ucell, int32_t* ustart,
                            int32_t* cbox, uint32_t* ncells_dev, hipStream_t s);
 
-// cnt[b] = 64-slot chunks of box b, scanned in place; *total_dev = chunks
-void launch_box_items(const int32_t* bstart, Count nbox, uint32_t* cnt, uint32_t* scan_tmp,
-                      uint32_t* total_dev, hipStream_t s);
-void launch_box_items_fill(const int32_t* bstart, Count nbox, const uint32_t* off, Count nitems,
-                           int2* items, hipStream_t s);
-
 // btight[b]: bit 0 tight, bit 1 tight with >= minPts rows, bit 2 in a cell
 // that can hold cores (cell_core); *nloose counts boxes of two or more rows
 // that are not tight
@@ -79,36 +73,43 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
                       unsigned int* nloose, hipStream_t s);
 
 // Components of the boxes with cores:
-//   launch_select_boxes  list of the boxes with cores (mode 0, v = bmincore),
-//                        of those with more than kSmallBox rows (mode 2,
-//                        with bstart) or of the roots (mode 1, v = rsnap);
-//                        *count += n
-//   launch_box_hook      hook forest over the listed boxes (bparent is
-//                        reset first): every box points at some earlier box
-//                        joined to it; big[0, *nbig) lists the boxes of
-//                        more than kSmallBox rows (launch_select_boxes mode
-//                        2), which take one wave each
-//   launch_box_roots     root of every box -> rsnap (-1 without cores)
+//   launch_list_boxes    list of the boxes with cores, *count += their
+//                        number; bparent reset
+//   launch_box_hook      hook forest over the listed boxes: every box points
+//                        at some earlier box joined to it
+//   launch_box_roots     root of every box -> rsnap (-1 without cores), the
+//                        roots to list (when not null), *count += their number
 //   launch_box_root_join every listed root joins the first tree of another
 //                        box it meets (kRootJoinRounds rounds, each followed
 //                        by launch_box_roots)
-//   then the open pairs (below), launch_box_clusters.
+//   launch_box_union     the pairs still open (different trees in rsnap,
+//                        within eps by their bounding boxes; *nopen += their
+//                        number), every one decided exactly
+//   then launch_box_clusters.
+// List lengths stay on the device (kernels of persistent grids).  heavy
+// holds heavy_cap entries of scratch; *nheavy, *nopen and every count are
+// zeroed by the caller.
 template <int D>
 constexpr int kRootJoinRounds = D <= 3 ? 1 : 2;
 
-void launch_select_boxes(Count nbox, int mode, const int32_t* v, int32_t* list,
-                         unsigned int* count, hipStream_t s, const int32_t* bstart = nullptr);
+void launch_list_boxes(Count nbox, const int32_t* bmincore, int32_t* list, unsigned int* count,
+                       int32_t* bparent, hipStream_t s);
 template <typename T, int D>
 void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
-                     Count nlist, int32_t* bparent, int32_t* big, unsigned int* nbig,
-                     hipStream_t s);
+                     const unsigned int* nlist, int32_t* bparent, hipStream_t s);
 void launch_box_roots(Count nbox, const int32_t* bmincore, int32_t* bparent, int32_t* rsnap,
-                      hipStream_t s);
+                      int32_t* list, unsigned int* count, hipStream_t s);
 template <typename T, int D>
 void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                          const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
-                          Count nlist, int32_t* bparent, hipStream_t s);
+                          const int32_t* rsnap, const uint8_t* core, const int32_t* roots,
+                          const unsigned int* nroots, int32_t* bparent, hipStream_t s);
+template <typename T, int D>
+void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
+                      const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
+                      const unsigned int* nlist, const int32_t* box_of_slot, int2* heavy,
+                      unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
+                      unsigned long long* nopen, hipStream_t s);
 // core[s] = 1 for the rows of tight boxes with >= minPts rows (btight bit 1),
 // 0 for every other row; bmincore[b] = inrow[bstart[b]] for those boxes
 // (every row is core and a box holds its rows in input order), INT_MAX for
@@ -118,50 +119,6 @@ void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btig
                       const int32_t* bstart, const int32_t* bcell, const uint32_t* inrow,
                       uint8_t* core, int32_t* bmincore, int2* rows, unsigned int* nrows,
                       hipStream_t s);
-// out[..] = the box chunks (items) of the boxes with open pairs (off[b+1] >
-// off[b]); *count += their number
-// (with min_rows > 0: only chunks of boxes of more than min_rows rows; the
-// thread-per-box union of launch_box_union_list takes the others)
-void launch_select_items(Count nitems, const int2* items, const uint32_t* off, int2* out,
-                         unsigned int* count, hipStream_t s, const int32_t* bstart = nullptr,
-                         int32_t min_rows = 0);
-// Boxes of at most this many rows take their open pairs one thread per box
-// (0: none): on when the boxes hold fewer than kSmallUnionMean rows on
-// average (sparse data, where a wave per box leaves most lanes idle), off
-// for denser data, whose small boxes meet large ones that a wave tests
-// faster.
-constexpr int kSmallUnionRows = 8;
-constexpr int kSmallUnionMean = 8;
-int32_t small_union_rows(int64_t n, int64_t nbox);
-// only_over (optional): the join runs only when *only_over > cap, i.e. when
-// the open-pair lists did not fit (decided on the device, no host check).
-template <typename T, int D>
-void launch_box_join(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                     const int32_t* bmincore, const uint8_t* core, const int32_t* rsnap,
-                     int32_t* bparent, hipStream_t s, const unsigned long long* only_over = nullptr,
-                     unsigned long long cap = 0);
-
-// The pairs the hook forest leaves open.  launch_box_scan with list ==
-// nullptr writes cnt[b] (nbox entries) and adds their sum to *total (64-bit,
-// zeroed by the caller); with a list it writes every box's open partners to
-// list[cnt[b] ..] (cnt scanned to offsets in between).
-// launch_box_union_list joins the listed pairs that hold a within-eps core
-// pair (boxes of at most small_rows rows one thread per box, the items --
-// chunks of the other boxes -- one wave each); off has nbox + 1 entries.  When the list does not fit, the caller
-// runs launch_box_join instead.  With total_chk (no host check in between),
-// both do nothing when *total_chk > cap, and launch_box_join with the same
-// check runs exactly then.
-template <typename T, int D>
-void launch_box_scan(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
-                     const int32_t* rsnap, uint32_t* cnt, int32_t* list,
-                     unsigned long long* total, hipStream_t s,
-                     const unsigned long long* total_chk = nullptr, unsigned long long cap = 0);
-template <typename T, int D>
-void launch_box_union_list(const BoxArgs<T>& a, const int2* items, Count nitems,
-                           const uint8_t* core, const uint32_t* off, const int32_t* list,
-                           int32_t* bparent, hipStream_t s,
-                           const unsigned long long* total_chk = nullptr,
-                           unsigned long long cap = 0, int32_t small_rows = 0);
 // p[0, n) = v
 void fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 

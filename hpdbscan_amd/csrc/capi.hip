@@ -442,7 +442,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     // reference's sorted positions are only materialised where needed
     uint32_t* pos_of_slot = nullptr;
     int32_t *box_of_slot = nullptr, *bstart = nullptr, *bcell = nullptr, *cbox = nullptr;
-    uint32_t* bcnt = nullptr;
     int32_t *bmincore = nullptr, *bparent = nullptr, *compmin = nullptr, *bcluster = nullptr;
     uint8_t* btight = nullptr;
     void* bbox = nullptr;
@@ -454,7 +453,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         bstart = A.take_n<int32_t>(nn + 1);
         bcell = A.take_n<int32_t>(nn);
         cbox = A.take_n<int32_t>(nn + 1);
-        bcnt = A.take_n<uint32_t>(nn + 1);
         bmincore = A.take_n<int32_t>(nn);
         bparent = A.take_n<int32_t>(nn);
         compmin = A.take_n<int32_t>(nn);
@@ -516,9 +514,8 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     if (!boxes) counts.a[ncounts++] = nchunks;
     exclusive_scan_set_u32(counts, ncounts, m, tmp, tmp_words, s);
     if (boxes) {
-        // the box chunks (counted and scanned) and the box flags (their
-        // loose count decides the union) before the read-back below
-        launch_box_items(bstart, host_count(nbox), bcnt, tmp, &counters[4], s);
+        // the box flags (their loose count decides the union) before the
+        // read-back below
         BoxArgs<T> bt;
         bt.nbox = nbox;
         bt.bstart = bstart;
@@ -543,7 +540,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     // 64-bit total first
     check_neighbor_rows(*hs_rows);
     const uint32_t total_ranges = hc[1];
-    const int32_t nbitems = boxes ? static_cast<int32_t>(hc[4]) : 0;
     // every box of two or more rows is tight: the union runs on boxes
     const bool all_tight = boxes && hc[5] == 0;
     const bool one_thread = ctx.border_rule == HPD_BORDER_ONE_THREAD;
@@ -555,14 +551,11 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
 
     const size_t range_bytes = align_up(static_cast<size_t>(total_ranges) * sizeof(int2), 256);
     X.reserve((boxes ? range_bytes : 0) + (row_tables ? 2 * range_bytes : 0) +
-              (row_tables ? align_up(max_items * sizeof(int2), 256) : 0) +
-              2 * align_up(static_cast<size_t>(nbitems) * sizeof(int2), 256) + 2048);
+              (row_tables ? align_up(max_items * sizeof(int2), 256) : 0) + 2048);
     int2* rboxes = boxes ? X.take_n<int2>(total_ranges) : nullptr;
     int2* ranges = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
     int2* rcells = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
     int2* items = row_tables ? X.take_n<int2>(max_items) : nullptr;
-    int2* bitems = boxes ? X.take_n<int2>(static_cast<size_t>(nbitems)) : nullptr;
-    int2* uitems = boxes ? X.take_n<int2>(static_cast<size_t>(nbitems)) : nullptr;
     if (boxes && stash)
         launch_neighbor_copy(stash, stash_rows, m, nranges, cbox, rboxes, rcenter, by_class, s);
     else if (boxes)
@@ -596,17 +589,16 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     BoxArgs<T> ba;
     bool box_union = false;
     if (boxes) {
-        launch_box_items_fill(bstart, host_count(nbox), bcnt, host_count(nbitems), bitems, s);
         ba.soa = soa;
         ba.ld = ld;
         ba.nbox = nbox;
         ba.bstart = bstart;
         ba.bcell = bcell;
         ba.cbox = cbox;
-        ba.bitems = bitems;
-        ba.nbitems = nbitems;
         ba.bbox = bbox;
         ba.jobs = jobs;
+        ba.njobs = njobs;
+        ba.nrows = n;
         ba.job_of_cell = job_of_cell;
         ba.rcenter = rcenter;
         a.box_of_slot = box_of_slot;
@@ -643,47 +635,29 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
 
     // box lists of the union (box mode leaves the slot-level parent free)
     // (the lists' lengths stay on the device: boxes with cores, and the
-    // roots of each join round, bounded by the number of boxes)
+    // roots of each join round)
     int32_t* blist = parent;
     box_union = all_tight;
     if (box_union) {
         // compmin holds the forest's roots until the clusters are known
         tm.mark(M_HOOK0);
-        launch_select_boxes(host_count(nbox), 0, bmincore, blist, &counters[8], s);
-        // (the slot-level union's rsnap is free in box mode: the list of
-        // the larger boxes)
-        launch_select_boxes(host_count(nbox), 2, bmincore, rsnap, &counters[14], s, bstart);
-        launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist,
-                              Count{nbox, &counters[8], true}, bparent, rsnap, &counters[14], s);
-        launch_box_roots(host_count(nbox), bmincore, bparent, compmin, s);
+        launch_list_boxes(host_count(nbox), bmincore, blist, &counters[8], bparent, s);
+        launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &counters[8], bparent, s);
+        // (the slot-level union's rsnap is free in box mode: the roots)
         for (int round = 0; round < kRootJoinRounds<D>; ++round) {
-            HPD_HIP(hipMemsetAsync(&counters[9], 0, sizeof(uint32_t), s));
-            launch_select_boxes(host_count(nbox), 1, compmin, blist, &counters[9], s);
-            launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, blist,
-                                       Count{nbox, &counters[9]}, bparent, s);
-            launch_box_roots(host_count(nbox), bmincore, bparent, compmin, s);
+            launch_box_roots(host_count(nbox), bmincore, bparent, compmin, rsnap,
+                             &counters[9 + round], s);
+            launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, rsnap,
+                                       &counters[9 + round], bparent, s);
         }
+        launch_box_roots(host_count(nbox), bmincore, bparent, compmin, nullptr, nullptr, s);
         tm.mark(M_HOOK1);
-        // the open pairs of every box, as a list in scratch64; offsets in
-        // bcnt (free after the box items)
-        int32_t* list = reinterpret_cast<int32_t*>(scratch64);
-        unsigned long long cap = 2 * static_cast<unsigned long long>(nn);
+        // pairs with a large box go through a list in scratch64
+        unsigned long long cap = static_cast<unsigned long long>(nn);
         if (ctx.open_pair_limit > 0 && ctx.open_pair_limit < cap) cap = ctx.open_pair_limit;
-        launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, nullptr, &dstats[5], s);
-        // offsets (meaningful when the total fits; the kernels that use them
-        // check the 64-bit total on the device, and the full join runs
-        // instead when it does not fit) and the chunks of the boxes that
-        // have open pairs
-        exclusive_scan_u32(bcnt, bcnt, nbox, tmp, &bcnt[nbox], s);
-        // sparse data: the small boxes' pairs one thread per box
-        const int32_t small_rows = small_union_rows(n, nbox);
-        launch_select_items(host_count(nbitems), bitems, bcnt, uitems, &counters[10], s, bstart,
-                            small_rows);
-        launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
-        launch_box_union_list<T, D>(ba, uitems, Count{nbitems, &counters[10]}, core, bcnt, list,
-                                    bparent, s, &dstats[5], cap, small_rows);
-        launch_box_join<T, D>(ba, nranges, rboxes, bmincore, core, compmin, bparent, s, &dstats[5],
-                              cap);
+        launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &counters[8], box_of_slot,
+                               reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,
+                               &dstats[5], s);
         tm.mark(M_JOIN1);
         launch_box_clusters(host_count(nbox), bmincore, bcell, cbox, bstart, inrow_of_slot, ustart,
                             bparent, reinterpret_cast<unsigned long long*>(scratch64), compmin,
@@ -790,7 +764,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
 // sequence can be captured in a hipGraph and replayed.  Conditions on which
 // run_keyed branches become flags read after the run; any of them hands the
 // run to the plain pipeline: non-finite input, grids beyond 64 key bits,
-// loose boxes, more open box pairs than the list holds.  Box mode only
+// loose boxes.  Box mode only
 // (floating-point data), smallest-cluster border rule.
 
 // Device words the static pipeline keeps its counts in.
@@ -798,24 +772,20 @@ enum StaticSlot : int {
     SS_M = 0,          // occupied cells
     SS_RANGES = 1,     // neighbour rows
     SS_NBOX = 3,       // boxes
-    SS_BITEMS = 4,     // 64-slot chunks of every box
     SS_LOOSE = 5,      // boxes of two or more rows that are not tight
     SS_CROWS = 6,      // rows to count
     SS_BROWS = 7,      // non-core rows
     SS_NLIST = 8,      // boxes with cores
     SS_JOIN0 = 9,      // roots of the first root-join round
-    SS_UITEMS = 10,    // box chunks with open pairs
     SS_JOIN1 = 13,     // roots of the second round
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
     SS_BITS = 16,      // key bits + sub-box bits
     SS_ROWTAB = 17,    // the row-order label table holds every key
-    SS_HOOKBIG = 18,   // boxes with cores of more than 32 rows
     SS_WORDS = 32
 };
 
-// worst-case sizes of the static pipeline's work lists
-static inline int64_t item_bound(int64_t n) { return n + n / 64 + 16; }  // chunks: <= m + n / 64
+// most neighbour rows of n rows: 3^(D-1) per cell
 template <int D>
 static inline int64_t range_bound(int64_t n) {
     int64_t r = n;
@@ -826,7 +796,7 @@ static inline int64_t range_bound(int64_t n) {
 template <typename T, int D>
 static size_t static_aux_bytes(int64_t n) {
     return align_up(static_cast<size_t>(range_bound<D>(n)) * sizeof(int2), 256) +
-           2 * align_up(static_cast<size_t>(item_bound(n)) * sizeof(int2), 256) + 4096;
+           4096;
 }
 
 template <typename T, int D>
@@ -852,7 +822,6 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     const size_t nn = static_cast<size_t>(n);
     const int64_t ld = (n + 15) & ~int64_t(15);
     const size_t L = static_cast<size_t>(ld);
-    const int64_t IB = item_bound(n);
     // zeroed by a kernel (no memset in a graph)
     fill_i32(reinterpret_cast<int32_t*>(sc), 0, SS_WORDS, s);
     fill_i32(reinterpret_cast<int32_t*>(dstats), 0, 2 * 16, s);
@@ -885,7 +854,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     uint32_t* nchunks = A.take_n<uint32_t>(nn + 1);
     uint8_t* core = A.take_n<uint8_t>(L);
     int32_t* parent = A.take_n<int32_t>(L);
-    int32_t* hook_big = A.take_n<int32_t>(L);  // (rsnap of the slot-level union)
+    int32_t* roots = A.take_n<int32_t>(L);  // (rsnap of the slot-level union)
     int32_t* rootslot = A.take_n<int32_t>(L);
     int32_t* cmin = A.take_n<int32_t>(nn);
     int32_t* cmax = A.take_n<int32_t>(nn);
@@ -897,7 +866,6 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     int32_t* bstart = A.take_n<int32_t>(nn + 1);
     int32_t* bcell = A.take_n<int32_t>(nn);
     int32_t* cbox = A.take_n<int32_t>(nn + 1);
-    uint32_t* bcnt = A.take_n<uint32_t>(nn + 1);
     int32_t* bmincore = A.take_n<int32_t>(nn);
     int32_t* bparent = A.take_n<int32_t>(nn);
     int32_t* compmin = A.take_n<int32_t>(nn);
@@ -928,15 +896,10 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
                                 &dstats[0], &dstats[4], nullptr, 1, rcenter, false, s);
     exclusive_scan_u32_dev(nranges, nranges, M, tmp, s);
     copy_at_count(nranges, &sc[SS_M], &sc[SS_RANGES], s);
-    launch_box_items(bstart, NB, bcnt, tmp, &sc[SS_BITEMS], s);
-
     const int64_t R = range_bound<D>(n);
     int2* rboxes = X.take_n<int2>(static_cast<size_t>(R));
-    int2* bitems = X.take_n<int2>(static_cast<size_t>(IB));
-    int2* uitems = X.take_n<int2>(static_cast<size_t>(IB));
     launch_neighbor_fill<K, T>(ucell, ustart, M, jobs, job_of_cell, nranges, nullptr, rboxes,
                                rcenter, s, nullptr, cbox);
-    launch_box_items_fill(bstart, NB, bcnt, Count{IB, &sc[SS_BITEMS]}, bitems, s);
 
     BoxArgs<T> ba;
     ba.soa = soa;
@@ -946,10 +909,10 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     ba.bstart = bstart;
     ba.bcell = bcell;
     ba.cbox = cbox;
-    ba.bitems = bitems;
-    ba.nbitems = static_cast<int32_t>(IB);
     ba.bbox = bbox;
     ba.jobs = jobs;
+    ba.njobs = njobs;
+    ba.nrows = n;
     ba.job_of_cell = job_of_cell;
     ba.rcenter = rcenter;
     launch_box_tight<T, D>(ba, cell_core, btight, &sc[SS_LOOSE], s);
@@ -983,30 +946,17 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
 
     // the box union (its result is discarded when a box is loose)
     int32_t* blist = parent;
-    launch_select_boxes(NB, 0, bmincore, blist, &sc[SS_NLIST], s);
-    launch_select_boxes(NB, 2, bmincore, hook_big, &sc[SS_HOOKBIG], s, bstart);
-    launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, Count{n, &sc[SS_NLIST]},
-                          bparent, hook_big, &sc[SS_HOOKBIG], s);
-    launch_box_roots(NB, bmincore, bparent, compmin, s);
+    launch_list_boxes(NB, bmincore, blist, &sc[SS_NLIST], bparent, s);
+    launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &sc[SS_NLIST], bparent, s);
     for (int round = 0; round < kRootJoinRounds<D>; ++round) {
         uint32_t* cnt = &sc[round == 0 ? SS_JOIN0 : SS_JOIN1];
-        launch_select_boxes(NB, 1, compmin, blist, cnt, s);
-        launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, blist, Count{n, cnt}, bparent,
-                                   s);
-        launch_box_roots(NB, bmincore, bparent, compmin, s);
+        launch_box_roots(NB, bmincore, bparent, compmin, roots, cnt, s);
+        launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, roots, cnt, bparent, s);
     }
-    int32_t* list = reinterpret_cast<int32_t*>(scratch64);
-    const unsigned long long cap = 2 * static_cast<unsigned long long>(nn);
-    launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, nullptr, &dstats[5], s);
-    exclusive_scan_u32_dev(bcnt, bcnt, NB, tmp, s);
-    // (the box count is on the device: the small boxes' pairs always one
-    // thread per box, the static pipeline's batches of small clouds being
-    // sparse)
-    launch_select_items(Count{IB, &sc[SS_BITEMS]}, bitems, bcnt, uitems, &sc[SS_UITEMS], s, bstart,
-                        kSmallUnionRows);
-    launch_box_scan<T, D>(ba, nranges, rboxes, compmin, bcnt, list, nullptr, s, &dstats[5], cap);
-    launch_box_union_list<T, D>(ba, uitems, Count{IB, &sc[SS_UITEMS]}, core, bcnt, list, bparent, s,
-                                &dstats[5], cap, kSmallUnionRows);
+    launch_box_roots(NB, bmincore, bparent, compmin, nullptr, nullptr, s);
+    launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &sc[SS_NLIST], box_of_slot,
+                           reinterpret_cast<int2*>(scratch64), &dstats[15],
+                           static_cast<unsigned long long>(nn), bparent, &dstats[5], s);
     launch_box_clusters(NB, bmincore, bcell, cbox, bstart, inrow_of_slot, ustart, bparent,
                         reinterpret_cast<unsigned long long*>(scratch64), compmin, bcluster, s);
 
@@ -1127,7 +1077,6 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     HPD_HIP(hipMemcpyAsync(hs, dstats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     HPD_HIP(hipStreamSynchronize(s));
     const bool ok = hc[SS_NONFINITE] == 0 && hc[SS_GRID] == 0 && hc[SS_LOOSE] == 0 &&
-                    hs[5] <= 2 * static_cast<unsigned long long>(n) &&
                     hs[4] <= static_cast<unsigned long long>(range_bound<D>(n));
     if (!ok) {
         ++ctx.graph_fallbacks;

@@ -79,21 +79,6 @@ __device__ __forceinline__ bool fetch_chunk(const int2* __restrict__ items, int3
     return true;
 }
 
-// Lanes per row of the row-group kernels, and the rows of a box up to which
-// the box's lane walks it by itself.
-template <int D>
-constexpr int kGroup = D <= 3 ? 8 : 16;
-constexpr int kLaneRows = 16;
-
-// Persistent grids: wave w of them takes items w, w + wave_stride(), ...
-__device__ __forceinline__ int32_t first_wave() {
-    return uniform(static_cast<int32_t>(blockIdx.x) * kWavesPerBlock +
-                   static_cast<int32_t>(threadIdx.x >> 6));
-}
-__device__ __forceinline__ int32_t wave_stride() {
-    return static_cast<int32_t>(gridDim.x) * kWavesPerBlock;
-}
-
 __device__ __forceinline__ int32_t wave_min(int32_t v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
@@ -188,7 +173,7 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
         uint32_t cnt = 0;
         bool need = on && min_pts > 0;
-        group_boxes<G>(need, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, INT_MAX,
+        group_boxes<G>(need, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
                        [&](bool valid, int32_t b) {
             int32_t q0 = 0, q1 = 0;
             bool part = false;
@@ -590,7 +575,7 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
         const double gap2_max = jp.gap2_max;
         const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
         int32_t best = INT_MAX, worst = -1;  // smallest, largest adjacent cluster so far
-        group_boxes<G>(on, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, INT_MAX,
+        group_boxes<G>(on, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
                        [&](bool valid, int32_t b) {
             const int32_t cl = valid ? bcluster[b] : -1;
             auto wanted = [&] { return cl >= 0 && cl != best && (cl < best || best == worst); };
@@ -839,14 +824,6 @@ __global__ __launch_bounds__(kThreads) void k_fill2(int32_t* __restrict__ a, int
 
 inline unsigned blocks_for(int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
 
-// Blocks of a persistent grid of the row-group kernels over at most n rows:
-// 8 blocks on each of the 256 CUs.
-template <int D>
-inline unsigned row_blocks(int64_t n) {
-    return static_cast<unsigned>(
-        std::min<int64_t>((n * kGroup<D> + kThreads - 1) / kThreads, 2048));
-}
-
 }  // namespace
 
 // *out += number of nonzero flags among f[0, n)
@@ -880,10 +857,10 @@ void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntes
                              a.bmincore, a.crows, a.ncrows_dev, s);
             if (count_start) HPD_HIP(hipEventRecord(count_start, s));
             if (ntests)
-                hipLaunchKernelGGL((k_core_rows<T, D, true>), dim3(row_blocks<D>(a.n)),
+                hipLaunchKernelGGL((k_core_rows<T, D, true>), dim3(group_blocks<D>(a.n)),
                                    dim3(kThreads), 0, s, a, core, ntests);
             else
-                hipLaunchKernelGGL((k_core_rows<T, D>), dim3(row_blocks<D>(a.n)), dim3(kThreads), 0,
+                hipLaunchKernelGGL((k_core_rows<T, D>), dim3(group_blocks<D>(a.n)), dim3(kThreads), 0,
                                    s, a, core, nullptr);
             HPD_HIP(hipGetLastError());
             return;
@@ -964,7 +941,7 @@ void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* b
     const unsigned gw = blocks_for(a.nitems, kWavesPerBlock);
     if constexpr (std::is_floating_point<T>::value) {
         if (bcluster && a.bbox) {
-            hipLaunchKernelGGL((k_border_rows<T, D>), dim3(row_blocks<D>(a.n)), dim3(kThreads), 0,
+            hipLaunchKernelGGL((k_border_rows<T, D>), dim3(group_blocks<D>(a.n)), dim3(kThreads), 0,
                                s, a, core, bcluster, static_cast<const int2*>(a.brows),
                                static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
                                amb_list);

@@ -234,79 +234,6 @@ __device__ __forceinline__ void point_box_lh(const double* lo, const double* hi,
     point_box_dd<D>(lo, hi, v, gmin2, gmax2);
 }
 
-// Visit the boxes of the neighbour rows [r0, r1) of an occupied cell, the
-// cell's own row (index `center`) first.  The box table is fetched up to 64
-// boxes at a time, one box per lane (the rows' box ranges likewise, one row
-// per lane), and handed to fn box by box with readlane, so a box costs no
-// dependent memory access of its own.  fn(b2, lo, hi, q0, q1, tag) gets the
-// box, its bounding box (double), its rows [q0, q1) and tag[b2] (0 without
-// tag), all wave-uniform; it returns true to stop the visit.  Only boxes
-// below bmax are visited.  With first >= 0 (a box of the own row), the own
-// row's boxes are visited from `first` on, wrapping round to the row's
-// earlier boxes: a visit that stops early sees the own cell's boxes first.
-template <typename T, int D, typename Fn>
-__device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t center,
-                                                 const int2* __restrict__ rboxes,
-                                                 const int32_t* __restrict__ bstart,
-                                                 const OrdKey<T>* __restrict__ bbox,
-                                                 const int32_t* __restrict__ tag, Fn&& fn,
-                                                 int32_t bmax = INT_MAX, int32_t first = -1) {
-    const int32_t nrows = r1 - r0;
-    const int lane = __lane_id();
-    for (int32_t g0 = 0; g0 < nrows; g0 += 64) {
-        const int32_t i = g0 + lane;  // visiting order: own row, then the others
-        int32_t rb0 = 0, rcnt = 0;
-        if (i < nrows) {
-            const int32_t r = i == 0 ? center : (r0 + i - 1 < center ? r0 + i - 1 : r0 + i);
-            const int2 bs = rboxes[r];
-            rb0 = bs.x;
-            rcnt = max(0, min(bs.y, bmax) - rb0);  // boxes below bmax only
-        }
-        int32_t incl = rcnt;  // inclusive prefix over the lanes
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int32_t t = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += t;
-        }
-        const int32_t excl = incl - rcnt;
-        const int32_t total = bcast(incl, 63);
-        const int32_t grows = min(64, nrows - g0);
-        // rotation of the own row (row 0 of the first group, lane 0)
-        int32_t rot = 0, rot_n = 0;
-        if (g0 == 0 && first >= 0) {
-            const int32_t b0 = bcast(rb0, 0);
-            rot_n = bcast(rcnt, 0);
-            rot = (first >= b0 && first < b0 + rot_n) ? first - b0 : 0;
-        }
-        for (int32_t k0 = 0; k0 < total; k0 += 64) {
-            const int32_t kk = min(k0 + lane, total - 1);
-            int32_t row = 0;  // last row whose first box index is <= kk
-            for (int32_t t = 1; t < grows; ++t) row = bcast(excl, t) <= kk ? t : row;
-            int32_t local = kk - __shfl(excl, row, 64);
-            if (row == 0 && rot > 0) local = local + rot < rot_n ? local + rot : local + rot - rot_n;
-            const int32_t bl = __shfl(rb0, row, 64) + local;
-            double lol[D], hil[D];
-#pragma unroll
-            for (int j = 0; j < D; ++j) {
-                lol[j] = box_lo<T, D>(bbox, bl, j);
-                hil[j] = box_hi<T, D>(bbox, bl, j);
-            }
-            const int32_t q0l = bstart[bl], q1l = bstart[bl + 1];
-            const int32_t tagl = tag ? tag[bl] : 0;
-            const int32_t nk = min(64, total - k0);
-            for (int32_t j = 0; j < nk; ++j) {
-                double lo[D], hi[D];
-#pragma unroll
-                for (int e = 0; e < D; ++e) {
-                    lo[e] = bcast(lol[e], j);
-                    hi[e] = bcast(hil[e], j);
-                }
-                if (fn(bcast(bl, j), lo, hi, bcast(q0l, j), bcast(q1l, j), bcast(tagl, j))) return;
-            }
-        }
-    }
-}
-
 // A wave split into groups of G lanes, each with a neighbourhood of its own:
 // the boxes of the neighbour rows [r0, r1) of an occupied cell (box ranges
 // rboxes, the own row `center` first, from the cell's first box `own` on and
@@ -314,7 +241,7 @@ __device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t
 // time, one per lane.  fn(valid, b) runs for the whole wave at once (it may
 // use wave-wide operations), with the lane's box b where valid; what it
 // returns must be equal over a group: true ends that group's visit.  Only
-// boxes below bmax are visited.  All arguments but G are per lane, equal over
+// boxes in [bmin, bmax) are visited.  All arguments but G are per lane, equal over
 // a group; inactive groups take part in the wave-wide steps only.
 //
 // Why groups: a neighbourhood holds some 10-30 boxes, so a whole wave per
@@ -323,7 +250,7 @@ __device__ __forceinline__ void for_each_row_box(int32_t r0, int32_t r1, int32_t
 template <int G, typename Fn>
 __device__ __forceinline__ void group_boxes(bool active, int32_t r0, int32_t r1, int32_t center,
                                             int32_t own, const int2* __restrict__ rboxes,
-                                            int32_t bmax, Fn&& fn) {
+                                            int32_t bmin, int32_t bmax, Fn&& fn) {
     const int gl = __lane_id() & (G - 1);
     const int32_t nrows = r1 - r0;
     for (int32_t g0 = 0; __any(active && g0 < nrows); g0 += G) {
@@ -333,7 +260,7 @@ __device__ __forceinline__ void group_boxes(bool active, int32_t r0, int32_t r1,
         if (active && i < nrows) {
             const int32_t r = i == 0 ? center : (r0 + i - 1 < center ? r0 + i - 1 : r0 + i);
             const int2 bs = rboxes[r];
-            b0 = bs.x;
+            b0 = max(bs.x, bmin);
             cnt = max(0, min(bs.y, bmax) - b0);
         }
         // the own row starts at box `own`
@@ -362,6 +289,28 @@ __device__ __forceinline__ void group_boxes(bool active, int32_t r0, int32_t r1,
             if (fn(active && kk < total, b)) active = false;
         }
     }
+}
+
+// Lanes per row or box of the group kernels, and the rows of a box up to
+// which the box's lane walks it by itself.
+template <int D>
+constexpr int kGroup = D <= 3 ? 8 : 16;
+constexpr int kLaneRows = 16;
+
+// Persistent grids: wave w of them takes items w, w + wave_stride(), ...
+constexpr int kGroupThreads = 256;
+__device__ __forceinline__ int32_t first_wave() {
+    return __builtin_amdgcn_readfirstlane(static_cast<int32_t>(blockIdx.x) * (kGroupThreads / 64) +
+                                          static_cast<int32_t>(threadIdx.x >> 6));
+}
+__device__ __forceinline__ int32_t wave_stride() {
+    return static_cast<int32_t>(gridDim.x) * (kGroupThreads / 64);
+}
+// Blocks of one over at most n items: 8 blocks on each of the 256 CUs.
+template <int D>
+inline unsigned group_blocks(int64_t n) {
+    const int64_t b = (n * kGroup<D> + kGroupThreads - 1) / kGroupThreads;
+    return static_cast<unsigned>(b < 2048 ? (b > 0 ? b : 1) : 2048);
 }
 
 // Sum, minimum and maximum over a group of G lanes.
