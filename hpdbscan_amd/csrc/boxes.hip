@@ -21,10 +21,9 @@
 // cores are joined when some core pair across them is within eps (tested
 // with the reference's expression, stopping at the first hit), unless they
 // are already joined; a core row farther than eps from the other box's
-// bounding box takes no part in the test.  Box pairs whose bounding boxes are farther apart than
-// eps * (1 + 1e-5) cannot hold such a pair (the float result of the
-// expression is within a few ulps of the exact squared distance) and are
-// skipped.
+// bounding box takes no part in the test.  Box pairs whose bounding boxes are
+// farther apart than eps by the same monotone expression (box_gap) cannot hold
+// such a pair and are skipped.
 #include <algorithm>
 #include <climits>
 
@@ -59,7 +58,7 @@ template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_gather_boxes(
     const T* __restrict__ pts, int64_t n, const uint32_t* __restrict__ inrow_of_slot,
     T* __restrict__ soa, int64_t ld, const int32_t* __restrict__ box_of_slot,
-    const int32_t* __restrict__ bstart, OrdKey<T>* __restrict__ bbox, OrdKey<T>* __restrict__ part) {
+    const int32_t* __restrict__ bstart, Span<T>* __restrict__ bbox, OrdKey<T>* __restrict__ part) {
     using U = OrdKey<T>;
     __shared__ U slo[kThreads][D];
     __shared__ U shi[kThreads][D];
@@ -107,13 +106,17 @@ __global__ __launch_bounds__(kThreads) void k_gather_boxes(
     __syncthreads();
     const int64_t blk1 = blk0 + kThreads < n ? blk0 + kThreads : n;  // end of the block's slots
     const int32_t nruns = box_of_slot[blk1 - 1] - b_first + 1;
-    const int t = threadIdx.x;
-    if (t < nruns) {
+    for (int t = threadIdx.x; t < nruns; t += kThreads) {
         const int32_t bb = b_first + t;
         const bool starts = bstart[bb] >= blk0;
         const bool ends = bstart[bb + 1] <= blk1;
-        U* dst = starts && ends ? &bbox[static_cast<int64_t>(bb) * D * 2]
-                                : &part[(2 * static_cast<int64_t>(blockIdx.x) + (starts ? 1 : 0)) * D * 2];
+        if (starts && ends) {
+#pragma unroll
+            for (int j = 0; j < D; ++j)
+                bbox[static_cast<int64_t>(bb) * D + j] = {ord_val(slo[t][j]), ord_val(shi[t][j])};
+            continue;
+        }
+        U* dst = &part[(2 * static_cast<int64_t>(blockIdx.x) + (starts ? 1 : 0)) * D * 2];
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             dst[2 * j] = slo[t][j];
@@ -134,7 +137,7 @@ constexpr int kBoundsTile = kThreads * kBoundsRows;
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_box_bounds(
     const T* __restrict__ soa, int64_t ld, int64_t n, const int32_t* __restrict__ box_of_slot,
-    const int32_t* __restrict__ bstart, OrdKey<T>* __restrict__ bbox, OrdKey<T>* __restrict__ part) {
+    const int32_t* __restrict__ bstart, Span<T>* __restrict__ bbox, OrdKey<T>* __restrict__ part) {
     using U = OrdKey<T>;
     static_assert(D * sizeof(T) <= 8, "rows of at most 8 bytes");
     __shared__ U slo[kBoundsTile][D];
@@ -218,8 +221,13 @@ __global__ __launch_bounds__(kThreads) void k_box_bounds(
         const int32_t bb = b_first + t;
         const bool starts = bstart[bb] >= blk0;
         const bool ends = bstart[bb + 1] <= blk1;
-        U* dst = starts && ends ? &bbox[static_cast<int64_t>(bb) * D * 2]
-                                : &part[(2 * static_cast<int64_t>(blockIdx.x) + (starts ? 1 : 0)) * D * 2];
+        if (starts && ends) {
+#pragma unroll
+            for (int j = 0; j < D; ++j)
+                bbox[static_cast<int64_t>(bb) * D + j] = {ord_val(slo[t][j]), ord_val(shi[t][j])};
+            continue;
+        }
+        U* dst = &part[(2 * static_cast<int64_t>(blockIdx.x) + (starts ? 1 : 0)) * D * 2];
 #pragma unroll
         for (int j = 0; j < D; ++j) {
             dst[2 * j] = slo[t][j];
@@ -237,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void k_box_span(int64_t n, int64_t nblock
                                                        const int32_t* __restrict__ box_of_slot,
                                                        const int32_t* __restrict__ bstart,
                                                        const OrdKey<T>* __restrict__ part,
-                                                       OrdKey<T>* __restrict__ bbox) {
+                                                       Span<T>* __restrict__ bbox) {
     using U = OrdKey<T>;
     const int64_t blk = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6);
     if (blk >= nblocks) return;
@@ -271,10 +279,8 @@ __global__ __launch_bounds__(kThreads) void k_box_span(int64_t n, int64_t nblock
     }
     if (lane_id() == 0) {
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            bbox[(static_cast<int64_t>(b) * D + j) * 2] = lo[j];
-            bbox[(static_cast<int64_t>(b) * D + j) * 2 + 1] = hi[j];
-        }
+        for (int j = 0; j < D; ++j)
+            bbox[static_cast<int64_t>(b) * D + j] = {ord_val(lo[j]), ord_val(hi[j])};
     }
 }
 
@@ -354,7 +360,7 @@ __global__ __launch_bounds__(kThreads) void k_cells_of_boxes(
 // flags per box: tight (dist2(extent) <= EPS2 in the reference's order),
 // full, in a cell that can hold cores
 template <typename T, int D>
-__global__ __launch_bounds__(kThreads) void k_box_tight(const OrdKey<T>* __restrict__ bbox,
+__global__ __launch_bounds__(kThreads) void k_box_tight(const Span<T>* __restrict__ bbox,
                                                         Count nbox_c,
                                                         const int32_t* __restrict__ bstart,
                                                         const int32_t* __restrict__ bcell,
@@ -371,8 +377,8 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const OrdKey<T>* __restr
     T lo[D], hi[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-        lo[j] = ord_val(bbox[(static_cast<int64_t>(b) * D + j) * 2]);
-        hi[j] = ord_val(bbox[(static_cast<int64_t>(b) * D + j) * 2 + 1]);
+        lo[j] = bbox[static_cast<int64_t>(b) * D + j].lo;
+        hi[j] = bbox[static_cast<int64_t>(b) * D + j].hi;
     }
     const bool tight = within<D>(hi, lo, jp.eps2);
     const int32_t size = bstart[b + 1] - bstart[b];
@@ -408,19 +414,18 @@ __device__ __forceinline__ bool any_pair(const T* __restrict__ soa, int64_t ld,
 template <typename T, int D>
 __device__ __forceinline__ bool wave_pair(const T* __restrict__ soa, int64_t ld,
                                           const uint8_t* __restrict__ core,
-                                          const OrdKey<T>* __restrict__ bbox, int32_t s0,
-                                          int32_t s1, int32_t b2, int32_t q0, int32_t q1, T eps2,
-                                          double gap2_max, double full2) {
+                                          const Span<T>* __restrict__ bbox, int32_t s0, int32_t s1,
+                                          int32_t b2, int32_t q0, int32_t q1, T eps2) {
     for (int32_t c = s0; c < s1; c += kWave) {
         const int32_t p = c + lane_id();
         const bool pcore = p < s1 && core[p];
         if (!__any(pcore)) continue;
         T pc[D];
         load_row<T, D>(soa, ld, pcore ? p : c, pc);
-        double gmin2, gmax2;
+        T gmin2, gmax2;
         point_box<T, D>(bbox, b2, pc, gmin2, gmax2);
-        const bool act = pcore && gmin2 <= gap2_max;
-        if (__any(act && gmax2 <= full2)) return true;
+        const bool act = pcore && gmin2 <= eps2;
+        if (__any(act && gmax2 <= eps2)) return true;
         if (__any(act) && any_pair<T, D>(soa, ld, core, q0, q1, pc, act, eps2)) return true;
     }
     return false;
@@ -445,26 +450,49 @@ __device__ __forceinline__ bool lane_pair(const T* __restrict__ soa, int64_t ld,
     return false;
 }
 
+// Whether one of the first and last rows of both boxes make such a pair.
+template <typename T, int D>
+__device__ __forceinline__ bool ends_pair(const T* __restrict__ soa, int64_t ld,
+                                          const uint8_t* __restrict__ core, int32_t s0, int32_t s1,
+                                          int32_t q0, int32_t q1, T eps2) {
+    const int32_t p[2] = {s0, s1 - 1}, q[2] = {q0, q1 - 1};
+    T pc[2][D], qc[2][D];
+    uint8_t cp[2], cq[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        load_row<T, D>(soa, ld, p[k], pc[k]);
+        load_row<T, D>(soa, ld, q[k], qc[k]);
+        cp[k] = core[p[k]];
+        cq[k] = core[q[k]];
+    }
+    bool hit = false;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        hit = hit || (cp[k & 1] && cq[k >> 1] && within<D>(pc[k & 1], qc[k >> 1], eps2));
+    return hit;
+}
+
 // The pair kernels below take the boxes with cores from blist, a group of G
 // lanes per box, a neighbour box per lane (group_boxes); box pairs of up to
 // kLanePair rows by rows are tested by their lane, larger ones by the wave.
-constexpr int kLanePair = 64;
+// (4096 clouds, hook and join ms: 16 4.79, 32 4.83, 64 4.91, 256 11.4 before
+// the first and last rows were tried first, 1024 13.2.)
+constexpr int kLanePair = 16;
 
-// squared distances between two bounding boxes: nearest and farthest points
+// The same bounds (point_box) for the rows of two boxes: gap2 <= dist2(p, q)
+// <= far2 for every pair of members.
 template <typename T, int D>
-__device__ __forceinline__ void box_gap(const OrdKey<T>* __restrict__ bbox, int32_t b2,
-                                        const double* lo, const double* hi, double& gap2,
-                                        double& far2) {
-    gap2 = 0.0;
-    far2 = 0.0;
+__device__ __forceinline__ void box_gap(const Span<T>* __restrict__ bbox, int32_t b2,
+                                        const Span<T>* mine, T& gap2, T& far2) {
+    T g[D], f[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-        const double l2 = box_lo<T, D>(bbox, b2, j), h2 = box_hi<T, D>(bbox, b2, j);
-        const double g = fmax(0.0, fmax(l2 - hi[j], lo[j] - h2));
-        const double f = fmax(h2 - lo[j], hi[j] - l2);
-        gap2 += g * g;
-        far2 += f * f;
+        const Span<T> s = bbox[static_cast<int64_t>(b2) * D + j];
+        g[j] = max(T(0), max(s.lo - mine[j].hi, mine[j].lo - s.hi));
+        f[j] = max(s.hi - mine[j].lo, mine[j].hi - s.lo);
     }
+    gap2 = sum2<D>(g);
+    far2 = sum2<D>(f);
 }
 
 // Hook forest (kJoin false): every listed box points at some earlier box
@@ -495,7 +523,7 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
     const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
     const int gl = lane_id() & (G - 1);
     const int grp = lane_id() / G;
-    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     for (int32_t base = first_wave() * kPer; base < nlist; base += wave_stride() * kPer) {
         const bool on = base + grp < nlist;
         const int32_t b = blist[on ? base + grp : nlist - 1];
@@ -503,14 +531,9 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
         const int32_t u = a.bcell[b];
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
-        const double gap2_max = jp.gap2_max;
-        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-        double lo[D], hi[D];
+        Span<T> mine[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            lo[j] = box_lo<T, D>(bbox, b, j);
-            hi[j] = box_hi<T, D>(bbox, b, j);
-        }
+        for (int j = 0; j < D; ++j) mine[j] = bbox[static_cast<int64_t>(b) * D + j];
         int32_t link = -1;  // equal over the group
         group_boxes<G>(on, static_cast<int32_t>(roff[u]), static_cast<int32_t>(roff[u + 1]),
                        a.rcenter[u], a.cbox[u], rboxes, 0, kJoin ? INT_MAX : b,
@@ -520,16 +543,23 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
             if (valid) {
                 const int32_t t = tag[b2];
                 if (kJoin ? (t >= 0 && t != b) : t != INT_MAX) {
-                    double gap2, far2;
-                    box_gap<T, D>(bbox, b2, lo, hi, gap2, far2);
-                    open = gap2 <= gap2_max;
-                    hit = far2 <= full2;
+                    T gap2, far2;
+                    box_gap<T, D>(bbox, b2, mine, gap2, far2);
+                    open = gap2 <= eps2;
+                    hit = far2 <= eps2;
                     q0 = a.bstart[b2];
                     q1 = a.bstart[b2 + 1];
                 }
             }
             const uint64_t gmask = ((G < 64 ? (uint64_t{1} << G) : 0) - 1) << (grp * G);
             uint64_t hits = ballot(hit) & gmask;
+            if (hits == 0 && open) {
+                // the first and last rows of both boxes first: neighbouring
+                // boxes mostly hold a pair among them, and a lane that runs
+                // into a box without one holds up its wave
+                hit = ends_pair<T, D>(a.soa, a.ld, core, s0, s1, q0, q1, eps2);
+            }
+            hits = ballot(hit) & gmask;
             if (hits == 0 && open) {
                 const int64_t tests = static_cast<int64_t>(s1 - s0) * (q1 - q0);
                 if (tests <= kLanePair) {
@@ -547,8 +577,7 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
                 if ((ballot(done) >> j) & 1) continue;
                 const int32_t t0 = bcast(s0, j);
                 if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, min(bcast(s1, j), t0 + kWave),
-                                    bcast(b2, j), bcast(q0, j), bcast(q1, j), bcast(eps2, j),
-                                    bcast(gap2_max, j), bcast(full2, j))) {
+                                    bcast(b2, j), bcast(q0, j), bcast(q1, j), bcast(eps2, j))) {
                     if (grp == j / G) {
                         done = true;
                         hits = uint64_t{1} << j;
@@ -586,7 +615,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
     constexpr int kPer = 64 / G;
     const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
     const int grp = lane_id() / G;
-    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     unsigned long long opened = 0;
     for (int32_t base = first_wave() * kPer; base < nlist; base += wave_stride() * kPer) {
         const bool on = base + grp < nlist;
@@ -596,24 +625,19 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
         const int32_t u = a.bcell[b];
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
-        const double gap2_max = jp.gap2_max;
-        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
-        double lo[D], hi[D];
+        Span<T> mine[D];
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            lo[j] = box_lo<T, D>(bbox, b, j);
-            hi[j] = box_hi<T, D>(bbox, b, j);
-        }
+        for (int j = 0; j < D; ++j) mine[j] = bbox[static_cast<int64_t>(b) * D + j];
         const int32_t r0 = static_cast<int32_t>(roff[u]);
         group_boxes<G>(on, r0, static_cast<int32_t>(roff[u + 1]), r0, -1, rboxes, b + 1, INT_MAX,
                        [&](bool valid, int32_t b2) {
             const int32_t s2 = valid ? rsnap[b2] : -1;
             bool open = false, whole = false;
             if (s2 >= 0 && s2 != sb) {
-                double gap2, far2;
-                box_gap<T, D>(bbox, b2, lo, hi, gap2, far2);
-                open = gap2 <= gap2_max;
-                whole = far2 <= full2;
+                T gap2, far2;
+                box_gap<T, D>(bbox, b2, mine, gap2, far2);
+                open = gap2 <= eps2;
+                whole = far2 <= eps2;
                 opened += open ? 1 : 0;
             }
             if (!__any(open)) return false;
@@ -655,8 +679,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
                                              : make_int2(-1, -1);
                     if (fits) continue;
                 }
-                if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, t1, b2j, v0, v1, bcast(eps2, j),
-                                    bcast(gap2_max, j), bcast(full2, j)) &&
+                if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, t1, b2j, v0, v1, bcast(eps2, j)) &&
                     lane_id() == 0)
                     uf_unite(bparent, r, r2);
             }
@@ -676,7 +699,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union_heavy(
     const unsigned long long* __restrict__ nheavy, unsigned long long heavy_cap) {
     const unsigned long long found = *nheavy;
     const int32_t n = uniform(static_cast<int32_t>(found < heavy_cap ? found : heavy_cap));
-    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     for (int32_t w = first_wave(); w < n; w += wave_stride()) {
         const int32_t x0 = uniform(heavy[w].x), b2 = uniform(heavy[w].y);
         if (x0 < 0) continue;
@@ -684,13 +707,12 @@ __global__ __launch_bounds__(kThreads) void k_box_union_heavy(
         const int32_t x1 = min(uniform(a.bstart[b + 1]), x0 + kHeavyRows);
         const int32_t q0 = uniform(a.bstart[b2]), q1 = uniform(a.bstart[b2 + 1]);
         const JobParams<T>& jp = a.jobs[uniform(a.job_of_cell[uniform(a.bcell[b])])];
-        const double full2 = static_cast<double>(jp.eps2) * (1.0 - 1e-5);
         for (int32_t c = x0; c < x1; c += kWave) {
             const int32_t r = uniform(uf_find(bparent, b));
             const int32_t r2 = uniform(uf_find(bparent, b2));
             if (r == r2) break;
-            if (wave_pair<T, D>(a.soa, a.ld, core, bbox, c, min(c + kWave, x1), b2, q0, q1, jp.eps2,
-                                jp.gap2_max, full2)) {
+            if (wave_pair<T, D>(a.soa, a.ld, core, bbox, c, min(c + kWave, x1), b2, q0, q1,
+                                jp.eps2)) {
                 if (lane_id() == 0) uf_unite(bparent, r, r2);
                 break;
             }
@@ -855,16 +877,16 @@ void launch_gather_boxes(const T* pts, int64_t n, const uint32_t* inrow_of_slot,
     if (tile == kThreads) {
         hipLaunchKernelGGL((k_gather_boxes<T, D>), dim3(static_cast<unsigned>(nb)), dim3(kThreads),
                            0, s, pts, n, inrow_of_slot, soa, ld, box_of_slot, bstart,
-                           static_cast<U*>(bbox), static_cast<U*>(part));
+                           static_cast<Span<T>*>(bbox), static_cast<U*>(part));
     } else {
         if constexpr (D * sizeof(T) <= 8)
             hipLaunchKernelGGL((k_box_bounds<T, D>), dim3(static_cast<unsigned>(nb)),
                                dim3(kThreads), 0, s, soa, ld, n, box_of_slot, bstart,
-                               static_cast<U*>(bbox), static_cast<U*>(part));
+                               static_cast<Span<T>*>(bbox), static_cast<U*>(part));
     }
     hipLaunchKernelGGL((k_box_span<T, D>), dim3(blocks_for(nb, kWavesPerBlock)), dim3(kThreads), 0,
                        s, n, nb, tile, box_of_slot, bstart, static_cast<const U*>(part),
-                       static_cast<U*>(bbox));
+                       static_cast<Span<T>*>(bbox));
     HPD_HIP(hipGetLastError());
 }
 
@@ -913,7 +935,7 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
     using U = OrdKey<T>;
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_tight<T, D>), dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0,
-                       s, reinterpret_cast<const U*>(a.bbox), Count{a.nbox, a.nbox_dev}, a.bstart,
+                       s, static_cast<const Span<T>*>(a.bbox), Count{a.nbox, a.nbox_dev}, a.bstart,
                        a.bcell, a.job_of_cell, a.jobs, cell_core, btight, nloose);
 }
 

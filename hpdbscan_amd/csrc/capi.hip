@@ -1013,7 +1013,6 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
         jp.row_end = offsets[j + 1];
         jp.min_pts = static_cast<uint32_t>(std::min<uint64_t>(min_pts[j], 0xffffffffull));
         jp.eps2 = eps2_as<T>(eps[j]);
-        jp.gap2_max = static_cast<double>(jp.eps2) * (1.0 + 1e-5) + 1e-30;
         jp.rcp_f = flushf(1.0f / flushf(eps[j]));
         jp.rcp_d = flushd(1.0 / flushd(static_cast<double>(eps[j])));
         jp.cp.d = D;
@@ -1158,7 +1157,6 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
         jp.key_base = key_total;
         jp.min_pts = static_cast<uint32_t>(std::min<uint64_t>(min_pts[j], 0xffffffffull));
         jp.eps2 = eps2_as<T>(eps[j]);
-        jp.gap2_max = static_cast<double>(jp.eps2) * (1.0 + 1e-5) + 1e-30;
         jp.cp.d = D;
         if (jp.row_end == jp.row_begin) continue;
         float rcp_f;

@@ -23,6 +23,7 @@ constexpr int kWave = 64;
 //           last single term.
 //   integer types: every step wraps modulo 2^bits(T).
 // Kernels are built with -ffp-contract=off, so no step is fused into an FMA.
+// sum2 is the part after the subtraction: the sum of the squares of u.
 // --------------------------------------------------------------------------
 template <typename T>
 struct Coord {
@@ -30,13 +31,10 @@ struct Coord {
 };
 
 template <int D>
-__device__ __forceinline__ float dist2(const float* p, const float* q) {
+__device__ __forceinline__ float sum2(const float* u) {
     float t[D];
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-        const float u = p[j] - q[j];
-        t[j] = u * u;
-    }
+    for (int j = 0; j < D; ++j) t[j] = u[j] * u[j];
     float s;
     int base;
     if constexpr (D >= 4) {
@@ -69,13 +67,10 @@ __device__ __forceinline__ float dist2(const float* p, const float* q) {
 }
 
 template <int D>
-__device__ __forceinline__ double dist2(const double* p, const double* q) {
+__device__ __forceinline__ double sum2(const double* u) {
     double t[D];
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-        const double u = p[j] - q[j];
-        t[j] = u * u;
-    }
+    for (int j = 0; j < D; ++j) t[j] = u[j] * u[j];
     if constexpr (D == 1) {
         return t[0];
     } else {
@@ -89,6 +84,15 @@ __device__ __forceinline__ double dist2(const double* p, const double* q) {
         if constexpr (D % 2 == 1) s = s + t[D - 1];
         return s;
     }
+}
+
+template <int D, typename T>
+__device__ __forceinline__ std::enable_if_t<std::is_floating_point<T>::value, T> dist2(const T* p,
+                                                                                      const T* q) {
+    T u[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) u[j] = p[j] - q[j];
+    return sum2<D>(u);
 }
 
 template <typename T>

@@ -139,10 +139,7 @@ __global__ __launch_bounds__(kThreads) void k_core(const DbscanArgs<T> a, uint8_
 // lane.  A box farther than eps from the row (bounding box) is skipped, one
 // within eps of its farthest corner counts whole, the others are tested row
 // by row: small ones by their lane, larger ones by the whole wave with the
-// candidates on the lanes.  Exactness: with d the exact distance and gmin2
-// <= d^2 <= gmax2, the reference's float expression is within a few ulps of
-// d^2, so gmin2 > EPS2 (1 + 1e-5) (+ 1e-30) rules every member out and
-// gmax2 <= EPS2 (1 - 1e-5) rules every member in.
+// candidates on the lanes.
 //
 // Bound by latency (list -> cell -> box ranges -> boxes) and VALU issue of
 // the box tests.  kCount: also add the row-row distance tests executed to
@@ -155,7 +152,7 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
     constexpr int kPer = 64 / G;  // rows of a wave
     const int32_t nrows = uniform(static_cast<int32_t>(*a.ncrows_dev));
     const int gl = lane_id() & (G - 1);
-    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     unsigned long long tests = 0;
     for (int32_t base = first_wave() * kPer; base < nrows; base += wave_stride() * kPer) {
         const int32_t i = base + lane_id() / G;
@@ -169,8 +166,6 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
         const uint32_t min_pts = jp.min_pts;
-        const double gap2_max = jp.gap2_max;
-        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
         uint32_t cnt = 0;
         bool need = on && min_pts > 0;
         group_boxes<G>(need, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
@@ -179,12 +174,12 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
             bool part = false;
             uint32_t w = 0;
             if (valid) {
-                double gmin2, gmax2;
+                T gmin2, gmax2;
                 point_box<T, D>(bbox, b, pc, gmin2, gmax2);
                 q0 = a.bstart[b];
                 q1 = a.bstart[b + 1];
-                const bool near = gmin2 <= gap2_max;
-                const bool whole = near && gmax2 <= full2;
+                const bool near = gmin2 <= eps2;
+                const bool whole = near && gmax2 <= eps2;
                 if (whole) w = static_cast<uint32_t>(q1 - q0);
                 part = near && !whole;
             }
@@ -559,7 +554,7 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
     constexpr int kPer = 64 / G;
     const int32_t nrows = uniform(static_cast<int32_t>(*nrows_dev));
     const int gl = lane_id() & (G - 1);
-    const OrdKey<T>* bbox = static_cast<const OrdKey<T>*>(a.bbox);
+    const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     unsigned long long noise = 0;
     for (int32_t base = first_wave() * kPer; base < nrows; base += wave_stride() * kPer) {
         const int32_t i = base + lane_id() / G;
@@ -572,8 +567,6 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
         const int32_t r1 = static_cast<int32_t>(a.roff[u + 1]);
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
-        const double gap2_max = jp.gap2_max;
-        const double full2 = static_cast<double>(eps2) * (1.0 - 1e-5);
         int32_t best = INT_MAX, worst = -1;  // smallest, largest adjacent cluster so far
         group_boxes<G>(on, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
                        [&](bool valid, int32_t b) {
@@ -582,12 +575,12 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
             int32_t q0 = 0, q1 = 0;
             bool part = false, hit = false;
             if (wanted()) {
-                double gmin2, gmax2;
+                T gmin2, gmax2;
                 point_box<T, D>(bbox, b, pc, gmin2, gmax2);
                 q0 = a.bstart[b];
                 q1 = a.bstart[b + 1];
-                const bool near = gmin2 <= gap2_max;
-                hit = near && gmax2 <= full2;
+                const bool near = gmin2 <= eps2;
+                hit = near && gmax2 <= eps2;
                 part = near && !hit;
             }
             if (__any(hit)) {

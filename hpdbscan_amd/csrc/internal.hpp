@@ -183,7 +183,6 @@ struct JobParams {
     T eps2{};               // EPS2 converted to T
     float rcp_f = 0.0f;     // 1/eps in float (float and integer data)
     double rcp_d = 0.0;     // 1/eps in double (double data)
-    double gap2_max = 0.0;  // box pairs farther apart than this cannot connect
     uint32_t min_pts = 0;
 };
 

@@ -91,33 +91,32 @@ __device__ __forceinline__ double ord_val(unsigned long long k) {
 template <typename T>
 using OrdKey = std::conditional_t<sizeof(T) == 8, unsigned long long, uint32_t>;
 
-template <typename T, int D>
-__device__ __forceinline__ double box_lo(const OrdKey<T>* __restrict__ bbox, int32_t b, int j) {
-    return static_cast<double>(ord_val(bbox[(static_cast<int64_t>(b) * D + j) * 2]));
-}
-template <typename T, int D>
-__device__ __forceinline__ double box_hi(const OrdKey<T>* __restrict__ bbox, int32_t b, int j) {
-    return static_cast<double>(ord_val(bbox[(static_cast<int64_t>(b) * D + j) * 2 + 1]));
-}
+// Bounding box of a box in one dimension: bbox[b * D + j].
+template <typename T>
+struct alignas(2 * sizeof(T)) Span {
+    T lo, hi;
+};
 
-// Squared distances from a row to a box's bounding box, in double: gmin2
-// to its nearest point, gmax2 to its farthest corner.  Every member q of the
-// box satisfies gmin2 <= |p - q|^2 <= gmax2.
+// Bounds of the reference's squared distance between a row and the members
+// of a box: gmin2 <= dist2(p, q) <= gmax2 for every member q, where gmin2 and
+// gmax2 are the reference's own expression (sum2) on the differences to the
+// box's nearest and farthest point.  Every step of it (subtract, square, each
+// add of the summation tree, the flush of tiny values) rounds monotonically,
+// so the bounds hold for the rounded values themselves: gmin2 > EPS2 rules
+// every member out and gmax2 <= EPS2 rules every member in, with no margin.
 template <typename T, int D>
-__device__ __forceinline__ void point_box(const OrdKey<T>* __restrict__ bbox, int32_t b,
-                                          const T* pc, double& gmin2, double& gmax2) {
-    gmin2 = 0.0;
-    gmax2 = 0.0;
+__device__ __forceinline__ void point_box(const Span<T>* __restrict__ bbox, int32_t b, const T* pc,
+                                          T& gmin2, T& gmax2) {
+    T g[D], f[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-        const double lo = box_lo<T, D>(bbox, b, j);
-        const double hi = box_hi<T, D>(bbox, b, j);
-        const double v = static_cast<double>(pc[j]);
-        const double g = fmax(0.0, fmax(lo - v, v - hi));
-        const double f = fmax(v - lo, hi - v);
-        gmin2 += g * g;
-        gmax2 += f * f;
+        const Span<T> s = bbox[static_cast<int64_t>(b) * D + j];
+        const T below = s.lo - pc[j], above = pc[j] - s.hi;
+        g[j] = max(T(0), max(below, above));
+        f[j] = max(-below, -above);
     }
+    gmin2 = sum2<D>(g);
+    gmax2 = sum2<D>(f);
 }
 
 // Wave-uniform copy of lane j's value (j wave-uniform): v_readlane.
@@ -210,30 +209,6 @@ __device__ __forceinline__ bool walk_wide(uint64_t rows, int32_t n) {
     return n > kWideMinRows && __popcll(rows) <= kWideRows;
 }
 
-// Squared distances from a row to the box [lo, hi] (double): gmin2 to its
-// nearest point, gmax2 to its farthest corner.
-template <int D>
-__device__ __forceinline__ void point_box_dd(const double* lo, const double* hi, const double* v,
-                                             double& gmin2, double& gmax2) {
-    gmin2 = 0.0;
-    gmax2 = 0.0;
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        const double g = fmax(0.0, fmax(lo[j] - v[j], v[j] - hi[j]));
-        const double f = fmax(v[j] - lo[j], hi[j] - v[j]);
-        gmin2 += g * g;
-        gmax2 += f * f;
-    }
-}
-template <typename T, int D>
-__device__ __forceinline__ void point_box_lh(const double* lo, const double* hi, const T* pc,
-                                             double& gmin2, double& gmax2) {
-    double v[D];
-#pragma unroll
-    for (int j = 0; j < D; ++j) v[j] = static_cast<double>(pc[j]);
-    point_box_dd<D>(lo, hi, v, gmin2, gmax2);
-}
-
 // A wave split into groups of G lanes, each with a neighbourhood of its own:
 // the boxes of the neighbour rows [r0, r1) of an occupied cell (box ranges
 // rboxes, the own row `center` first, from the cell's first box `own` on and
@@ -295,7 +270,7 @@ __device__ __forceinline__ void group_boxes(bool active, int32_t r0, int32_t r1,
 // which the box's lane walks it by itself.
 template <int D>
 constexpr int kGroup = D <= 3 ? 8 : 16;
-constexpr int kLaneRows = 16;
+constexpr int kLaneRows = 8;
 
 // Persistent grids: wave w of them takes items w, w + wave_stride(), ...
 constexpr int kGroupThreads = 256;
@@ -331,50 +306,6 @@ __device__ __forceinline__ int32_t group_max(int32_t v) {
 #pragma unroll
     for (int o = G / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
     return v;
-}
-
-// Box-to-box squared distances (double): gmin2 between the nearest points
-// of [alo, ahi] and [blo, bhi], gmax2 between the farthest.  For every row p
-// inside box a, gmin2 <= gmin2(p, b) and gmax2(p, b) <= gmax2, also as
-// computed in double: every step (subtract, max, square, add) rounds
-// monotonically.
-template <int D>
-__device__ __forceinline__ void box_box(const double* alo, const double* ahi, const double* blo,
-                                        const double* bhi, double& gmin2, double& gmax2) {
-    gmin2 = 0.0;
-    gmax2 = 0.0;
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        const double g = fmax(0.0, fmax(blo[j] - ahi[j], alo[j] - bhi[j]));
-        const double f = fmax(bhi[j] - alo[j], ahi[j] - blo[j]);
-        gmin2 += g * g;
-        gmax2 += f * f;
-    }
-}
-
-// A wave-uniform double held in scalar registers (v_readfirstlane).
-__device__ __forceinline__ double uniform_d(double v) {
-    const long long x = __double_as_longlong(v);
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x)));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(x >> 32)));
-    return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
-}
-
-// Wave-uniform bounding box (double) of the rows of the lanes where `on`.
-template <typename T, int D>
-__device__ __forceinline__ void rows_bbox(const T* pc, bool on, double* lo, double* hi) {
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-        double a = on ? static_cast<double>(pc[j]) : __builtin_huge_val();
-        double b = on ? static_cast<double>(pc[j]) : -__builtin_huge_val();
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            a = fmin(a, __shfl_xor(a, o, 64));
-            b = fmax(b, __shfl_xor(b, o, 64));
-        }
-        lo[j] = uniform_d(a);
-        hi[j] = uniform_d(b);
-    }
 }
 
 // Runs of equal `key` over consecutive lanes (boxes are contiguous slot
