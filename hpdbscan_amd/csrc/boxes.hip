@@ -738,14 +738,15 @@ __global__ __launch_bounds__(kThreads) void k_core_init(
     int64_t n, const int32_t* __restrict__ box_of_slot, const uint8_t* __restrict__ btight,
     const int32_t* __restrict__ bstart, const int32_t* __restrict__ bcell,
     const uint32_t* __restrict__ inrow, uint8_t* __restrict__ core, int32_t* __restrict__ bmincore,
-    int2* __restrict__ rows, unsigned int* __restrict__ nrows) {
+    int2* __restrict__ rows, unsigned int* __restrict__ nrows, int chunk) {
     block_collect(n, rows, nrows, [&](int64_t s, int2& v) {
         const int32_t b = box_of_slot[s];
         const uint8_t t = btight[b];
         const bool full = (t & 2) != 0;
         core[s] = full ? 1 : 0;
-        if (bstart[b] == s) bmincore[b] = full ? static_cast<int32_t>(inrow[s]) : INT_MAX;
-        if (full || !(t & 4)) return false;
+        const int32_t at = static_cast<int32_t>(s) - bstart[b];
+        if (at == 0) bmincore[b] = full ? static_cast<int32_t>(inrow[s]) : INT_MAX;
+        if (full || !(t & 4) || (at & (chunk - 1)) != 0) return false;
         v = make_int2(static_cast<int32_t>(s), bcell[b]);
         return true;
     });
@@ -952,8 +953,9 @@ void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbox
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
                      const unsigned int* nlist, int32_t* bparent, hipStream_t s) {
     if (a.nbox <= 0) return;
-    hipLaunchKernelGGL((k_box_link<T, D, false>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0,
-                       s, a, roff, rboxes, bmincore, core, blist, nlist, bparent);
+    hipLaunchKernelGGL((k_box_link<T, D, false>),
+                       dim3(persistent_blocks<k_box_link<T, D, false>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(kThreads), 0, s, a, roff, rboxes, bmincore, core, blist, nlist, bparent);
     HPD_HIP(hipGetLastError());
 }
 
@@ -970,18 +972,19 @@ void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2*
                           const int32_t* rsnap, const uint8_t* core, const int32_t* roots,
                           const unsigned int* nroots, int32_t* bparent, hipStream_t s) {
     if (a.nbox <= 0) return;
-    hipLaunchKernelGGL((k_box_link<T, D, true>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0,
-                       s, a, roff, rboxes, rsnap, core, roots, nroots, bparent);
+    hipLaunchKernelGGL((k_box_link<T, D, true>),
+                       dim3(persistent_blocks<k_box_link<T, D, true>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, roots, nroots, bparent);
     HPD_HIP(hipGetLastError());
 }
 
 void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
                       const int32_t* bstart, const int32_t* bcell, const uint32_t* inrow,
                       uint8_t* core, int32_t* bmincore, int2* rows, unsigned int* nrows,
-                      hipStream_t s) {
+                      int chunk, hipStream_t s) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_core_init, dim3(collect_blocks(n)), dim3(kCollectThreads), 0, s, n,
-                       box_of_slot, btight, bstart, bcell, inrow, core, bmincore, rows, nrows);
+                       box_of_slot, btight, bstart, bcell, inrow, core, bmincore, rows, nrows, chunk);
     HPD_HIP(hipGetLastError());
 }
 
@@ -992,12 +995,14 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
                       unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
                       unsigned long long* nopen, hipStream_t s) {
     if (a.nbox <= 0) return;
-    hipLaunchKernelGGL((k_box_union<T, D>), dim3(group_blocks<D>(a.nbox)), dim3(kThreads), 0, s, a,
-                       roff, rboxes, rsnap, core, blist, nlist, bparent, heavy, nheavy, heavy_cap,
+    hipLaunchKernelGGL((k_box_union<T, D>),
+                       dim3(persistent_blocks<k_box_union<T, D>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, blist, nlist, bparent, heavy, nheavy, heavy_cap,
                        nopen);
     // (its waves leave at once when there are no entries)
-    hipLaunchKernelGGL((k_box_union_heavy<T, D>), dim3(group_blocks<1>(a.nrows)), dim3(kThreads), 0,
-                       s, a, box_of_slot, core, bparent, static_cast<const int2*>(heavy),
+    hipLaunchKernelGGL((k_box_union_heavy<T, D>),
+                       dim3(persistent_blocks<k_box_union_heavy<T, D>>(a.nrows / kHeavyRows + 1, 1)),
+                       dim3(kThreads), 0, s, a, box_of_slot, core, bparent, static_cast<const int2*>(heavy),
                        static_cast<const unsigned long long*>(nheavy), heavy_cap);
     HPD_HIP(hipGetLastError());
 }

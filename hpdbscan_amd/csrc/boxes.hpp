@@ -113,12 +113,13 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
 // core[s] = 1 for the rows of tight boxes with >= minPts rows (btight bit 1),
 // 0 for every other row; bmincore[b] = inrow[bstart[b]] for those boxes
 // (every row is core and a box holds its rows in input order), INT_MAX for
-// the others; rows[..] = the other rows whose cell can hold cores (btight
-// bit 2), as (slot, cell), *nrows += their number
+// the others; rows[..] = the chunks of up to `chunk` (a power of two) rows of
+// those other boxes whose cell can hold cores (btight bit 2), as (first slot,
+// cell), *nrows += their number
 void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btight,
                       const int32_t* bstart, const int32_t* bcell, const uint32_t* inrow,
                       uint8_t* core, int32_t* bmincore, int2* rows, unsigned int* nrows,
-                      hipStream_t s);
+                      int chunk, hipStream_t s);
 // p[0, n) = v
 void fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 

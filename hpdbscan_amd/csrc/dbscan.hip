@@ -134,98 +134,137 @@ __global__ __launch_bounds__(kThreads) void k_core(const DbscanArgs<T> a, uint8_
     (void)ncore;
 }
 
-// Box-mode core counts: the rows listed in a.crows (rows outside the full
-// boxes, in cells that can hold cores), G lanes per row, a neighbour box per
-// lane.  A box farther than eps from the row (bounding box) is skipped, one
-// within eps of its farthest corner counts whole, the others are tested row
-// by row: small ones by their lane, larger ones by the whole wave with the
-// candidates on the lanes.
+// Orders the LDS accesses of a wave's lanes among each other (the hardware
+// keeps a wave's LDS operations in order; this keeps the compiler from moving
+// or caching them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Box-mode core counts: the chunks listed in a.crows (up to G rows of one
+// box, boxes outside the full ones, in cells that can hold cores), G lanes per
+// chunk, a neighbour box per lane: the chunk's rows and counts lie in LDS, and
+// each lane holds its box against one row after the other.  A box farther
+// than eps from the row is skipped, one within eps of its farthest corner
+// counts whole, the others are tested row by row: small ones by their lane,
+// larger ones by the whole wave with the candidates on the lanes.
 //
-// Bound by latency (list -> cell -> box ranges -> boxes) and VALU issue of
-// the box tests.  kCount: also add the row-row distance tests executed to
-// *ntests (the instrumented variant).
+// Bound by VALU issue of the box tests and by the latency of list -> cell ->
+// box ranges -> boxes, which the rows of a chunk share.  kCount: also add the
+// row-row distance tests executed to *ntests (the instrumented variant).
 template <typename T, int D, bool kCount = false>
 __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                                                         uint8_t* __restrict__ core,
                                                         unsigned long long* __restrict__ ntests) {
     constexpr int G = kGroup<D>;
-    constexpr int kPer = 64 / G;  // rows of a wave
-    const int32_t nrows = uniform(static_cast<int32_t>(*a.ncrows_dev));
-    const int gl = lane_id() & (G - 1);
+    constexpr int kPer = 64 / G;  // chunks of a wave
+    __shared__ T rows_lds[kWavesPerBlock][64][D];
+    __shared__ uint32_t cnt_lds[kWavesPerBlock][64];
+    const int w = static_cast<int>(threadIdx.x >> 6);
+    const int32_t nitems = uniform(static_cast<int32_t>(*a.ncrows_dev));
+    const int lane = lane_id();
+    const int g0 = lane & ~(G - 1);  // first lane of the group
+    T(*rx)[D] = rows_lds[w];
+    uint32_t* rc = cnt_lds[w];
+    // the lanes of the caller's group where `on`, as G bits
+    auto group_bits = [&](bool on) {
+        return static_cast<uint32_t>(ballot(on) >> g0) & ((1u << G) - 1u);
+    };
     const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     unsigned long long tests = 0;
-    for (int32_t base = first_wave() * kPer; base < nrows; base += wave_stride() * kPer) {
-        const int32_t i = base + lane_id() / G;
-        const bool on = i < nrows;
-        const int2 it = a.crows[on ? i : nrows - 1];
-        const int32_t p = it.x, u = it.y;
+    for (int32_t base = first_wave() * kPer; base < nitems; base += wave_stride() * kPer) {
+        const int32_t i = base + lane / G;
+        const bool on = i < nitems;
+        const int2 it = a.crows[on ? i : nitems - 1];
+        const int32_t u = it.y;
+        const int32_t b = a.box_of_slot[it.x];
+        const int32_t p = it.x + (lane & (G - 1));
+        const bool has = on && p < a.bstart[b + 1];
         T pc[D];
-        load_row<T, D>(a.soa, a.ld, p, pc);
+        load_row<T, D>(a.soa, a.ld, has ? p : it.x, pc);
+#pragma unroll
+        for (int j = 0; j < D; ++j) rx[lane][j] = pc[j];
+        rc[lane] = 0;
+        wave_lds_fence();
         const int32_t r0 = static_cast<int32_t>(a.roff[u]);
         const int32_t r1 = static_cast<int32_t>(a.roff[u + 1]);
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
         const uint32_t min_pts = jp.min_pts;
-        uint32_t cnt = 0;
-        bool need = on && min_pts > 0;
-        group_boxes<G>(need, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
-                       [&](bool valid, int32_t b) {
+        bool need = has && min_pts > 0;
+        group_boxes<G>(on && min_pts > 0, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
+                       [&](bool valid, int32_t b2) {
             int32_t q0 = 0, q1 = 0;
-            bool part = false;
-            uint32_t w = 0;
+            uint32_t part = 0;  // rows of the chunk the box is undecided for
+            const uint32_t open = group_bits(need);
             if (valid) {
-                T gmin2, gmax2;
-                point_box<T, D>(bbox, b, pc, gmin2, gmax2);
-                q0 = a.bstart[b];
-                q1 = a.bstart[b + 1];
-                const bool near = gmin2 <= eps2;
-                const bool whole = near && gmax2 <= eps2;
-                if (whole) w = static_cast<uint32_t>(q1 - q0);
-                part = near && !whole;
-            }
-            cnt += group_sum<G>(w);
-            need = need && cnt < min_pts;
-            if (__any(need && part)) {
-                const bool lane_walk = q1 - q0 <= kLaneRows;
-                uint32_t c = 0;
-                if (need && part && lane_walk) {
-                    for (int32_t q = q0; q < q1; ++q) {
-                        T qc[D];
-                        load_row<T, D>(a.soa, a.ld, q, qc);
-                        c += within<D>(pc, qc, eps2) ? 1u : 0u;
-                    }
-                    if constexpr (kCount) tests += static_cast<unsigned long long>(q1 - q0);
-                }
-                cnt += group_sum<G>(c);
-                need = need && cnt < min_pts;
-                for (uint64_t todo = ballot(need && part && !lane_walk); todo != 0;
-                     todo &= todo - 1) {
-                    const int j = static_cast<int>(__builtin_ctzll(todo));
-                    if (!((ballot(need) >> j) & 1)) continue;  // an earlier box was enough
-                    T pr[D];
+                Span<T> s[D];
 #pragma unroll
-                    for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], j);
-                    const uint32_t left =
-                        static_cast<uint32_t>(bcast(static_cast<int32_t>(min_pts - cnt), j));
-                    uint32_t visited = 0;
-                    const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, bcast(q0, j),
-                                                          bcast(q1, j), pr, bcast(eps2, j), left,
-                                                          visited);
-                    if (lane_id() / G == j / G) {
-                        cnt += got;
-                        need = need && cnt < min_pts;
-                    }
-                    if constexpr (kCount)
-                        if (lane_id() == 0) tests += visited;
+                for (int j = 0; j < D; ++j) s[j] = bbox[static_cast<int64_t>(b2) * D + j];
+                q0 = a.bstart[b2];
+                q1 = a.bstart[b2 + 1];
+                for (uint32_t m = open; m != 0; m &= m - 1) {
+                    const int k = __builtin_ctz(m);
+                    T gmin2, gmax2;
+                    point_box<T, D>(s, 0, rx[g0 + k], gmin2, gmax2);
+                    if (gmin2 > eps2) continue;
+                    if (gmax2 <= eps2) atomicAdd(&rc[g0 + k], static_cast<uint32_t>(q1 - q0));
+                    else part |= 1u << k;
                 }
             }
-            return !need;
+            wave_lds_fence();
+            need = need && rc[lane] < min_pts;
+            if (__any(part != 0)) {
+                const bool lane_walk = q1 - q0 <= kLaneRows;
+                part &= group_bits(need);
+                if (lane_walk) {
+                    for (uint32_t m = part; m != 0; m &= m - 1) {
+                        const int k = __builtin_ctz(m);
+                        uint32_t c = 0;
+                        for (int32_t q = q0; q < q1; ++q) {
+                            T qc[D];
+                            load_row<T, D>(a.soa, a.ld, q, qc);
+                            c += within<D>(rx[g0 + k], qc, eps2) ? 1u : 0u;
+                        }
+                        if (c) atomicAdd(&rc[g0 + k], c);
+                        if constexpr (kCount) tests += static_cast<unsigned long long>(q1 - q0);
+                    }
+                }
+                for (uint64_t todo = ballot(part != 0 && !lane_walk); todo != 0; todo &= todo - 1) {
+                    const int j = static_cast<int>(__builtin_ctzll(todo));
+                    const uint32_t mp = static_cast<uint32_t>(bcast(static_cast<int32_t>(min_pts), j));
+                    for (uint32_t m = static_cast<uint32_t>(bcast(static_cast<int32_t>(part), j));
+                         m != 0; m &= m - 1) {
+                        const int row = (j & ~(G - 1)) + __builtin_ctz(m);
+                        wave_lds_fence();
+                        const uint32_t now =
+                            static_cast<uint32_t>(uniform(static_cast<int32_t>(rc[row])));
+                        if (now >= mp) continue;  // an earlier box was enough
+                        T pr[D];
+#pragma unroll
+                        for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], row);
+                        uint32_t visited = 0;
+                        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, bcast(q0, j),
+                                                              bcast(q1, j), pr, bcast(eps2, j),
+                                                              mp - now, visited);
+                        if (lane == 0) rc[row] = now + got;
+                        if constexpr (kCount)
+                            if (lane == 0) tests += visited;
+                    }
+                }
+                wave_lds_fence();
+                need = need && rc[lane] < min_pts;
+            }
+            return group_bits(need) == 0;
         });
-        // (launch_core_rows_init wrote 0 for every listed row)
-        if (on && gl == 0 && cnt >= min_pts) {
-            core[p] = 1;
-            atomicMin(&a.bmincore[a.box_of_slot[p]], static_cast<int32_t>(a.inrow[p]));
-        }
+        // (launch_core_init wrote 0 for every listed row)
+        wave_lds_fence();
+        const bool is_core = has && rc[lane] >= min_pts;
+        if (is_core) core[p] = 1;
+        const int32_t first =
+            group_min<G>(is_core ? static_cast<int32_t>(a.inrow[p]) : INT_MAX);
+        if (lane == g0 && first != INT_MAX) atomicMin(&a.bmincore[b], first);
+        wave_lds_fence();
     }
     if constexpr (kCount) block_add<kThreads>(tests, ntests);
 }
@@ -847,14 +886,17 @@ void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntes
             // rows of tight boxes with >= minPts rows are core, every other
             // row starts non-core; the rows that can be core are listed
             launch_core_init(a.n, a.box_of_slot, a.btight, a.bstart, a.bcell, a.inrow, core,
-                             a.bmincore, a.crows, a.ncrows_dev, s);
+                             a.bmincore, a.crows, a.ncrows_dev, kGroup<D>, s);
             if (count_start) HPD_HIP(hipEventRecord(count_start, s));
+            constexpr int per_wave = 64 / kGroup<D>;
             if (ntests)
-                hipLaunchKernelGGL((k_core_rows<T, D, true>), dim3(group_blocks<D>(a.n)),
+                hipLaunchKernelGGL((k_core_rows<T, D, true>),
+                                   dim3(persistent_blocks<k_core_rows<T, D, true>>(a.n, per_wave)),
                                    dim3(kThreads), 0, s, a, core, ntests);
             else
-                hipLaunchKernelGGL((k_core_rows<T, D>), dim3(group_blocks<D>(a.n)), dim3(kThreads), 0,
-                                   s, a, core, nullptr);
+                hipLaunchKernelGGL((k_core_rows<T, D, false>),
+                                   dim3(persistent_blocks<k_core_rows<T, D, false>>(a.n, per_wave)),
+                                   dim3(kThreads), 0, s, a, core, nullptr);
             HPD_HIP(hipGetLastError());
             return;
         }
@@ -934,8 +976,9 @@ void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* b
     const unsigned gw = blocks_for(a.nitems, kWavesPerBlock);
     if constexpr (std::is_floating_point<T>::value) {
         if (bcluster && a.bbox) {
-            hipLaunchKernelGGL((k_border_rows<T, D>), dim3(group_blocks<D>(a.n)), dim3(kThreads), 0,
-                               s, a, core, bcluster, static_cast<const int2*>(a.brows),
+            hipLaunchKernelGGL((k_border_rows<T, D>),
+                               dim3(persistent_blocks<k_border_rows<T, D>>(a.n, 64 / kGroup<D>)),
+                               dim3(kThreads), 0, s, a, core, bcluster, static_cast<const int2*>(a.brows),
                                static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
                                amb_list);
             HPD_HIP(hipGetLastError());

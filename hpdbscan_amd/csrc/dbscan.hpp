@@ -39,9 +39,9 @@ struct DbscanArgs {
     const void* bbox = nullptr;
     // box mode: box ranges of the neighbour rows (in place of rcells)
     const int2* rboxes = nullptr;
-    // box mode: the rows to count (outside the full boxes, in cells that can
-    // hold cores) and the non-core rows of the border pass, as (slot, cell),
-    // with their numbers (device words, zeroed by the caller)
+    // box mode: the chunks of rows to count (launch_core_init) and the
+    // non-core rows of the border pass, as (slot, cell), with their numbers
+    // (device words, zeroed by the caller)
     int2* crows = nullptr;
     unsigned int* ncrows_dev = nullptr;
     int2* brows = nullptr;

@@ -273,19 +273,41 @@ constexpr int kGroup = D <= 3 ? 8 : 16;
 constexpr int kLaneRows = 8;
 
 // Persistent grids: wave w of them takes items w, w + wave_stride(), ...
+// Workgroups go to the 8 XCDs in turn, and each XCD has an L2 of its own, so
+// the waves are numbered XCD by XCD: of the stretch of items that the grid
+// works on together, each XCD takes one eighth, and neighbouring items, which
+// read the same boxes, meet in one L2.
 constexpr int kGroupThreads = 256;
+constexpr unsigned kXcds = 8;
 __device__ __forceinline__ int32_t first_wave() {
-    return __builtin_amdgcn_readfirstlane(static_cast<int32_t>(blockIdx.x) * (kGroupThreads / 64) +
+    unsigned blk = blockIdx.x;
+    if (gridDim.x % kXcds == 0) blk = (blk % kXcds) * (gridDim.x / kXcds) + blk / kXcds;
+    return __builtin_amdgcn_readfirstlane(static_cast<int32_t>(blk) * (kGroupThreads / 64) +
                                           static_cast<int32_t>(threadIdx.x >> 6));
 }
 __device__ __forceinline__ int32_t wave_stride() {
     return static_cast<int32_t>(gridDim.x) * (kGroupThreads / 64);
 }
-// Blocks of one over at most n items: 8 blocks on each of the 256 CUs.
-template <int D>
-inline unsigned group_blocks(int64_t n) {
-    const int64_t b = (n * kGroup<D> + kGroupThreads - 1) / kGroupThreads;
-    return static_cast<unsigned>(b < 2048 ? (b > 0 ? b : 1) : 2048);
+// Blocks of one over at most `items` items, `per_wave` per wave: no more than
+// run at once (every block then starts at once, and none is left to run by
+// itself after the others), a multiple of the XCDs when there are that many.
+template <auto Kernel>
+inline unsigned persistent_blocks(int64_t items, int per_wave) {
+    static const int64_t resident = [] {
+        int dev = 0, cus = 0, per_cu = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void*>(Kernel), kGroupThreads, 0) != hipSuccess ||
+            cus < 1 || per_cu < 1)
+            return int64_t{2048};
+        return static_cast<int64_t>(cus) * per_cu;
+    }();
+    const int64_t per_block = static_cast<int64_t>(per_wave) * (kGroupThreads / 64);
+    int64_t b = (items + per_block - 1) / per_block;
+    if (b > resident) b = resident;
+    if (b >= kXcds) b -= b % kXcds;
+    return static_cast<unsigned>(b > 0 ? b : 1);
 }
 
 // Sum, minimum and maximum over a group of G lanes.
