@@ -337,6 +337,23 @@ static inline int bits_for(uint64_t max_value) {
     return max_value == 0 ? 0 : 64 - __builtin_clzll(max_value);
 }
 
+// device bytes of the job table and the min/max pass of a run
+template <typename T, int D>
+static size_t table_bytes(int64_t n, int64_t njobs) {
+    const size_t nn = static_cast<size_t>(n), nj = static_cast<size_t>(njobs);
+    const size_t mm_blocks = nn / static_cast<size_t>(minmax_rows_per_block()) + nj + 1;
+    return sizeof(T) * 2 * D * (mm_blocks + nj) + 4 * (mm_blocks + nj + 2) + 64 +
+           sizeof(JobParams<T>) * nj + 8 * 256;
+}
+
+// most neighbour rows of n rows: 3^(D-1) per cell
+template <int D>
+constexpr int64_t range_bound(int64_t n) {
+    int64_t r = n;
+    for (int j = 1; j < D; ++j) r *= 3;
+    return r;
+}
+
 // worst-case device workspace of one run with n rows
 template <typename T, int D>
 static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
@@ -355,10 +372,7 @@ static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
     b += 2 * D * 8 * nn;                       // box bounding boxes
     b += gather_part_bytes(n, D, static_cast<int>(sizeof(T)));  // their per-block shares
     if (sort_moves_rows<T, D>()) b += 2 * sizeof(T) * D * nn;   // rows between sort passes
-    const size_t nj = static_cast<size_t>(njobs);
-    const size_t mm_blocks = nn / static_cast<size_t>(minmax_rows_per_block()) + nj + 1;
-    b += sizeof(T) * 2 * D * (mm_blocks + nj) + 4 * (mm_blocks + nj + 2) + 64;  // min/max
-    b += sizeof(JobParams<T>) * nj + 4 * nn;   // job table, job of every cell
+    b += table_bytes<T, D>(n, njobs) + 4 * nn;  // job table, min/max, job of every cell
     if (one_thread) b += 8 * nn + 4 * nn + nn + 4;  // ambiguous rows, f, involved, flag
     b += 8 * 16;                               // statistics, counters
     b += 54 * 256 + 64 * 1024;                 // alignment
@@ -494,15 +508,15 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     uint8_t* cell_core = boxes ? A.take_n<uint8_t>(nn) : nullptr;
     // the count pass keeps the rows it finds in scratch64 (idle until the
     // core count) when every cell's 3^(D-1) rows fit, and the fill copies them
-    int32_t stash_rows = 1;
-    for (int j = 1; j < D; ++j) stash_rows *= 3;
-    int2* stash = scratch64 && static_cast<uint64_t>(m) * static_cast<uint64_t>(stash_rows) <= nn
+    constexpr int32_t max_rows = static_cast<int32_t>(range_bound<D>(1));
+    int2* stash = scratch64 && !neighbor_rows_wide(m, max_rows) &&
+                          static_cast<uint64_t>(m) * static_cast<uint64_t>(max_rows) <= nn
                       ? reinterpret_cast<int2*>(scratch64)
                       : nullptr;
     // up to 27 rows per cell (D <= 4): the copy puts the nearest rows first
     const bool by_class = stash && D <= 4;
     launch_neighbor_count<K, T>(ucell, ustart, host_count(m), jobs, njobs, job_of_cell, nranges,
-                                cell_core, &dstats[0], &dstats[4], stash, stash_rows, rcenter,
+                                cell_core, &dstats[0], &dstats[4], stash, max_rows, rcenter,
                                 by_class, s, ctab);
     // the per-cell counts, scanned together (totals at entry m); box mode
     // has no use for the 64-row chunks of every cell unless the union runs on
@@ -557,13 +571,13 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     int2* rcells = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
     int2* items = row_tables ? X.take_n<int2>(max_items) : nullptr;
     if (boxes && stash)
-        launch_neighbor_copy(stash, stash_rows, m, nranges, cbox, rboxes, rcenter, by_class, s);
+        launch_neighbor_copy(stash, max_rows, m, nranges, cbox, rboxes, rcenter, by_class, s);
     else if (boxes)
         launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
-                                   nullptr, rboxes, rcenter, s, ctab, cbox);
+                                   nullptr, rboxes, rcenter, max_rows, s, ctab, cbox);
     else
         launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
-                                   ranges, rcells, rcenter, s);
+                                   ranges, rcells, rcenter, max_rows, s);
     if (!boxes)
         launch_work_items(ustart, host_count(m), nchunks, host_count(static_cast<int64_t>(hc[2])),
                           items, s);
@@ -626,7 +640,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         a.nitems = static_cast<int32_t>(*h);
         launch_work_items(ustart, host_count(m), nchunks, host_count(a.nitems), items, s);
         launch_neighbor_fill<K, T>(ucell, ustart, host_count(m), jobs, job_of_cell, nranges,
-                                   ranges, rcells, rcenter, s);
+                                   ranges, rcells, rcenter, max_rows, s);
     };
     tm.mark(M_INDEX);
 
@@ -785,14 +799,6 @@ enum StaticSlot : int {
     SS_WORDS = 32
 };
 
-// most neighbour rows of n rows: 3^(D-1) per cell
-template <int D>
-static inline int64_t range_bound(int64_t n) {
-    int64_t r = n;
-    for (int j = 1; j < D; ++j) r *= 3;
-    return r;
-}
-
 template <typename T, int D>
 static size_t static_aux_bytes(int64_t n) {
     return align_up(static_cast<size_t>(range_bound<D>(n)) * sizeof(int2), 256) +
@@ -893,13 +899,14 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     const Count M{n, &sc[SS_M]};
     const Count NB{n, &sc[SS_NBOX]};
     launch_neighbor_count<K, T>(ucell, ustart, M, jobs, njobs, job_of_cell, nranges, cell_core,
-                                &dstats[0], &dstats[4], nullptr, 1, rcenter, false, s);
+                                &dstats[0], &dstats[4], nullptr,
+                                static_cast<int32_t>(range_bound<D>(1)), rcenter, false, s);
     exclusive_scan_u32_dev(nranges, nranges, M, tmp, s);
     copy_at_count(nranges, &sc[SS_M], &sc[SS_RANGES], s);
     const int64_t R = range_bound<D>(n);
     int2* rboxes = X.take_n<int2>(static_cast<size_t>(R));
     launch_neighbor_fill<K, T>(ucell, ustart, M, jobs, job_of_cell, nranges, nullptr, rboxes,
-                               rcenter, s, nullptr, cbox);
+                               rcenter, static_cast<int32_t>(range_bound<D>(1)), s, nullptr, cbox);
 
     BoxArgs<T> ba;
     ba.soa = soa;

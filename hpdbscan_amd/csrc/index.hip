@@ -168,6 +168,139 @@ __device__ __forceinline__ int32_t job_of_key(const JobParams<T>* __restrict__ j
     return lo;
 }
 
+// The same for the cells of a wave, consecutive and ascending over its lanes
+// (several lanes may hold one cell): one search for the first active lane's
+// key (wave-uniform, scalar loads), then each lane steps past the jobs that
+// end before its key.
+template <typename T>
+__device__ __forceinline__ int32_t job_of_key_wave(const JobParams<T>* __restrict__ jobs,
+                                                   int32_t njobs, uint64_t key) {
+    if (njobs == 1) return 0;
+    const uint64_t key0 =
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(key))) |
+        (static_cast<uint64_t>(static_cast<uint32_t>(
+             __builtin_amdgcn_readfirstlane(static_cast<int>(key >> 32))))
+         << 32);
+    int32_t j = job_of_key(jobs, njobs, key0);
+    while (j + 1 < njobs && jobs[j + 1].key_base <= key) ++j;
+    return j;
+}
+
+// Neighbour rows of a cell by a group of L lanes (L >= 16 dividing 64), one
+// row per lane and round: for few cells, where one thread per cell leaves the
+// chip idle and walks up to 3^(D-1) searches one after the other (6-D: 243
+// rows for each of 5947 cells, 625 us counted and 635 us filled; by groups of
+// 64 lanes 33 us each).  Count (kFill false) and fill write what
+// k_neighbor_rows_count and k_neighbor_rows_fill write; with by_class (all
+// rows in one round) each cell's rows are filled nearest first.
+template <typename K, typename T, int L, bool kFill>
+__global__ __launch_bounds__(256) void k_neighbor_rows_wide(
+    const K* __restrict__ ucell, const int32_t* __restrict__ ustart, Count mc,
+    const JobParams<T>* __restrict__ jobs, int32_t njobs, int32_t* __restrict__ job_of_cell,
+    uint32_t* __restrict__ nranges, uint8_t* __restrict__ cell_core,
+    unsigned long long* __restrict__ sumcand, unsigned long long* __restrict__ rows_total,
+    int2* __restrict__ ranges, int2* __restrict__ rcells, int32_t* __restrict__ rcenter,
+    const int32_t* __restrict__ ctab, const int32_t* __restrict__ cbox, bool by_class) {
+    const int32_t m = static_cast<int32_t>(mc.get());
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const bool on = t / L < m;
+    const int32_t u = on ? static_cast<int32_t>(t / L) : m - 1;
+    const int gl = static_cast<int>(t % L);
+    const int g0 = __lane_id() & ~(L - 1);
+    constexpr uint64_t kMask = L == 64 ? ~uint64_t{0} : (uint64_t{1} << (L & 63)) - 1;
+    auto group = [&](bool v) { return (ballot(v) >> g0) & kMask; };
+    const uint64_t lt = (uint64_t{1} << gl) - 1;
+    uint64_t cand = 0;
+    uint32_t cnt = 0;
+    uint64_t count_u = 0;
+    if (m > 0) {
+        const uint64_t key = static_cast<uint64_t>(ucell[u]);
+        const int32_t j = kFill ? job_of_cell[u] : job_of_key_wave(jobs, njobs, key);
+        const uint64_t base = jobs[j].key_base;
+        const CellParams& cp = jobs[j].cp;
+        uint64_t idx[kMaxDims];
+        decode_cell(key - base, cp, idx);
+        const uint64_t lo0 = idx[0] > 0 ? 1 : 0;
+        const uint64_t hi0 = idx[0] + 1 < cp.ncell[0] ? 1 : 0;
+        int nrows = 1;
+        for (int k = 1; k < cp.d; ++k) nrows *= 3;
+        const uint32_t w0 = kFill ? nranges[u] : 0u;
+        for (int r0 = 0; r0 < nrows; r0 += L) {
+            // row r of the odometer of for_each_row
+            const int r = r0 + gl;
+            int rem = r, nz = 0;
+            bool inside = r < nrows;
+            uint64_t c = key;
+#pragma unroll
+            for (int k = 1; k < kMaxDims; ++k) {
+                if (k >= cp.d) break;
+                const int dgt = rem % 3;
+                rem /= 3;
+                if (dgt == 0) {
+                    if (idx[k] == 0) inside = false;
+                    c -= cp.stride[k];
+                    ++nz;
+                } else if (dgt == 2) {
+                    if (idx[k] + 1 >= cp.ncell[k]) inside = false;
+                    c += cp.stride[k];
+                    ++nz;
+                }
+            }
+            int2 ab = make_int2(0, 0);
+            if (inside)
+                ab = ctab ? row_cells_tab(ctab, c - lo0, c + hi0)
+                          : row_cells(ucell, m, c - lo0, c + hi0, 0);
+            const bool found = ab.y > ab.x;
+            const uint64_t mask = group(found);
+            if (kFill) {
+                uint32_t at = cnt + static_cast<uint32_t>(__popcll(mask & lt));
+                if (by_class) {
+                    at = 0;
+#pragma unroll
+                    for (int cl = 0; cl < 4; ++cl) {
+                        const uint64_t mine = group(found && nz == cl);
+                        if (cl < nz) at += static_cast<uint32_t>(__popcll(mine));
+                        else if (cl == nz) at += static_cast<uint32_t>(__popcll(mine & lt));
+                    }
+                }
+                if (found && on) {
+                    const uint32_t w = w0 + at;
+                    if (r == (nrows - 1) / 2) rcenter[u] = static_cast<int32_t>(w);
+                    if (ranges) ranges[w] = make_int2(ustart[ab.x], ustart[ab.y]);
+                    rcells[w] = cbox ? make_int2(cbox[ab.x], cbox[ab.y]) : ab;
+                }
+            } else if (found) {
+                cand += static_cast<uint64_t>(ustart[ab.y] - ustart[ab.x]);
+            }
+            cnt += static_cast<uint32_t>(__popcll(mask));
+        }
+        if (!kFill) {
+#pragma unroll
+            for (int o = L / 2; o > 0; o >>= 1) cand += __shfl_xor(cand, o, 64);
+            count_u = static_cast<uint64_t>(ustart[u + 1] - ustart[u]);
+            if (on && gl == 0) {
+                job_of_cell[u] = j;
+                nranges[u] = cnt;
+                if (cell_core) cell_core[u] = cand >= jobs[j].min_pts ? 1 : 0;
+            }
+        }
+    }
+    if constexpr (!kFill) {
+        const bool lead = on && gl == 0;
+        block_add2<256>(lead ? static_cast<unsigned long long>(cand * count_u) : 0ull,
+                        lead ? static_cast<unsigned long long>(cnt) : 0ull, sumcand, rows_total);
+    }
+}
+
+// Lanes per cell of the kernel above (0: one thread per cell instead).  Up to
+// 2^22 threads, about 8 times what the chip holds; above, one thread per cell
+// fills it (5M 4-D rows, 362k cells: 87 us against 118).  D <= 2 has at most
+// 3 rows.
+inline int wide_lanes(int64_t cells, int32_t rows) {
+    const int lanes = rows <= 3 ? 0 : rows <= 9 ? 16 : rows <= 27 ? 32 : 64;
+    return cells * lanes <= (int64_t{1} << 22) ? lanes : 0;
+}
+
 template <typename K, typename T>
 __global__ __launch_bounds__(256) void k_neighbor_rows_count(const K* __restrict__ ucell,
                                                              const int32_t* __restrict__ ustart,
@@ -191,7 +324,7 @@ __global__ __launch_bounds__(256) void k_neighbor_rows_count(const K* __restrict
     uint32_t nranges_u = 0;
     if (u < m) {
         const uint64_t key = static_cast<uint64_t>(ucell[u]);
-        const int32_t j = job_of_key(jobs, njobs, key);
+        const int32_t j = job_of_key_wave(jobs, njobs, key);
         job_of_cell[u] = j;
         const uint64_t base = jobs[j].key_base;
         uint32_t cnt = 0;
@@ -395,16 +528,44 @@ void launch_cells(const K* keys, int64_t n, int shift, uint32_t* flags, uint32_t
     HPD_HIP(hipGetLastError());
 }
 
+bool neighbor_rows_wide(int64_t cells, int32_t rows) { return wide_lanes(cells, rows) > 0; }
+
+template <typename K, typename T, bool kFill>
+static void launch_wide(int lanes, const K* ucell, const int32_t* ustart, Count m,
+                        const JobParams<T>* jobs, int32_t njobs, int32_t* job_of_cell,
+                        uint32_t* nranges, uint8_t* cell_core, unsigned long long* sumcand,
+                        unsigned long long* rows_total, int2* ranges, int2* rcells,
+                        int32_t* rcenter, const int32_t* ctab, const int32_t* cbox, bool by_class,
+                        hipStream_t s) {
+    const dim3 grid(blocks_for(m.host * lanes, 256));
+#define HPD_WIDE(L)                                                                            \
+    hipLaunchKernelGGL((k_neighbor_rows_wide<K, T, L, kFill>), grid, dim3(256), 0, s, ucell,   \
+                       ustart, m, jobs, njobs, job_of_cell, nranges, cell_core, sumcand,       \
+                       rows_total, ranges, rcells, rcenter, ctab, cbox, by_class)
+    if (lanes == 16) HPD_WIDE(16);
+    else if (lanes == 32) HPD_WIDE(32);
+    else HPD_WIDE(64);
+#undef HPD_WIDE
+    HPD_HIP(hipGetLastError());
+}
+
 template <typename K, typename T>
 void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
                            const JobParams<T>* jobs, int32_t njobs, int32_t* job_of_cell,
                            uint32_t* nranges, uint8_t* cell_core, unsigned long long* sumcand,
-                           unsigned long long* rows_total, int2* stash, int32_t stash_rows,
+                           unsigned long long* rows_total, int2* stash, int32_t max_rows,
                            int32_t* rcenter, bool by_class, hipStream_t s, const int32_t* ctab) {
     if (m.host <= 0) return;
+    const int lanes = stash ? 0 : wide_lanes(m.host, max_rows);
+    if (lanes > 0) {
+        launch_wide<K, T, false>(lanes, ucell, ustart, m, jobs, njobs, job_of_cell, nranges,
+                                 cell_core, sumcand, rows_total, nullptr, nullptr, nullptr, ctab,
+                                 nullptr, false, s);
+        return;
+    }
     hipLaunchKernelGGL((k_neighbor_rows_count<K, T>), dim3(blocks_for(m.host, 256)), dim3(256), 0, s,
                        ucell, ustart, m, jobs, njobs, job_of_cell, nranges, cell_core, sumcand,
-                       rows_total, stash, stash_rows, rcenter, by_class, ctab);
+                       rows_total, stash, max_rows, rcenter, by_class, ctab);
     HPD_HIP(hipGetLastError());
 }
 
@@ -435,10 +596,19 @@ void launch_neighbor_copy(const int2* stash, int32_t stash_rows, int32_t m, cons
 
 template <typename K, typename T>
 void launch_neighbor_fill(const K* ucell, const int32_t* ustart, Count m,
-                          const JobParams<T>* jobs, const int32_t* job_of_cell,
-                          const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
+                          const JobParams<T>* jobs, int32_t* job_of_cell, uint32_t* roff,
+                          int2* ranges, int2* rcells, int32_t* rcenter, int32_t max_rows,
                           hipStream_t s, const int32_t* ctab, const int32_t* cbox) {
     if (m.host <= 0) return;
+    const int lanes = wide_lanes(m.host, max_rows);
+    if (lanes > 0) {
+        // nearest first where a cell's rows fit one round (D <= 4) and the
+        // box kernels read them
+        launch_wide<K, T, true>(lanes, ucell, ustart, m, jobs, 0, job_of_cell, roff, nullptr,
+                                nullptr, nullptr, ranges, rcells, rcenter, ctab, cbox,
+                                cbox && max_rows <= 27, s);
+        return;
+    }
     hipLaunchKernelGGL((k_neighbor_rows_fill<K, T>), dim3(blocks_for(m.host, 256)), dim3(256), 0, s,
                        ucell, ustart, m, jobs, job_of_cell, roff, ranges, rcells, rcenter, ctab, cbox);
     HPD_HIP(hipGetLastError());
@@ -477,13 +647,13 @@ HPD_INST_INDEX(uint64_t)
                                                      int32_t*, bool, hipStream_t,               \
                                                      const int32_t*);                           \
     template void launch_neighbor_fill<uint32_t, T>(const uint32_t*, const int32_t*, Count,     \
-                                                    const JobParams<T>*, const int32_t*,        \
-                                                    const uint32_t*, int2*, int2*, int32_t*,    \
+                                                    const JobParams<T>*, int32_t*, uint32_t*,   \
+                                                    int2*, int2*, int32_t*, int32_t,            \
                                                     hipStream_t, const int32_t*,                \
                                                     const int32_t*);                            \
     template void launch_neighbor_fill<uint64_t, T>(const uint64_t*, const int32_t*, Count,     \
-                                                    const JobParams<T>*, const int32_t*,        \
-                                                    const uint32_t*, int2*, int2*, int32_t*,    \
+                                                    const JobParams<T>*, int32_t*, uint32_t*,   \
+                                                    int2*, int2*, int32_t*, int32_t,            \
                                                     hipStream_t, const int32_t*,                \
                                                     const int32_t*);
 HPD_FOR_EACH_DTYPE(HPD_INST_ROWS)

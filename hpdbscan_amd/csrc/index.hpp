@@ -20,9 +20,9 @@ void launch_cells(const K* keys, int64_t n, int shift, uint32_t* flags, uint32_t
 // neighbour rows of cell u; cell_core[u] (when not null) = 1 if cell u has
 // >= minPts candidates (only then can it hold cores), else 0; adds
 // Σ_u count(u) * |candidates(u)| to *sumcand and Σ_u nranges[u] to
-// *rows_total (64-bit, unlike the scan of nranges).  With a stash (m * stash_rows
-// entries, stash_rows >= the most neighbour rows a cell can have) the
-// rows' cell ranges go to stash[u * stash_rows ..] and the own row's index
+// *rows_total (64-bit, unlike the scan of nranges).  max_rows = 3^(D-1), the
+// most neighbour rows a cell can have.  With a stash (m * max_rows entries) the
+// rows' cell ranges go to stash[u * max_rows ..] and the own row's index
 // among them to rcenter[u], for launch_neighbor_copy; with by_class (D <= 4)
 // each row's offset class (the number of dimensions it is offset in) rides
 // in the top bits of its two cell indices.
@@ -30,7 +30,7 @@ template <typename K, typename T>
 void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
                            const JobParams<T>* jobs, int32_t njobs, int32_t* job_of_cell,
                            uint32_t* nranges, uint8_t* cell_core, unsigned long long* sumcand,
-                           unsigned long long* rows_total, int2* stash, int32_t stash_rows,
+                           unsigned long long* rows_total, int2* stash, int32_t max_rows,
                            int32_t* rcenter, bool by_class, hipStream_t s,
                            const int32_t* ctab = nullptr);
 
@@ -56,10 +56,13 @@ void launch_neighbor_copy(const int2* stash, int32_t stash_rows, int32_t m, cons
 // load, not three dependent ones.  ranges may be null.
 template <typename K, typename T>
 void launch_neighbor_fill(const K* ucell, const int32_t* ustart, Count m,
-                          const JobParams<T>* jobs, const int32_t* job_of_cell,
-                          const uint32_t* roff, int2* ranges, int2* rcells, int32_t* rcenter,
+                          const JobParams<T>* jobs, int32_t* job_of_cell, uint32_t* roff,
+                          int2* ranges, int2* rcells, int32_t* rcenter, int32_t max_rows,
                           hipStream_t s, const int32_t* ctab = nullptr,
                           const int32_t* cbox = nullptr);
+// Whether the two take few cells by groups of lanes (no stash then: the fill
+// searches again).
+bool neighbor_rows_wide(int64_t cells, int32_t max_rows);
 
 void launch_chunk_counts(const int32_t* ustart, Count m, uint32_t* nchunks, hipStream_t s);
 
