@@ -381,8 +381,10 @@ static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
 
 template <typename T, int D, typename K>
 static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>* jobs,
-                      int32_t njobs, int key_bits, uint64_t key_total, bool boxes,
+                      int32_t njobs, int key_bits, uint64_t key_total, bool use_boxes,
                       int64_t* labels, hipStream_t s, PhaseTimer& tm) {
+    // (known false for integer rows: their box kernels are not compiled)
+    const bool boxes = std::is_floating_point<T>::value && use_boxes;
     Arena& A = *ctx.main_use;
     Arena& X = *ctx.aux_use;
     const size_t nn = static_cast<size_t>(n);
@@ -1103,6 +1105,56 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     return true;
 }
 
+// --------------------------------------------------------------------------
+// integer rows as float rows
+// --------------------------------------------------------------------------
+// Integer rows whose arithmetic float reproduces exactly run as float rows,
+// on boxes (200k lattice rows in 3-D: 5.1 ms by the row-level union of the
+// integer path, whose wrapping distance is not monotone in general):
+//   * coordinates and their spans at most 2^24: they are exact in float, and
+//     so is every (x - min), whose float the reference's cell index takes;
+//   * for any two rows that are candidates of each other, the squared
+//     differences and their sum at most 2^24 (exact in float, in any order)
+//     and at most the largest T (nothing wraps).  Candidates lie in the same
+//     or in adjacent cells, so |x - y| / eps < 2 plus the rounding of the two
+//     scaled values, each below span / eps <= 2^24 / eps.
+// EPS2 is the integer path's (truncated) value.
+
+// most |x - y| of candidates in a dimension of span `span` (both integers)
+static double candidate_span(double span, float eps) {
+    const double e = static_cast<double>(eps);
+    const double b = (2.0 + span / e * (1.0 / (1 << 21))) * e * 1.00001 + 1.0;
+    return std::min(span, std::floor(b));
+}
+
+// whether the sum of the squares of per-dimension spans stays exact
+template <typename T>
+static bool sum_exact(double sum) {
+    return sum <= 16777216.0 && sum <= static_cast<double>(std::numeric_limits<T>::max());
+}
+
+template <typename T, int D>
+static bool float_exact(const T* mn, const T* mx, float eps) {
+    double sum = 0.0;
+    for (int k = 0; k < D; ++k) {
+        const double lo = static_cast<double>(mn[k]), hi = static_cast<double>(mx[k]);
+        if (std::fabs(lo) > 16777216.0 || std::fabs(hi) > 16777216.0 || hi - lo > 16777216.0)
+            return false;
+        const double c = candidate_span(hi - lo, eps);
+        sum += c * c;
+    }
+    return sum_exact<T>(sum);
+}
+
+// What float_exact needs whatever the data: whether it can hold for eps at
+// all (the workspace for it is only taken then).  Spans below 2 eps can still
+// pass it; such data has a few cells and stays on the integer path.
+template <typename T, int D>
+static bool float_possible(float eps) {
+    return sum_exact<T>(static_cast<double>(D) * 4.0 * static_cast<double>(eps) *
+                        static_cast<double>(eps));
+}
+
 // A batch of jobs: rows [offsets[j], offsets[j+1]) of `pts` form job j with
 // its own eps[j] and min_pts[j].  A plain call is a batch of one.
 template <typename T, int D>
@@ -1121,7 +1173,25 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     PhaseTimer tm(ctx, s);
     tm.mark(M_START);
     Arena& A = *ctx.main_use;
-    A.reserve(workspace_bytes<T, D>(n, njobs, ctx.border_rule == HPD_BORDER_ONE_THREAD));
+    const bool one_thread = ctx.border_rule == HPD_BORDER_ONE_THREAD;
+    bool as_float = false;  // integer rows: room for them as float rows
+    if constexpr (std::is_integral<T>::value) {
+        // (not in a fixed workspace, whose size the integer path's needs set)
+        as_float = ctx.main_use == &ctx.main;
+        for (int32_t j = 0; j < njobs && as_float; ++j) as_float = float_possible<T, D>(eps[j]);
+        if (as_float) {
+            try {
+                A.reserve(workspace_bytes<float, D>(n, njobs, one_thread) +
+                          table_bytes<T, D>(n, njobs) +
+                          align_up(sizeof(float) * D * static_cast<size_t>(n), 256));
+            } catch (const Error& e) {
+                if (e.code != HPD_ENOMEM) throw;
+                (void)hipGetLastError();
+                as_float = false;
+            }
+        }
+    }
+    if (!as_float) A.reserve(workspace_bytes<T, D>(n, njobs, one_thread));
 
     // job table, first pass: row ranges and min/max blocks.  The host
     // vectors outlive every copy from them: the run ends with a stream sync.
@@ -1170,6 +1240,8 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
         double rcp_d;
         const T* mn = &hmm[static_cast<size_t>(j) * 2 * D];
         const Geometry g = make_geometry<T>(mn, mn + D, D, eps[j], &rcp_f, &rcp_d);
+        if constexpr (std::is_integral<T>::value)
+            as_float = as_float && float_exact<T, D>(mn, mn + D, eps[j]);
         if (g.overflow)
             throw Error(HPD_EUNSUPPORTED,
                         "the eps-grid has more than 2^64 cells (the reference's cell ids wrap)");
@@ -1192,20 +1264,51 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     if (njobs != 1) ctx.stats.total_cells = key_total;
     const int key_bits = bits_for(key_total > 0 ? key_total - 1 : 0);
     ctx.stats.key_bits = key_bits;
-    HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs, hipMemcpyHostToDevice, s));
 
-    // floating-point data runs on sub-boxes (the sort key then carries the
-    // sub-box digit below the cell id); integer data, or a grid so large
-    // that the digit does not fit beside the cell id, runs on cells
+    // floating-point data (and integer data that float reproduces) runs on
+    // sub-boxes (the sort key then carries the sub-box digit below the cell
+    // id); other integer data, or a grid so large that the digit does not fit
+    // beside the cell id, runs on cells
     const int split_bits = box_sub_bits(D, split_of(ctx, D));
-    const bool boxes = std::is_floating_point<T>::value && key_bits + split_bits <= 64;
+    const bool boxes = (std::is_floating_point<T>::value || as_float) && key_bits + split_bits <= 64;
     const int sort_bits = key_bits + (boxes ? split_bits : 0);
-    if (sort_bits <= 32)
-        run_keyed<T, D, uint32_t>(ctx, pts, n, jobs_dev, njobs, key_bits, key_total, boxes, labels,
-                                  s, tm);
-    else
-        run_keyed<T, D, uint64_t>(ctx, pts, n, jobs_dev, njobs, key_bits, key_total, boxes, labels,
-                                  s, tm);
+    auto run = [&](auto* rows, auto* table) {
+        using R = std::remove_const_t<std::remove_pointer_t<decltype(rows)>>;
+        if (sort_bits <= 32)
+            run_keyed<R, D, uint32_t>(ctx, rows, n, table, njobs, key_bits, key_total, boxes,
+                                      labels, s, tm);
+        else
+            run_keyed<R, D, uint64_t>(ctx, rows, n, table, njobs, key_bits, key_total, boxes,
+                                      labels, s, tm);
+    };
+    if constexpr (std::is_integral<T>::value) {
+        if (as_float && boxes) {
+            HostArray<JobParams<float>, 1> hf(static_cast<size_t>(njobs));
+            for (int32_t j = 0; j < njobs; ++j) {
+                JobParams<float>& f = hf[j];
+                f.cp = hj[j].cp;
+                f.key_base = hj[j].key_base;
+                f.row_begin = hj[j].row_begin;
+                f.row_end = hj[j].row_end;
+                for (int k = 0; k < D; ++k) f.minv[k] = static_cast<float>(hj[j].minv[k]);
+                f.eps2 = static_cast<float>(hj[j].eps2);
+                f.rcp_f = hj[j].rcp_f;
+                f.rcp_d = hj[j].rcp_d;
+                f.min_pts = hj[j].min_pts;
+            }
+            JobParams<float>* table = A.take_n<JobParams<float>>(static_cast<size_t>(njobs));
+            float* rows = A.take_n<float>(static_cast<size_t>(n) * D);
+            HPD_HIP(hipMemcpyAsync(table, hf.data(), sizeof(JobParams<float>) * njobs,
+                                   hipMemcpyHostToDevice, s));
+            launch_to_float<T>(pts, n * D, rows, s);
+            run(static_cast<const float*>(rows), table);
+        }
+    }
+    if (std::is_floating_point<T>::value || !as_float || !boxes) {
+        HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs,
+                               hipMemcpyHostToDevice, s));
+        run(pts, jobs_dev);
+    }
     if (ctx.timing) {
         ctx.stats.ms_grid = tm.ms(M_START, M_GRID);
         ctx.stats.ms_sort = tm.ms(M_GRID, M_SORT);

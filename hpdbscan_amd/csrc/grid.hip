@@ -310,6 +310,17 @@ __global__ __launch_bounds__(256) void k_geometry(JobParams<T>* __restrict__ job
 
 inline unsigned blocks_for(int64_t n, int t) { return static_cast<unsigned>((n + t - 1) / t); }
 
+// out[i] = in[i] as float; four values per thread, the block's loads of one
+// round side by side (no alignment of `in` beyond its own type's)
+template <typename T>
+__global__ __launch_bounds__(256) void k_to_float(const T* __restrict__ in, int64_t count,
+                                                  float* __restrict__ out) {
+    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 1024 + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (i0 + k * 256 < count) out[i0 + k * 256] = static_cast<float>(in[i0 + k * 256]);
+}
+
 }  // namespace
 
 template <typename T, int D>
@@ -321,6 +332,14 @@ void launch_geometry(JobParams<T>* jobs, int32_t njobs, const T* mm, int sub_bit
 }
 
 int minmax_rows_per_block() { return kMMRows; }
+
+template <typename T>
+void launch_to_float(const T* in, int64_t count, float* out, hipStream_t s) {
+    if (count <= 0) return;
+    hipLaunchKernelGGL(k_to_float<T>, dim3(blocks_for((count + 3) / 4, 256)), dim3(256), 0, s, in,
+                       count, out);
+    HPD_HIP(hipGetLastError());
+}
 
 template <typename T, int D>
 void launch_minmax(const T* pts, const JobParams<T>* jobs, int32_t njobs, const int32_t* bfirst,
@@ -375,5 +394,8 @@ void launch_gather_soa(const T* pts, int64_t n, const uint32_t* order, T* soa, i
     HPD_INST_GRID(T, 8)
 
 HPD_FOR_EACH_DTYPE(HPD_INST_GRID_ALL_D)
+
+#define HPD_INST_TO_FLOAT(T) template void launch_to_float<T>(const T*, int64_t, float*, hipStream_t);
+HPD_FOR_EACH_DTYPE(HPD_INST_TO_FLOAT)
 
 }  // namespace hpd

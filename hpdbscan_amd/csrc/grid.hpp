@@ -51,6 +51,10 @@ template <typename T, int D, typename K>
 void launch_cell_ids(const T* pts, int64_t n, const JobParams<T>* jobs, int32_t njobs, int sub_k,
                      int sub_bits, K* keys, uint32_t* vals, hipStream_t s);
 
+// out[i] = in[i] as float (integer rows whose values float holds exactly)
+template <typename T>
+void launch_to_float(const T* in, int64_t count, float* out, hipStream_t s);
+
 // soa[j * ld + i] = pts[order[i] * D + j]
 template <typename T, int D>
 void launch_gather_soa(const T* pts, int64_t n, const uint32_t* order, T* soa, int64_t ld,
