@@ -39,7 +39,8 @@ ROCM_LIB = "/opt/rocm/lib"
 
 # "file.hip:MACRO=value": one part of a file compiled in parts (side by side)
 SOURCES = ["capi.hip", "scan.hip", "radix_sort.hip", "grid.hip", "index.hip",
-           *(f"dbscan.hip:HPD_DBSCAN_PART={p}" for p in range(4)), "boxes.hip", "server.cpp"]
+           *(f"dbscan.hip:HPD_DBSCAN_PART={p}" for p in range(4)), "boxes.hip", "small.hip",
+           "server.cpp"]
 
 ARCH = os.environ.get("HPD_OFFLOAD_ARCH", "gfx950")
 

@@ -26,6 +26,7 @@
 #include "grid.hpp"
 #include "index.hpp"
 #include "internal.hpp"
+#include "small.hpp"
 
 namespace hpd {
 
@@ -768,6 +769,55 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
 }
 
 // --------------------------------------------------------------------------
+// small inputs
+// --------------------------------------------------------------------------
+// Waits for a small run's result and takes its statistics; false when it
+// refused the input (the general path then runs it, or reports why not), or
+// left ambiguous border rows to the one-thread rule.
+static bool read_small(Context& ctx, hipStream_t s) {
+    HPD_HIP(hipStreamSynchronize(s));
+    const SmallResult* r = reinterpret_cast<const SmallResult*>(ctx.host_scratch);
+    if (r->nonfinite || r->overflow || r->unfit ||
+        (r->ambiguous > 0 && ctx.border_rule == HPD_BORDER_ONE_THREAD))
+        return false;
+    ctx.stats.total_cells = r->total_cells;
+    ctx.stats.key_bits = bits_for(r->total_cells - 1);
+    ctx.stats.sum_candidates = r->sum_candidates;
+    ctx.stats.core_points = r->cores;
+    ctx.stats.noise_points = r->noise;
+    ctx.stats.ambiguous_borders = r->ambiguous;
+    ctx.stats.occupied_cells = r->cells;
+    ctx.stats.neighbor_rows = r->neighbor_rows;
+    ctx.stats.boxes = r->boxes;
+    return true;
+}
+
+template <typename T, int D>
+static size_t small_call_bytes(int64_t n) {
+    return small_workspace_bytes<T, D>(n) + align_up(sizeof(SmallResult), 256);
+}
+
+// One job of few rows through the all-pairs kernels (small.hip).
+template <typename T, int D>
+static bool run_small(Context& ctx, const T* pts, int64_t n, float eps, uint64_t min_pts,
+                      int64_t* labels, hipStream_t s) {
+    Arena& A = *ctx.main_use;
+    A.reserve(small_call_bytes<T, D>(n));
+    SmallResult* result = A.take_n<SmallResult>(1);
+    void* work = A.take(small_workspace_bytes<T, D>(n));
+    JobParams<T> jp{};
+    jp.row_end = n;
+    jp.min_pts = static_cast<uint32_t>(std::min<uint64_t>(min_pts, 0xffffffffull));
+    jp.eps2 = eps2_as<T>(eps);
+    jp.rcp_f = flushf(1.0f / flushf(eps));
+    jp.rcp_d = flushd(1.0 / flushd(static_cast<double>(eps)));
+    const int sub_k = split_of(ctx, D);
+    launch_small<T, D>(pts, n, jp, nullptr, sub_k, box_sub_bits(D, sub_k), work, result,
+                       reinterpret_cast<SmallResult*>(ctx.host_scratch), labels, s);
+    return read_small(ctx, s);
+}
+
+// --------------------------------------------------------------------------
 // the static pipeline (hpd_context_set_graph)
 // --------------------------------------------------------------------------
 // The same kernels as run_keyed, with every table sized by its worst case
@@ -810,7 +860,7 @@ static size_t static_aux_bytes(int64_t n) {
 template <typename T, int D>
 static size_t static_main_bytes(int64_t n, int32_t njobs) {
     return workspace_bytes<T, D>(n, njobs, false) + sizeof(uint64_t) * static_cast<size_t>(njobs) +
-           SS_WORDS * 4 + 64 * 1024 + 8 * 256;
+           SS_WORDS * 4 + sizeof(SmallResult) + 64 * 1024 + 8 * 256;
 }
 
 // The body of a static run on stream s: every launch of the run, nothing
@@ -822,11 +872,19 @@ static size_t static_main_bytes(int64_t n, int32_t njobs) {
 template <typename T, int D>
 static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
                         const int32_t* bfirst_dev, int32_t njobs, int32_t nblocks, int64_t* labels,
-                        uint32_t* sc, unsigned long long* dstats, hipStream_t s) {
+                        uint32_t* sc, unsigned long long* dstats, SmallResult* small,
+                        hipStream_t s) {
     using K = uint64_t;
     Arena& A = ctx.main;
     Arena& X = ctx.aux;
     X.reset();
+    if (njobs == 1 && n <= small_rows()) {
+        const int parts = split_of(ctx, D);
+        void* work = A.take(small_workspace_bytes<T, D>(n));
+        launch_small<T, D>(pts, n, JobParams<T>{}, jobs, parts, box_sub_bits(D, parts), work, small,
+                           reinterpret_cast<SmallResult*>(ctx.host_scratch), labels, s);
+        return;
+    }
     const size_t nn = static_cast<size_t>(n);
     const int64_t ld = (n + 15) & ~int64_t(15);
     const size_t L = static_cast<size_t>(ld);
@@ -1009,6 +1067,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     int32_t* bfirst_dev = A.take_n<int32_t>(static_cast<size_t>(njobs) + 1);
     uint32_t* sc = A.take_n<uint32_t>(SS_WORDS);
     unsigned long long* dstats = A.take_n<unsigned long long>(16);
+    SmallResult* small = A.take_n<SmallResult>(1);
 
     // host-made part of the job table: row ranges, eps2, minPts, reciprocals
     HostArray<JobParams<T>, 1> hj(static_cast<size_t>(njobs));
@@ -1052,7 +1111,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
         HPD_HIP(hipStreamBeginCapture(ctx.stream, hipStreamCaptureModeThreadLocal));
         CaptureGuard guard{ctx.stream};
         static_body<T, D>(ctx, pts, n, jobs_dev, bfirst_dev, njobs, nblocks, labels, sc, dstats,
-                          ctx.stream);
+                          small, ctx.stream);
         hipGraph_t g = nullptr;
         guard.open = false;
         HPD_HIP(hipStreamEndCapture(ctx.stream, &g));
@@ -1078,6 +1137,11 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     }
     HPD_HIP(hipGraphLaunch(ge.exec, s));
     ++ctx.graph_launches;
+    if (njobs == 1 && n <= small_rows()) {
+        const bool taken = read_small(ctx, s);
+        if (!taken) ++ctx.graph_fallbacks;
+        return taken;
+    }
     // one read-back after the run: counts, flags and statistics
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx.host_scratch);
     unsigned long long* hs = reinterpret_cast<unsigned long long*>(ctx.host_scratch) + 16;
@@ -1168,6 +1232,13 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
             !ctx.timing &&
             run_static<T, D>(ctx, static_cast<int>(sizeof(T)), pts, n, offsets, njobs, eps, min_pts,
                              labels, s))
+            return;
+    }
+    if constexpr (std::is_floating_point<T>::value) {
+        // few rows: all pairs compared (the timing marks and the executed
+        // tests are the general path's)
+        if (njobs == 1 && n <= small_rows() && !ctx.timing &&
+            run_small<T, D>(ctx, pts, n, eps[0], min_pts[0], labels, s))
             return;
     }
     PhaseTimer tm(ctx, s);
@@ -1378,18 +1449,27 @@ static void run_any(Context& ctx, int dt, const void* pts, int64_t n, int d,
 #undef HPD_RUN_CASE
 }
 
-// workspace_bytes of a plain call (one job) of any dtype and dimension
+// workspace of a plain call (one job) of any dtype and dimension: the general
+// path's, and that of the all-pairs kernels where they are tried first
+template <typename T, int D>
+static size_t workspace_call(int64_t n, bool one_thread) {
+    size_t b = workspace_bytes<T, D>(n, 1, one_thread);
+    if constexpr (std::is_floating_point<T>::value)
+        if (n <= small_rows()) b = std::max(b, small_call_bytes<T, D>(n));
+    return b;
+}
+
 template <typename T>
 static size_t workspace_typed(int64_t n, int d, bool one_thread) {
     switch (d) {
-        case 1: return workspace_bytes<T, 1>(n, 1, one_thread);
-        case 2: return workspace_bytes<T, 2>(n, 1, one_thread);
-        case 3: return workspace_bytes<T, 3>(n, 1, one_thread);
-        case 4: return workspace_bytes<T, 4>(n, 1, one_thread);
-        case 5: return workspace_bytes<T, 5>(n, 1, one_thread);
-        case 6: return workspace_bytes<T, 6>(n, 1, one_thread);
-        case 7: return workspace_bytes<T, 7>(n, 1, one_thread);
-        case 8: return workspace_bytes<T, 8>(n, 1, one_thread);
+        case 1: return workspace_call<T, 1>(n, one_thread);
+        case 2: return workspace_call<T, 2>(n, one_thread);
+        case 3: return workspace_call<T, 3>(n, one_thread);
+        case 4: return workspace_call<T, 4>(n, one_thread);
+        case 5: return workspace_call<T, 5>(n, one_thread);
+        case 6: return workspace_call<T, 6>(n, one_thread);
+        case 7: return workspace_call<T, 7>(n, one_thread);
+        case 8: return workspace_call<T, 8>(n, one_thread);
         default:
             throw Error(HPD_EUNSUPPORTED, "dimensions above " + std::to_string(kMaxDims) +
                                               " are not supported by this build");

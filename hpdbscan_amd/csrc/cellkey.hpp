@@ -1,13 +1,14 @@
 // The cell key of a row: the reference's linearised cell id
 // (spatial_index.h:144-165) offset by the job's key base, followed by the
-// row's sub-box digit.  Shared by the kernel that keys the rows for the sort
-// and the one that labels rows in input order, which must find the very key
-// the sort used.
+// row's sub-box digit, and the grid it lies in.  Shared by the kernel that keys
+// the rows for the sort and the one that labels rows in input order, which must
+// find the very key the sort used, and by the kernels of small inputs.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <limits>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -113,6 +114,97 @@ __device__ __forceinline__ uint64_t row_key(const T* __restrict__ p, const JobPa
         }
     }
     return ((jp.key_base + cell) << sub_bits) | sub;
+}
+
+// The reference starts max at numeric_limits<T>::min(): FLT_MIN / DBL_MIN for
+// floating types (the smallest positive normal), the lowest value for
+// integers.
+template <typename T>
+__device__ __forceinline__ T max_init() {
+    return std::numeric_limits<T>::min();
+}
+template <typename T>
+__device__ __forceinline__ T min_init() {
+    return std::numeric_limits<T>::max();
+}
+
+// std::min(m, c) == (c < m) ? c : m ; std::max(m, c) == (m < c) ? c : m
+template <typename T>
+__device__ __forceinline__ T ref_min(T m, T c) {
+    return (c < m) ? c : m;
+}
+template <typename T>
+__device__ __forceinline__ T ref_max(T m, T c) {
+    return (m < c) ? c : m;
+}
+
+// float / double -> integer as x86-64 cvttss2si / cvttsd2si produce it
+// (out of range or NaN: the "integer indefinite" value)
+__device__ __forceinline__ int64_t d2i64_x86(double v) {
+    if (!(v >= -9223372036854775808.0 && v < 9223372036854775808.0)) return INT64_MIN;
+    return static_cast<int64_t>(v);
+}
+__device__ __forceinline__ uint64_t d2u64_x86(double v) {
+    if (v < 9223372036854775808.0) return static_cast<uint64_t>(d2i64_x86(v));
+    return static_cast<uint64_t>(d2i64_x86(v - 9223372036854775808.0)) ^ 0x8000000000000000ull;
+}
+
+// cells of one dimension, ceil((max - min) / eps) + 1 (spatial_index.h:124-131)
+// with the reciprocal form and the flushing of the reference's build (device
+// code flushes denormal inputs and results itself)
+template <typename T>
+__device__ __forceinline__ uint64_t cells_of_dev(T mx, T mn, float rcp_f, double rcp_d) {
+    if constexpr (std::is_same<T, float>::value) {
+        const float v = (mx - mn) * rcp_f;
+        return d2u64_x86(static_cast<double>(ceilf(v))) + 1;
+    } else if constexpr (std::is_same<T, double>::value) {
+        const double v = (mx - mn) * rcp_d;
+        return d2u64_x86(ceil(v)) + 1;
+    } else {
+        const float v = int_diff_f32<T>(mx, mn) * rcp_f;
+        return d2u64_x86(static_cast<double>(ceilf(v))) + 1;
+    }
+}
+
+// The grid of one job from its min / max (mm: D minima, D maxima), into jp
+// (whose reciprocals the host wrote): cells per dimension, dimension order (an
+// insertion sort ascending by cells, which is what std::sort does for so few
+// keys: ties keep their order), strides, minima.  Returns the number of
+// cells; overflow becomes true when they exceed 2^64.
+template <typename T, int D>
+__device__ __forceinline__ uint64_t make_grid(const T* mm, JobParams<T>& jp, bool& overflow) {
+    uint64_t c[D];
+    uint64_t tot = 1;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        c[k] = cells_of_dev<T>(mm[D + k], mm[k], jp.rcp_f, jp.rcp_d);
+        uint64_t t;
+        if (__builtin_mul_overflow(tot, c[k], &t)) overflow = true;
+        tot = t;
+    }
+    int sw[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) sw[k] = k;
+    for (int k = 1; k < D; ++k) {
+        const int v = sw[k];
+        int i = k - 1;
+        while (i >= 0 && c[v] < c[sw[i]]) {
+            sw[i + 1] = sw[i];
+            --i;
+        }
+        sw[i + 1] = v;
+    }
+    uint64_t acc = 1;
+    jp.cp.d = D;
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+        jp.minv[k] = mm[k];
+        jp.cp.swapped[k] = sw[k];
+        jp.cp.stride[k] = acc;
+        jp.cp.ncell[k] = c[sw[k]];
+        acc *= c[sw[k]];
+    }
+    return tot;
 }
 
 }  // namespace hpd

@@ -22,28 +22,6 @@ namespace {
 constexpr int kMMThreads = 256;
 constexpr int kMMRows = 8 * kMMThreads;  // rows per partial block
 
-// The reference starts max at numeric_limits<T>::min(): FLT_MIN / DBL_MIN for
-// floating types (the smallest positive normal), the lowest value for
-// integers.
-template <typename T>
-__device__ __forceinline__ T max_init() {
-    return std::numeric_limits<T>::min();
-}
-template <typename T>
-__device__ __forceinline__ T min_init() {
-    return std::numeric_limits<T>::max();
-}
-
-// std::min(m, c) == (c < m) ? c : m ; std::max(m, c) == (m < c) ? c : m
-template <typename T>
-__device__ __forceinline__ T ref_min(T m, T c) {
-    return (c < m) ? c : m;
-}
-template <typename T>
-__device__ __forceinline__ T ref_max(T m, T c) {
-    return (m < c) ? c : m;
-}
-
 // first job whose partial-block range contains block b (bfirst ascending)
 __device__ __forceinline__ int32_t job_of_block(const int32_t* __restrict__ bfirst, int32_t njobs,
                                                 int32_t b) {
@@ -185,38 +163,8 @@ __global__ __launch_bounds__(256) void k_gather_soa(const T* __restrict__ pts, i
     for (int j = 0; j < D; ++j) soa[static_cast<int64_t>(j) * ld + i] = pts[o * D + j];
 }
 
-// float / double -> integer as x86-64 cvttss2si / cvttsd2si produce it
-// (out of range or NaN: the "integer indefinite" value)
-__device__ __forceinline__ int64_t d2i64_x86(double v) {
-    if (!(v >= -9223372036854775808.0 && v < 9223372036854775808.0)) return INT64_MIN;
-    return static_cast<int64_t>(v);
-}
-__device__ __forceinline__ uint64_t d2u64_x86(double v) {
-    if (v < 9223372036854775808.0) return static_cast<uint64_t>(d2i64_x86(v));
-    return static_cast<uint64_t>(d2i64_x86(v - 9223372036854775808.0)) ^ 0x8000000000000000ull;
-}
-
-// cells of one dimension, ceil((max - min) / eps) + 1 (spatial_index.h:124-131)
-// with the reciprocal form and the flushing of the reference's build (device
-// code flushes denormal inputs and results itself)
-template <typename T>
-__device__ __forceinline__ uint64_t cells_of_dev(T mx, T mn, float rcp_f, double rcp_d) {
-    if constexpr (std::is_same<T, float>::value) {
-        const float v = (mx - mn) * rcp_f;
-        return d2u64_x86(static_cast<double>(ceilf(v))) + 1;
-    } else if constexpr (std::is_same<T, double>::value) {
-        const double v = (mx - mn) * rcp_d;
-        return d2u64_x86(ceil(v)) + 1;
-    } else {
-        const float v = int_diff_f32<T>(mx, mn) * rcp_f;
-        return d2u64_x86(static_cast<double>(ceilf(v))) + 1;
-    }
-}
-
 // The grid of every job from its min / max (mm: 2D values per job), as the
-// host computes it after reading them back: cells per dimension, dimension
-// order (an insertion sort ascending by cells, which is what std::sort does
-// for so few keys: ties keep their order), strides; then key bases in job
+// host computes it after reading them back (make_grid); then key bases in job
 // order.  flags[0] |= 1: a grid of more than 2^64 cells; *sort_bits = bits
 // of the largest key + sub_bits; *total = all jobs' cells.  One block.
 template <typename T, int D>
@@ -235,40 +183,9 @@ __global__ __launch_bounds__(256) void k_geometry(JobParams<T>* __restrict__ job
         JobParams<T>& jp = jobs[j];
         uint64_t tot = 0;
         if (jp.row_end > jp.row_begin) {
-            const T* mn = &mm[static_cast<int64_t>(j) * 2 * D];
-            uint64_t c[D];
-            tot = 1;
             bool of = false;
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                c[k] = cells_of_dev<T>(mn[D + k], mn[k], jp.rcp_f, jp.rcp_d);
-                uint64_t t;
-                if (__builtin_mul_overflow(tot, c[k], &t)) of = true;
-                tot = t;
-            }
+            tot = make_grid<T, D>(&mm[static_cast<int64_t>(j) * 2 * D], jp, of);
             if (of) atomicOr(&bad, 1);
-            int sw[D];
-#pragma unroll
-            for (int k = 0; k < D; ++k) sw[k] = k;
-            for (int k = 1; k < D; ++k) {
-                const int v = sw[k];
-                int i = k - 1;
-                while (i >= 0 && c[v] < c[sw[i]]) {
-                    sw[i + 1] = sw[i];
-                    --i;
-                }
-                sw[i + 1] = v;
-            }
-            uint64_t acc = 1;
-            jp.cp.d = D;
-#pragma unroll
-            for (int k = 0; k < D; ++k) {
-                jp.minv[k] = mn[k];
-                jp.cp.swapped[k] = sw[k];
-                jp.cp.stride[k] = acc;
-                jp.cp.ncell[k] = c[sw[k]];
-                acc *= c[sw[k]];
-            }
         }
         cells[j] = tot;
     }
