@@ -878,7 +878,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     Arena& A = ctx.main;
     Arena& X = ctx.aux;
     X.reset();
-    if (njobs == 1 && n <= small_rows()) {
+    if (njobs == 1 && n <= small_rows(D)) {
         const int parts = split_of(ctx, D);
         void* work = A.take(small_workspace_bytes<T, D>(n));
         launch_small<T, D>(pts, n, JobParams<T>{}, jobs, parts, box_sub_bits(D, parts), work, small,
@@ -1137,7 +1137,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     }
     HPD_HIP(hipGraphLaunch(ge.exec, s));
     ++ctx.graph_launches;
-    if (njobs == 1 && n <= small_rows()) {
+    if (njobs == 1 && n <= small_rows(D)) {
         const bool taken = read_small(ctx, s);
         if (!taken) ++ctx.graph_fallbacks;
         return taken;
@@ -1237,7 +1237,7 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     if constexpr (std::is_floating_point<T>::value) {
         // few rows: all pairs compared (the timing marks and the executed
         // tests are the general path's)
-        if (njobs == 1 && n <= small_rows() && !ctx.timing &&
+        if (njobs == 1 && n <= small_rows(D) && !ctx.timing &&
             run_small<T, D>(ctx, pts, n, eps[0], min_pts[0], labels, s))
             return;
     }
@@ -1455,7 +1455,7 @@ template <typename T, int D>
 static size_t workspace_call(int64_t n, bool one_thread) {
     size_t b = workspace_bytes<T, D>(n, 1, one_thread);
     if constexpr (std::is_floating_point<T>::value)
-        if (n <= small_rows()) b = std::max(b, small_call_bytes<T, D>(n));
+        if (n <= small_rows(D)) b = std::max(b, small_call_bytes<T, D>(n));
     return b;
 }
 

@@ -2,9 +2,9 @@
 //
 // Replaces the reference's cell histogram + serial counting-sort scatter
 // (spatial_index.h:144-216).  Per pass:
-//   1. k_radix_hist    per-tile digit histogram, stored digit-major
-//                      hist[digit * ntiles + tile]
-//   2. exclusive scan  of hist -> global offset of (digit, tile)
+//   1. k_radix_hist    digit histogram of every block's run of tiles
+//   2. exclusive scan  of the histograms -> global offset of (digit, block);
+//                      for few blocks each block of 3. adds them up itself
 //   3. k_radix_scatter stable rank of every key inside its tile (wave
 //                      ballots + per-wave LDS counters), the tile staged
 //                      in LDS in digit order, then written out so that
@@ -12,6 +12,13 @@
 // A tile is 4096 keys: 4 waves x 16 iterations x 64 lanes; the stable order
 // inside a tile is (wave, iteration, lane), i.e. input order.  9-bit digits
 // (512 buckets, two per thread) are used where they save a pass.
+//
+// A block takes a run of tiles (SortPlan) where there are more than
+// kRunBlocks of them: with one tile per block the histograms of 100M keys are
+// 50 MB per pass, written, scanned and read back in single words.  Longer runs
+// save more there but leave too few blocks to hide a tile's chain of barriers
+// (100M rows, 2 passes, sort phase in ms by the blocks left: 2048 4.05, 4096
+// 4.10, 8192 3.93, 16384 3.87, all 48828 3.98).
 #include "common.hpp"
 #include "hpdbscan_capi.h"
 #include "internal.hpp"
@@ -33,10 +40,29 @@ __host__ __device__ inline int64_t tiles_of(int64_t n, int64_t tile = kTile) {
     return (n + tile - 1) / tile;
 }
 
+// How a sort of n keys splits: blocks of `run` tiles; with self, each scatter
+// block adds up the histograms (hist[block * buckets + digit], written and
+// read in rows) instead of a scan of hist[digit * blocks + block]: two launches
+// fewer per pass for up to kSelfBlocks * 1 KB read by every block (100k rows, 3
+// passes: 456 -> 423 us; replayed, 8 passes: 514 -> 435 us).
+constexpr int64_t kRunBlocks = 16384;
+constexpr int64_t kSelfBlocks = 192;
+struct SortPlan {
+    int64_t blocks;
+    int run;
+    bool self;
+};
+inline SortPlan sort_plan(int64_t n, int64_t tile) {
+    const int64_t tiles = tiles_of(n, tile);
+    const int64_t run = tiles_of(tiles, kRunBlocks);
+    const int64_t blocks = tiles_of(tiles, run);
+    return SortPlan{blocks, static_cast<int>(run), blocks <= kSelfBlocks};
+}
+
 template <typename K, int kBits, int kIt = kIters>
 __global__ __launch_bounds__(kThreads) void k_radix_hist(const K* __restrict__ keys, int64_t n,
                                                          int shift, uint32_t* __restrict__ hist,
-                                                         int64_t ntiles,
+                                                         SortPlan plan,
                                                          const int* __restrict__ bits_dev) {
     if (bits_dev && shift >= *bits_dev) return;  // a pass beyond the key's bits
     constexpr int B = 1 << kBits;
@@ -44,21 +70,29 @@ __global__ __launch_bounds__(kThreads) void k_radix_hist(const K* __restrict__ k
     __shared__ uint32_t cnt[B];
     for (int dg = threadIdx.x; dg < B; dg += kThreads) cnt[dg] = 0;
     __syncthreads();
-    const int w = threadIdx.x >> 6;
-    const int l = threadIdx.x & 63;
     constexpr int tile = kThreads * kIt;
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * tile + w * (tile / 4);
-#pragma unroll 4
-    for (int it = 0; it < kIt; ++it) {
-        const int64_t idx = base + it * 64 + l;
-        if (idx < n) {
-            const uint32_t dgt = static_cast<uint32_t>((keys[idx] >> shift) & kMask);
-            atomicAdd(&cnt[dgt], 1u);
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * plan.run * tile;
+    const int64_t end = base + static_cast<int64_t>(plan.run) * tile;
+    const int64_t stop = end < n ? end : n;
+    for (int64_t t = base + threadIdx.x; t < stop; t += tile) {
+        K k[kIt];
+#pragma unroll
+        for (int it = 0; it < kIt; ++it) {
+            const int64_t idx = t + it * kThreads;
+            k[it] = idx < stop ? keys[idx] : K(0);
         }
+#pragma unroll
+        for (int it = 0; it < kIt; ++it)
+            if (t + it * kThreads < stop)
+                atomicAdd(&cnt[static_cast<uint32_t>((k[it] >> shift) & kMask)], 1u);
     }
     __syncthreads();
-    for (int dg = threadIdx.x; dg < B; dg += kThreads)
-        hist[static_cast<int64_t>(dg) * ntiles + blockIdx.x] = cnt[dg];
+    for (int dg = threadIdx.x; dg < B; dg += kThreads) {
+        if (plan.self)
+            hist[static_cast<int64_t>(blockIdx.x) * B + dg] = cnt[dg];
+        else
+            hist[static_cast<int64_t>(dg) * plan.blocks + blockIdx.x] = cnt[dg];
+    }
 }
 
 // Rows that a pass carries along with the pairs: row i of `in` (one word W
@@ -100,7 +134,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const K* __restrict_
                                                             uint32_t* __restrict__ vout, int64_t n,
                                                             int shift,
                                                             const uint32_t* __restrict__ offs,
-                                                            int64_t ntiles,
+                                                            SortPlan plan,
                                                             const int* __restrict__ bits_dev,
                                                             Rows rows = Rows{}) {
     if (bits_dev && shift >= *bits_dev) return;  // a pass beyond the key's bits
@@ -117,106 +151,164 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const K* __restrict_
     __shared__ typename Rows::W srow[Rows::kOn ? tile : 1];
     const int w = threadIdx.x >> 6;
     const int l = threadIdx.x & 63;
-    for (int dg = threadIdx.x; dg < B; dg += kThreads) {
+    if (plan.self) {
+        // digits of thread t: t, t + kThreads.  Own offset: the digit's keys
+        // in earlier blocks plus all keys of smaller digits.
+        uint32_t before[kOwn], all[kOwn];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) cnt[i][dg] = 0;
-        gbase[dg] = offs[static_cast<int64_t>(dg) * ntiles + blockIdx.x];
+        for (int o = 0; o < kOwn; ++o) {
+            before[o] = 0;
+            all[o] = 0;
+        }
+        for (int64_t b = 0; b < plan.blocks; b += 4) {
+            uint32_t v[4][kOwn];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int o = 0; o < kOwn; ++o)
+                    v[j][o] = b + j < plan.blocks
+                                  ? offs[(b + j) * B + o * kThreads + threadIdx.x] : 0u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int o = 0; o < kOwn; ++o) {
+                    if (b + j < static_cast<int64_t>(blockIdx.x)) before[o] += v[j][o];
+                    all[o] += v[j][o];
+                }
+        }
+        uint32_t below = 0;  // keys of the digits of earlier rounds
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) {
+            uint32_t inc = all[o];
+#pragma unroll
+            for (int st = 1; st < 64; st <<= 1) {
+                const uint32_t t = __shfl_up(inc, st, 64);
+                if (l >= st) inc += t;
+            }
+            if (l == 63) wsum[w] = inc;
+            __syncthreads();
+            uint32_t woff = 0, total = 0;
+#pragma unroll
+            for (int i = 0; i < kThreads / 64; ++i) {
+                if (i < w) woff += wsum[i];
+                total += wsum[i];
+            }
+            gbase[o * kThreads + threadIdx.x] = below + woff + inc - all[o] + before[o];
+            below += total;
+            __syncthreads();
+        }
+    } else {
+        for (int dg = threadIdx.x; dg < B; dg += kThreads)
+            gbase[dg] = offs[static_cast<int64_t>(dg) * plan.blocks + blockIdx.x];
     }
-    __syncthreads();
+    const int64_t run0 = static_cast<int64_t>(blockIdx.x) * plan.run * tile;
+    for (int r = 0; r < plan.run; ++r) {
+        const int64_t tile0 = run0 + static_cast<int64_t>(r) * tile;
+        if (tile0 >= n) break;
+        for (int dg = threadIdx.x; dg < B; dg += kThreads) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cnt[i][dg] = 0;
+        }
+        __syncthreads();
 
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * tile + w * (tile / 4);
-    const uint64_t lt = lanemask_lt();
-    K key[kIt];
-    uint32_t val[kIt];
-    uint32_t rank[kIt];
-    uint32_t dgt[kIt];
-    typename Rows::W row[Rows::kOn ? kIt : 1];
+        const int64_t base = tile0 + w * (tile / 4);
+        const uint64_t lt = lanemask_lt();
+        K key[kIt];
+        uint32_t val[kIt];
+        uint32_t rank[kIt];
+        uint32_t dgt[kIt];
+        typename Rows::W row[Rows::kOn ? kIt : 1];
 #pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-        const int64_t idx = base + it * 64 + l;
-        const bool valid = idx < n;
-        const K k = valid ? kin[idx] : K(0);
-        const uint32_t d = static_cast<uint32_t>((k >> shift) & kMask);
-        uint64_t peers = ballot(valid);
-#pragma unroll
-        for (int b = 0; b < kBits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t m = ballot(bit);
-            peers &= bit ? m : ~m;
-        }
-        uint32_t c = 0;
-        if (valid) c = cnt[w][d];
-        if (valid && (peers & lt) == 0) cnt[w][d] = c + static_cast<uint32_t>(__popcll(peers));
-        rank[it] = c + static_cast<uint32_t>(__popcll(peers & lt));
-        dgt[it] = valid ? d : 0xffffffffu;
-        key[it] = k;
-        val[it] = valid ? vin[idx] : 0u;
-        if constexpr (Rows::kOn) row[it] = valid ? rows.load(idx) : 0;
-    }
-    __syncthreads();
-    // exclusive prefix of each digit over the four waves, and of the digits'
-    // tile totals over the digits (thread t owns digits [t * kOwn, ..))
-    uint32_t tot[kOwn];
-    uint32_t run = 0;
-#pragma unroll
-    for (int o = 0; o < kOwn; ++o) {
-        const int dg = threadIdx.x * kOwn + o;
-        uint32_t acc = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t c = cnt[i][dg];
-            cnt[i][dg] = acc;
-            acc += c;
-        }
-        tot[o] = acc;
-        run += acc;
-    }
-    uint32_t inc = run;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t t = __shfl_up(inc, o, 64);
-        if (l >= o) inc += t;
-    }
-    if (l == 63) wsum[w] = inc;
-    __syncthreads();
-    uint32_t woff = 0;
-#pragma unroll
-    for (int i = 0; i < kThreads / 64; ++i)
-        if (i < w) woff += wsum[i];
-    uint32_t first = woff + inc - run;
-#pragma unroll
-    for (int o = 0; o < kOwn; ++o) {
-        tbase[threadIdx.x * kOwn + o] = first;
-        first += tot[o];
-    }
-    __syncthreads();
-    // stage the tile in digit order (stable: waves, iterations and lanes are
-    // in input order) ...
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-        if (dgt[it] != 0xffffffffu) {
-            const uint32_t at = tbase[dgt[it]] + cnt[w][dgt[it]] + rank[it];
-            skey[at] = key[it];
-            sval[at] = val[it];
-            if constexpr (Rows::kOn) srow[at] = row[it];
-        }
-    }
-    __syncthreads();
-    // ... and write it out: consecutive threads write consecutive places of
-    // one digit's run
-    const int64_t left = n - static_cast<int64_t>(blockIdx.x) * tile;
-    const int valid_in_tile = left < tile ? static_cast<int>(left) : tile;
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-        const int at = it * kThreads + threadIdx.x;
-        if (at < valid_in_tile) {
-            const K k = skey[at];
+        for (int it = 0; it < kIt; ++it) {
+            const int64_t idx = base + it * 64 + l;
+            const bool valid = idx < n;
+            const K k = valid ? kin[idx] : K(0);
             const uint32_t d = static_cast<uint32_t>((k >> shift) & kMask);
-            const uint32_t dst = gbase[d] + (static_cast<uint32_t>(at) - tbase[d]);
-            kout[dst] = k;
-            vout[dst] = sval[at];
-            if constexpr (Rows::kOn) rows.store(dst, srow[at]);
+            uint64_t peers = ballot(valid);
+#pragma unroll
+            for (int b = 0; b < kBits; ++b) {
+                const bool bit = (d >> b) & 1u;
+                const uint64_t m = ballot(bit);
+                peers &= bit ? m : ~m;
+            }
+            uint32_t c = 0;
+            if (valid) c = cnt[w][d];
+            if (valid && (peers & lt) == 0) cnt[w][d] = c + static_cast<uint32_t>(__popcll(peers));
+            rank[it] = c + static_cast<uint32_t>(__popcll(peers & lt));
+            dgt[it] = valid ? d : 0xffffffffu;
+            key[it] = k;
+            val[it] = valid ? vin[idx] : 0u;
+            if constexpr (Rows::kOn) row[it] = valid ? rows.load(idx) : 0;
         }
+        __syncthreads();
+        // exclusive prefix of each digit over the four waves, and of the digits'
+        // tile totals over the digits (thread t owns digits [t * kOwn, ..))
+        uint32_t tot[kOwn];
+        uint32_t run = 0;
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) {
+            const int dg = threadIdx.x * kOwn + o;
+            uint32_t acc = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t c = cnt[i][dg];
+                cnt[i][dg] = acc;
+                acc += c;
+            }
+            tot[o] = acc;
+            run += acc;
+        }
+        uint32_t inc = run;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = __shfl_up(inc, o, 64);
+            if (l >= o) inc += t;
+        }
+        if (l == 63) wsum[w] = inc;
+        __syncthreads();
+        uint32_t woff = 0;
+#pragma unroll
+        for (int i = 0; i < kThreads / 64; ++i)
+            if (i < w) woff += wsum[i];
+        uint32_t first = woff + inc - run;
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) {
+            tbase[threadIdx.x * kOwn + o] = first;
+            first += tot[o];
+        }
+        __syncthreads();
+        // stage the tile in digit order (stable: waves, iterations and lanes are
+        // in input order) ...
+#pragma unroll
+        for (int it = 0; it < kIt; ++it) {
+            if (dgt[it] != 0xffffffffu) {
+                const uint32_t at = tbase[dgt[it]] + cnt[w][dgt[it]] + rank[it];
+                skey[at] = key[it];
+                sval[at] = val[it];
+                if constexpr (Rows::kOn) srow[at] = row[it];
+            }
+        }
+        __syncthreads();
+        // ... and write it out: consecutive threads write consecutive places of
+        // one digit's run
+        const int64_t left = n - tile0;
+        const int valid_in_tile = left < tile ? static_cast<int>(left) : tile;
+#pragma unroll
+        for (int it = 0; it < kIt; ++it) {
+            const int at = it * kThreads + threadIdx.x;
+            if (at < valid_in_tile) {
+                const K k = skey[at];
+                const uint32_t d = static_cast<uint32_t>((k >> shift) & kMask);
+                const uint32_t dst = gbase[d] + (static_cast<uint32_t>(at) - tbase[d]);
+                kout[dst] = k;
+                vout[dst] = sval[at];
+                if constexpr (Rows::kOn) rows.store(dst, srow[at]);
+            }
+        }
+        __syncthreads();
+        // the next tile's keys go after this one's
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) gbase[threadIdx.x * kOwn + o] += tot[o];
     }
 }
 
@@ -242,20 +334,19 @@ __global__ __launch_bounds__(kThreads) void k_radix_settle(K* __restrict__ keys_
 template <typename K, int kBits>
 bool sort_passes(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n, int bits,
                  uint32_t* hist, uint32_t* tmp, hipStream_t s, const int* bits_dev = nullptr) {
-    const int64_t nt = tiles_of(n);
-    const int64_t nh = static_cast<int64_t>(1 << kBits) * nt;
+    const SortPlan plan = sort_plan(n, kTile);
+    const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
     K* kout = keys_b;
     uint32_t* vout = vals_b;
     bool in_b = false;
     for (int shift = 0; shift < bits; shift += kBits) {
-        hipLaunchKernelGGL((k_radix_hist<K, kBits>), dim3(static_cast<unsigned>(nt)),
-                           dim3(kThreads), 0, s, kin, n, shift, hist, nt, bits_dev);
-        exclusive_scan_u32(hist, hist, nh, tmp, nullptr, s);
-        hipLaunchKernelGGL((k_radix_scatter<K, kBits>), dim3(static_cast<unsigned>(nt)),
-                           dim3(kThreads), 0, s, kin, vin, kout, vout, n, shift, hist, nt,
-                           bits_dev);
+        hipLaunchKernelGGL((k_radix_hist<K, kBits>), grid, dim3(kThreads), 0, s, kin, n, shift,
+                           hist, plan, bits_dev);
+        if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
+        hipLaunchKernelGGL((k_radix_scatter<K, kBits>), grid, dim3(kThreads), 0, s, kin, vin, kout,
+                           vout, n, shift, hist, plan, bits_dev);
         HPD_HIP(hipGetLastError());
         K* tk = kin;
         kin = kout;
@@ -274,8 +365,8 @@ template <typename K, int kBits, typename T, int D>
 bool sort_passes_rows(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n,
                       int bits, uint32_t* hist, uint32_t* tmp, const T* pts, T* rows_a,
                       T* rows_b, T* soa, int64_t ld, hipStream_t s) {
-    const int64_t nt = tiles_of(n, kTileMin);
-    const int64_t nh = static_cast<int64_t>(1 << kBits) * nt;
+    const SortPlan plan = sort_plan(n, kTileMin);
+    const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
     K* kout = keys_b;
@@ -288,12 +379,12 @@ bool sort_passes_rows(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, 
         using W = typename MoveRows<T, D>::W;
         MoveRows<T, D> mv{reinterpret_cast<const W*>(rin), reinterpret_cast<W*>(rnext), soa,
                           last ? ld : 0};
-        hipLaunchKernelGGL((k_radix_hist<K, kBits, kItersRows>), dim3(static_cast<unsigned>(nt)),
-                           dim3(kThreads), 0, s, kin, n, shift, hist, nt, nullptr);
-        exclusive_scan_u32(hist, hist, nh, tmp, nullptr, s);
-        hipLaunchKernelGGL((k_radix_scatter<K, kBits, MoveRows<T, D>, kItersRows>),
-                           dim3(static_cast<unsigned>(nt)), dim3(kThreads), 0, s, kin, vin, kout,
-                           vout, n, shift, hist, nt, nullptr, mv);
+        hipLaunchKernelGGL((k_radix_hist<K, kBits, kItersRows>), grid, dim3(kThreads), 0, s, kin, n,
+                           shift, hist, plan, nullptr);
+        if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
+        hipLaunchKernelGGL((k_radix_scatter<K, kBits, MoveRows<T, D>, kItersRows>), grid,
+                           dim3(kThreads), 0, s, kin, vin, kout, vout, n, shift, hist, plan, nullptr,
+                           mv);
         HPD_HIP(hipGetLastError());
         K* tk = kin;
         kin = kout;

@@ -490,10 +490,11 @@ __global__ __launch_bounds__(kLabelThreads) void k_small_label(int32_t n, SmallL
 
 }  // namespace
 
-// All pairs against the general path, us: 1000 rows 71 / 263, 4000 155 / 330,
-// 8000 317 / 380 (3-D float, blobs of 150 rows); 2-D alike, 6-D and 8-D ahead
-// by more.  The two meet near 10000 rows; denser data meets sooner.
-int64_t small_rows() { return 6000; }
+// All pairs against the general path, us (3-D float, blobs of 150 rows): 1000
+// rows 55 / 263, 6000 147 / 340, 9000 245 / 370; the densest 2-D data measured
+// meets it at 8000 rows.  From 5-D on the general path's neighbourhoods grow
+// with 3^D (6-D, 12000 rows: 471 / 590 and, dense, 590 / 850).
+int64_t small_rows(int d) { return d <= 4 ? 6000 : 12000; }
 
 template <typename T, int D>
 size_t small_workspace_bytes(int64_t n) {

@@ -28,12 +28,12 @@ struct SmallResult {
 // Most rows of a small run.  All pairs of rows are compared, so the time grows
 // with their square; the general path costs some 55 launches whatever the
 // size.
-int64_t small_rows();
+int64_t small_rows(int d);
 
 template <typename T, int D>
 size_t small_workspace_bytes(int64_t n);
 
-// Labels of n <= small_rows() rows of one job (jp: eps2, min_pts and
+// Labels of n <= small_rows(D) rows of one job (jp: eps2, min_pts and
 // reciprocals; jp_dev, when not null, holds them in device memory instead)
 // under the smallest-cluster border rule, by comparing all pairs: no sort, no
 // index, no read-back.  work: small_workspace_bytes.  The result is

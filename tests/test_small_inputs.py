@@ -57,6 +57,11 @@ def test_sizes(contexts, n, d, dtype):
     check(contexts, cloud(n, d, dtype, 100 * d + n), 0.2 + 0.1 * d, 5, "small")
 
 
+@pytest.mark.parametrize("d,n", [(5, 12000), (6, 12001)])
+def test_sizes_from_five_dimensions(contexts, n, d):
+    check(contexts, cloud(n, d, np.float32, d), 0.6, 5, "small, 5-D and above")
+
+
 @pytest.mark.parametrize("min_points", [0, 1, 2, 4000])
 def test_min_points(contexts, min_points):
     check(contexts, cloud(3000, 3, np.float32, 1), 0.4, min_points, "small minPts")
