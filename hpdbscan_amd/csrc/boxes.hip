@@ -368,7 +368,9 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const Span<T>* __restric
                                                         const JobParams<T>* __restrict__ jobs,
                                                         const uint8_t* __restrict__ cell_core,
                                                         uint8_t* __restrict__ btight,
-                                                        unsigned int* __restrict__ nloose) {
+                                                        unsigned int* __restrict__ nloose,
+                                                        int32_t large,
+                                                        unsigned int* __restrict__ nlarge) {
     const int32_t nbox = static_cast<int32_t>(nbox_c.get());
     const int32_t b = static_cast<int32_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (b >= nbox) return;
@@ -387,6 +389,7 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const Span<T>* __restric
                                      ((tight && static_cast<uint32_t>(size) >= jp.min_pts) ? 2 : 0) |
                                      (cell_core[u] ? 4 : 0));
     if (!tight && size > 1) atomicAdd(nloose, 1u);
+    if (size > large) atomicAdd(nlarge, 1u);
 }
 
 // Whether a core row of a box, [q0, q1), is within eps of the row of a lane
@@ -478,6 +481,7 @@ __device__ __forceinline__ bool ends_pair(const T* __restrict__ soa, int64_t ld,
 // (4096 clouds, hook and join ms: 16 4.79, 32 4.83, 64 4.91, 256 11.4 before
 // the first and last rows were tried first, 1024 13.2.)
 constexpr int kLanePair = 16;
+constexpr int kLinkRows = 4096;
 
 // The same bounds (point_box) for the rows of two boxes: gap2 <= dist2(p, q)
 // <= far2 for every pair of members.
@@ -498,9 +502,9 @@ __device__ __forceinline__ void box_gap(const Span<T>* __restrict__ bbox, int32_
 // Hook forest (kJoin false): every listed box points at some earlier box
 // holding a core within eps of one of its cores, the own neighbour row
 // searched first from the own cell on (any such box will do, and a box
-// without one stays a root; larger boxes search from their first 64 rows
-// only, here and in the root join: a missed link is found by the exact union
-// later).  bparent stays <=
+// without one stays a root; boxes search from their first 64 rows and through
+// the other box's first kLinkRows only, here and in the root join: a missed
+// link is found by the exact union later).  bparent stays <=
 // the box index, so the hooks form a forest whose trees are connected sets
 // of boxes.
 // Root join (kJoin): every root of that forest (blist) looks through its
@@ -576,8 +580,10 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
                 const int j = static_cast<int>(__builtin_ctzll(todo));
                 if ((ballot(done) >> j) & 1) continue;
                 const int32_t t0 = bcast(s0, j);
+                const int32_t v0 = bcast(q0, j);
                 if (wave_pair<T, D>(a.soa, a.ld, core, bbox, t0, min(bcast(s1, j), t0 + kWave),
-                                    bcast(b2, j), bcast(q0, j), bcast(q1, j), bcast(eps2, j))) {
+                                    bcast(b2, j), v0, min(bcast(q1, j), v0 + kLinkRows),
+                                    bcast(eps2, j))) {
                     if (grp == j / G) {
                         done = true;
                         hits = uint64_t{1} << j;
@@ -932,12 +938,12 @@ void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* b
 
 template <typename T, int D>
 void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
-                      unsigned int* nloose, hipStream_t s) {
+                      unsigned int* nloose, int32_t large, unsigned int* nlarge, hipStream_t s) {
     using U = OrdKey<T>;
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_tight<T, D>), dim3(blocks_for(a.nbox, kThreads)), dim3(kThreads), 0,
                        s, static_cast<const Span<T>*>(a.bbox), Count{a.nbox, a.nbox_dev}, a.bstart,
-                       a.bcell, a.job_of_cell, a.jobs, cell_core, btight, nloose);
+                       a.bcell, a.job_of_cell, a.jobs, cell_core, btight, nloose, large, nlarge);
 }
 
 void launch_list_boxes(Count nbox, const int32_t* bmincore, int32_t* list, unsigned int* count,
@@ -1069,7 +1075,8 @@ void launch_positions(int64_t n, int32_t m, const int32_t* box_of_slot, const in
                                             const int32_t*, const int32_t*, void*, void*,         \
                                             hipStream_t);                                         \
     template void launch_box_tight<T, D>(const BoxArgs<T>&, const uint8_t*, uint8_t*,            \
-                                         unsigned int*, hipStream_t);                                            \
+                                         unsigned int*, int32_t, unsigned int*,           \
+                                         hipStream_t);                                            \
     template void launch_box_hook<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,          \
                                         const int32_t*, const uint8_t*, const int32_t*,           \
                                         const unsigned int*, int32_t*, hipStream_t);              \

@@ -67,10 +67,10 @@ void launch_cells_of_boxes(const K* keys, int64_t n, int shift, const int32_t* b
 
 // btight[b]: bit 0 tight, bit 1 tight with >= minPts rows, bit 2 in a cell
 // that can hold cores (cell_core); *nloose counts boxes of two or more rows
-// that are not tight
+// that are not tight, *nlarge boxes of more than `large` rows
 template <typename T, int D>
 void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
-                      unsigned int* nloose, hipStream_t s);
+                      unsigned int* nloose, int32_t large, unsigned int* nlarge, hipStream_t s);
 
 // Components of the boxes with cores:
 //   launch_list_boxes    list of the boxes with cores, *count += their

@@ -322,6 +322,10 @@ private:
 // kernels' loops).
 constexpr uint64_t kMaxNeighborRows = 0x7fffffffull;
 constexpr int kWaveRows = 64;  // rows of a work item
+// 64-bit device words of a run: statistics (0-7), 32-bit counters (8-15, of
+// which 15 counts the union's heavy entries), put-off walks of the core count
+// (16) and of the border pass (17, 18)
+constexpr int kStatWords = 24;
 
 static void check_neighbor_rows(uint64_t total) {
     if (total > kMaxNeighborRows)
@@ -375,7 +379,7 @@ static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
     if (sort_moves_rows<T, D>()) b += 2 * sizeof(T) * D * nn;   // rows between sort passes
     b += table_bytes<T, D>(n, njobs) + 4 * nn;  // job table, min/max, job of every cell
     if (one_thread) b += 8 * nn + 4 * nn + nn + 4;  // ambiguous rows, f, involved, flag
-    b += 8 * 16;                               // statistics, counters
+    b += 8 * kStatWords;                       // statistics, counters
     b += 54 * 256 + 64 * 1024;                 // alignment
     return b;
 }
@@ -415,10 +419,11 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     int32_t* cmax = A.take_n<int32_t>(nn);
     int32_t* rcenter = A.take_n<int32_t>(nn);
     int32_t* job_of_cell = A.take_n<int32_t>(nn);
-    unsigned long long* dstats = A.take_n<unsigned long long>(16);
-    // m, ranges, items, boxes, box items, loose, rows to count, non-core rows
+    unsigned long long* dstats = A.take_n<unsigned long long>(kStatWords);
+    // 0 m, 1 ranges, 2 items, 3 boxes, 5 loose, 6 chunks to count, 7 non-core
+    // rows, 8 boxes with cores, 9 and 10 roots, 11 large boxes, 13 full-row table
     uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
-    HPD_HIP(hipMemsetAsync(dstats, 0, 16 * sizeof(unsigned long long), s));
+    HPD_HIP(hipMemsetAsync(dstats, 0, kStatWords * sizeof(unsigned long long), s));
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx.host_scratch);
 
     // cell ids (spatial_index.h:144-165), offset by the job's key base; in
@@ -540,7 +545,8 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         bt.bbox = bbox;
         bt.jobs = jobs;
         bt.job_of_cell = job_of_cell;
-        launch_box_tight<T, D>(bt, cell_core, btight, &counters[5], s);
+        launch_box_tight<T, D>(bt, cell_core, btight, &counters[5], heavy_walk_rows(), &counters[11],
+                               s);
     }
     // the scans' totals into the counters (one launch), then one read-back
     // of the 64-bit row total (dstats[4]) and the counters (dstats + 8)
@@ -631,6 +637,15 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         a.ncrows_dev = &counters[6];
         a.brows = reinterpret_cast<int2*>(scratch64);
         a.nbrows_dev = &counters[7];
+        if (hc[11] > 0) {  // boxes of millions of rows: their walks in parts
+            a.heavy = reinterpret_cast<int2*>(flags);
+            a.nheavy = &dstats[16];
+            a.heavy_cap = static_cast<unsigned long long>(nn);
+            a.slot_a = parent;  // free before and after the union
+            a.slot_b = rsnap;
+            a.late = cmin;
+            a.nlate = reinterpret_cast<unsigned int*>(&dstats[18]);
+        }
     }
     // box mode: the row-level tables when they turn out to be needed (the
     // neighbour rows ascending again, their own-row index with them)
@@ -711,6 +726,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
                           box_union && !one_thread ? nullptr : rootslot, cmin, cmax, labels,
                           &dstats[1], s, full_ok);
     tm.mark(M_BORDER0);
+    a.nheavy = &dstats[17];
     launch_border<T, D>(a, core, box_union ? bcluster : nullptr, rootslot, cmin, cmax, labels,
                         &dstats[2], amb, s);
 
@@ -843,6 +859,7 @@ enum StaticSlot : int {
     SS_BROWS = 7,      // non-core rows
     SS_NLIST = 8,      // boxes with cores
     SS_JOIN0 = 9,      // roots of the first root-join round
+    SS_LARGE = 11,     // (boxes above a size: not counted here)
     SS_JOIN1 = 13,     // roots of the second round
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
@@ -867,7 +884,7 @@ static size_t static_main_bytes(int64_t n, int32_t njobs) {
 // else (no read-back, no synchronisation, no memset), in the workspace the
 // caller reserved and started taking from; jobs / bfirst_dev hold the
 // host-made job table (row ranges, eps2, minPts, reciprocals) and min/max
-// blocks.  sc (SS_WORDS words) and dstats (16 words) end up
+// blocks.  sc (SS_WORDS words) and dstats (kStatWords words) end up
 // holding the counts read afterwards.
 template <typename T, int D>
 static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
@@ -890,7 +907,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     const size_t L = static_cast<size_t>(ld);
     // zeroed by a kernel (no memset in a graph)
     fill_i32(reinterpret_cast<int32_t*>(sc), 0, SS_WORDS, s);
-    fill_i32(reinterpret_cast<int32_t*>(dstats), 0, 2 * 16, s);
+    fill_i32(reinterpret_cast<int32_t*>(dstats), 0, 2 * kStatWords, s);
 
     // min / max, then every job's grid on the device
     T* part = A.take_n<T>(static_cast<size_t>(nblocks) * 2 * D + 1);
@@ -982,7 +999,7 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     ba.nrows = n;
     ba.job_of_cell = job_of_cell;
     ba.rcenter = rcenter;
-    launch_box_tight<T, D>(ba, cell_core, btight, &sc[SS_LOOSE], s);
+    launch_box_tight<T, D>(ba, cell_core, btight, &sc[SS_LOOSE], INT32_MAX, &sc[SS_LARGE], s);
 
     DbscanArgs<T> a;
     a.soa = soa;
@@ -1066,7 +1083,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     JobParams<T>* jobs_dev = A.take_n<JobParams<T>>(static_cast<size_t>(njobs));
     int32_t* bfirst_dev = A.take_n<int32_t>(static_cast<size_t>(njobs) + 1);
     uint32_t* sc = A.take_n<uint32_t>(SS_WORDS);
-    unsigned long long* dstats = A.take_n<unsigned long long>(16);
+    unsigned long long* dstats = A.take_n<unsigned long long>(kStatWords);
     SmallResult* small = A.take_n<SmallResult>(1);
 
     // host-made part of the job table: row ranges, eps2, minPts, reciprocals

@@ -141,6 +141,31 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
+// Boxes of more rows are walked in parts of this many, one wave each
+// (100M skewed rows: 26 us a part).
+constexpr int32_t kHeavyWalk = 16384;
+
+// An entry (slot, first row) per part of the rows [q0, q1) of a box; false
+// when the list is full (every argument wave-uniform).
+template <typename T>
+__device__ __forceinline__ bool put_heavy(const DbscanArgs<T>& a, int32_t slot, int32_t q0,
+                                          int32_t q1) {
+    const int32_t k = (q1 - q0 + kHeavyWalk - 1) / kHeavyWalk;
+    unsigned long long at = 0;
+    if (lane_id() == 0) at = atomicAdd(a.nheavy, static_cast<unsigned long long>(k));
+    at = bcast64(at, 0);
+    const bool fits = at + static_cast<unsigned long long>(k) <= a.heavy_cap;
+    // (the entries of a range that does not fit do nothing)
+    for (int32_t e = lane_id(); e < k && at + e < a.heavy_cap; e += kWave)
+        a.heavy[at + e] = fits ? make_int2(slot, q0 + e * kHeavyWalk) : make_int2(-1, -1);
+    return fits;
+}
+template <typename T>
+__device__ __forceinline__ int32_t heavy_count(const DbscanArgs<T>& a) {
+    const unsigned long long n = *a.nheavy;
+    return uniform(static_cast<int32_t>(n < a.heavy_cap ? n : a.heavy_cap));
+}
+
 // Box-mode core counts: the chunks listed in a.crows (up to G rows of one
 // box, boxes outside the full ones, in cells that can hold cores), G lanes per
 // chunk, a neighbour box per lane: the chunk's rows and counts lie in LDS, and
@@ -152,6 +177,9 @@ __device__ __forceinline__ void wave_lds_fence() {
 // Bound by VALU issue of the box tests and by the latency of list -> cell ->
 // box ranges -> boxes, which the rows of a chunk share.  kCount: also add the
 // row-row distance tests executed to *ntests (the instrumented variant).
+// With a.heavy (boxes of more than kHeavyWalk rows exist) a row's walk of such
+// a box leaves an entry per kHeavyWalk of its rows for k_core_heavy: one wave
+// takes 0.4 us per 256 rows, 8 ms for a box of five million.
 template <typename T, int D, bool kCount = false>
 __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                                                         uint8_t* __restrict__ core,
@@ -192,6 +220,7 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         const T eps2 = jp.eps2;
         const uint32_t min_pts = jp.min_pts;
         bool need = has && min_pts > 0;
+        bool put_off = false;  // the lane's row has entries in a.heavy
         group_boxes<G>(on && min_pts > 0, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
                        [&](bool valid, int32_t b2) {
             int32_t q0 = 0, q1 = 0;
@@ -233,6 +262,7 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                 for (uint64_t todo = ballot(part != 0 && !lane_walk); todo != 0; todo &= todo - 1) {
                     const int j = static_cast<int>(__builtin_ctzll(todo));
                     const uint32_t mp = static_cast<uint32_t>(bcast(static_cast<int32_t>(min_pts), j));
+                    const int32_t v0 = bcast(q0, j), v1 = bcast(q1, j);
                     for (uint32_t m = static_cast<uint32_t>(bcast(static_cast<int32_t>(part), j));
                          m != 0; m &= m - 1) {
                         const int row = (j & ~(G - 1)) + __builtin_ctz(m);
@@ -240,13 +270,17 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                         const uint32_t now =
                             static_cast<uint32_t>(uniform(static_cast<int32_t>(rc[row])));
                         if (now >= mp) continue;  // an earlier box was enough
+                        if (a.heavy_cap > 0 && v1 - v0 > kHeavyWalk &&
+                            put_heavy(a, bcast(p, row), v0, v1)) {
+                            if (lane == row) put_off = true;
+                            continue;
+                        }
                         T pr[D];
 #pragma unroll
                         for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], row);
                         uint32_t visited = 0;
-                        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, bcast(q0, j),
-                                                              bcast(q1, j), pr, bcast(eps2, j),
-                                                              mp - now, visited);
+                        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, v0, v1, pr,
+                                                              bcast(eps2, j), mp - now, visited);
                         if (lane == 0) rc[row] = now + got;
                         if constexpr (kCount)
                             if (lane == 0) tests += visited;
@@ -260,6 +294,7 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         // (launch_core_init wrote 0 for every listed row)
         wave_lds_fence();
         const bool is_core = has && rc[lane] >= min_pts;
+        if (put_off) a.slot_a[p] = static_cast<int32_t>(min(rc[lane], min_pts));
         if (is_core) core[p] = 1;
         const int32_t first =
             group_min<G>(is_core ? static_cast<int32_t>(a.inrow[p]) : INT_MAX);
@@ -267,6 +302,44 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         wave_lds_fence();
     }
     if constexpr (kCount) block_add<kThreads>(tests, ntests);
+}
+
+// The put-off walks of k_core_rows, a wave per entry (slot, first row of the
+// part): the counts meet in a.slot_a, and the part that brings a row to minPts
+// makes it a core.
+template <typename T, int D>
+__global__ __launch_bounds__(kThreads) void k_core_heavy(const DbscanArgs<T> a,
+                                                         uint8_t* __restrict__ core,
+                                                         unsigned long long* __restrict__ ntests) {
+    const int32_t n = heavy_count(a);
+    unsigned long long tests = 0;
+    for (int32_t w = first_wave(); w < n; w += wave_stride()) {
+        const int32_t p = uniform(a.heavy[w].x), q0 = uniform(a.heavy[w].y);
+        if (p < 0) continue;
+        const int32_t b = uniform(a.box_of_slot[p]);
+        const JobParams<T>& jp = a.jobs[uniform(a.job_of_cell[uniform(a.bcell[b])])];
+        const uint32_t min_pts = jp.min_pts;
+        const uint32_t now = static_cast<uint32_t>(uniform(ld_agent(&a.slot_a[p])));
+        if (now >= min_pts) continue;
+        const int32_t q1 = min(q0 + kHeavyWalk, uniform(a.bstart[uniform(a.box_of_slot[q0]) + 1]));
+        T pc[D];
+        load_row<T, D>(a.soa, a.ld, p, pc);
+        uint32_t visited = 0;
+        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, q0, q1, pc, jp.eps2,
+                                              min_pts - now, visited);
+        if (lane_id() == 0) {
+            tests += visited;
+            if (got > 0) {
+                const uint32_t old = static_cast<uint32_t>(
+                    atomicAdd(&a.slot_a[p], static_cast<int32_t>(got)));
+                if (old < min_pts && old + got >= min_pts) {
+                    core[p] = 1;
+                    atomicMin(&a.bmincore[b], static_cast<int32_t>(a.inrow[p]));
+                }
+            }
+        }
+    }
+    if (ntests) block_add<kThreads>(tests, ntests);
 }
 
 template <typename T, int D>
@@ -575,6 +648,32 @@ __global__ __launch_bounds__(kThreads) void k_border(const DbscanArgs<T> a,
     }
 }
 
+// Label of a non-core row (lanes where `on`) next to clusters from `best` to
+// `worst` (INT_MAX and -1: none): the smallest, or noise (returns 1).  Rows next
+// to two or more are counted in stats[1] and listed.  The whole wave calls it.
+__device__ __forceinline__ unsigned int border_label(bool on, int32_t p, int32_t u,
+                                                     const uint32_t* __restrict__ inrow,
+                                                     int32_t best, int32_t worst, int64_t first_pos,
+                                                     int64_t* __restrict__ labels,
+                                                     unsigned long long* __restrict__ stats,
+                                                     int2* __restrict__ amb_list) {
+    if (on) labels[inrow[p]] = best == INT_MAX ? 0 : static_cast<int64_t>(best) - first_pos + 1;
+    const bool is_amb = on && best != INT_MAX && best != worst;
+    const uint64_t amb = ballot(is_amb);
+    if (amb != 0) {
+        unsigned long long at = 0;
+        if (lane_id() == 0)
+            at = atomicAdd(&stats[1], static_cast<unsigned long long>(__popcll(amb)));
+        if (amb_list) {
+            at = bcast64(at, 0);
+            if (is_amb)
+                amb_list[at + static_cast<unsigned long long>(__popcll(amb & lanemask_lt()))] =
+                    make_int2(p, u);
+        }
+    }
+    return on && best == INT_MAX ? 1u : 0u;
+}
+
 // Box-mode border labels: every core of a box lies in the box's cluster
 // (bcluster), so a non-core row only needs, per neighbour box whose cluster
 // could change its answer, one within-eps core of that box (or a box within
@@ -582,7 +681,9 @@ __global__ __launch_bounds__(kThreads) void k_border(const DbscanArgs<T> a,
 // k_core_rows; a box is skipped when its cluster is the row's current one, or
 // larger once two clusters were met; the smallest adjacent cluster and the
 // two-cluster flag come out exact.  stats[0] += noise rows, stats[1] += rows
-// next to two or more clusters.
+// next to two or more clusters.  Walks of boxes of more than kHeavyWalk rows
+// are put off as in k_core_rows: the row's clusters so far go to a.slot_a and
+// a.slot_b, k_border_heavy adds the parts' and k_border_late labels the row.
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_border_rows(
     const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
@@ -607,6 +708,7 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
         const JobParams<T>& jp = a.jobs[a.njobs == 1 ? 0 : a.job_of_cell[u]];
         const T eps2 = jp.eps2;
         int32_t best = INT_MAX, worst = -1;  // smallest, largest adjacent cluster so far
+        bool put_off = false;                // the row has entries in a.heavy
         group_boxes<G>(on, r0, r1, a.rcenter[u], a.cbox[u], a.rboxes, 0, INT_MAX,
                        [&](bool valid, int32_t b) {
             const int32_t cl = valid ? bcluster[b] : -1;
@@ -645,12 +747,18 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
                      todo &= todo - 1) {
                     const int j = static_cast<int>(__builtin_ctzll(todo));
                     if (!((ballot(wanted()) >> j) & 1)) continue;
+                    const int32_t v0 = bcast(q0, j), v1 = bcast(q1, j);
+                    if (a.heavy_cap > 0 && v1 - v0 > kHeavyWalk &&
+                        put_heavy(a, bcast(p, j), v0, v1)) {
+                        if (lane_id() / G == j / G) put_off = true;
+                        continue;
+                    }
                     T pr[D];
 #pragma unroll
                     for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], j);
                     uint32_t visited = 0;
-                    if (wide_count<T, D>(a.soa, a.ld, core, bcast(q0, j), bcast(q1, j), pr,
-                                         bcast(eps2, j), 1u, visited) != 0) {
+                    if (wide_count<T, D>(a.soa, a.ld, core, v0, v1, pr, bcast(eps2, j), 1u,
+                                         visited) != 0) {
                         const int32_t c = bcast(cl, j);
                         if (lane_id() / G == j / G) {
                             best = min(best, c);
@@ -661,24 +769,60 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
             }
             return false;
         });
-        const bool lead = on && gl == 0;
-        if (lead) {
-            labels[a.inrow[p]] =
-                best == INT_MAX ? 0 : static_cast<int64_t>(best) - jp.row_begin + 1;
-            noise += best == INT_MAX ? 1 : 0;
+        if (on && gl == 0 && put_off) {
+            a.slot_a[p] = best;
+            a.slot_b[p] = worst;
+            a.late[atomicAdd(a.nlate, 1u)] = p;
         }
-        const bool is_amb = lead && best != INT_MAX && best != worst;
-        const uint64_t amb_mask = ballot(is_amb);
-        if (amb_mask == 0) continue;
-        unsigned long long at = 0;
-        if (lane_id() == 0)
-            at = atomicAdd(&stats[1], static_cast<unsigned long long>(__popcll(amb_mask)));
-        if (amb_list) {
-            at = __shfl(at, 0, 64);
-            if (is_amb)
-                amb_list[at + static_cast<unsigned long long>(__popcll(amb_mask & lanemask_lt()))] =
-                    make_int2(p, u);
+        noise += border_label(on && gl == 0 && !put_off, p, u, a.inrow, best, worst, jp.row_begin,
+                              labels, stats, amb_list);
+    }
+    block_add<kThreads>(noise, &stats[0]);
+}
+
+// The put-off walks of k_border_rows, a wave per entry.
+template <typename T, int D>
+__global__ __launch_bounds__(kThreads) void k_border_heavy(const DbscanArgs<T> a,
+                                                           const uint8_t* __restrict__ core,
+                                                           const int32_t* __restrict__ bcluster) {
+    const int32_t n = heavy_count(a);
+    for (int32_t w = first_wave(); w < n; w += wave_stride()) {
+        const int32_t p = uniform(a.heavy[w].x), q0 = uniform(a.heavy[w].y);
+        if (p < 0) continue;
+        const int32_t b2 = uniform(a.box_of_slot[q0]);
+        const int32_t cl = uniform(bcluster[b2]);
+        const int32_t best = uniform(ld_agent(&a.slot_a[p]));
+        const int32_t worst = uniform(ld_agent(&a.slot_b[p]));
+        // nothing new: between the two, or beyond two that differ already
+        if ((cl >= best && cl <= worst) || (cl > best && best != worst)) continue;
+        const int32_t q1 = min(q0 + kHeavyWalk, uniform(a.bstart[b2 + 1]));
+        const T eps2 = a.jobs[uniform(a.job_of_cell[uniform(a.bcell[b2])])].eps2;
+        T pc[D];
+        load_row<T, D>(a.soa, a.ld, p, pc);
+        uint32_t visited = 0;
+        if (wide_count<T, D>(a.soa, a.ld, core, q0, q1, pc, eps2, 1u, visited) == 0) continue;
+        if (lane_id() == 0) {
+            atomicMin(&a.slot_a[p], cl);
+            atomicMax(&a.slot_b[p], cl);
         }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_border_late(const DbscanArgs<T> a,
+                                                          int64_t* __restrict__ labels,
+                                                          unsigned long long* __restrict__ stats,
+                                                          int2* __restrict__ amb_list) {
+    const int32_t n = static_cast<int32_t>(*a.nlate);
+    unsigned long long noise = 0;
+    const int32_t stride = static_cast<int32_t>(gridDim.x) * kThreads;
+    for (int32_t i0 = static_cast<int32_t>(blockIdx.x) * kThreads; i0 < n; i0 += stride) {
+        const int32_t i = i0 + static_cast<int32_t>(threadIdx.x);
+        const bool on = i < n;
+        const int32_t p = a.late[on ? i : 0];
+        const int32_t u = a.bcell[a.box_of_slot[p]];
+        noise += border_label(on, p, u, a.inrow, a.slot_a[p], a.slot_b[p],
+                              a.jobs[a.job_of_cell[u]].row_begin, labels, stats, amb_list);
     }
     block_add<kThreads>(noise, &stats[0]);
 }
@@ -876,6 +1020,10 @@ static void count_noise(const int64_t* labels, int64_t n, unsigned long long* ou
     HPD_HIP(hipGetLastError());
 }
 
+#if !defined(HPD_DBSCAN_PART) || HPD_DBSCAN_PART == 0
+int32_t heavy_walk_rows() { return kHeavyWalk; }
+#endif
+
 template <typename T, int D>
 void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntests, hipStream_t s,
                  hipEvent_t count_start) {
@@ -897,6 +1045,10 @@ void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntes
                 hipLaunchKernelGGL((k_core_rows<T, D, false>),
                                    dim3(persistent_blocks<k_core_rows<T, D, false>>(a.n, per_wave)),
                                    dim3(kThreads), 0, s, a, core, nullptr);
+            if (a.heavy_cap > 0)
+                hipLaunchKernelGGL((k_core_heavy<T, D>),
+                                   dim3(persistent_blocks<k_core_heavy<T, D>>(a.n, 1)),
+                                   dim3(kThreads), 0, s, a, core, ntests);
             HPD_HIP(hipGetLastError());
             return;
         }
@@ -981,6 +1133,13 @@ void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* b
                                dim3(kThreads), 0, s, a, core, bcluster, static_cast<const int2*>(a.brows),
                                static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
                                amb_list);
+            if (a.heavy_cap > 0) {
+                hipLaunchKernelGGL((k_border_heavy<T, D>),
+                                   dim3(persistent_blocks<k_border_heavy<T, D>>(a.n, 1)),
+                                   dim3(kThreads), 0, s, a, core, bcluster);
+                hipLaunchKernelGGL(k_border_late<T>, dim3(256), dim3(kThreads), 0, s, a, labels,
+                                   stats, amb_list);
+            }
             HPD_HIP(hipGetLastError());
             return;
         }

@@ -46,10 +46,24 @@ struct DbscanArgs {
     unsigned int* ncrows_dev = nullptr;
     int2* brows = nullptr;
     unsigned int* nbrows_dev = nullptr;
+    // box mode, when boxes of more than heavy_walk_rows() rows exist (else
+    // heavy_cap 0): walks of such boxes are put off to heavy[0, heavy_cap), with
+    // their number *nheavy (a word of its own for the core count and for the
+    // border pass) and that of the rows in late, *nlate (device words, zeroed by
+    // the caller), scratch by slot
+    int2* heavy = nullptr;
+    unsigned long long* nheavy = nullptr;
+    unsigned long long heavy_cap = 0;
+    int32_t* slot_a = nullptr;
+    int32_t* slot_b = nullptr;
+    int32_t* late = nullptr;
+    unsigned int* nlate = nullptr;
     // box mode: the core count also writes the smallest input row of a core
     // row per box (INT_MAX without cores)
     int32_t* bmincore = nullptr;
 };
+
+int32_t heavy_walk_rows();
 
 // core flag of every slot; with box tables the candidates are visited box
 // by box (boxes beyond eps skipped, boxes within eps counted whole).  The
