@@ -177,10 +177,12 @@ __device__ __forceinline__ int32_t heavy_count(const DbscanArgs<T>& a) {
 // Bound by VALU issue of the box tests and by the latency of list -> cell ->
 // box ranges -> boxes, which the rows of a chunk share.  kCount: also add the
 // row-row distance tests executed to *ntests (the instrumented variant).
-// With a.heavy (boxes of more than kHeavyWalk rows exist) a row's walk of such
-// a box leaves an entry per kHeavyWalk of its rows for k_core_heavy: one wave
-// takes 0.4 us per 256 rows, 8 ms for a box of five million.
-template <typename T, int D, bool kCount = false>
+// kHeavy: with a.heavy (boxes of more than kHeavyWalk rows exist) a row's walk
+// of such a box leaves an entry per kHeavyWalk of its rows for k_core_heavy:
+// one wave takes 0.4 us per 256 rows, 8 ms for a box of five million.  A
+// variant of its own, since the code costs scalar registers (4096 clouds of 8k
+// rows: 5.3 ms without, 9.0 ms with it).
+template <typename T, int D, bool kCount, bool kHeavy>
 __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                                                         uint8_t* __restrict__ core,
                                                         unsigned long long* __restrict__ ntests) {
@@ -262,7 +264,6 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                 for (uint64_t todo = ballot(part != 0 && !lane_walk); todo != 0; todo &= todo - 1) {
                     const int j = static_cast<int>(__builtin_ctzll(todo));
                     const uint32_t mp = static_cast<uint32_t>(bcast(static_cast<int32_t>(min_pts), j));
-                    const int32_t v0 = bcast(q0, j), v1 = bcast(q1, j);
                     for (uint32_t m = static_cast<uint32_t>(bcast(static_cast<int32_t>(part), j));
                          m != 0; m &= m - 1) {
                         const int row = (j & ~(G - 1)) + __builtin_ctz(m);
@@ -270,17 +271,19 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
                         const uint32_t now =
                             static_cast<uint32_t>(uniform(static_cast<int32_t>(rc[row])));
                         if (now >= mp) continue;  // an earlier box was enough
-                        if (a.heavy_cap > 0 && v1 - v0 > kHeavyWalk &&
-                            put_heavy(a, bcast(p, row), v0, v1)) {
-                            if (lane == row) put_off = true;
-                            continue;
-                        }
+                        if constexpr (kHeavy)
+                            if (a.heavy_cap > 0 && bcast(q1 - q0, j) > kHeavyWalk &&
+                                put_heavy(a, bcast(p, row), bcast(q0, j), bcast(q1, j))) {
+                                if (lane == row) put_off = true;
+                                continue;
+                            }
                         T pr[D];
 #pragma unroll
                         for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], row);
                         uint32_t visited = 0;
-                        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, v0, v1, pr,
-                                                              bcast(eps2, j), mp - now, visited);
+                        const uint32_t got = wide_count<T, D>(a.soa, a.ld, nullptr, bcast(q0, j),
+                                                              bcast(q1, j), pr, bcast(eps2, j),
+                                                              mp - now, visited);
                         if (lane == 0) rc[row] = now + got;
                         if constexpr (kCount)
                             if (lane == 0) tests += visited;
@@ -294,7 +297,8 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
         // (launch_core_init wrote 0 for every listed row)
         wave_lds_fence();
         const bool is_core = has && rc[lane] >= min_pts;
-        if (put_off) a.slot_a[p] = static_cast<int32_t>(min(rc[lane], min_pts));
+        if constexpr (kHeavy)
+            if (put_off) a.slot_a[p] = static_cast<int32_t>(min(rc[lane], min_pts));
         if (is_core) core[p] = 1;
         const int32_t first =
             group_min<G>(is_core ? static_cast<int32_t>(a.inrow[p]) : INT_MAX);
@@ -684,7 +688,7 @@ __device__ __forceinline__ unsigned int border_label(bool on, int32_t p, int32_t
 // next to two or more clusters.  Walks of boxes of more than kHeavyWalk rows
 // are put off as in k_core_rows: the row's clusters so far go to a.slot_a and
 // a.slot_b, k_border_heavy adds the parts' and k_border_late labels the row.
-template <typename T, int D>
+template <typename T, int D, bool kHeavy>
 __global__ __launch_bounds__(kThreads) void k_border_rows(
     const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
     const int2* __restrict__ rows, const unsigned int* __restrict__ nrows_dev,
@@ -748,11 +752,11 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
                     const int j = static_cast<int>(__builtin_ctzll(todo));
                     if (!((ballot(wanted()) >> j) & 1)) continue;
                     const int32_t v0 = bcast(q0, j), v1 = bcast(q1, j);
-                    if (a.heavy_cap > 0 && v1 - v0 > kHeavyWalk &&
-                        put_heavy(a, bcast(p, j), v0, v1)) {
-                        if (lane_id() / G == j / G) put_off = true;
-                        continue;
-                    }
+                    if constexpr (kHeavy)
+                        if (v1 - v0 > kHeavyWalk && put_heavy(a, bcast(p, j), v0, v1)) {
+                            if (lane_id() / G == j / G) put_off = true;
+                            continue;
+                        }
                     T pr[D];
 #pragma unroll
                     for (int e = 0; e < D; ++e) pr[e] = bcast(pc[e], j);
@@ -769,11 +773,12 @@ __global__ __launch_bounds__(kThreads) void k_border_rows(
             }
             return false;
         });
-        if (on && gl == 0 && put_off) {
-            a.slot_a[p] = best;
-            a.slot_b[p] = worst;
-            a.late[atomicAdd(a.nlate, 1u)] = p;
-        }
+        if constexpr (kHeavy)
+            if (on && gl == 0 && put_off) {
+                a.slot_a[p] = best;
+                a.slot_b[p] = worst;
+                a.late[atomicAdd(a.nlate, 1u)] = p;
+            }
         noise += border_label(on && gl == 0 && !put_off, p, u, a.inrow, best, worst, jp.row_begin,
                               labels, stats, amb_list);
     }
@@ -1037,14 +1042,15 @@ void launch_core(const DbscanArgs<T>& a, uint8_t* core, unsigned long long* ntes
                              a.bmincore, a.crows, a.ncrows_dev, kGroup<D>, s);
             if (count_start) HPD_HIP(hipEventRecord(count_start, s));
             constexpr int per_wave = 64 / kGroup<D>;
-            if (ntests)
-                hipLaunchKernelGGL((k_core_rows<T, D, true>),
-                                   dim3(persistent_blocks<k_core_rows<T, D, true>>(a.n, per_wave)),
+            auto rows = [&](auto count, auto heavy) {
+                constexpr auto kernel = k_core_rows<T, D, decltype(count)::value,
+                                                    decltype(heavy)::value>;
+                hipLaunchKernelGGL(kernel, dim3(persistent_blocks<kernel>(a.n, per_wave)),
                                    dim3(kThreads), 0, s, a, core, ntests);
-            else
-                hipLaunchKernelGGL((k_core_rows<T, D, false>),
-                                   dim3(persistent_blocks<k_core_rows<T, D, false>>(a.n, per_wave)),
-                                   dim3(kThreads), 0, s, a, core, nullptr);
+            };
+            if (ntests) rows(std::true_type{}, std::true_type{});
+            else if (a.heavy_cap > 0) rows(std::false_type{}, std::true_type{});
+            else rows(std::false_type{}, std::false_type{});
             if (a.heavy_cap > 0)
                 hipLaunchKernelGGL((k_core_heavy<T, D>),
                                    dim3(persistent_blocks<k_core_heavy<T, D>>(a.n, 1)),
@@ -1128,11 +1134,16 @@ void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* b
     const unsigned gw = blocks_for(a.nitems, kWavesPerBlock);
     if constexpr (std::is_floating_point<T>::value) {
         if (bcluster && a.bbox) {
-            hipLaunchKernelGGL((k_border_rows<T, D>),
-                               dim3(persistent_blocks<k_border_rows<T, D>>(a.n, 64 / kGroup<D>)),
-                               dim3(kThreads), 0, s, a, core, bcluster, static_cast<const int2*>(a.brows),
-                               static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
-                               amb_list);
+            auto rows = [&](auto heavy) {
+                constexpr auto kernel = k_border_rows<T, D, decltype(heavy)::value>;
+                hipLaunchKernelGGL(kernel, dim3(persistent_blocks<kernel>(a.n, 64 / kGroup<D>)),
+                                   dim3(kThreads), 0, s, a, core, bcluster,
+                                   static_cast<const int2*>(a.brows),
+                                   static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
+                                   amb_list);
+            };
+            if (a.heavy_cap > 0) rows(std::true_type{});
+            else rows(std::false_type{});
             if (a.heavy_cap > 0) {
                 hipLaunchKernelGGL((k_border_heavy<T, D>),
                                    dim3(persistent_blocks<k_border_heavy<T, D>>(a.n, 1)),
