@@ -9,8 +9,9 @@
 //                      ballots + per-wave LDS counters), the tile staged
 //                      in LDS in digit order, then written out so that
 //                      consecutive threads write consecutive places
-// A tile is 4096 keys: 4 waves x 16 iterations x 64 lanes; the stable order
-// inside a tile is (wave, iteration, lane), i.e. input order.  9-bit digits
+// A tile is 4096 keys: 4 waves x 16 iterations x 64 lanes (fewer iterations for
+// few keys); the stable order inside a tile is (wave, iteration, lane), i.e.
+// input order.  9-bit digits
 // (512 buckets, two per thread) are used where they save a pass.
 //
 // A block takes a run of tiles (SortPlan) where there are more than
@@ -19,6 +20,9 @@
 // save more there but leave too few blocks to hide a tile's chain of barriers
 // (100M rows, 2 passes, sort phase in ms by the blocks left: 2048 4.05, 4096
 // 4.10, 8192 3.93, 16384 3.87, all 48828 3.98).
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 #include "hpdbscan_capi.h"
 #include "internal.hpp"
@@ -29,37 +33,51 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kIters = 16;
-constexpr int kTile = kThreads * kIters;  // 4096
 // passes that carry rows stage them in LDS too: half the tile keeps two
 // more blocks resident per CU
 constexpr int kItersRows = 8;
-constexpr int kTileMin = kThreads * kItersRows;
+constexpr int kItersMin = 4;
 constexpr int kMaxBuckets = 512;          // 9-bit digits
 
-__host__ __device__ inline int64_t tiles_of(int64_t n, int64_t tile = kTile) {
+__host__ __device__ inline int64_t tiles_of(int64_t n, int64_t tile) {
     return (n + tile - 1) / tile;
 }
 
-// How a sort of n keys splits: blocks of `run` tiles; with self, each scatter
-// block adds up the histograms (hist[block * buckets + digit], written and
-// read in rows) instead of a scan of hist[digit * blocks + block]: two launches
-// fewer per pass for up to kSelfBlocks * 1 KB read by every block (100k rows, 3
-// passes: 456 -> 423 us; replayed, 8 passes: 514 -> 435 us).
+// How a sort of n keys splits: blocks of `run` tiles of kThreads * iters keys;
+// with self, each scatter block adds up the histograms (hist[block * buckets +
+// digit], written and read in rows) instead of a scan of hist[digit * blocks +
+// block]: two launches fewer per pass for up to kSelfBlocks * 1 KB read by
+// every block.  Where that is so the tiles are the smallest that leave no more
+// than kSelfBlocks of them: a tile's ranking is a serial chain of its
+// iterations, and 100k rows fill 25 of 256 CUs with tiles of 4096 (sort phase,
+// tiles of 4096 against this rule: 100k rows of 3 floats 126 -> 102 us, 30k of 6
+// doubles 159 -> 109, 200k of 3 136 -> 117; with up to 768 blocks 102, 110, 113).
 constexpr int64_t kRunBlocks = 16384;
 constexpr int64_t kSelfBlocks = 192;
 struct SortPlan {
     int64_t blocks;
+    int iters;
     int run;
     bool self;
 };
-inline SortPlan sort_plan(int64_t n, int64_t tile) {
-    const int64_t tiles = tiles_of(n, tile);
+inline SortPlan sort_plan(int64_t n, int max_iters) {
+    int iters = kItersMin;
+    while (iters < max_iters && tiles_of(n, kThreads * iters) > kSelfBlocks) iters *= 2;
+    const int64_t tiles = tiles_of(n, kThreads * iters);
     const int64_t run = tiles_of(tiles, kRunBlocks);
     const int64_t blocks = tiles_of(tiles, run);
-    return SortPlan{blocks, static_cast<int>(run), blocks <= kSelfBlocks};
+    return SortPlan{blocks, iters, static_cast<int>(run), blocks <= kSelfBlocks};
+}
+// fn(std::integral_constant<int, iters>)
+template <int kMax, typename Fn>
+void with_iters(const SortPlan& plan, Fn&& fn) {
+    static_assert(kMax == 8 || kMax == 16, "the iterations of a full tile");
+    if (plan.iters == 4) fn(std::integral_constant<int, 4>{});
+    else if (plan.iters == 8) fn(std::integral_constant<int, 8>{});
+    else fn(std::integral_constant<int, kMax>{});
 }
 
-template <typename K, int kBits, int kIt = kIters>
+template <typename K, int kBits, int kIt>
 __global__ __launch_bounds__(kThreads) void k_radix_hist(const K* __restrict__ keys, int64_t n,
                                                          int shift, uint32_t* __restrict__ hist,
                                                          SortPlan plan,
@@ -127,7 +145,7 @@ struct MoveRows {
     }
 };
 
-template <typename K, int kBits, typename Rows = NoRows, int kIt = kIters>
+template <typename K, int kBits, int kIt, typename Rows = NoRows>
 __global__ __launch_bounds__(kThreads) void k_radix_scatter(const K* __restrict__ kin,
                                                             const uint32_t* __restrict__ vin,
                                                             K* __restrict__ kout,
@@ -152,34 +170,59 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const K* __restrict_
     const int w = threadIdx.x >> 6;
     const int l = threadIdx.x & 63;
     if (plan.self) {
-        // digits of thread t: t, t + kThreads.  Own offset: the digit's keys
-        // in earlier blocks plus all keys of smaller digits.
-        uint32_t before[kOwn], all[kOwn];
+        // Own offset of a digit: its keys in earlier blocks (gbase) plus all
+        // keys of smaller digits (from tbase).  The waves take the blocks'
+        // histograms in turn, four digits per lane and load.
+        constexpr int kQ = B / 256;
+        constexpr int kDeep = 8;  // rows in flight per wave
+        for (int dg = threadIdx.x; dg < B; dg += kThreads) gbase[dg] = tbase[dg] = 0;
+        uint4 before[kQ], all[kQ];
 #pragma unroll
-        for (int o = 0; o < kOwn; ++o) {
-            before[o] = 0;
-            all[o] = 0;
-        }
-        for (int64_t b = 0; b < plan.blocks; b += 4) {
-            uint32_t v[4][kOwn];
+        for (int q = 0; q < kQ; ++q) before[q] = all[q] = make_uint4(0, 0, 0, 0);
+        const uint4* rows4 = reinterpret_cast<const uint4*>(offs);
+        const int nblk = static_cast<int>(plan.blocks);
+        for (int b = w; b < nblk; b += 4 * kDeep) {
+            uint4 v[kDeep][kQ];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < kDeep; ++j)
 #pragma unroll
-                for (int o = 0; o < kOwn; ++o)
-                    v[j][o] = b + j < plan.blocks
-                                  ? offs[(b + j) * B + o * kThreads + threadIdx.x] : 0u;
+                for (int q = 0; q < kQ; ++q)
+                    v[j][q] = b + 4 * j < nblk ? rows4[(b + 4 * j) * (B / 4) + q * 64 + l]
+                                               : make_uint4(0, 0, 0, 0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < kDeep; ++j)
 #pragma unroll
-                for (int o = 0; o < kOwn; ++o) {
-                    if (b + j < static_cast<int64_t>(blockIdx.x)) before[o] += v[j][o];
-                    all[o] += v[j][o];
+                for (int q = 0; q < kQ; ++q) {
+                    const uint32_t in = b + 4 * j < static_cast<int>(blockIdx.x) ? ~0u : 0u;
+                    before[q].x += v[j][q].x & in;
+                    before[q].y += v[j][q].y & in;
+                    before[q].z += v[j][q].z & in;
+                    before[q].w += v[j][q].w & in;
+                    all[q].x += v[j][q].x;
+                    all[q].y += v[j][q].y;
+                    all[q].z += v[j][q].z;
+                    all[q].w += v[j][q].w;
                 }
         }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) {
+            const int dg = q * 256 + 4 * l;
+            atomicAdd(&gbase[dg], before[q].x);
+            atomicAdd(&gbase[dg + 1], before[q].y);
+            atomicAdd(&gbase[dg + 2], before[q].z);
+            atomicAdd(&gbase[dg + 3], before[q].w);
+            atomicAdd(&tbase[dg], all[q].x);
+            atomicAdd(&tbase[dg + 1], all[q].y);
+            atomicAdd(&tbase[dg + 2], all[q].z);
+            atomicAdd(&tbase[dg + 3], all[q].w);
+        }
+        __syncthreads();
         uint32_t below = 0;  // keys of the digits of earlier rounds
 #pragma unroll
         for (int o = 0; o < kOwn; ++o) {
-            uint32_t inc = all[o];
+            const uint32_t sum = tbase[o * kThreads + threadIdx.x];
+            uint32_t inc = sum;
 #pragma unroll
             for (int st = 1; st < 64; st <<= 1) {
                 const uint32_t t = __shfl_up(inc, st, 64);
@@ -193,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(const K* __restrict_
                 if (i < w) woff += wsum[i];
                 total += wsum[i];
             }
-            gbase[o * kThreads + threadIdx.x] = below + woff + inc - all[o] + before[o];
+            gbase[o * kThreads + threadIdx.x] += below + woff + inc - sum;
             below += total;
             __syncthreads();
         }
@@ -334,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_settle(K* __restrict__ keys_
 template <typename K, int kBits>
 bool sort_passes(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n, int bits,
                  uint32_t* hist, uint32_t* tmp, hipStream_t s, const int* bits_dev = nullptr) {
-    const SortPlan plan = sort_plan(n, kTile);
+    const SortPlan plan = sort_plan(n, kIters);
     const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
@@ -342,11 +385,14 @@ bool sort_passes(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64
     uint32_t* vout = vals_b;
     bool in_b = false;
     for (int shift = 0; shift < bits; shift += kBits) {
-        hipLaunchKernelGGL((k_radix_hist<K, kBits>), grid, dim3(kThreads), 0, s, kin, n, shift,
-                           hist, plan, bits_dev);
-        if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
-        hipLaunchKernelGGL((k_radix_scatter<K, kBits>), grid, dim3(kThreads), 0, s, kin, vin, kout,
-                           vout, n, shift, hist, plan, bits_dev);
+        with_iters<kIters>(plan, [&](auto iters) {
+            constexpr int kIt = decltype(iters)::value;
+            hipLaunchKernelGGL((k_radix_hist<K, kBits, kIt>), grid, dim3(kThreads), 0, s, kin, n,
+                               shift, hist, plan, bits_dev);
+            if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
+            hipLaunchKernelGGL((k_radix_scatter<K, kBits, kIt>), grid, dim3(kThreads), 0, s, kin,
+                               vin, kout, vout, n, shift, hist, plan, bits_dev);
+        });
         HPD_HIP(hipGetLastError());
         K* tk = kin;
         kin = kout;
@@ -365,7 +411,7 @@ template <typename K, int kBits, typename T, int D>
 bool sort_passes_rows(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n,
                       int bits, uint32_t* hist, uint32_t* tmp, const T* pts, T* rows_a,
                       T* rows_b, T* soa, int64_t ld, hipStream_t s) {
-    const SortPlan plan = sort_plan(n, kTileMin);
+    const SortPlan plan = sort_plan(n, kItersRows);
     const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
@@ -379,12 +425,15 @@ bool sort_passes_rows(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, 
         using W = typename MoveRows<T, D>::W;
         MoveRows<T, D> mv{reinterpret_cast<const W*>(rin), reinterpret_cast<W*>(rnext), soa,
                           last ? ld : 0};
-        hipLaunchKernelGGL((k_radix_hist<K, kBits, kItersRows>), grid, dim3(kThreads), 0, s, kin, n,
-                           shift, hist, plan, nullptr);
-        if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
-        hipLaunchKernelGGL((k_radix_scatter<K, kBits, MoveRows<T, D>, kItersRows>), grid,
-                           dim3(kThreads), 0, s, kin, vin, kout, vout, n, shift, hist, plan, nullptr,
-                           mv);
+        with_iters<kItersRows>(plan, [&](auto iters) {
+            constexpr int kIt = decltype(iters)::value;
+            hipLaunchKernelGGL((k_radix_hist<K, kBits, kIt>), grid, dim3(kThreads), 0, s, kin, n,
+                               shift, hist, plan, nullptr);
+            if (!plan.self) exclusive_scan_u32(hist, hist, plan.blocks << kBits, tmp, nullptr, s);
+            hipLaunchKernelGGL((k_radix_scatter<K, kBits, kIt, MoveRows<T, D>>), grid,
+                               dim3(kThreads), 0, s, kin, vin, kout, vout, n, shift, hist, plan,
+                               nullptr, mv);
+        });
         HPD_HIP(hipGetLastError());
         K* tk = kin;
         kin = kout;
@@ -408,7 +457,11 @@ int radix_pass_count(int bits) {
 }
 
 size_t radix_hist_words(int64_t n) {
-    return static_cast<size_t>(kMaxBuckets) * static_cast<size_t>(tiles_of(n > 0 ? n : 1, kTileMin));
+    const int64_t k = n > 0 ? n : 1;
+    // (a bound that grows with n over the plans of all tile sizes)
+    const int64_t blocks = std::max(tiles_of(k, kThreads * kItersRows),
+                                    std::min(kSelfBlocks, tiles_of(k, kThreads * kItersMin)));
+    return static_cast<size_t>(kMaxBuckets) * static_cast<size_t>(blocks);
 }
 
 // 9-bit digits where they save a pass (e.g. 25-27 key bits: 3 passes, not 4)
