@@ -467,6 +467,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     int32_t *bmincore = nullptr, *bparent = nullptr, *compmin = nullptr, *bcluster = nullptr;
     uint8_t* btight = nullptr;
     void* bbox = nullptr;
+    int32_t* ctab = nullptr;
     uint64_t* scratch64 = nullptr;  // n words: open-pair lists, cluster keys, position sort
     if (boxes) {
         scratch64 = A.take_n<uint64_t>(nn);
@@ -482,15 +483,16 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         btight = A.take_n<uint8_t>(nn);
         bbox = A.take(2 * D * sizeof(T) * nn);
         void* bpart = A.take(gather_part_bytes(n, D, static_cast<int>(sizeof(T))));
-        // box flags and their scan in the sort's free buffers; then the
-        // occupied cells from the boxes (per-box cell flags and their scan
-        // in the run-flag buffer)
-        launch_box_table<K>(keys, n, nullptr, nullptr, vals_free,
-                            reinterpret_cast<uint32_t*>(keys_free), tmp, bstart, bcell, box_of_slot,
-                            &counters[3], nullptr, 2 * D, static_cast<int>(sizeof(T)), s, sub_bits,
-                            flags);
-        launch_cells_of_boxes<K>(keys, n, sub_bits, bstart, &counters[3], flags, flags + nn + 1,
-                                 tmp, bcell, ucell, ustart, cbox, &counters[0], s);
+        // a dense table of every cell id in the sort's spare key buffer, when
+        // the grid is small enough (the neighbour rows then read the table
+        // instead of searching the occupied cells)
+        const size_t free_pair = align_up(nn * sizeof(K), 256) + nn * sizeof(uint32_t);
+        if (key_total > 0 && key_total <= free_pair / sizeof(int32_t)) {
+            ctab = reinterpret_cast<int32_t*>(keys_free);  // keys_free and vals_free
+            fill_i32(ctab, -1, static_cast<int64_t>(key_total), s);
+        }
+        launch_box_table<K>(keys, n, sub_bits, flags, box_of_slot, bstart, bcell, ucell, ustart,
+                            cbox, ctab, &counters[3], &counters[0], s);
         launch_gather_boxes<T, D>(rows_sorted ? nullptr : pts, n, inrow_of_slot, soa, ld,
                                   box_of_slot, bstart, bbox, bpart, s);
     } else if (!rows_sorted) {
@@ -501,15 +503,6 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     HPD_HIP(hipStreamSynchronize(s));
     const int32_t m = static_cast<int32_t>(hc[0]);
     const int32_t nbox = boxes ? static_cast<int32_t>(hc[3]) : 0;
-    // box mode: a dense table of every cell id in the sort's spare key
-    // buffer, when the grid is small enough (the neighbour rows then read
-    // the table instead of searching the occupied cells)
-    int32_t* ctab = nullptr;
-    const size_t free_pair = align_up(nn * sizeof(K), 256) + nn * sizeof(uint32_t);
-    if (boxes && key_total > 0 && key_total <= free_pair / sizeof(int32_t)) {
-        ctab = reinterpret_cast<int32_t*>(keys_free);  // keys_free and vals_free
-        launch_cell_table<K>(ucell, host_count(m), ctab, key_total, s);
-    }
     tm.mark(M_SORT);
 
     // neighbour ranges (spatial_index.h:682-737)
@@ -964,12 +957,8 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
                             reinterpret_cast<const int*>(&sc[SS_BITS]), hist, tmp, s);
     K* keys = keys_a;
     uint32_t* inrow_of_slot = vals_a;
-    // the boxes, then the occupied cells from them
-    launch_box_table<K>(keys, n, nullptr, nullptr, vals_b, reinterpret_cast<uint32_t*>(keys_b), tmp,
-                        bstart, bcell, box_of_slot, &sc[SS_NBOX], nullptr, 2 * D,
-                        static_cast<int>(sizeof(T)), s, sub_bits, flags);
-    launch_cells_of_boxes<K>(keys, n, sub_bits, bstart, &sc[SS_NBOX], flags, flags + nn + 1, tmp,
-                             bcell, ucell, ustart, cbox, &sc[SS_M], s);
+    launch_box_table<K>(keys, n, sub_bits, flags, box_of_slot, bstart, bcell, ucell, ustart, cbox,
+                        nullptr, &sc[SS_NBOX], &sc[SS_M], s);
     launch_gather_boxes<T, D>(pts, n, inrow_of_slot, soa, ld, box_of_slot, bstart, bbox, bpart, s);
 
     // neighbour rows and work lists, counted and laid out on the device

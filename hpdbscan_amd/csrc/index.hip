@@ -96,14 +96,6 @@ __device__ __forceinline__ int2 row_cells_tab(const int32_t* __restrict__ ctab, 
     return b >= 0 ? make_int2(a, b + 1) : make_int2(0, 0);
 }
 
-// ctab[id] = u for every occupied cell u (the table filled with -1 before)
-template <typename K>
-__global__ __launch_bounds__(256) void k_cell_table(const K* __restrict__ ucell, Count mc,
-                                                    int32_t* __restrict__ ctab) {
-    const int32_t u = static_cast<int32_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (u < static_cast<int32_t>(mc.get())) ctab[static_cast<uint64_t>(ucell[u])] = u;
-}
-
 // Decode a cell id into per-swapped-dimension indices.
 __device__ __forceinline__ void decode_cell(uint64_t key, const CellParams& cp, uint64_t* idx) {
 #pragma unroll
@@ -569,15 +561,6 @@ void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
     HPD_HIP(hipGetLastError());
 }
 
-template <typename K>
-void launch_cell_table(const K* ucell, Count m, int32_t* ctab, uint64_t ids, hipStream_t s) {
-    if (m.host <= 0) return;
-    fill_i32(ctab, -1, static_cast<int64_t>(ids), s);
-    hipLaunchKernelGGL(k_cell_table<K>, dim3(blocks_for(m.host, 256)), dim3(256), 0, s, ucell, m,
-                       ctab);
-    HPD_HIP(hipGetLastError());
-}
-
 void launch_neighbor_copy(const int2* stash, int32_t stash_rows, int32_t m, const uint32_t* roff,
                           const int32_t* cbox, int2* rboxes, int32_t* rcenter, bool by_class,
                           hipStream_t s) {
@@ -628,8 +611,7 @@ void launch_work_items(const int32_t* ustart, Count m, const uint32_t* coff, Cou
 
 #define HPD_INST_INDEX(K)                                                                     \
     template void launch_cells<K>(const K*, int64_t, int, uint32_t*, uint32_t*, K*, int32_t*, \
-                                  uint32_t*, hipStream_t);                                    \
-    template void launch_cell_table<K>(const K*, Count, int32_t*, uint64_t, hipStream_t);
+                                  uint32_t*, hipStream_t);
 HPD_INST_INDEX(uint32_t)
 HPD_INST_INDEX(uint64_t)
 

@@ -34,12 +34,6 @@ void launch_neighbor_count(const K* ucell, const int32_t* ustart, Count m,
                            int32_t* rcenter, bool by_class, hipStream_t s,
                            const int32_t* ctab = nullptr);
 
-// Dense table of every cell id below `ids`: ctab[id] = its occupied-cell
-// index, -1 for an empty cell (ids int32 entries).  With it the neighbour
-// kernels read a row's cells from the table instead of searching.
-template <typename K>
-void launch_cell_table(const K* ucell, Count m, int32_t* ctab, uint64_t ids, hipStream_t s);
-
 // Box mode: launch_neighbor_fill's box ranges and rcenter from the count
 // pass's stash (roff scanned); with by_class the rows of each cell go
 // nearest first (own row, then by the number of offset dimensions) instead of
