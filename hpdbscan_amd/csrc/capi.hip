@@ -869,8 +869,11 @@ static size_t static_aux_bytes(int64_t n) {
 
 template <typename T, int D>
 static size_t static_main_bytes(int64_t n, int32_t njobs) {
-    return workspace_bytes<T, D>(n, njobs, false) + sizeof(uint64_t) * static_cast<size_t>(njobs) +
-           SS_WORDS * 4 + sizeof(SmallResult) + 64 * 1024 + 8 * 256;
+    size_t b = workspace_bytes<T, D>(n, njobs, false);
+    if (njobs == 1 && n <= small_rows(D))  // all pairs compared: a bit per pair
+        b = std::max(b, table_bytes<T, D>(n, 1) + small_workspace_bytes<T, D>(n));
+    return b + sizeof(uint64_t) * static_cast<size_t>(njobs) + SS_WORDS * 4 + sizeof(SmallResult) +
+           64 * 1024 + 8 * 256;
 }
 
 // The body of a static run on stream s: every launch of the run, nothing
