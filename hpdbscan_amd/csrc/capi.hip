@@ -208,6 +208,8 @@ private:
 // --------------------------------------------------------------------------
 // context
 // --------------------------------------------------------------------------
+constexpr int kHostMinMax = 64, kHostWords = 128;  // of Context::host_scratch
+
 struct Context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -232,7 +234,9 @@ struct Context {
     bool timing = false;
     bool count_tests = false;  // hpd_context_set_timing level 2
     hpd_run_stats stats{};
-    uint64_t* host_scratch = nullptr;  // pinned, 64 words
+    // pinned: small results and read-backs; from kHostMinMax on the min / max of a
+    // run of one job (2 * kMaxDims values, then the non-finite flag)
+    uint64_t* host_scratch = nullptr;
     std::vector<hipEvent_t> events;
     // hpd_context_set_graph: floating-point runs go through the static
     // pipeline, captured in a hipGraph and replayed while the shape stays
@@ -346,7 +350,7 @@ static inline int bits_for(uint64_t max_value) {
 template <typename T, int D>
 static size_t table_bytes(int64_t n, int64_t njobs) {
     const size_t nn = static_cast<size_t>(n), nj = static_cast<size_t>(njobs);
-    const size_t mm_blocks = nn / static_cast<size_t>(minmax_rows_per_block()) + nj + 1;
+    const size_t mm_blocks = nn / static_cast<size_t>(minmax_rows_per_block(n)) + nj + 1;
     return sizeof(T) * 2 * D * (mm_blocks + nj) + 4 * (mm_blocks + nj + 2) + 64 +
            sizeof(JobParams<T>) * nj + 8 * 256;
 }
@@ -385,8 +389,8 @@ static size_t workspace_bytes(int64_t n, int64_t njobs, bool one_thread) {
 }
 
 template <typename T, int D, typename K>
-static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>* jobs,
-                      int32_t njobs, int key_bits, uint64_t key_total, bool use_boxes,
+static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
+                      const JobParams<T>* host_jobs, int32_t njobs, int key_bits, uint64_t key_total, bool use_boxes,
                       int64_t* labels, hipStream_t s, PhaseTimer& tm) {
     // (known false for integer rows: their box kernels are not compiled)
     const bool boxes = std::is_floating_point<T>::value && use_boxes;
@@ -423,7 +427,14 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     // 0 m, 1 ranges, 2 items, 3 boxes, 5 loose, 6 chunks to count, 7 non-core
     // rows, 8 boxes with cores, 9 and 10 roots, 11 large boxes, 13 full-row table
     uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
-    HPD_HIP(hipMemsetAsync(dstats, 0, kStatWords * sizeof(unsigned long long), s));
+    // the job table and the zeroed counters
+    if (njobs == 1) {
+        launch_put_job<T>(host_jobs[0], jobs, dstats, kStatWords * sizeof(unsigned long long), s);
+    } else {
+        HPD_HIP(hipMemcpyAsync(jobs, host_jobs, sizeof(JobParams<T>) * njobs,
+                               hipMemcpyHostToDevice, s));
+        HPD_HIP(hipMemsetAsync(dstats, 0, kStatWords * sizeof(unsigned long long), s));
+    }
     uint32_t* hc = reinterpret_cast<uint32_t*>(ctx.host_scratch);
 
     // cell ids (spatial_index.h:144-165), offset by the job's key base; in
@@ -499,7 +510,11 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
         launch_gather_soa<T, D>(pts, n, inrow_of_slot, soa, ld, s);
     }
     // one read-back for the occupied cells and the boxes
-    HPD_HIP(hipMemcpyAsync(hc, counters, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    ReadBack cells;
+    cells.src[0] = counters;
+    cells.host[0] = hc;
+    cells.words[0] = 4;
+    read_back(cells, s);
     HPD_HIP(hipStreamSynchronize(s));
     const int32_t m = static_cast<int32_t>(hc[0]);
     const int32_t nbox = boxes ? static_cast<int32_t>(hc[3]) : 0;
@@ -543,13 +558,14 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
     }
     // the scans' totals into the counters (one launch), then one read-back
     // of the 64-bit row total (dstats[4]) and the counters (dstats + 8)
-    WordCopies totals;
-    totals.add(&nranges[m], &counters[1]);
-    if (!boxes) totals.add(&nchunks[m], &counters[2]);
-    copy_words(totals, s);
+    ReadBack totals;
+    totals.first.add(&nranges[m], &counters[1]);
+    if (!boxes) totals.first.add(&nchunks[m], &counters[2]);
     unsigned long long* hs_rows = reinterpret_cast<unsigned long long*>(ctx.host_scratch) + 12;
-    HPD_HIP(hipMemcpyAsync(hs_rows, &dstats[4], 10 * sizeof(unsigned long long),
-                           hipMemcpyDeviceToHost, s));
+    totals.src[0] = &dstats[4];
+    totals.host[0] = hs_rows;
+    totals.words[0] = 20;
+    read_back(totals, s);
     HPD_HIP(hipStreamSynchronize(s));
     hc = reinterpret_cast<uint32_t*>(hs_rows + 4);  // the counters as read back
     // the scan of nranges and every range index are 32-bit: check the
@@ -724,7 +740,11 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, const JobParams<T>*
                         &dstats[2], amb, s);
 
     unsigned long long* hs = reinterpret_cast<unsigned long long*>(ctx.host_scratch);
-    HPD_HIP(hipMemcpyAsync(hs, dstats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    ReadBack sums;
+    sums.src[0] = dstats;
+    sums.host[0] = hs;
+    sums.words[0] = 16;
+    read_back(sums, s);
     HPD_HIP(hipStreamSynchronize(s));
     if (box_union) ctx.stats.open_box_pairs = hs[5];
     ctx.stats.core_tests = hs[7];
@@ -910,8 +930,9 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     T* mm = A.take_n<T>(static_cast<size_t>(njobs) * 2 * D + 16);
     uint64_t* jcells = A.take_n<uint64_t>(static_cast<size_t>(njobs));
     unsigned long long* total_cells = dstats + 6;
-    launch_minmax<T, D>(pts, jobs, njobs, bfirst_dev, nblocks, part, mm,
-                        reinterpret_cast<int*>(&sc[SS_NONFINITE]), s);
+    int* bad_part = A.take_n<int>(static_cast<size_t>(nblocks) + 1);
+    launch_minmax<T, D>(pts, 0, n, jobs, njobs, bfirst_dev, nblocks, minmax_rows_per_block(n), part,
+                        bad_part, mm, reinterpret_cast<int*>(&sc[SS_NONFINITE]), s);
     const int sub_k = split_of(ctx, D);
     const int sub_bits = box_sub_bits(D, sub_k);
     launch_geometry<T, D>(jobs, njobs, mm, sub_bits, jcells, reinterpret_cast<int*>(&sc[SS_GRID]),
@@ -1045,6 +1066,15 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     launch_label_cores<T>(a, core, bcluster, parent, compmin, nullptr, cmin, cmax, labels,
                           &dstats[1], s, &sc[SS_ROWTAB]);
     launch_border<T, D>(a, core, bcluster, rootslot, cmin, cmax, labels, &dstats[2], nullptr, s);
+    // counts, flags and statistics for the host
+    ReadBack r;
+    r.src[0] = sc;
+    r.host[0] = ctx.host_scratch;
+    r.words[0] = SS_WORDS;
+    r.src[1] = dstats;
+    r.host[1] = ctx.host_scratch + SS_WORDS / 2;
+    r.words[1] = 16;
+    read_back(r, s);
 }
 
 // Ends a stream capture if the body throws halfway.
@@ -1081,7 +1111,7 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     // host-made part of the job table: row ranges, eps2, minPts, reciprocals
     HostArray<JobParams<T>, 1> hj(static_cast<size_t>(njobs));
     HostArray<int32_t, 2> bfirst(static_cast<size_t>(njobs) + 1);
-    const int rpb = minmax_rows_per_block();
+    const int64_t rpb = minmax_rows_per_block(n);
     int32_t nblocks = 0;
     for (int32_t j = 0; j < njobs; ++j) {
         JobParams<T>& jp = hj[j];
@@ -1097,10 +1127,14 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
         nblocks += static_cast<int32_t>((offsets[j + 1] - offsets[j] + rpb - 1) / rpb);
     }
     bfirst[njobs] = nblocks;
-    HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs, hipMemcpyHostToDevice,
-                           s));
-    HPD_HIP(hipMemcpyAsync(bfirst_dev, bfirst.data(), sizeof(int32_t) * (njobs + 1),
-                           hipMemcpyHostToDevice, s));
+    if (njobs == 1) {
+        launch_put_job<T>(hj[0], jobs_dev, nullptr, 0, s);
+    } else {
+        HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs,
+                               hipMemcpyHostToDevice, s));
+        HPD_HIP(hipMemcpyAsync(bfirst_dev, bfirst.data(), sizeof(int32_t) * (njobs + 1),
+                               hipMemcpyHostToDevice, s));
+    }
 
     Context::GraphEntry& ge = ctx.graph_entry;
     const bool same = ge.exec && ge.dtype == dtype && ge.d == D && ge.n == n && ge.data == pts &&
@@ -1151,11 +1185,10 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
         if (!taken) ++ctx.graph_fallbacks;
         return taken;
     }
-    // one read-back after the run: counts, flags and statistics
-    uint32_t* hc = reinterpret_cast<uint32_t*>(ctx.host_scratch);
-    unsigned long long* hs = reinterpret_cast<unsigned long long*>(ctx.host_scratch) + 16;
-    HPD_HIP(hipMemcpyAsync(hc, sc, SS_WORDS * 4, hipMemcpyDeviceToHost, s));
-    HPD_HIP(hipMemcpyAsync(hs, dstats, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    // the run's last kernel left the counts, flags and statistics here
+    const uint32_t* hc = reinterpret_cast<const uint32_t*>(ctx.host_scratch);
+    const unsigned long long* hs =
+        reinterpret_cast<const unsigned long long*>(ctx.host_scratch) + SS_WORDS / 2;
     HPD_HIP(hipStreamSynchronize(s));
     const bool ok = hc[SS_NONFINITE] == 0 && hc[SS_GRID] == 0 && hc[SS_LOOSE] == 0 &&
                     hs[4] <= static_cast<unsigned long long>(range_bound<D>(n));
@@ -1277,7 +1310,7 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     // vectors outlive every copy from them: the run ends with a stream sync.
     HostArray<JobParams<T>, 1> hj(static_cast<size_t>(njobs));
     HostArray<int32_t, 2> bfirst(static_cast<size_t>(njobs) + 1);
-    const int rpb = minmax_rows_per_block();
+    const int64_t rpb = minmax_rows_per_block(n);
     int32_t nblocks = 0;
     for (int32_t j = 0; j < njobs; ++j) {
         hj[j] = JobParams<T>{};
@@ -1292,19 +1325,36 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     T* part = A.take_n<T>(static_cast<size_t>(nblocks) * 2 * D + 1);
     T* mm = A.take_n<T>(static_cast<size_t>(njobs) * 2 * D + 16);
     int* nonfinite = reinterpret_cast<int*>(A.take_n<int>(4));
-    HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs, hipMemcpyHostToDevice, s));
-    HPD_HIP(hipMemcpyAsync(bfirst_dev, bfirst.data(), sizeof(int32_t) * (njobs + 1),
-                           hipMemcpyHostToDevice, s));
-    HPD_HIP(hipMemsetAsync(nonfinite, 0, sizeof(int), s));
+    int* bad_part = A.take_n<int>(static_cast<size_t>(nblocks) + 1);
 
-    // min / max per job (spatial_index.h:99-122)
-    launch_minmax<T, D>(pts, jobs_dev, njobs, bfirst_dev, nblocks, part, mm, nonfinite, s);
+    // min / max per job (spatial_index.h:99-122).  One job needs no table for
+    // that, and its result goes to pinned memory by itself: 100k rows 362 -> 331 us
+    // with the job table as a kernel argument and the read-backs as kernels.
     HostArray<T, 2 * D> hmm(static_cast<size_t>(njobs) * 2 * D);
     int hbad = 0;
-    HPD_HIP(hipMemcpyAsync(hmm.data(), mm, sizeof(T) * njobs * 2 * D, hipMemcpyDeviceToHost, s));
-    HPD_HIP(hipMemcpyAsync(ctx.host_scratch, nonfinite, sizeof(int), hipMemcpyDeviceToHost, s));
-    HPD_HIP(hipStreamSynchronize(s));
-    std::memcpy(&hbad, ctx.host_scratch, sizeof(int));
+    if (njobs == 1) {
+        T* host_mm = reinterpret_cast<T*>(ctx.host_scratch + kHostMinMax);
+        int* host_bad = reinterpret_cast<int*>(ctx.host_scratch + kHostMinMax + 2 * kMaxDims);
+        launch_minmax<T, D>(pts, offsets[0], offsets[1], nullptr, 1, nullptr, nblocks, rpb, part,
+                            bad_part, host_mm, host_bad, s);
+        HPD_HIP(hipStreamSynchronize(s));
+        std::memcpy(hmm.data(), host_mm, sizeof(T) * 2 * D);
+        hbad = *host_bad;
+    } else {
+        HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs,
+                               hipMemcpyHostToDevice, s));
+        HPD_HIP(hipMemcpyAsync(bfirst_dev, bfirst.data(), sizeof(int32_t) * (njobs + 1),
+                               hipMemcpyHostToDevice, s));
+        HPD_HIP(hipMemsetAsync(nonfinite, 0, sizeof(int), s));
+        launch_minmax<T, D>(pts, 0, n, jobs_dev, njobs, bfirst_dev, nblocks, rpb, part, bad_part,
+                            mm, nonfinite, s);
+        HPD_HIP(hipMemcpyAsync(hmm.data(), mm, sizeof(T) * njobs * 2 * D, hipMemcpyDeviceToHost,
+                               s));
+        HPD_HIP(hipMemcpyAsync(ctx.host_scratch, nonfinite, sizeof(int), hipMemcpyDeviceToHost,
+                               s));
+        HPD_HIP(hipStreamSynchronize(s));
+        std::memcpy(&hbad, ctx.host_scratch, sizeof(int));
+    }
     if (hbad) throw Error(HPD_EINVAL, "input contains NaN or infinite coordinates");
 
     // per-job grid (spatial_index.h:124-142) and key ranges
@@ -1352,13 +1402,13 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     const int split_bits = box_sub_bits(D, split_of(ctx, D));
     const bool boxes = (std::is_floating_point<T>::value || as_float) && key_bits + split_bits <= 64;
     const int sort_bits = key_bits + (boxes ? split_bits : 0);
-    auto run = [&](auto* rows, auto* table) {
+    auto run = [&](auto* rows, auto* table, auto* host_table) {
         using R = std::remove_const_t<std::remove_pointer_t<decltype(rows)>>;
         if (sort_bits <= 32)
-            run_keyed<R, D, uint32_t>(ctx, rows, n, table, njobs, key_bits, key_total, boxes,
+            run_keyed<R, D, uint32_t>(ctx, rows, n, table, host_table, njobs, key_bits, key_total, boxes,
                                       labels, s, tm);
         else
-            run_keyed<R, D, uint64_t>(ctx, rows, n, table, njobs, key_bits, key_total, boxes,
+            run_keyed<R, D, uint64_t>(ctx, rows, n, table, host_table, njobs, key_bits, key_total, boxes,
                                       labels, s, tm);
     };
     if constexpr (std::is_integral<T>::value) {
@@ -1378,16 +1428,12 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
             }
             JobParams<float>* table = A.take_n<JobParams<float>>(static_cast<size_t>(njobs));
             float* rows = A.take_n<float>(static_cast<size_t>(n) * D);
-            HPD_HIP(hipMemcpyAsync(table, hf.data(), sizeof(JobParams<float>) * njobs,
-                                   hipMemcpyHostToDevice, s));
             launch_to_float<T>(pts, n * D, rows, s);
-            run(static_cast<const float*>(rows), table);
+            run(static_cast<const float*>(rows), table, hf.data());
         }
     }
     if (std::is_floating_point<T>::value || !as_float || !boxes) {
-        HPD_HIP(hipMemcpyAsync(jobs_dev, hj.data(), sizeof(JobParams<T>) * njobs,
-                               hipMemcpyHostToDevice, s));
-        run(pts, jobs_dev);
+        run(pts, jobs_dev, hj.data());
     }
     if (ctx.timing) {
         ctx.stats.ms_grid = tm.ms(M_START, M_GRID);
@@ -1625,7 +1671,7 @@ int hpd_context_create(int device, hpd_context** out) {
             hpd::init_scratch_for_current_device(device);
             HPD_HIP(hipStreamCreateWithFlags(&c->impl.stream, hipStreamNonBlocking));
             void* hs = nullptr;
-            HPD_HIP(hipHostMalloc(&hs, 64 * sizeof(uint64_t), hipHostMallocDefault));
+            HPD_HIP(hipHostMalloc(&hs, hpd::kHostWords * sizeof(uint64_t), hipHostMallocDefault));
             c->impl.host_scratch = static_cast<uint64_t*>(hs);
         } catch (...) {
             if (c->impl.stream) (void)hipStreamDestroy(c->impl.stream);

@@ -520,22 +520,24 @@ __global__ __launch_bounds__(kThreads) void k_full_box_table(
 // own place (coalesced, where labelling in slot order stores at permuted
 // places).  Rows of other boxes (table value 0) are left to
 // k_label_cores_boxes.  Nothing when the table did not fit.
+constexpr int kFullRows = 256;  // rows per wave
 template <typename T, int D, typename K>
 __global__ __launch_bounds__(kThreads) void k_label_full_rows(
     const T* __restrict__ pts, int64_t n, const JobParams<T>* __restrict__ jobs, int32_t njobs,
     int sub_k, int sub_bits, const int32_t* __restrict__ tab, int64_t cap,
     const unsigned int* __restrict__ ok, int64_t* __restrict__ labels) {
     if (*ok == 0) return;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * kThreads) {
-        const JobParams<T>& jp = jobs[job_of_row_wave(jobs, njobs, i)];
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + (threadIdx.x >> 6)) *
+                       kFullRows;
+    for_job_rows(jobs, njobs, r0, r0 + kFullRows < n ? r0 + kFullRows : n,
+                 [&](const JobParams<T>& jp, int64_t i) {
         const K key = static_cast<K>(row_key<T, D>(pts + i * D, jp, sub_k, sub_bits));
         // (every row's key is a box's key, below cap when *ok is set)
         const int32_t v = static_cast<uint64_t>(key) < static_cast<uint64_t>(cap)
                               ? tab[static_cast<int64_t>(key)]
                               : 0;
         if (v != 0) labels[i] = -static_cast<int64_t>(v);
-    }
+    });
 }
 
 template <typename T, int D>
@@ -1073,7 +1075,8 @@ void launch_label_full_rows(const T* pts, const DbscanArgs<T>& a, int sub_k, int
     hipLaunchKernelGGL((k_full_box_table<T, K>), dim3(blocks_for(nbox.host, kThreads)),
                        dim3(kThreads), 0, s, keys, a.n, a.bstart, nbox, a.bcell, a.job_of_cell,
                        a.jobs, a.btight, bcluster, tab, cap, ok);
-    hipLaunchKernelGGL((k_label_full_rows<T, D, K>), dim3(blocks_for(a.n, kThreads)),
+    hipLaunchKernelGGL((k_label_full_rows<T, D, K>),
+                       dim3(blocks_for(a.n, kWavesPerBlock * kFullRows)),
                        dim3(kThreads), 0, s, pts, a.n,
                        a.jobs, a.njobs, sub_k, sub_bits, static_cast<const int32_t*>(tab), cap,
                        static_cast<const unsigned int*>(ok), labels);

@@ -20,33 +20,25 @@ namespace hpd {
 namespace {
 
 constexpr int kMMThreads = 256;
-constexpr int kMMRows = 8 * kMMThreads;  // rows per partial block
+constexpr int kMMRows = 8 * kMMThreads;  // rows per partial block, at least
+// the final pass is one block per job: a job's partials stay below this
+constexpr int64_t kMMBlocks = 2048;
 
-// first job whose partial-block range contains block b (bfirst ascending)
-__device__ __forceinline__ int32_t job_of_block(const int32_t* __restrict__ bfirst, int32_t njobs,
-                                                int32_t b) {
-    int32_t lo = 0, hi = njobs - 1;
-    while (lo < hi) {
-        const int32_t mid = (lo + hi + 1) >> 1;
-        if (bfirst[mid] <= b) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-// One block reduces up to kMMRows rows of one job; bfirst[j] is the first
-// block of job j.
+// One block reduces up to `rpb` rows of one job; bfirst[j] is the first block
+// of job j (one job: rows [row0, row1), jobs and bfirst not read).
 template <typename T, int D>
-__global__ __launch_bounds__(kMMThreads) void k_minmax_partial(const T* __restrict__ pts,
-                                                               const JobParams<T>* __restrict__ jobs,
-                                                               int32_t njobs,
-                                                               const int32_t* __restrict__ bfirst,
-                                                               T* __restrict__ part,
-                                                               int* __restrict__ nonfinite) {
+__global__ __launch_bounds__(kMMThreads) void k_minmax_partial(
+    const T* __restrict__ pts, int64_t row0, int64_t row1, const JobParams<T>* __restrict__ jobs,
+    int32_t njobs, const int32_t* __restrict__ bfirst, int64_t rpb, T* __restrict__ part,
+    int* __restrict__ bad_part) {
     const int32_t b = static_cast<int32_t>(blockIdx.x);
-    const int32_t j = job_of_block(bfirst, njobs, b);
-    const int64_t r0 = jobs[j].row_begin + static_cast<int64_t>(b - bfirst[j]) * kMMRows;
-    const int64_t r1 = min(r0 + kMMRows, jobs[j].row_end);
+    int64_t r0 = row0 + b * rpb, r1 = row1;
+    if (njobs > 1) {
+        const int32_t j = wave_last(njobs, [&](int32_t k) { return bfirst[k] <= b; });
+        r0 = jobs[j].row_begin + (b - bfirst[j]) * rpb;
+        r1 = jobs[j].row_end;
+    }
+    r1 = min(r0 + rpb, r1);
     T mn[D], mx[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) {
@@ -65,7 +57,7 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_partial(const T* __restri
     }
     // NaN never wins the comparisons above, so non-finite input is flagged
     // separately (the host rejects it)
-    if (__any(bad) && __lane_id() == 0) atomicOr(nonfinite, 1);
+    const int any_bad = __syncthreads_or(bad ? 1 : 0);
     __shared__ T smn[D][kMMThreads];
     __shared__ T smx[D][kMMThreads];
 #pragma unroll
@@ -85,6 +77,7 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_partial(const T* __restri
         __syncthreads();
     }
     if (threadIdx.x == 0) {
+        bad_part[b] = any_bad;
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             part[static_cast<int64_t>(b) * 2 * D + k] = smn[k][0];
@@ -93,12 +86,20 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_partial(const T* __restri
     }
 }
 
-// One block per job: min/max over the job's partial blocks.
+// One block per job: min/max over the job's partial blocks; *nonfinite |= 1 (one
+// job: stored) when a row is not finite.  out and nonfinite may be pinned host
+// memory for one job.
 template <typename T, int D>
 __global__ __launch_bounds__(kMMThreads) void k_minmax_final(const T* __restrict__ part,
+                                                             const int* __restrict__ bad_part,
                                                              const int32_t* __restrict__ bfirst,
-                                                             T* __restrict__ out) {
+                                                             int32_t njobs, int32_t nblocks,
+                                                             T* __restrict__ out,
+                                                             int* __restrict__ nonfinite) {
     const int32_t j = static_cast<int32_t>(blockIdx.x);
+    const int32_t b0 = njobs == 1 ? 0 : bfirst[j];
+    const int32_t b1 = njobs == 1 ? nblocks : bfirst[j + 1];
+    int bad = 0;
     __shared__ T smn[D][kMMThreads];
     __shared__ T smx[D][kMMThreads];
     T mn[D], mx[D];
@@ -107,7 +108,8 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_final(const T* __restrict
         mn[k] = min_init<T>();
         mx[k] = max_init<T>();
     }
-    for (int32_t b = bfirst[j] + threadIdx.x; b < bfirst[j + 1]; b += kMMThreads) {
+    for (int32_t b = b0 + static_cast<int32_t>(threadIdx.x); b < b1; b += kMMThreads) {
+        bad |= bad_part[b];
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             mn[k] = ref_min(mn[k], part[static_cast<int64_t>(b) * 2 * D + k]);
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_final(const T* __restrict
         smn[k][threadIdx.x] = mn[k];
         smx[k][threadIdx.x] = mx[k];
     }
-    __syncthreads();
+    bad = __syncthreads_or(bad);
     for (int o = kMMThreads / 2; o > 0; o >>= 1) {
         if (threadIdx.x < o) {
 #pragma unroll
@@ -131,6 +133,8 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_final(const T* __restrict
         __syncthreads();
     }
     if (threadIdx.x == 0) {
+        if (njobs == 1) *nonfinite = bad ? 1 : 0;
+        else if (bad) atomicOr(nonfinite, 1);
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             out[static_cast<int64_t>(j) * 2 * D + k] = smn[k][0];
@@ -139,17 +143,27 @@ __global__ __launch_bounds__(kMMThreads) void k_minmax_final(const T* __restrict
     }
 }
 
+// A wave takes kIdRows consecutive rows.
+constexpr int kIdRows = 256;
 template <typename T, int D, typename K>
 __global__ __launch_bounds__(256) void k_cell_ids(const T* __restrict__ pts, int64_t n,
                                                   const JobParams<T>* __restrict__ jobs,
                                                   int32_t njobs, int sub_k, int sub_bits,
                                                   K* __restrict__ keys,
                                                   uint32_t* __restrict__ vals) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= n) return;
-    const JobParams<T>& jp = jobs[job_of_row_wave(jobs, njobs, i)];
-    keys[i] = static_cast<K>(row_key<T, D>(pts + i * D, jp, sub_k, sub_bits));
-    vals[i] = static_cast<uint32_t>(i);
+    const int64_t r0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kIdRows;
+    for_job_rows(jobs, njobs, r0, r0 + kIdRows < n ? r0 + kIdRows : n,
+                 [&](const JobParams<T>& jp, int64_t i) {
+        keys[i] = static_cast<K>(row_key<T, D>(pts + i * D, jp, sub_k, sub_bits));
+        vals[i] = static_cast<uint32_t>(i);
+    });
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_put_job(const JobParams<T> v, JobParams<T>* __restrict__ dst,
+                                                 uint32_t* __restrict__ zero, int nzero) {
+    if (threadIdx.x == 0) *dst = v;
+    for (int i = threadIdx.x; i < nzero; i += 256) zero[i] = 0u;
 }
 
 template <typename T, int D>
@@ -248,7 +262,18 @@ void launch_geometry(JobParams<T>* jobs, int32_t njobs, const T* mm, int sub_bit
     HPD_HIP(hipGetLastError());
 }
 
-int minmax_rows_per_block() { return kMMRows; }
+int64_t minmax_rows_per_block(int64_t n) {
+    const int64_t per = static_cast<int64_t>(kMMRows) * kMMBlocks;
+    return kMMRows * (n > per ? (n + per - 1) / per : 1);
+}
+
+template <typename T>
+void launch_put_job(const JobParams<T>& v, JobParams<T>* dst, void* zero, size_t zero_bytes,
+                    hipStream_t s) {
+    hipLaunchKernelGGL(k_put_job<T>, dim3(1), dim3(256), 0, s, v, dst, static_cast<uint32_t*>(zero),
+                       static_cast<int>(zero_bytes / 4));
+    HPD_HIP(hipGetLastError());
+}
 
 template <typename T>
 void launch_to_float(const T* in, int64_t count, float* out, hipStream_t s) {
@@ -259,12 +284,15 @@ void launch_to_float(const T* in, int64_t count, float* out, hipStream_t s) {
 }
 
 template <typename T, int D>
-void launch_minmax(const T* pts, const JobParams<T>* jobs, int32_t njobs, const int32_t* bfirst,
-                   int32_t nblocks, T* part, T* out, int* nonfinite, hipStream_t s) {
+void launch_minmax(const T* pts, int64_t row0, int64_t row1, const JobParams<T>* jobs,
+                   int32_t njobs, const int32_t* bfirst, int32_t nblocks, int64_t rpb, T* part,
+                   int* bad_part, T* out, int* nonfinite, hipStream_t s) {
     if (nblocks > 0)
-        hipLaunchKernelGGL((k_minmax_partial<T, D>), dim3(nblocks), dim3(kMMThreads), 0, s, pts, jobs,
-                           njobs, bfirst, part, nonfinite);
-    hipLaunchKernelGGL((k_minmax_final<T, D>), dim3(njobs), dim3(kMMThreads), 0, s, part, bfirst, out);
+        hipLaunchKernelGGL((k_minmax_partial<T, D>), dim3(nblocks), dim3(kMMThreads), 0, s, pts,
+                           row0, row1, jobs, njobs, bfirst, rpb, part, bad_part);
+    hipLaunchKernelGGL((k_minmax_final<T, D>), dim3(njobs), dim3(kMMThreads), 0, s,
+                       static_cast<const T*>(part), static_cast<const int*>(bad_part), bfirst,
+                       njobs, nblocks, out, nonfinite);
     HPD_HIP(hipGetLastError());
 }
 
@@ -272,7 +300,7 @@ template <typename T, int D, typename K>
 void launch_cell_ids(const T* pts, int64_t n, const JobParams<T>* jobs, int32_t njobs, int sub_k,
                      int sub_bits, K* keys, uint32_t* vals, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL((k_cell_ids<T, D, K>), dim3(blocks_for(n, 256)), dim3(256), 0, s, pts, n,
+    hipLaunchKernelGGL((k_cell_ids<T, D, K>), dim3(blocks_for(n, 4 * kIdRows)), dim3(256), 0, s, pts, n,
                        jobs, njobs, sub_k, sub_bits, keys, vals);
     HPD_HIP(hipGetLastError());
 }
@@ -289,8 +317,9 @@ void launch_gather_soa(const T* pts, int64_t n, const uint32_t* order, T* soa, i
 #define HPD_INST_GRID(T, D)                                                                     \
     template void launch_geometry<T, D>(JobParams<T>*, int32_t, const T*, int, uint64_t*, int*,  \
                                         int*, unsigned long long*, hipStream_t);                  \
-    template void launch_minmax<T, D>(const T*, const JobParams<T>*, int32_t, const int32_t*,    \
-                                      int32_t, T*, T*, int*, hipStream_t);                       \
+    template void launch_minmax<T, D>(const T*, int64_t, int64_t, const JobParams<T>*, int32_t,  \
+                                      const int32_t*, int32_t, int64_t, T*, int*, T*, int*,      \
+                                      hipStream_t);                                              \
     template void launch_cell_ids<T, D, uint32_t>(const T*, int64_t, const JobParams<T>*,        \
                                                   int32_t, int, int, uint32_t*, uint32_t*,       \
                                                   hipStream_t);                                  \
@@ -314,5 +343,9 @@ HPD_FOR_EACH_DTYPE(HPD_INST_GRID_ALL_D)
 
 #define HPD_INST_TO_FLOAT(T) template void launch_to_float<T>(const T*, int64_t, float*, hipStream_t);
 HPD_FOR_EACH_DTYPE(HPD_INST_TO_FLOAT)
+
+#define HPD_INST_PUT_JOB(T) \
+    template void launch_put_job<T>(const JobParams<T>&, JobParams<T>*, void*, size_t, hipStream_t);
+HPD_FOR_EACH_DTYPE(HPD_INST_PUT_JOB)
 
 }  // namespace hpd

@@ -23,8 +23,13 @@
 
 namespace hpd {
 
-// rows reduced by one block of the min/max kernel
-int minmax_rows_per_block();
+// rows reduced by one block of the min/max kernel in a run of n rows
+int64_t minmax_rows_per_block(int64_t n);
+
+// *dst = v, and zero_bytes bytes (a multiple of 4) at zero cleared, in one launch
+template <typename T>
+void launch_put_job(const JobParams<T>& v, JobParams<T>* dst, void* zero, size_t zero_bytes,
+                    hipStream_t s);
 
 // The static pipeline's grid of every job, on the device: from the jobs'
 // min / max (mm) it fills cp, minv and key_base of every job (host-written
@@ -37,12 +42,15 @@ void launch_geometry(JobParams<T>* jobs, int32_t njobs, const T* mm, int sub_bit
 
 // Per job j: out[j*2D .. j*2D+D) = min, out[j*2D+D .. (j+1)*2D) = max over
 // the job's rows.  bfirst[j] = first partial block of job j (host-made,
-// ceil(rows / minmax_rows_per_block()) blocks per job, bfirst[njobs] =
-// nblocks); part holds 2*D*nblocks values; *nonfinite (zeroed by the caller)
-// becomes 1 if a coordinate is NaN or infinite.
+// ceil(rows / rpb) blocks per job, bfirst[njobs] = nblocks); part holds
+// 2*D*nblocks values, bad_part nblocks; *nonfinite becomes 1 if a coordinate is
+// NaN or infinite (several jobs: zeroed by the caller; one job: written).  One
+// job: rows [row0, row1), jobs and bfirst unused, out and nonfinite may be
+// pinned host memory.
 template <typename T, int D>
-void launch_minmax(const T* pts, const JobParams<T>* jobs, int32_t njobs, const int32_t* bfirst,
-                   int32_t nblocks, T* part, T* out, int* nonfinite, hipStream_t s);
+void launch_minmax(const T* pts, int64_t row0, int64_t row1, const JobParams<T>* jobs,
+                   int32_t njobs, const int32_t* bfirst, int32_t nblocks, int64_t rpb, T* part,
+                   int* bad_part, T* out, int* nonfinite, hipStream_t s);
 
 // key = (job key_base + linearised cell id (spatial_index.h:144-165)) <<
 // sub_bits | sub-box digit (sub_bits = 0: no digit; the cell's k^D split

@@ -245,14 +245,21 @@ void exclusive_scan_u32_dev(const uint32_t* in, uint32_t* out, Count n, uint32_t
 }
 
 namespace {
-__global__ void k_copy_words(const WordCopies c) {
-    if (static_cast<int>(threadIdx.x) < c.k) *c.dst[threadIdx.x] = *c.src[threadIdx.x];
+// one wave: the copied words are read after its own stores
+__global__ __launch_bounds__(64) void k_read_back(const ReadBack r) {
+    const int t = static_cast<int>(threadIdx.x);
+    if (t < r.first.k) *r.first.dst[t] = *r.first.src[t];
+    __syncthreads();
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t* src = static_cast<const uint32_t*>(r.src[k]);
+        uint32_t* host = static_cast<uint32_t*>(r.host[k]);
+        for (int i = t; i < r.words[k]; i += 64) host[i] = src[i];
+    }
 }
 }  // namespace
 
-void copy_words(const WordCopies& c, hipStream_t s) {
-    if (c.k <= 0) return;
-    hipLaunchKernelGGL(k_copy_words, dim3(1), dim3(64), 0, s, c);
+void read_back(const ReadBack& r, hipStream_t s) {
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(64), 0, s, r);
     HPD_HIP(hipGetLastError());
 }
 
