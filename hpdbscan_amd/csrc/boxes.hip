@@ -564,6 +564,13 @@ __device__ __forceinline__ bool ends_pair(const T* __restrict__ soa, int64_t ld,
 // (4096 clouds, hook and join ms: 16 4.79, 32 4.83, 64 4.91, 256 11.4 before
 // the first and last rows were tried first, 1024 13.2.)
 constexpr int kLanePair = 16;
+// Lanes per box: neighbourhoods grow with 3^D, and a group hands its lanes one
+// box each per round of dependent loads.  Hook and join / union ms by lanes:
+// 10M rows of 3 (8 lanes) 0.169 / 0.133, (16) 0.196 / 0.152, (32) 0.265 / 0.196;
+// 5M of 4 (16) 0.299 / 0.614, (32) 0.243 / 0.624, (64) 0.286 / 0.673; 30k of 6
+// doubles (16) 0.220 / 0.119, (32) 0.147 / 0.109, (64) 0.123 / 0.112.
+template <int D>
+constexpr int kPairGroup = D <= 3 ? 8 : D == 4 ? 32 : 64;
 constexpr int kLinkRows = 4096;
 
 // The same bounds (point_box) for the rows of two boxes: gap2 <= dist2(p, q)
@@ -605,7 +612,7 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
                                                        const int32_t* __restrict__ blist,
                                                        const unsigned int* __restrict__ nlist_dev,
                                                        int32_t* bparent) {
-    constexpr int G = kGroup<D>;
+    constexpr int G = kPairGroup<D>;
     constexpr int kPer = 64 / G;
     const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
     const int gl = lane_id() & (G - 1);
@@ -700,7 +707,7 @@ __global__ __launch_bounds__(kThreads) void k_box_union(
     const int32_t* __restrict__ blist, const unsigned int* __restrict__ nlist_dev,
     int32_t* bparent, int2* __restrict__ heavy, unsigned long long* __restrict__ nheavy,
     unsigned long long heavy_cap, unsigned long long* __restrict__ nopen) {
-    constexpr int G = kGroup<D>;
+    constexpr int G = kPairGroup<D>;
     constexpr int kPer = 64 / G;
     const int32_t nlist = uniform(static_cast<int32_t>(*nlist_dev));
     const int grp = lane_id() / G;
@@ -1070,7 +1077,7 @@ void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbox
                      const unsigned int* nlist, int32_t* bparent, hipStream_t s) {
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_link<T, D, false>),
-                       dim3(persistent_blocks<k_box_link<T, D, false>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(persistent_blocks<k_box_link<T, D, false>>(a.nbox, 64 / kPairGroup<D>)),
                        dim3(kThreads), 0, s, a, roff, rboxes, bmincore, core, blist, nlist, bparent);
     HPD_HIP(hipGetLastError());
 }
@@ -1089,7 +1096,7 @@ void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2*
                           const unsigned int* nroots, int32_t* bparent, hipStream_t s) {
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_link<T, D, true>),
-                       dim3(persistent_blocks<k_box_link<T, D, true>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(persistent_blocks<k_box_link<T, D, true>>(a.nbox, 64 / kPairGroup<D>)),
                        dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, roots, nroots, bparent);
     HPD_HIP(hipGetLastError());
 }
@@ -1112,7 +1119,7 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
                       unsigned long long* nopen, hipStream_t s) {
     if (a.nbox <= 0) return;
     hipLaunchKernelGGL((k_box_union<T, D>),
-                       dim3(persistent_blocks<k_box_union<T, D>>(a.nbox, 64 / kGroup<D>)),
+                       dim3(persistent_blocks<k_box_union<T, D>>(a.nbox, 64 / kPairGroup<D>)),
                        dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, blist, nlist, bparent, heavy, nheavy, heavy_cap,
                        nopen);
     // (its waves leave at once when there are no entries)

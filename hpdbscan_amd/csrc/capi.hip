@@ -425,7 +425,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     int32_t* job_of_cell = A.take_n<int32_t>(nn);
     unsigned long long* dstats = A.take_n<unsigned long long>(kStatWords);
     // 0 m, 1 ranges, 2 items, 3 boxes, 5 loose, 6 chunks to count, 7 non-core
-    // rows, 8 boxes with cores, 9 and 10 roots, 11 large boxes, 13 full-row table
+    // rows, 8 boxes with cores, 9 roots, 11 large boxes, 13 full-row table
     uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
     // the job table and the zeroed counters
     if (njobs == 1) {
@@ -685,12 +685,9 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         launch_list_boxes(host_count(nbox), bmincore, blist, &counters[8], bparent, s);
         launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &counters[8], bparent, s);
         // (the slot-level union's rsnap is free in box mode: the roots)
-        for (int round = 0; round < kRootJoinRounds<D>; ++round) {
-            launch_box_roots(host_count(nbox), bmincore, bparent, compmin, rsnap,
-                             &counters[9 + round], s);
-            launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, rsnap,
-                                       &counters[9 + round], bparent, s);
-        }
+        launch_box_roots(host_count(nbox), bmincore, bparent, compmin, rsnap, &counters[9], s);
+        launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, rsnap, &counters[9], bparent,
+                                   s);
         launch_box_roots(host_count(nbox), bmincore, bparent, compmin, nullptr, nullptr, s);
         tm.mark(M_HOOK1);
         // pairs with a large box go through a list in scratch64
@@ -871,9 +868,8 @@ enum StaticSlot : int {
     SS_CROWS = 6,      // rows to count
     SS_BROWS = 7,      // non-core rows
     SS_NLIST = 8,      // boxes with cores
-    SS_JOIN0 = 9,      // roots of the first root-join round
+    SS_JOIN = 9,      // roots of the first root-join round
     SS_LARGE = 11,     // (boxes above a size: not counted here)
-    SS_JOIN1 = 13,     // roots of the second round
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
     SS_BITS = 16,      // key bits + sub-box bits
@@ -1045,11 +1041,8 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     int32_t* blist = parent;
     launch_list_boxes(NB, bmincore, blist, &sc[SS_NLIST], bparent, s);
     launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &sc[SS_NLIST], bparent, s);
-    for (int round = 0; round < kRootJoinRounds<D>; ++round) {
-        uint32_t* cnt = &sc[round == 0 ? SS_JOIN0 : SS_JOIN1];
-        launch_box_roots(NB, bmincore, bparent, compmin, roots, cnt, s);
-        launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, roots, cnt, bparent, s);
-    }
+    launch_box_roots(NB, bmincore, bparent, compmin, roots, &sc[SS_JOIN], s);
+    launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, roots, &sc[SS_JOIN], bparent, s);
     launch_box_roots(NB, bmincore, bparent, compmin, nullptr, nullptr, s);
     launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &sc[SS_NLIST], box_of_slot,
                            reinterpret_cast<int2*>(scratch64), &dstats[15],

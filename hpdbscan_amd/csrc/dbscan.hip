@@ -198,7 +198,8 @@ __global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
     uint32_t* rc = cnt_lds[w];
     // the lanes of the caller's group where `on`, as G bits
     auto group_bits = [&](bool on) {
-        return static_cast<uint32_t>(ballot(on) >> g0) & ((1u << G) - 1u);
+        static_assert(G <= 32, "a group's lanes in 32 bits");
+        return static_cast<uint32_t>(ballot(on) >> g0) & (~0u >> (32 - G));
     };
     const Span<T>* bbox = static_cast<const Span<T>*>(a.bbox);
     unsigned long long tests = 0;
@@ -690,13 +691,17 @@ __device__ __forceinline__ unsigned int border_label(bool on, int32_t p, int32_t
 // next to two or more clusters.  Walks of boxes of more than kHeavyWalk rows
 // are put off as in k_core_rows: the row's clusters so far go to a.slot_a and
 // a.slot_b, k_border_heavy adds the parts' and k_border_late labels the row.
+// Lanes per row (ms by lanes: 5M rows of 4 (16) 0.256, (32) 0.241, (64) 0.302;
+// 30k of 6 doubles (16) 0.079, (32) 0.053, (64) 0.040).
+template <int D>
+constexpr int kBorderGroup = D <= 3 ? 8 : D == 4 ? 32 : 64;
 template <typename T, int D, bool kHeavy>
 __global__ __launch_bounds__(kThreads) void k_border_rows(
     const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
     const int2* __restrict__ rows, const unsigned int* __restrict__ nrows_dev,
     int64_t* __restrict__ labels, unsigned long long* __restrict__ stats,
     int2* __restrict__ amb_list) {
-    constexpr int G = kGroup<D>;
+    constexpr int G = kBorderGroup<D>;
     constexpr int kPer = 64 / G;
     const int32_t nrows = uniform(static_cast<int32_t>(*nrows_dev));
     const int gl = lane_id() & (G - 1);
@@ -1139,7 +1144,7 @@ void launch_border(const DbscanArgs<T>& a, const uint8_t* core, const int32_t* b
         if (bcluster && a.bbox) {
             auto rows = [&](auto heavy) {
                 constexpr auto kernel = k_border_rows<T, D, decltype(heavy)::value>;
-                hipLaunchKernelGGL(kernel, dim3(persistent_blocks<kernel>(a.n, 64 / kGroup<D>)),
+                hipLaunchKernelGGL(kernel, dim3(persistent_blocks<kernel>(a.n, 64 / kBorderGroup<D>)),
                                    dim3(kThreads), 0, s, a, core, bcluster,
                                    static_cast<const int2*>(a.brows),
                                    static_cast<const unsigned int*>(a.nbrows_dev), labels, stats,
