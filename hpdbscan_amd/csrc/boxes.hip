@@ -523,14 +523,23 @@ __device__ __forceinline__ bool lane_pair(const T* __restrict__ soa, int64_t ld,
                                           const uint8_t* __restrict__ core, int32_t s0, int32_t s1,
                                           int32_t q0, int32_t q1, T eps2) {
     for (int32_t p = s0; p < s1; ++p) {
-        if (!core[p]) continue;
+        const bool cp = core[p] != 0;
         T pc[D];
         load_row<T, D>(soa, ld, p, pc);
-        for (int32_t q = q0; q < q1; ++q) {
-            if (!core[q]) continue;
-            T qc[D];
-            load_row<T, D>(soa, ld, q, qc);
-            if (within<D>(pc, qc, eps2)) return true;
+        // (four rows side by side: their loads don't wait for each other)
+        for (int32_t q = q0; q < q1; q += 4) {
+            T qc[4][D];
+            bool cq[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int32_t at = min(q + k, q1 - 1);
+                cq[k] = core[at] != 0;
+                load_row<T, D>(soa, ld, at, qc[k]);
+            }
+            bool hit = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) hit = hit || (cq[k] && within<D>(pc, qc[k], eps2));
+            if (hit && cp) return true;
         }
     }
     return false;
@@ -688,6 +697,85 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
             else bparent[b] = link;
         }
     }
+}
+
+// The boxes with cores of the cells whose own boxes and later neighbour boxes
+// lie in different snapshot trees (rsnap) go to `list`: only they can have open
+// pairs.  A group of lanes per cell, which ends at the first box of another
+// tree; a cell's boxes share the neighbourhood, and most cells lie inside one
+// tree.  From 4-D on and for many boxes: the neighbourhoods are large, or a launch
+// is cheap beside them (union with this kernel and without, us: 5M rows of 4
+// floats 203, 630; 30k of 6 doubles 33, 112; 4096 clouds of 3 3218, 4720; 10M
+// rows of 3 116, 137; 100k of 3 60, 42; 300k of 2 38, 26).
+constexpr int64_t kMixedBoxes = 250000;
+constexpr int kMixedStage = 512;  // list entries staged per wave
+template <int D>
+__global__ __launch_bounds__(kThreads) void k_mixed_cells(
+    Count m_c, const int32_t* __restrict__ cbox, const uint32_t* __restrict__ roff,
+    const int2* __restrict__ rboxes, const int32_t* __restrict__ rsnap, int32_t* __restrict__ list,
+    unsigned int* __restrict__ count) {
+    constexpr int G = kPairGroup<D>;
+    constexpr int kPer = 64 / G;
+    __shared__ int32_t stage[kWavesPerBlock][kMixedStage];
+    __shared__ unsigned int left[kWavesPerBlock], at0;
+    const int32_t m = uniform(static_cast<int32_t>(m_c.get()));
+    const int w = static_cast<int>(threadIdx.x >> 6);
+    const int gl = lane_id() & (G - 1);
+    const int grp = lane_id() / G;
+    const uint64_t gmask = ((G < 64 ? (uint64_t{1} << G) : 0) - 1) << (grp * G);
+    unsigned int fill = 0;  // of the wave's stage
+    for (int32_t base = first_wave() * kPer; base < m; base += wave_stride() * kPer) {
+        const bool on = base + grp < m;
+        const int32_t u = on ? base + grp : m - 1;
+        const int32_t c0 = cbox[u], c1 = cbox[u + 1];
+        const int32_t r0 = static_cast<int32_t>(roff[u]), r1 = static_cast<int32_t>(roff[u + 1]);
+        int32_t lo = INT_MAX, hi = -1;
+        for (int32_t k = c0; __any(on && k < c1); k += G) {
+            const int32_t t = on && k + gl < c1 ? rsnap[k + gl] : -1;
+            if (t >= 0) {
+                lo = min(lo, t);
+                hi = max(hi, t);
+            }
+        }
+        const int32_t root = group_min<G>(lo);
+        bool mixed = group_max<G>(hi) > root;
+        group_boxes<G>(on && root != INT_MAX && !mixed, r0, r1, r0, -1, rboxes, c1, INT_MAX,
+                       [&](bool valid, int32_t b2) {
+            const int32_t t = valid ? rsnap[b2] : -1;
+            const bool other = (ballot(t >= 0 && t != root) & gmask) != 0;
+            mixed = mixed || other;
+            return other;
+        });
+        mixed = mixed && on && root != INT_MAX;
+        for (int32_t k = c0; __any(mixed && k < c1); k += G) {
+            const bool put = mixed && k + gl < c1 && rsnap[k + gl] >= 0;
+            const uint64_t puts = ballot(put);
+            const unsigned int add = static_cast<unsigned int>(__popcll(puts));
+            if (fill + add > kMixedStage) {
+                unsigned int at = 0;
+                if (lane_id() == 0) at = atomicAdd(count, fill);
+                at = static_cast<unsigned int>(bcast(static_cast<int32_t>(at), 0));
+                wave_lds_fence();
+                for (unsigned int e = lane_id(); e < fill; e += kWave) list[at + e] = stage[w][e];
+                wave_lds_fence();
+                fill = 0;
+            }
+            if (put) stage[w][fill + __popcll(puts & lanemask_lt())] = k + gl;
+            fill += add;
+        }
+    }
+    // the rest, one reservation per block
+    if (lane_id() == 0) left[w] = fill;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned int sum = 0;
+        for (int k = 0; k < kWavesPerBlock; ++k) sum += left[k];
+        at0 = sum > 0 ? atomicAdd(count, sum) : 0u;
+    }
+    __syncthreads();
+    unsigned int at = at0;
+    for (int k = 0; k < w; ++k) at += left[k];
+    for (unsigned int e = lane_id(); e < fill; e += kWave) list[at + e] = stage[w][e];
 }
 
 // The exact union: every listed box meets the later boxes of its
@@ -1114,14 +1202,24 @@ void launch_core_init(int64_t n, const int32_t* box_of_slot, const uint8_t* btig
 template <typename T, int D>
 void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                       const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
-                      const unsigned int* nlist, const int32_t* box_of_slot, int2* heavy,
+                      const unsigned int* nblist, Count m, int32_t* list, unsigned int* nlist,
+                      const int32_t* box_of_slot, int2* heavy,
                       unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
                       unsigned long long* nopen, hipStream_t s) {
     if (a.nbox <= 0) return;
+    // (a device-written number of boxes: the bound is the rows)
+    const int64_t boxes = a.nbox_dev ? a.nbox / 8 : a.nbox;
+    if (D >= 4 || boxes > kMixedBoxes) {
+        hipLaunchKernelGGL(k_mixed_cells<D>,
+                           dim3(persistent_blocks<k_mixed_cells<D>>(m.host, 64 / kPairGroup<D>)),
+                           dim3(kThreads), 0, s, m, a.cbox, roff, rboxes, rsnap, list, nlist);
+        blist = list;
+        nblist = nlist;
+    }
     hipLaunchKernelGGL((k_box_union<T, D>),
                        dim3(persistent_blocks<k_box_union<T, D>>(a.nbox, 64 / kPairGroup<D>)),
-                       dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, blist, nlist, bparent, heavy, nheavy, heavy_cap,
-                       nopen);
+                       dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, blist, nblist, bparent,
+                       heavy, nheavy, heavy_cap, nopen);
     // (its waves leave at once when there are no entries)
     hipLaunchKernelGGL((k_box_union_heavy<T, D>),
                        dim3(persistent_blocks<k_box_union_heavy<T, D>>(a.nrows / kHeavyRows + 1, 1)),
@@ -1204,7 +1302,8 @@ void launch_positions(int64_t n, int32_t m, const int32_t* box_of_slot, const in
                                              const unsigned int*, int32_t*, hipStream_t);         \
     template void launch_box_union<T, D>(const BoxArgs<T>&, const uint32_t*, const int2*,         \
                                          const int32_t*, const uint8_t*, const int32_t*,          \
-                                         const unsigned int*, const int32_t*, int2*,              \
+                                         const unsigned int*, Count, int32_t*, unsigned int*,     \
+                                         const int32_t*, int2*,                                   \
                                          unsigned long long*, unsigned long long, int32_t*,       \
                                          unsigned long long*, hipStream_t);
 #define HPD_INST_BOX_ALL_D(T) \

@@ -69,7 +69,9 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
 //                        box it meets (one round: a second one costs more than
 //                        the union then saves, 30k of 6 doubles 599 -> 637 us,
 //                        100k of 3 floats 324 -> 340); then launch_box_roots
-//   launch_box_union     the pairs still open (different trees in rsnap,
+//   launch_box_union     (list: scratch for the boxes, out of the *nblist of
+//                        blist, of those of the m cells that can have open
+//                        pairs, *nlist += their number) the pairs still open (different trees in rsnap,
 //                        within eps by their bounding boxes; *nopen += their
 //                        number), every one decided exactly
 //   then launch_box_clusters.
@@ -91,7 +93,8 @@ void launch_box_root_join(const BoxArgs<T>& a, const uint32_t* roff, const int2*
 template <typename T, int D>
 void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                       const int32_t* rsnap, const uint8_t* core, const int32_t* blist,
-                      const unsigned int* nlist, const int32_t* box_of_slot, int2* heavy,
+                      const unsigned int* nblist, Count m, int32_t* list, unsigned int* nlist,
+                      const int32_t* box_of_slot, int2* heavy,
                       unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
                       unsigned long long* nopen, hipStream_t s);
 // core[s] = 1 for the rows of tight boxes with >= minPts rows (btight bit 1),

@@ -425,7 +425,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     int32_t* job_of_cell = A.take_n<int32_t>(nn);
     unsigned long long* dstats = A.take_n<unsigned long long>(kStatWords);
     // 0 m, 1 ranges, 2 items, 3 boxes, 5 loose, 6 chunks to count, 7 non-core
-    // rows, 8 boxes with cores, 9 roots, 11 large boxes, 13 full-row table
+    // rows, 8 boxes with cores, 9 roots, 10 boxes near several trees, 11 large boxes, 13 full-row table
     uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
     // the job table and the zeroed counters
     if (njobs == 1) {
@@ -693,8 +693,8 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         // pairs with a large box go through a list in scratch64
         unsigned long long cap = static_cast<unsigned long long>(nn);
         if (ctx.open_pair_limit > 0 && ctx.open_pair_limit < cap) cap = ctx.open_pair_limit;
-        launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &counters[8], box_of_slot,
-                               reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,
+        launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &counters[8],
+                               host_count(m), rsnap, &counters[10], box_of_slot, reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,
                                &dstats[5], s);
         tm.mark(M_JOIN1);
         launch_box_clusters(host_count(nbox), bmincore, bcell, cbox, bstart, inrow_of_slot, ustart,
@@ -868,7 +868,8 @@ enum StaticSlot : int {
     SS_CROWS = 6,      // rows to count
     SS_BROWS = 7,      // non-core rows
     SS_NLIST = 8,      // boxes with cores
-    SS_JOIN = 9,      // roots of the first root-join round
+    SS_JOIN = 9,       // roots of the hook forest
+    SS_MIXED = 10,     // boxes of cells next to several trees
     SS_LARGE = 11,     // (boxes above a size: not counted here)
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
@@ -1044,7 +1045,8 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     launch_box_roots(NB, bmincore, bparent, compmin, roots, &sc[SS_JOIN], s);
     launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, roots, &sc[SS_JOIN], bparent, s);
     launch_box_roots(NB, bmincore, bparent, compmin, nullptr, nullptr, s);
-    launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &sc[SS_NLIST], box_of_slot,
+    launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &sc[SS_NLIST], M, roots,
+                           &sc[SS_MIXED], box_of_slot,
                            reinterpret_cast<int2*>(scratch64), &dstats[15],
                            static_cast<unsigned long long>(nn), bparent, &dstats[5], s);
     launch_box_clusters(NB, bmincore, bcell, cbox, bstart, inrow_of_slot, ustart, bparent,

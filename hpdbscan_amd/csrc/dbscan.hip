@@ -134,13 +134,6 @@ __global__ __launch_bounds__(kThreads) void k_core(const DbscanArgs<T> a, uint8_
     (void)ncore;
 }
 
-// Orders the LDS accesses of a wave's lanes among each other (the hardware
-// keeps a wave's LDS operations in order; this keeps the compiler from moving
-// or caching them).
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-}
-
 // Boxes of more rows are walked in parts of this many, one wave each
 // (100M skewed rows: 26 us a part).
 constexpr int32_t kHeavyWalk = 16384;

@@ -312,6 +312,13 @@ inline unsigned persistent_blocks(int64_t items, int per_wave) {
     return static_cast<unsigned>(b > 0 ? b : 1);
 }
 
+// Orders the LDS accesses of a wave's lanes among each other (the hardware
+// keeps a wave's LDS operations in order; this keeps the compiler from moving
+// or caching them).
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Sum, minimum and maximum over a group of G lanes.
 template <int G>
 __device__ __forceinline__ uint32_t group_sum(uint32_t v) {

@@ -49,3 +49,20 @@ def test_clouds(ctx, d, dtype, eps, spread):
             np.testing.assert_array_equal(c.cluster(x, eps, mp), got)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("d,eps", [(2, 0.06), (3, 0.4)])
+def test_many_boxes(ctx, d, eps):
+    """Above 250000 boxes the union looks at cells first in 2-D and 3-D too."""
+    n = 700_000
+    rng = np.random.default_rng(d)
+    centres = rng.uniform(0, 60, (400, d))
+    x = centres[rng.integers(0, 400, n)] + rng.normal(0, 1.2 if d == 2 else 0.9, (n, d))
+    far = rng.integers(0, n, n // 10)
+    x[far] = rng.uniform(0, 60, (len(far), d))
+    x = x.astype(np.float32)
+    print(f"[gpu-case] many boxes d={d}", flush=True)
+    got = ctx.cluster(x, eps, 5)
+    assert ctx.stats()["boxes"] > 250_000
+    r = oracle.check_parallel(x, eps, 5, got, threads=16)
+    assert r["mismatches"] == 0 and r["bad_ambiguous"] == 0
