@@ -11,7 +11,8 @@ namespace hpd {
 
 constexpr int kCollectThreads = 256;
 constexpr int kCollectWaves = kCollectThreads / kWave;
-constexpr int kCollectPer = 4;  // indices per thread and round
+constexpr int kCollectPer = 2;  // indices per thread and round (100k rows, whole call
+                                // in us: 1 309-317, 2 298-315, 4 325-330, 8 345)
 constexpr int kCollectTile = kCollectThreads * kCollectPer;
 constexpr int kCollectCap = 2048;  // entries staged in LDS
 
