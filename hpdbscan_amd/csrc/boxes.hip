@@ -440,6 +440,9 @@ __global__ __launch_bounds__(kThreads) void k_table_write(
     }
 }
 
+// rows of a box from which its pairs of the union go by parts (k_box_union)
+constexpr int kHeavyRows = 2048;
+
 // flags per box: tight (dist2(extent) <= EPS2 in the reference's order),
 // full, in a cell that can hold cores
 template <typename T, int D>
@@ -472,7 +475,8 @@ __global__ __launch_bounds__(kThreads) void k_box_tight(const Span<T>* __restric
                                      ((tight && static_cast<uint32_t>(size) >= jp.min_pts) ? 2 : 0) |
                                      (cell_core[u] ? 4 : 0));
     if (!tight && size > 1) atomicAdd(nloose, 1u);
-    if (size > large) atomicAdd(nlarge, 1u);
+    if (size > large) atomicAdd(&nlarge[0], 1u);
+    if (size > kHeavyRows) atomicAdd(&nlarge[1], 1u);
 }
 
 // Whether a core row of a box, [q0, q1), is within eps of the row of a lane
@@ -786,7 +790,6 @@ __global__ __launch_bounds__(kThreads) void k_mixed_cells(
 // pair with a box of more than kHeavyRows rows leaves an entry per kHeavyRows
 // of that box in heavy (up to heavy_cap entries; beyond, the wave tests it
 // here) and the others are tested by the wave.
-constexpr int kHeavyRows = 2048;
 
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void k_box_union(
@@ -905,15 +908,18 @@ __global__ __launch_bounds__(kThreads) void k_box_union_heavy(
 }
 
 // list[...] = every box with cores (v = bmincore != INT_MAX); *count +=
-// their number; every box a root of its own (bparent)
+// their number; every box a root of its own (bparent), its smallest core key
+// (cmin) none yet
 __global__ __launch_bounds__(kThreads) void k_list_boxes(Count nbox_c,
                                                          const int32_t* __restrict__ bmincore,
                                                          int32_t* __restrict__ list,
                                                          unsigned int* __restrict__ count,
-                                                         int32_t* __restrict__ bparent) {
+                                                         int32_t* __restrict__ bparent,
+                                                         unsigned long long* __restrict__ cmin) {
     block_collect(nbox_c.get(), list, count, [&](int64_t b, int32_t& v) {
         v = static_cast<int32_t>(b);
         bparent[b] = v;
+        cmin[b] = ~0ull;
         return bmincore[b] != INT_MAX;
     });
 }
@@ -1064,12 +1070,6 @@ __global__ __launch_bounds__(kThreads) void k_box_cluster(Count nbox_c,
     bcluster[b] = bmincore[b] == INT_MAX ? -1 : compmin[uf_find(bparent, b)];
 }
 
-__global__ __launch_bounds__(kThreads) void k_fill_u64(unsigned long long* __restrict__ a,
-                                                       unsigned long long v, int64_t n) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i < n) a[i] = v;
-}
-
 // 16 bytes per store, then the rest
 __global__ __launch_bounds__(kThreads) void k_fill_i32(int32_t* __restrict__ a, int32_t v,
                                                        int64_t n) {
@@ -1152,10 +1152,10 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
 }
 
 void launch_list_boxes(Count nbox, const int32_t* bmincore, int32_t* list, unsigned int* count,
-                       int32_t* bparent, hipStream_t s) {
+                       int32_t* bparent, unsigned long long* cmin, hipStream_t s) {
     if (nbox.host <= 0) return;
     hipLaunchKernelGGL(k_list_boxes, dim3(collect_blocks(nbox.host)), dim3(kThreads), 0, s, nbox,
-                       bmincore, list, count, bparent);
+                       bmincore, list, count, bparent, cmin);
     HPD_HIP(hipGetLastError());
 }
 
@@ -1205,7 +1205,7 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
                       const unsigned int* nblist, Count m, int32_t* list, unsigned int* nlist,
                       const int32_t* box_of_slot, int2* heavy,
                       unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
-                      unsigned long long* nopen, hipStream_t s) {
+                      unsigned long long* nopen, bool large, hipStream_t s) {
     if (a.nbox <= 0) return;
     // (a device-written number of boxes: the bound is the rows)
     const int64_t boxes = a.nbox_dev ? a.nbox / 8 : a.nbox;
@@ -1221,7 +1221,8 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
                        dim3(kThreads), 0, s, a, roff, rboxes, rsnap, core, blist, nblist, bparent,
                        heavy, nheavy, heavy_cap, nopen);
     // (its waves leave at once when there are no entries)
-    hipLaunchKernelGGL((k_box_union_heavy<T, D>),
+    if (large)
+        hipLaunchKernelGGL((k_box_union_heavy<T, D>),
                        dim3(persistent_blocks<k_box_union_heavy<T, D>>(a.nrows / kHeavyRows + 1, 1)),
                        dim3(kThreads), 0, s, a, box_of_slot, core, bparent, static_cast<const int2*>(heavy),
                        static_cast<const unsigned long long*>(nheavy), heavy_cap);
@@ -1241,7 +1242,6 @@ void launch_box_clusters(Count nbox, const int32_t* bmincore, const int32_t* bce
                          int32_t* compmin, int32_t* bcluster, hipStream_t s) {
     if (nbox.host <= 0) return;
     const dim3 g(blocks_for(nbox.host, kThreads));
-    hipLaunchKernelGGL(k_fill_u64, g, dim3(kThreads), 0, s, cmin, ~0ull, nbox.host);
     hipLaunchKernelGGL(k_box_compmin, g, dim3(kThreads), 0, s, nbox, bmincore, bcell, bparent, cmin);
     hipLaunchKernelGGL(k_box_resolve, g, dim3(kThreads), 0, s, nbox,
                        static_cast<const int32_t*>(bparent),
@@ -1305,7 +1305,7 @@ void launch_positions(int64_t n, int32_t m, const int32_t* box_of_slot, const in
                                          const unsigned int*, Count, int32_t*, unsigned int*,     \
                                          const int32_t*, int2*,                                   \
                                          unsigned long long*, unsigned long long, int32_t*,       \
-                                         unsigned long long*, hipStream_t);
+                                         unsigned long long*, bool, hipStream_t);
 #define HPD_INST_BOX_ALL_D(T) \
     HPD_INST_BOX_KEYS(T, 1)   \
     HPD_INST_BOX_KEYS(T, 2)   \

@@ -53,14 +53,16 @@ void launch_box_table(const K* keys, int64_t n, int shift, uint32_t* sums, int32
 
 // btight[b]: bit 0 tight, bit 1 tight with >= minPts rows, bit 2 in a cell
 // that can hold cores (cell_core); *nloose counts boxes of two or more rows
-// that are not tight, *nlarge boxes of more than `large` rows
+// that are not tight, nlarge[0] boxes of more than `large` rows, nlarge[1] those
+// whose pairs the union takes by parts
 template <typename T, int D>
 void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* btight,
                       unsigned int* nloose, int32_t large, unsigned int* nlarge, hipStream_t s);
 
 // Components of the boxes with cores:
 //   launch_list_boxes    list of the boxes with cores, *count += their
-//                        number; bparent reset
+//                        number; bparent and cmin (of launch_box_clusters)
+//                        reset
 //   launch_box_hook      hook forest over the listed boxes: every box points
 //                        at some earlier box joined to it
 //   launch_box_roots     root of every box -> rsnap (-1 without cores), the
@@ -73,13 +75,14 @@ void launch_box_tight(const BoxArgs<T>& a, const uint8_t* cell_core, uint8_t* bt
 //                        blist, of those of the m cells that can have open
 //                        pairs, *nlist += their number) the pairs still open (different trees in rsnap,
 //                        within eps by their bounding boxes; *nopen += their
-//                        number), every one decided exactly
+//                        number), every one decided exactly (large: boxes of
+//                        launch_box_tight's nlarge[1] may exist)
 //   then launch_box_clusters.
 // List lengths stay on the device (kernels of persistent grids).  heavy
 // holds heavy_cap entries of scratch; *nheavy, *nopen and every count are
 // zeroed by the caller.
 void launch_list_boxes(Count nbox, const int32_t* bmincore, int32_t* list, unsigned int* count,
-                       int32_t* bparent, hipStream_t s);
+                       int32_t* bparent, unsigned long long* cmin, hipStream_t s);
 template <typename T, int D>
 void launch_box_hook(const BoxArgs<T>& a, const uint32_t* roff, const int2* rboxes,
                      const int32_t* bmincore, const uint8_t* core, const int32_t* blist,
@@ -96,7 +99,7 @@ void launch_box_union(const BoxArgs<T>& a, const uint32_t* roff, const int2* rbo
                       const unsigned int* nblist, Count m, int32_t* list, unsigned int* nlist,
                       const int32_t* box_of_slot, int2* heavy,
                       unsigned long long* nheavy, unsigned long long heavy_cap, int32_t* bparent,
-                      unsigned long long* nopen, hipStream_t s);
+                      unsigned long long* nopen, bool large, hipStream_t s);
 // core[s] = 1 for the rows of tight boxes with >= minPts rows (btight bit 1),
 // 0 for every other row; bmincore[b] = inrow[bstart[b]] for those boxes
 // (every row is core and a box holds its rows in input order), INT_MAX for

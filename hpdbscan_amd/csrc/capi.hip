@@ -425,7 +425,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     int32_t* job_of_cell = A.take_n<int32_t>(nn);
     unsigned long long* dstats = A.take_n<unsigned long long>(kStatWords);
     // 0 m, 1 ranges, 2 items, 3 boxes, 5 loose, 6 chunks to count, 7 non-core
-    // rows, 8 boxes with cores, 9 roots, 10 boxes near several trees, 11 large boxes, 13 full-row table
+    // rows, 8 boxes with cores, 9 roots, 10 boxes near several trees, 11 and 12 large boxes, 13 full-row table
     uint32_t* counters = reinterpret_cast<uint32_t*>(dstats + 8);
     // the job table and the zeroed counters
     if (njobs == 1) {
@@ -479,7 +479,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     uint8_t* btight = nullptr;
     void* bbox = nullptr;
     int32_t* ctab = nullptr;
-    uint64_t* scratch64 = nullptr;  // n words: open-pair lists, cluster keys, position sort
+    uint64_t* scratch64 = nullptr;  // n words: open-pair lists, position sort
     if (boxes) {
         scratch64 = A.take_n<uint64_t>(nn);
         pos_of_slot = A.take_n<uint32_t>(nn);
@@ -564,7 +564,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     unsigned long long* hs_rows = reinterpret_cast<unsigned long long*>(ctx.host_scratch) + 12;
     totals.src[0] = &dstats[4];
     totals.host[0] = hs_rows;
-    totals.words[0] = 20;
+    totals.words[0] = 24;
     read_back(totals, s);
     HPD_HIP(hipStreamSynchronize(s));
     hc = reinterpret_cast<uint32_t*>(hs_rows + 4);  // the counters as read back
@@ -680,9 +680,12 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
     int32_t* blist = parent;
     box_union = all_tight;
     if (box_union) {
-        // compmin holds the forest's roots until the clusters are known
+        // compmin holds the forest's roots until the clusters are known; the
+        // smallest key of every cluster lies in flags, between the put-off
+        // walks of the core count and those of the border pass
+        unsigned long long* cluster_keys = reinterpret_cast<unsigned long long*>(flags);
         tm.mark(M_HOOK0);
-        launch_list_boxes(host_count(nbox), bmincore, blist, &counters[8], bparent, s);
+        launch_list_boxes(host_count(nbox), bmincore, blist, &counters[8], bparent, cluster_keys, s);
         launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &counters[8], bparent, s);
         // (the slot-level union's rsnap is free in box mode: the roots)
         launch_box_roots(host_count(nbox), bmincore, bparent, compmin, rsnap, &counters[9], s);
@@ -694,11 +697,12 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         unsigned long long cap = static_cast<unsigned long long>(nn);
         if (ctx.open_pair_limit > 0 && ctx.open_pair_limit < cap) cap = ctx.open_pair_limit;
         launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &counters[8],
-                               host_count(m), rsnap, &counters[10], box_of_slot, reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,
-                               &dstats[5], s);
+                               host_count(m), rsnap, &counters[10], box_of_slot,
+                               reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,
+                               &dstats[5], hc[12] > 0, s);
         tm.mark(M_JOIN1);
         launch_box_clusters(host_count(nbox), bmincore, bcell, cbox, bstart, inrow_of_slot, ustart,
-                            bparent, reinterpret_cast<unsigned long long*>(scratch64), compmin,
+                            bparent, cluster_keys, compmin,
                             bcluster, s);
     } else {
         if (boxes) {
@@ -870,7 +874,7 @@ enum StaticSlot : int {
     SS_NLIST = 8,      // boxes with cores
     SS_JOIN = 9,       // roots of the hook forest
     SS_MIXED = 10,     // boxes of cells next to several trees
-    SS_LARGE = 11,     // (boxes above a size: not counted here)
+    SS_LARGE = 11,     // and 12 (boxes above a size: not used here)
     SS_NONFINITE = 14, // non-finite coordinates
     SS_GRID = 15,      // grid beyond 64 key bits
     SS_BITS = 16,      // key bits + sub-box bits
@@ -1039,8 +1043,9 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     launch_core<T, D>(a, core, ctx.count_tests ? &dstats[7] : nullptr, s);
 
     // the box union (its result is discarded when a box is loose)
+    unsigned long long* cluster_keys = reinterpret_cast<unsigned long long*>(flags);
     int32_t* blist = parent;
-    launch_list_boxes(NB, bmincore, blist, &sc[SS_NLIST], bparent, s);
+    launch_list_boxes(NB, bmincore, blist, &sc[SS_NLIST], bparent, cluster_keys, s);
     launch_box_hook<T, D>(ba, nranges, rboxes, bmincore, core, blist, &sc[SS_NLIST], bparent, s);
     launch_box_roots(NB, bmincore, bparent, compmin, roots, &sc[SS_JOIN], s);
     launch_box_root_join<T, D>(ba, nranges, rboxes, compmin, core, roots, &sc[SS_JOIN], bparent, s);
@@ -1048,9 +1053,9 @@ static void static_body(Context& ctx, const T* pts, int64_t n, JobParams<T>* job
     launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &sc[SS_NLIST], M, roots,
                            &sc[SS_MIXED], box_of_slot,
                            reinterpret_cast<int2*>(scratch64), &dstats[15],
-                           static_cast<unsigned long long>(nn), bparent, &dstats[5], s);
+                           static_cast<unsigned long long>(nn), bparent, &dstats[5], true, s);
     launch_box_clusters(NB, bmincore, bcell, cbox, bstart, inrow_of_slot, ustart, bparent,
-                        reinterpret_cast<unsigned long long*>(scratch64), compmin, bcluster, s);
+                        cluster_keys, compmin, bcluster, s);
 
     // the rows of full boxes labelled in input order when the keys fit the
     // table (in the sort's spare key buffer), the other cores in slot order
