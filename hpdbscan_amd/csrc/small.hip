@@ -1,7 +1,7 @@
 // Clustering of small inputs by comparing all pairs of rows.
 //
-// The general path takes some 55 launches and four read-backs whatever the
-// size: 1000 rows took 263 us, of which no kernel did work worth a launch.
+// The general path takes some 35 launches and four read-backs whatever the
+// size: 2000 rows take 194 us, of which no kernel does work worth a launch.
 // Without a sort and an index five kernels do (a row's sorted position is the
 // number of rows with a smaller (cell, row), its candidates are the rows
 // whose cell differs by at most one in every dimension):
@@ -490,11 +490,21 @@ __global__ __launch_bounds__(kLabelThreads) void k_small_label(int32_t n, SmallL
 
 }  // namespace
 
-// All pairs against the general path, us (3-D float, blobs of 150 rows): 1000
-// rows 55 / 263, 6000 147 / 340, 9000 245 / 370; the densest 2-D data measured
-// meets it at 8000 rows.  From 5-D on the general path's neighbourhoods grow
-// with 3^D (6-D, 12000 rows: 471 / 590 and, dense, 590 / 850).
-int64_t small_rows(int d) { return d <= 4 ? 6000 : 12000; }
+// All pairs against the general path, us, clouds of 60 blobs and (dense) of 5:
+// 3-D float 2000 rows 69 / 194 and 91 / 214, 6000 148 / 211 and 170 / 196, 9000
+// 242 / 228 and 282 / 197; 2-D 6000 155 / 213 and 192 / 202.  From 5-D on the
+// general path's neighbourhoods grow with 3^D: 6-D double 6000 187 / 295 and
+// 238 / 307, 9000 328 / 330 and 387 / 337; 8-D float 12000 477 / 903 and 643 /
+// 721 (5-D and 7-D: between).
+int64_t small_rows(int d) {
+    switch (d) {
+        case 5: return 7000;
+        case 6: return 8000;
+        case 7: return 10000;
+        case 8: return 12000;
+        default: return 6000;
+    }
+}
 
 template <typename T, int D>
 size_t small_workspace_bytes(int64_t n) {

@@ -26,7 +26,7 @@ struct SmallResult {
 };
 
 // Most rows of a small run.  All pairs of rows are compared, so the time grows
-// with their square; the general path costs some 55 launches whatever the
+// with their square; the general path costs some 35 launches whatever the
 // size.
 int64_t small_rows(int d);
 
