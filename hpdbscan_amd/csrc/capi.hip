@@ -221,15 +221,12 @@ struct Context {
     Arena* main_use = &main;
     Arena* aux_use = &aux;
     int border_rule = HPD_BORDER_MIN_CLUSTER;
-    // box mode: cells with at most this many rows are handled one thread
-    // per row in the border pass (and in the core count if sparse_core),
-    // the others one wave per 64-row chunk (hpd_context_set_work_split;
-    // defaults picked by hpdbscan_amd.autotune on the 10M x 3-D workload)
+    // hpd_context_set_work_split: kept for its getter
     int32_t sparse_max = 8;
     // sub-boxes per cell and dimension (hpd_context_set_box_split; 0: 2 up
     // to 3-D, 3 above, which keeps every sub-box's diagonal below eps)
     int32_t box_split = 0;
-    uint64_t open_pair_limit = 0;  // 0: 2n
+    uint64_t open_pair_limit = 0;  // 0: one entry per row
     bool sparse_core = false;
     bool timing = false;
     bool count_tests = false;  // hpd_context_set_timing level 2
@@ -582,11 +579,12 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         boxes ? static_cast<size_t>(m) + nn / kWaveRows + 1 : static_cast<size_t>(hc[2]);
 
     const size_t range_bytes = align_up(static_cast<size_t>(total_ranges) * sizeof(int2), 256);
-    X.reserve((boxes ? range_bytes : 0) + (row_tables ? 2 * range_bytes : 0) +
+    // (the cell ranges take the box ranges' place when they are made)
+    X.reserve((boxes ? range_bytes : 0) + (row_tables ? (boxes ? 1 : 2) * range_bytes : 0) +
               (row_tables ? align_up(max_items * sizeof(int2), 256) : 0) + 2048);
     int2* rboxes = boxes ? X.take_n<int2>(total_ranges) : nullptr;
     int2* ranges = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
-    int2* rcells = row_tables ? X.take_n<int2>(total_ranges) : nullptr;
+    int2* rcells = !row_tables ? nullptr : boxes ? rboxes : X.take_n<int2>(total_ranges);
     int2* items = row_tables ? X.take_n<int2>(max_items) : nullptr;
     if (boxes && stash)
         launch_neighbor_copy(stash, max_rows, m, nranges, cbox, rboxes, rcenter, by_class, s);
@@ -657,7 +655,8 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         }
     }
     // box mode: the row-level tables when they turn out to be needed (the
-    // neighbour rows ascending again, their own-row index with them)
+    // neighbour rows ascending again, their own-row index with them); the box
+    // ranges are gone after it, no kernel on boxes follows
     auto fill_row_tables = [&] {
         launch_chunk_counts(ustart, host_count(m), nchunks, s);
         exclusive_scan_u32(nchunks, nchunks, m, tmp, &nchunks[m], s);

@@ -20,7 +20,6 @@
 // save more there but leave too few blocks to hide a tile's chain of barriers
 // (100M rows, 2 passes, sort phase in ms by the blocks left: 2048 4.05, 4096
 // 4.10, 8192 3.93, 16384 3.87, all 48828 3.98).
-#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -60,8 +59,10 @@ struct SortPlan {
     int run;
     bool self;
 };
-inline SortPlan sort_plan(int64_t n, int max_iters) {
-    int iters = kItersMin;
+// (9-bit digits from 2048 keys on: half the blocks, so that no plan needs more
+// histogram words than kMaxBuckets per 2048 keys)
+inline SortPlan sort_plan(int64_t n, int max_iters, int bits) {
+    int iters = bits > 8 ? 2 * kItersMin : kItersMin;
     while (iters < max_iters && tiles_of(n, kThreads * iters) > kSelfBlocks) iters *= 2;
     const int64_t tiles = tiles_of(n, kThreads * iters);
     const int64_t run = tiles_of(tiles, kRunBlocks);
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_settle(K* __restrict__ keys_
 template <typename K, int kBits>
 bool sort_passes(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n, int bits,
                  uint32_t* hist, uint32_t* tmp, hipStream_t s, const int* bits_dev = nullptr) {
-    const SortPlan plan = sort_plan(n, kIters);
+    const SortPlan plan = sort_plan(n, kIters, kBits);
     const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
@@ -411,7 +412,7 @@ template <typename K, int kBits, typename T, int D>
 bool sort_passes_rows(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, int64_t n,
                       int bits, uint32_t* hist, uint32_t* tmp, const T* pts, T* rows_a,
                       T* rows_b, T* soa, int64_t ld, hipStream_t s) {
-    const SortPlan plan = sort_plan(n, kItersRows);
+    const SortPlan plan = sort_plan(n, kItersRows, kBits);
     const dim3 grid(static_cast<unsigned>(plan.blocks));
     K* kin = keys_a;
     uint32_t* vin = vals_a;
@@ -457,11 +458,8 @@ int radix_pass_count(int bits) {
 }
 
 size_t radix_hist_words(int64_t n) {
-    const int64_t k = n > 0 ? n : 1;
-    // (a bound that grows with n over the plans of all tile sizes)
-    const int64_t blocks = std::max(tiles_of(k, kThreads * kItersRows),
-                                    std::min(kSelfBlocks, tiles_of(k, kThreads * kItersMin)));
-    return static_cast<size_t>(kMaxBuckets) * static_cast<size_t>(blocks);
+    return static_cast<size_t>(kMaxBuckets) *
+           static_cast<size_t>(tiles_of(n > 0 ? n : 1, kThreads * kItersRows));
 }
 
 // 9-bit digits where they save a pass (e.g. 25-27 key bits: 3 passes, not 4)
