@@ -57,42 +57,40 @@ PEAK_HBM_GBS = 8000.0  # MI355X HBM3E
 # The kernels that compare rows with their neighbours, keyed by the
 # per-kernel time the library reports (HIP events on its stream).
 PAIR_KERNELS = {
-    "ms_core_kernel": "k_core_boxes",
-    "ms_hook_kernel": "k_box_hook+k_box_hook_small",
-    "ms_union_kernel": "k_box_scan+k_box_union_list+k_box_union",
-    "ms_border_kernel": "k_border_boxes+k_border_sparse",
+    "ms_core_kernel": "k_core_rows+k_core_heavy",
+    "ms_hook_kernel": "k_box_link+k_box_roots+k_list_boxes",
+    "ms_union_kernel": "k_mixed_cells+k_box_union+k_box_union_heavy",
+    "ms_border_kernel": "k_border_rows+k_border_heavy",
 }
 
 
 def compulsory_bytes(kernel: str, st: dict, n: int, d: int, s: int) -> int:
     """Bytes a kernel must move at least once: every array it reads, once,
     and every array it writes, once (n rows, D dims, s-byte values, nb boxes,
-    m occupied cells, R neighbour rows).
+    m occupied cells, R neighbour rows; the rows are those that are not core,
+    which every one of the row kernels has to look at, a lower bound).
 
-      k_core_boxes    rows n*D*s, box of row n*4, core flag written n;
-                      per box first row 4, bounding box 2*D*s, flags 1;
-                      per cell first row, ranges offset, own row, job (16);
-                      per neighbour row its cells (8)
-      k_box_hook*     (the hook forest) rows n*D*s, core flag n; per box
-                      first row, cell, smallest core, parent written (16) +
-                      bounding box; per cell ranges offset, first box, job
-                      (12); 8 per row
-      k_box_scan*     (the open-pair union) as the hook forest plus the
-                      hook roots (4 per box)
-      k_border_*      rows n*D*s, core flag n, input row 4n, box of row 4n,
-                      labels written 8 per non-core row; per box first row,
-                      cluster, cell (12) + bounding box; per cell 16; 8 per
-                      neighbour row
+      k_core_rows     per non-core row its values, box and flag; per box first
+                      row, flags (8), bounding box; per cell ranges offset, own
+                      row, first box, job (16); per neighbour row its boxes (8)
+      k_box_link      (the hook forest, its roots and joins) per box first row,
+                      cell, smallest core, parent, root (20) + bounding box; per
+                      cell ranges offset, first box, job (12); 8 per row
+      k_mixed_cells   (and the exact union) per box its root (4); per cell
+                      ranges offset, first box (8); 8 per neighbour row
+      k_border_rows   per non-core row its entry (8), values, input row, label
+                      (12); per box first row, cluster (8) + bounding box; per
+                      cell 16; 8 per neighbour row
     """
     nb, m, r = int(st["boxes"]), int(st["occupied_cells"]), int(st["neighbor_rows"])
     noncore = n - int(st["core_points"])
-    if kernel == "k_core_boxes":
-        return n * (d * s + 5) + nb * (2 * d * s + 5) + m * 16 + r * 8
-    if kernel.startswith("k_box_hook"):
-        return n * (d * s + 1) + nb * (2 * d * s + 16) + m * 12 + r * 8
-    if kernel.startswith("k_box_scan"):
-        return n * (d * s + 1) + nb * (2 * d * s + 20) + m * 12 + r * 8
-    return n * (d * s + 9) + 8 * noncore + nb * (2 * d * s + 12) + m * 16 + r * 8
+    if kernel.startswith("k_core_rows"):
+        return noncore * (d * s + 5) + nb * (2 * d * s + 8) + m * 16 + r * 8
+    if kernel.startswith("k_box_link"):
+        return nb * (2 * d * s + 20) + m * 12 + r * 8
+    if kernel.startswith("k_mixed_cells"):
+        return nb * 4 + m * 8 + r * 8
+    return noncore * (d * s + 20) + nb * (2 * d * s + 8) + m * 16 + r * 8
 
 
 def measured_traffic(workload: str, kernel: str):

@@ -226,13 +226,14 @@ class Context:
         check(load().hpd_context_set_border_rule(self._h, rule))
 
     def set_work_split(self, sparse_max: int, sparse_core: bool = False) -> None:
-        """Cells with at most sparse_max rows go one thread per row (border
-        pass; core count too with sparse_core).  Results do not change."""
+        """Checked and kept (work_split()); the kernels split their work by
+        box, so neither results nor speed change."""
         check(load().hpd_context_set_work_split(self._h, int(sparse_max), 1 if sparse_core else 0))
 
     def set_open_pair_limit(self, limit: int) -> None:
-        """Most open box pairs the union lists hold (0: 2n); beyond it the
-        union walks every box's neighbourhood.  Results do not change."""
+        """Most list entries for the parts of large boxes' pairs in the union
+        (0: one per row); beyond it they are tested in place.  Results do not
+        change."""
         check(load().hpd_context_set_open_pair_limit(self._h, int(limit)))
 
     def set_box_split(self, parts: int) -> None:

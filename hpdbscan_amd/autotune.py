@@ -10,9 +10,9 @@ Two settings change the speed of a run and never its labels:
   distance tests.  More parts give tighter boxes (more groups decided
   without row tests) at the price of more boxes to walk and more key bits
   to sort;
-* the work split (hpd_context_set_work_split): the core count and the
-  border pass run one 64-lane wavefront per 64-row chunk of a dense cell
-  and one thread per row of a sparse cell; the line between the two.
+* the work split (hpd_context_set_work_split): kept for callers that store
+  tuned settings; the kernels split their work by box, so its candidates
+  differ by noise only.
 
 Where each pays off depends on the data (density spread, D, eps), so this
 module times candidates on the GPU for a given workload: first the box
@@ -21,8 +21,8 @@ fastest box split.  Every candidate must reproduce the first candidate's
 labels exactly; a mismatch raises.  `apply` sets a tuned result on a
 Context.
 
-The library's defaults (box split 2 up to 3-D, sparse_max 8, core count not
-split) are what this tuner picks on the 10M x 3-D workload.
+The library's default box split (2 up to 3-D) is what this tuner picks on the
+10M x 3-D workload.
 """
 from __future__ import annotations
 

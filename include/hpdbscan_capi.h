@@ -132,28 +132,24 @@ int hpd_context_get_stats(const hpd_context* ctx, hpd_run_stats* out);
  * replayed by later calls with the same shape (dtype, d, rows, job offsets,
  * data and label buffers, options); eps, minPts and the data itself may
  * change.  The labels are identical to the plain pipeline's.  It uses more
- * device memory (about 3^(d-1) * 16 + 260 bytes per row) and falls back to
- * the plain pipeline, transparently, for loose sub-boxes, grids beyond 64
- * key bits or too many open box pairs; non-finite input then fails as
- * usual.  Disabling it frees the graph. */
+ * device memory (about 3^(d-1) * 8 + 260 bytes per row) and falls back to
+ * the plain pipeline, transparently, for loose sub-boxes or grids beyond 64
+ * key bits; non-finite input then fails as usual.  Disabling it frees the graph. */
 int hpd_context_set_graph(hpd_context* ctx, int enabled);
 /* Graph launches, captures and fallbacks to the plain pipeline so far. */
 int hpd_context_get_graph_stats(const hpd_context* ctx, uint64_t* launches, uint64_t* captures,
                                 uint64_t* fallbacks);
 
-/* Work split of the neighbour kernels on sub-boxes (floating-point data):
- * cells with at most sparse_max rows (0..64) are processed one GPU thread
- * per row in the border pass, and in the core count too when sparse_core is
- * nonzero; other cells one 64-lane wavefront per 64-row chunk.  Results do
- * not depend on it; hpdbscan_amd.autotune picks it for a workload.  No
+/* Work split of the neighbour kernels: sparse_max in 0..64, checked and kept
+ * for the getter.  The kernels take chunks of rows of one box by groups of
+ * lanes, whatever the cells' sizes, so it changes neither results nor speed.  No
  * counterpart in the reference (OpenMP schedule(dynamic, 32), hpdbscan.h:65). */
 int hpd_context_set_work_split(hpd_context* ctx, int32_t sparse_max, int sparse_core);
 int hpd_context_get_work_split(const hpd_context* ctx, int32_t* sparse_max, int* sparse_core);
 
-/* Most box pairs the union keeps in its open-pair lists (0: the default,
- * 2n for n rows, which the lists' memory holds).  When a run has more, the
- * union walks every box's neighbourhood instead (decided on the device).
- * Results do not depend on it.  No counterpart in the reference. */
+/* Most entries of the list in which the union keeps the pairs of large boxes
+ * by parts (0, and the most: n for n rows).  Pairs that do not fit are tested
+ * in place (decided on the device).  Results do not depend on it.  No counterpart in the reference. */
 int hpd_context_set_open_pair_limit(hpd_context* ctx, uint64_t limit);
 
 /* Sub-boxes per cell and dimension (the tile of the pair kernels): each
