@@ -174,11 +174,12 @@ __device__ __forceinline__ int32_t heavy_count(const DbscanArgs<T>& a) {
 // of such a box leaves an entry per kHeavyWalk of its rows for k_core_heavy:
 // one wave takes 0.4 us per 256 rows, 8 ms for a box of five million.  A
 // variant of its own, since the code costs scalar registers (4096 clouds of 8k
-// rows: 5.3 ms without, 9.0 ms with it).
+// rows: 5.3 ms without, 9.0 ms with it).  Float rows up to 3-D fit 8 waves per
+// SIMD (64 VGPRs, nothing spilled): the same clouds 5.35 ms at 7 waves, 4.95 at 8.
 template <typename T, int D, bool kCount, bool kHeavy>
-__global__ __launch_bounds__(kThreads) void k_core_rows(const DbscanArgs<T> a,
-                                                        uint8_t* __restrict__ core,
-                                                        unsigned long long* __restrict__ ntests) {
+__global__ __launch_bounds__(kThreads, D <= 3 && sizeof(T) == 4 && !kCount ? 8 : 1)
+void k_core_rows(const DbscanArgs<T> a, uint8_t* __restrict__ core,
+                 unsigned long long* __restrict__ ntests) {
     constexpr int G = kGroup<D>;
     constexpr int kPer = 64 / G;  // chunks of a wave
     __shared__ T rows_lds[kWavesPerBlock][64][D];
@@ -686,10 +687,13 @@ __device__ __forceinline__ unsigned int border_label(bool on, int32_t p, int32_t
 // a.slot_b, k_border_heavy adds the parts' and k_border_late labels the row.
 // Lanes per row (ms by lanes: 5M rows of 4 (16) 0.256, (32) 0.241, (64) 0.302;
 // 30k of 6 doubles (16) 0.079, (32) 0.053, (64) 0.040).
+// Float rows up to 3-D run at 7 waves per SIMD (4096 clouds of 8k rows: 6 waves
+// 2.38 ms, 7 2.16, 8 2.24; 10M rows 101 us, 98, 114).
 template <int D>
 constexpr int kBorderGroup = D <= 3 ? 8 : D == 4 ? 32 : 64;
 template <typename T, int D, bool kHeavy>
-__global__ __launch_bounds__(kThreads) void k_border_rows(
+__global__ __launch_bounds__(kThreads, D <= 3 && sizeof(T) == 4 && !kHeavy ? 7 : 1)
+void k_border_rows(
     const DbscanArgs<T> a, const uint8_t* __restrict__ core, const int32_t* __restrict__ bcluster,
     const int2* __restrict__ rows, const unsigned int* __restrict__ nrows_dev,
     int64_t* __restrict__ labels, unsigned long long* __restrict__ stats,
