@@ -43,6 +43,7 @@
 #include "dbscan.hpp"
 #include "grid.hpp"
 #include "internal.hpp"
+#include "put_off.hpp"
 #include "visit.hpp"
 
 namespace hpd {
@@ -802,8 +803,7 @@ __global__ __launch_bounds__(kThreads) void k_border_heavy(const DbscanArgs<T> a
         const int32_t cl = uniform(bcluster[b2]);
         const int32_t best = uniform(ld_agent(&a.slot_a[p]));
         const int32_t worst = uniform(ld_agent(&a.slot_b[p]));
-        // nothing new: between the two, or beyond two that differ already
-        if ((cl >= best && cl <= worst) || (cl > best && best != worst)) continue;
+        if (cluster_settled(best, worst, cl)) continue;
         const int32_t q1 = min(q0 + kHeavyWalk, uniform(a.bstart[b2 + 1]));
         const T eps2 = a.jobs[uniform(a.job_of_cell[uniform(a.bcell[b2])])].eps2;
         T pc[D];
