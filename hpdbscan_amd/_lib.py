@@ -231,9 +231,9 @@ class Context:
         check(load().hpd_context_set_work_split(self._h, int(sparse_max), 1 if sparse_core else 0))
 
     def set_open_pair_limit(self, limit: int) -> None:
-        """Most list entries for the parts of large boxes' pairs in the union
-        (0: one per row); beyond it they are tested in place.  Results do not
-        change."""
+        """Most list entries for the parts of large boxes in the core count, the
+        union and the border pass (0: one per row); what is beyond it is done in
+        place.  Results do not change."""
         check(load().hpd_context_set_open_pair_limit(self._h, int(limit)))
 
     def set_box_split(self, parts: int) -> None:

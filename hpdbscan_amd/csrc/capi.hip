@@ -227,6 +227,10 @@ struct Context {
     // to 3-D, 3 above, which keeps every sub-box's diagonal below eps)
     int32_t box_split = 0;
     uint64_t open_pair_limit = 0;  // 0: one entry per row
+    // entries of a list of put-off work of a run of n rows
+    unsigned long long put_off_cap(uint64_t n) const {
+        return open_pair_limit > 0 && open_pair_limit < n ? open_pair_limit : n;
+    }
     bool sparse_core = false;
     bool timing = false;
     bool count_tests = false;  // hpd_context_set_timing level 2
@@ -647,7 +651,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         if (hc[11] > 0) {  // boxes of millions of rows: their walks in parts
             a.heavy = reinterpret_cast<int2*>(flags);
             a.nheavy = &dstats[16];
-            a.heavy_cap = static_cast<unsigned long long>(nn);
+            a.heavy_cap = ctx.put_off_cap(nn);
             a.slot_a = parent;  // free before and after the union
             a.slot_b = rsnap;
             a.late = cmin;
@@ -693,8 +697,7 @@ static void run_keyed(Context& ctx, const T* pts, int64_t n, JobParams<T>* jobs,
         launch_box_roots(host_count(nbox), bmincore, bparent, compmin, nullptr, nullptr, s);
         tm.mark(M_HOOK1);
         // pairs with a large box go through a list in scratch64
-        unsigned long long cap = static_cast<unsigned long long>(nn);
-        if (ctx.open_pair_limit > 0 && ctx.open_pair_limit < cap) cap = ctx.open_pair_limit;
+        const unsigned long long cap = ctx.put_off_cap(nn);
         launch_box_union<T, D>(ba, nranges, rboxes, compmin, core, blist, &counters[8],
                                host_count(m), rsnap, &counters[10], box_of_slot,
                                reinterpret_cast<int2*>(scratch64), &dstats[15], cap, bparent,

@@ -147,9 +147,10 @@ int hpd_context_get_graph_stats(const hpd_context* ctx, uint64_t* launches, uint
 int hpd_context_set_work_split(hpd_context* ctx, int32_t sparse_max, int sparse_core);
 int hpd_context_get_work_split(const hpd_context* ctx, int32_t* sparse_max, int* sparse_core);
 
-/* Most entries of the list in which the union keeps the pairs of large boxes
- * by parts (0, and the most: n for n rows).  Pairs that do not fit are tested
- * in place (decided on the device).  Results do not depend on it.  No counterpart in the reference. */
+/* Most entries of a list in which the core count, the union and the border
+ * pass keep their work on large boxes by parts (0, and the most: n for n rows).
+ * What does not fit is done in place (decided on the device).  Results do not
+ * depend on it.  No counterpart in the reference. */
 int hpd_context_set_open_pair_limit(hpd_context* ctx, uint64_t limit);
 
 /* Sub-boxes per cell and dimension (the tile of the pair kernels): each

@@ -201,3 +201,27 @@ def test_put_off_borders_of_two_clusters(crowds, d, dtype, rule):
             assert st["noise_points"] == int((want == 0).sum())
     finally:
         ctx.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("limit", [1, 2, 5, 101])
+@pytest.mark.parametrize("d,dtype", CASES)
+def test_lists_that_overflow(crowds, d, dtype, limit):
+    """The lists of put-off walks cut short: walks in place (1 holds no box of
+    two parts), partly filled ranges, and rows with one crowd's walk put off and
+    the other's in place, in the core count and in the border pass."""
+    from hpdbscan_amd import BORDER_ONE_THREAD, _lib
+    x, _, r = crowds(d, dtype)
+    ctx = _lib.Context(0)
+    try:
+        ctx.set_open_pair_limit(limit)
+        for rule, want in ((0, min_rule(r, x)), (BORDER_ONE_THREAD, r["labels"])):
+            print(f"[gpu-case] two crowds d={d} {np.dtype(dtype).name} limit={limit} rule={rule}",
+                  flush=True)
+            ctx.set_border_rule(rule)
+            np.testing.assert_array_equal(ctx.cluster(x, EPS, MIN_POINTS), want)
+            st = ctx.stats()
+            assert st["ambiguous_borders"] == int(r["ambiguous"].sum())
+            assert st["core_points"] == int(r["core"].sum())
+    finally:
+        ctx.close()
