@@ -1280,8 +1280,9 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     }
     if constexpr (std::is_floating_point<T>::value) {
         // few rows: all pairs compared (the timing marks and the executed
-        // tests are the general path's)
-        if (njobs == 1 && n <= small_rows(D) && !ctx.timing &&
+        // tests are the general path's; a fixed workspace turns the marks off,
+        // not the tests)
+        if (njobs == 1 && n <= small_rows(D) && !ctx.timing && !ctx.count_tests &&
             run_small<T, D>(ctx, pts, n, eps[0], min_pts[0], labels, s))
             return;
     }

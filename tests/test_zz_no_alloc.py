@@ -103,3 +103,21 @@ def test_noalloc_rejects_inputs_beyond_the_scratch():
         xd.close()
         out.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("n", [800, 6000, 20_000])
+def test_noalloc_counts_executed_tests(n):
+    """Timing level 2: the executed distance tests are counted for inputs of
+    every size, those that all pairs would be compared of among them."""
+    from hpdbscan_amd import _lib
+    x = blobs(n, 3, 8, 0.3, 5.0, 11)
+    ctx = _lib.Context(0)
+    try:
+        ctx.set_timing(2)
+        say(f"noalloc executed tests n={n}")
+        want, got, sw, sg, _, _ = run_both(ctx, x, 0.3, 8)
+        np.testing.assert_array_equal(got, want)
+        assert 0 < sw["core_tests"] < sw["sum_candidates"]
+        assert 0 < sg["core_tests"] < sg["sum_candidates"]
+    finally:
+        ctx.close()
