@@ -223,6 +223,7 @@ struct Context {
     int border_rule = HPD_BORDER_MIN_CLUSTER;
     // hpd_context_set_work_split: kept for its getter
     int32_t sparse_max = 8;
+    bool sparse_core = false;
     // sub-boxes per cell and dimension (hpd_context_set_box_split; 0: 2 up
     // to 3-D, 3 above, which keeps every sub-box's diagonal below eps)
     int32_t box_split = 0;
@@ -231,7 +232,6 @@ struct Context {
     unsigned long long put_off_cap(uint64_t n) const {
         return open_pair_limit > 0 && open_pair_limit < n ? open_pair_limit : n;
     }
-    bool sparse_core = false;
     bool timing = false;
     bool count_tests = false;  // hpd_context_set_timing level 2
     hpd_run_stats stats{};
@@ -244,9 +244,8 @@ struct Context {
     bool graph = false;
     struct GraphEntry {
         hipGraphExec_t exec = nullptr;
-        int dtype = -1, d = 0, border_rule = -1, sparse_max = -1, box_split = -1;
+        int dtype = -1, d = 0, border_rule = -1, box_split = -1;
         bool count_tests = false;
-        bool sparse_core = false;
         int64_t n = 0;
         const void* data = nullptr;
         const void* labels = nullptr;
@@ -1142,7 +1141,6 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
     const bool same = ge.exec && ge.dtype == dtype && ge.d == D && ge.n == n && ge.data == pts &&
                       ge.labels == labels && ge.arena_main == A.base() &&
                       ge.arena_aux == ctx.aux.base() && ge.border_rule == ctx.border_rule &&
-                      ge.sparse_max == ctx.sparse_max && ge.sparse_core == ctx.sparse_core &&
                       ge.box_split == ctx.box_split && ge.count_tests == ctx.count_tests &&
                       ge.offsets.size() == static_cast<size_t>(njobs) + 1 &&
                       std::equal(ge.offsets.begin(), ge.offsets.end(), offsets);
@@ -1173,10 +1171,8 @@ static bool run_static(Context& ctx, int dtype, const T* pts, int64_t n, const i
         ge.arena_main = A.base();
         ge.arena_aux = ctx.aux.base();
         ge.border_rule = ctx.border_rule;
-        ge.sparse_max = ctx.sparse_max;
         ge.box_split = ctx.box_split;
         ge.count_tests = ctx.count_tests;
-        ge.sparse_core = ctx.sparse_core;
         ge.offsets.assign(offsets, offsets + njobs + 1);
         ++ctx.graph_captures;
     }

@@ -180,3 +180,31 @@ def test_graph_sparse_rows_beyond_the_likely_grid(plain, graph, split):
     finally:
         xd.close()
         ld.close()
+
+
+def test_graph_settings_that_make_a_new_capture(plain, graph):
+    """The box split changes what the captured kernels do and makes a new capture;
+    the work split, which no kernel reads, does not."""
+    from hpdbscan_amd import _lib
+    rng = np.random.default_rng(22)
+    x = rng.uniform(0, 20.0, (20_000, 2)).astype(np.float32)
+    want = plain.cluster(x, 0.15, 4)
+    assert oracle.check(x, 0.15, 4, want) == (0, 0)
+    xd = _lib.DeviceBuffer.from_array(graph, x)
+    ld = _lib.DeviceBuffer(graph, 8 * len(x))
+    try:
+        captures = []
+        for split, box in [((8, False), 0), ((16, True), 0), ((0, False), 0), ((0, False), 3),
+                           ((8, False), 3)]:
+            say(f"graph work split {split} box split {box}")
+            graph.set_work_split(*split)
+            assert graph.work_split() == split
+            graph.set_box_split(box)
+            graph.cluster_device(xd.ptr, len(x), 2, np.float32, 0.15, 4, ld.ptr)
+            np.testing.assert_array_equal(ld.to_array(np.int64, len(x)), want)
+            captures.append(graph.graph_stats()["captures"])
+        assert captures == [1, 1, 1, 2, 2]
+        assert graph.graph_stats()["fallbacks"] == 0
+    finally:
+        xd.close()
+        ld.close()
