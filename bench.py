@@ -23,7 +23,7 @@ The JSON line also carries
   batched       the batched workload (4096 clouds, 1k-200k rows each) in one
                 hpd_cluster_batch_device call vs a loop of one call per
                 cloud: jobs/s of both, per-call p50/p99 of the loop, and
-                equality of the labels; the work split of both comes from
+                equality of the labels; the box split of both comes from
                 hpdbscan_amd.autotune run on the batch first; graph_* is the
                 same batch through the static pipeline captured once in a
                 hipGraph and replayed (hpd_context_set_graph)
@@ -211,14 +211,14 @@ def batched_leg(a) -> dict:
     print(f"[bench] batched: {nj} clouds, {len(rows)} rows (generated in {time.time() - t0:.1f}s)",
           file=sys.stderr, flush=True)
     ctx = _lib.Context(0)
-    # the work split comes from the autotuner, run on this batch (every
+    # the box split comes from the autotuner, run on this batch (every
     # candidate must give the same labels); the plain loop uses it too
     t0 = time.time()
     tuned = autotune.tune_batch(rows, off, eps, mps, ctx=ctx, reps=1) if a.autotune else None
     if tuned:
         autotune.apply(ctx, tuned)
-        print(f"[bench] batched: work split {tuned['best']} (autotuned in {time.time() - t0:.1f}s)",
-              file=sys.stderr, flush=True)
+        print(f"[bench] batched: box split {tuned['best']['box_split']} "
+              f"(autotuned in {time.time() - t0:.1f}s)", file=sys.stderr, flush=True)
     xd = _lib.DeviceBuffer.from_array(ctx, rows)
     ld = _lib.DeviceBuffer(ctx, 8 * len(rows))
     # warm up both paths (allocations)
@@ -237,7 +237,6 @@ def batched_leg(a) -> dict:
     graph = {}
     if a.graph:
         gctx = _lib.Context(0)
-        gctx.set_work_split(*ctx.work_split())
         gctx.set_box_split(ctx.box_split())
         gctx.set_graph(True)
         gl = _lib.DeviceBuffer(gctx, 8 * len(rows))
@@ -291,8 +290,7 @@ def batched_leg(a) -> dict:
         "batched_latency_ms": round(t_batch * 1e3, 2),
         "speedup_jobs_per_s": round(t_plain / t_batch, 2),
         "labels_equal": equal,
-        "work_split": tuned["best"] if tuned else {"box_split": 0, "sparse_max": 8,
-                                                   "sparse_core": False},
+        "box_split": tuned["best"]["box_split"] if tuned else 0,
         "note": "device-resident rows; a batched job's latency is the whole batch's",
         **graph,
     }
@@ -614,7 +612,7 @@ def main() -> None:
     ap.add_argument("--no-graph", dest="graph", action="store_false",
                     help="batched leg: skip the hipGraph-captured static pipeline")
     ap.add_argument("--no-autotune", dest="autotune", action="store_false",
-                    help="batched leg: library default work split instead of the autotuned one")
+                    help="batched leg: library default box split instead of the autotuned one")
     ap.add_argument("--no-serving", action="store_true")
     ap.add_argument("--serve-requests", type=int, default=400)
     ap.add_argument("--serve-rate", type=float, default=200.0)

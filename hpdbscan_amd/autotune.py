@@ -1,25 +1,22 @@
-"""Autotuner of the pair kernels' tile and work split.
+"""Autotuner of the pair kernels' tile.
 
     python -m hpdbscan_amd.autotune [--workload blobs_10m] [--n N] [--reps 3]
                                     [--batch] [--out split.json]
 
-Two settings change the speed of a run and never its labels:
+One setting changes the speed of a run and never its labels: the box split
+(hpd_context_set_box_split).  Every eps-cell is cut into parts^d sub-boxes, the
+tiles whose bounding boxes decide whole groups of distance tests.  More parts
+give tighter boxes (more groups decided without row tests) at the price of more
+boxes to walk and more key bits to sort.
 
-* the box split (hpd_context_set_box_split): every eps-cell is cut into
-  parts^d sub-boxes, the tiles whose bounding boxes decide whole groups of
-  distance tests.  More parts give tighter boxes (more groups decided
-  without row tests) at the price of more boxes to walk and more key bits
-  to sort;
-* the work split (hpd_context_set_work_split): kept for callers that store
-  tuned settings; the kernels split their work by box, so its candidates
-  differ by noise only.
+Where that pays off depends on the data (density spread, D, eps), so this module
+times the box splits on the GPU for a given workload.  Every candidate must
+reproduce the first candidate's labels exactly; a mismatch raises.  `apply` sets
+a tuned result on a Context.
 
-Where each pays off depends on the data (density spread, D, eps), so this
-module times candidates on the GPU for a given workload: first the box
-splits under the library's work split, then the work splits under the
-fastest box split.  Every candidate must reproduce the first candidate's
-labels exactly; a mismatch raises.  `apply` sets a tuned result on a
-Context.
+The work split (hpd_context_set_work_split) has no effect since the kernels split
+their work by box: the result carries its default, and work splits are timed
+only when a caller names some as `candidates`.
 
 The library's default box split (2 up to 3-D) is what this tuner picks on the
 10M x 3-D workload.
@@ -34,7 +31,7 @@ import numpy as np
 
 from . import _lib, datagen
 
-# work splits (sparse_max, sparse_core)
+# work splits (sparse_max, sparse_core) that the setting takes; no kernel reads it
 CANDIDATES = [(0, False), (4, False), (8, False), (16, False), (32, False), (8, True), (16, True)]
 DEFAULT_WORK_SPLIT = (8, False)
 # box splits: 0 is the library's choice for the dimension
@@ -100,6 +97,9 @@ def _two_stage(ctx, run, fetch, reps: int, d: int, candidates) -> dict:
     boxes = _sweep(ctx, run, fetch, reps, [{"box_split": k} for k in box_split_candidates(d)])
     k = boxes["best"]["box_split"]
     ctx.set_box_split(k)
+    if not candidates:
+        return {"best": {"box_split": k, "sparse_max": sm, "sparse_core": sc},
+                "box_split_results": boxes["results"], "results": []}
     works = _sweep(ctx, run, fetch, reps,
                    [{"sparse_max": a, "sparse_core": b} for a, b in candidates], ref=boxes["ref"])
     best = {"box_split": k, **works["best"]}
@@ -107,9 +107,9 @@ def _two_stage(ctx, run, fetch, reps: int, d: int, candidates) -> dict:
 
 
 def tune(data: np.ndarray, eps: float, min_points: int, ctx=None, reps: int = 3,
-         candidates=CANDIDATES) -> dict:
-    """Fastest box split and work split for clustering `data` (2-D array)
-    once."""
+         candidates=()) -> dict:
+    """Fastest box split (and work split, of `candidates`) for clustering `data`
+    (2-D array) once."""
     own = ctx is None
     ctx = ctx or _lib.Context(0)
     a = np.ascontiguousarray(data)
@@ -130,9 +130,9 @@ def tune(data: np.ndarray, eps: float, min_points: int, ctx=None, reps: int = 3,
 
 
 def tune_batch(data: np.ndarray, offsets, eps, min_points, ctx=None, reps: int = 3,
-               candidates=CANDIDATES) -> dict:
-    """Fastest box split and work split for one batched call over the jobs
-    of `offsets`."""
+               candidates=()) -> dict:
+    """Fastest box split (and work split, of `candidates`) for one batched call
+    over the jobs of `offsets`."""
     own = ctx is None
     ctx = ctx or _lib.Context(0)
     a = np.ascontiguousarray(data)

@@ -2,6 +2,8 @@
 the GPU, a real sweep whose candidates must all give equal labels."""
 from __future__ import annotations
 
+import inspect
+
 import numpy as np
 import pytest
 
@@ -73,6 +75,26 @@ def test_two_stage_box_split_then_work_split(monkeypatch):
     calls = iter([np.arange(5)] * 3 + [np.arange(5) + 1])
     with pytest.raises(RuntimeError, match="changed the labels"):
         autotune._two_stage(ctx, lambda: None, lambda: next(calls), 1, 3, [(0, False)])
+
+
+def test_without_candidates_only_box_splits_are_timed(monkeypatch):
+    """No work split is timed unless the caller names some: the result carries
+    the default, and every timed run had it."""
+    ctx = FakeContext(cost={})
+    t = [0.0]
+    seen = []
+    monkeypatch.setattr(autotune.time, "perf_counter", lambda: t[0])
+
+    def run():
+        seen.append((ctx.box, ctx.split))
+        t[0] += {0: 2.0, 3: 1.0, 4: 4.0}[ctx.box]
+
+    for fn in (autotune.tune, autotune.tune_batch):
+        assert inspect.signature(fn).parameters["candidates"].default == ()
+    res = autotune._two_stage(ctx, run, lambda: np.arange(5), 1, 3, ())
+    assert res["best"] == {"box_split": 3, "sparse_max": 8, "sparse_core": False}
+    assert res["results"] == [] and ctx.box == 3
+    assert {split for _, split in seen} == {autotune.DEFAULT_WORK_SPLIT}
 
 
 def test_box_split_candidates():
