@@ -56,16 +56,19 @@ void Arena::reserve(size_t bytes) {
         throw Error(HPD_EUNSUPPORTED, "the run needs " + std::to_string(bytes) +
                                           " bytes of device workspace here; " +
                                           std::to_string(cap_) + " are available");
-    if (base_) {
-        HPD_HIP(hipFree(base_));
-        base_ = nullptr;
-        cap_ = 0;
-    }
+    release();
     const size_t want = align_up(bytes + bytes / 8, size_t(1) << 20);
     void* p = nullptr;
     HPD_HIP(hipMalloc(&p, want));
     base_ = static_cast<char*>(p);
     cap_ = want;
+}
+
+void Arena::release() {
+    if (!base_ || !owned_) return;
+    HPD_HIP(hipFree(base_));
+    base_ = nullptr;
+    cap_ = used_ = 0;
 }
 
 void* Arena::take(size_t bytes) {
@@ -1261,10 +1264,11 @@ static bool float_possible(float eps) {
 
 // A batch of jobs: rows [offsets[j], offsets[j+1]) of `pts` form job j with
 // its own eps[j] and min_pts[j].  A plain call is a batch of one.
+// try_float: integer rows may run as float rows.
 template <typename T, int D>
 static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offsets,
                       int32_t njobs, const float* eps, const uint64_t* min_pts, int64_t* labels,
-                      hipStream_t s) {
+                      hipStream_t s, bool try_float = true) {
     if constexpr (std::is_floating_point<T>::value) {
         // the static pipeline, captured once per shape and replayed; it hands
         // the run back when one of its flags says so
@@ -1289,7 +1293,7 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
     bool as_float = false;  // integer rows: room for them as float rows
     if constexpr (std::is_integral<T>::value) {
         // (not in a fixed workspace, whose size the integer path's needs set)
-        as_float = ctx.main_use == &ctx.main;
+        as_float = try_float && ctx.main_use == &ctx.main;
         for (int32_t j = 0; j < njobs && as_float; ++j) as_float = float_possible<T, D>(eps[j]);
         if (as_float) {
             try {
@@ -1428,7 +1432,21 @@ static void run_batch(Context& ctx, const T* pts, int64_t n, const int64_t* offs
             JobParams<float>* table = A.take_n<JobParams<float>>(static_cast<size_t>(njobs));
             float* rows = A.take_n<float>(static_cast<size_t>(n) * D);
             launch_to_float<T>(pts, n * D, rows, s);
-            run(static_cast<const float*>(rows), table, hf.data());
+            bool room = true;
+            try {
+                run(static_cast<const float*>(rows), table, hf.data());
+            } catch (const Error& e) {
+                if (e.code != HPD_ENOMEM) throw;
+                (void)hipGetLastError();
+                room = false;
+            }
+            if (!room) {
+                // the float rows' workspace left none for the neighbour tables
+                // (sized after the index, before any label is written): the
+                // integer path, whose workspace is smaller
+                A.release();
+                return run_batch<T, D>(ctx, pts, n, offsets, njobs, eps, min_pts, labels, s, false);
+            }
         }
     }
     if (std::is_floating_point<T>::value || !as_float || !boxes) {

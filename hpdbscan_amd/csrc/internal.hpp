@@ -44,6 +44,8 @@ public:
     }
     // Make sure at least `bytes` are available in one block (drops contents).
     void reserve(size_t bytes);
+    // Give an allocation of its own back.
+    void release();
     void reset() { used_ = 0; }
     void* take(size_t bytes);
     template <typename T>
