@@ -252,8 +252,9 @@ class Context:
         return int(sm.value), bool(sc.value)
 
     def set_timing(self, enabled) -> None:
-        """True / 1: phase events; 2: also count the core count's executed
-        distance tests (an instrumented, slower kernel)."""
+        """True / 1: phase events of the general path (small inputs and graph
+        mode take other paths without timing; same labels); 2: also count the
+        core count's executed distance tests (an instrumented, slower kernel)."""
         check(load().hpd_context_set_timing(self._h, int(enabled)))
 
     def set_graph(self, enabled: bool) -> None:

@@ -91,9 +91,11 @@ typedef struct hpd_run_stats {
     double ms_union_kernel;      /* box union: union of the remaining pairs */
     double ms_border_kernel;     /* border / noise labels of non-core rows */
     uint64_t boxes;              /* sub-boxes of the occupied cells */
-    int32_t box_union;           /* 1 if the union ran on sub-boxes */
+    int32_t box_union;           /* 1 if the union ran on sub-boxes (0 for small
+                                    inputs, of which all pairs are compared) */
     uint64_t neighbor_rows;      /* [first, end) slot ranges of all cells */
-    uint64_t open_box_pairs;     /* box pairs the hook forest left open */
+    uint64_t open_box_pairs;     /* box pairs the hook forest left open (0
+                                    without a box union) */
     double ms_core_kernel;       /* the core count kernel alone (part of ms_core) */
     uint64_t core_tests;         /* row-row distance tests the core count executed
                                     (box mode, timing level 2; bounding boxes
@@ -119,7 +121,12 @@ int hpd_context_destroy(hpd_context* ctx);
 int hpd_context_set_border_rule(hpd_context* ctx, int rule);
 /* Phase timing: 1 records HIP events between the phases (ms_* of the
  * statistics); 2 also runs an instrumented core count kernel that counts
- * the distance tests it executes (core_tests; slower, for measurement). */
+ * the distance tests it executes (core_tests; slower, for measurement).
+ * The phases are the general path's.  Without timing, floating-point calls of
+ * one job with few rows (6000 up to 4-D, 7000 in 5-D, 8000 in 6-D, 10000 in
+ * 7-D, 12000 in 8-D) compare all pairs instead, which is faster, so that their
+ * phase times are not parts of the untimed call's time; labels are the same.
+ * Graph mode is left out while timing is on, too. */
 int hpd_context_set_timing(hpd_context* ctx, int enabled);
 int hpd_context_get_stats(const hpd_context* ctx, hpd_run_stats* out);
 
