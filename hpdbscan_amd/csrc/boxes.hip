@@ -676,8 +676,8 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
             }
             const bool none = hits == 0;
             hits = none ? ballot(hit) & gmask : hits;
-            // (the ballot above is taken by every lane: `none` differs
-            // between groups only in which value they keep)
+            // (the ballot is taken where `none` holds, which is equal over a
+            // group: a group takes it whole and reads its own lanes only)
             bool done = hits != 0;
             for (uint64_t todo = ballot(open && !done); todo != 0; todo &= todo - 1) {
                 const int j = static_cast<int>(__builtin_ctzll(todo));
@@ -710,7 +710,12 @@ __global__ __launch_bounds__(kThreads) void k_box_link(const BoxArgs<T> a,
 // tree.  From 4-D on and for many boxes: the neighbourhoods are large, or a launch
 // is cheap beside them (union with this kernel and without, us: 5M rows of 4
 // floats 203, 630; 30k of 6 doubles 33, 112; 4096 clouds of 3 3218, 4720; 10M
-// rows of 3 116, 137; 100k of 3 60, 42; 300k of 2 38, 26).
+// rows of 3, 1.0M boxes, 116, 137; 100k of 3 60, 42; 300k of 2 38, 26).  Near the
+// line it is the data that decides: blobs with 10 % noise of 3 by boxes 128k
+// 75, 64; 224k 95, 83; 376k 123, 112; 942k 262, 250; of 2 174k 71, 61; 694k 124,
+// 111; 1.3M 144, 147.  So between the line and about a million boxes such a
+// cloud loses some 12 us (1 to 2 % of its call); the 10M rows gain a seventh of
+// the union, the batch of clouds a third.
 constexpr int64_t kMixedBoxes = 250000;
 constexpr int kMixedStage = 512;  // list entries staged per wave
 template <int D>

@@ -20,7 +20,7 @@ constexpr int kCollectCap = 2048;  // entries staged in LDS
 // together read and write one stretch of memory (with a slice of [0, n) per
 // block the core labels' scattered writes of 4096 clouds took 5.2 ms, with
 // tiles in turn 2.7).  One reservation per scanned tile would be an atomic on
-// one address per 1024 slots (10M rows: 10k of them); staged, it is one per
+// one address per 512 slots (10M rows: 20k of them); staged, it is one per
 // 2048 entries found.
 constexpr unsigned kCollectBlocks = 2048;
 inline unsigned collect_blocks(int64_t n) {

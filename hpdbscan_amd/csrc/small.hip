@@ -493,9 +493,11 @@ __global__ __launch_bounds__(kLabelThreads) void k_small_label(int32_t n, SmallL
 // All pairs against the general path, us, clouds of 60 blobs and (dense) of 5:
 // 3-D float 2000 rows 69 / 194 and 91 / 214, 6000 148 / 211 and 170 / 196, 9000
 // 242 / 228 and 282 / 197; 2-D 6000 155 / 213 and 192 / 202.  From 5-D on the
-// general path's neighbourhoods grow with 3^D: 6-D double 6000 187 / 295 and
-// 238 / 307, 9000 328 / 330 and 387 / 337; 8-D float 12000 477 / 903 and 643 /
-// 721 (5-D and 7-D: between).
+// general path's neighbourhoods grow with 3^D: 5-D float 7000 195 / 259 and 229 /
+// 260, 9000 273 / 270 and 348 / 266 (double 7000 216 / 267 and 251 / 269); 6-D
+// double 6000 187 / 295 and 238 / 307, 9000 328 / 330 and 387 / 337; 7-D float
+// 9000 304 / 369 and 370 / 407, 11000 398 / 393 and 478 / 416 (double 9000 342 /
+// 385 and 416 / 420); 8-D float 12000 477 / 903 and 643 / 721.
 int64_t small_rows(int d) {
     switch (d) {
         case 5: return 7000;
